@@ -50,7 +50,8 @@ static_assert(sizeof(Staged) == 48, "48-byte staged splat");
 // loads waited for batch by batch (ListWalk), and takes 91.7 in groups of four,
 // 92.6 in twos and 93.8 in eights; at 40k Gaussians and 333x251, where 1344
 // blocks leave most of the chip idle and latency is all, 138.9 and 98.0 us
-// (103.5 and 98.9).
+// (103.5 and 98.9). The backward pass evaluates in the same groups: 189.7 us one
+// by one, 180.8 in twos, 178.8 in fours at 1M.
 constexpr uint32_t kGroup = 4;
 constexpr uint32_t kBlock = 64; // pixels of an 8x8 block, threads of its workgroup, entries per batch
 
@@ -122,7 +123,6 @@ __device__ __forceinline__ Staged stage(const Splat &s, const BlockGeometry &geo
 
 // Lane l's pixel in its block and its two mask bits.
 __device__ __forceinline__ uint32_t lane_bits(uint32_t lx, uint32_t ly) { return (1u << lx) | (1u << (16u + ly)); }
-__device__ __forceinline__ bool covers(const Staged &s, uint32_t bits) { return (s.cols & bits) == bits; }
 
 // The wave votes as scalar masks: a ballot of one comparison is that
 // comparison's lane mask, so the loops vote with the AND of the ballots of
@@ -147,59 +147,6 @@ __device__ __forceinline__ uint32_t kth_set_bit(uint64_t m, uint32_t k) {
     }
   }
   return at;
-}
-
-// The next entries of the block's walk over its tile's list, from `pos` on
-// towards `limit` (up: pos, pos + 1, ...; down: pos - 1, pos - 2, ...), that
-// have the block's bit (blockBit) in their key: up to kBlock of them, in walk
-// order, into `queue`; `pos` is left at the first entry not yet looked at (up)
-// or one past it (down). The keys are read a window of kBlock at a time; a
-// window is taken up to the first wanted entry that does not fit. Returns how
-// many were queued. The caller has made sure the previous queue is read.
-template <bool Down>
-__device__ __forceinline__ uint32_t gather_entries(const uint32_t *__restrict__ entryKeys, uint32_t blockBit, uint32_t &pos,
-                                                   uint32_t limit, uint32_t *queue) {
-  const uint32_t lane = threadIdx.x;
-  uint32_t queued = 0;
-  while (queued < kBlock && pos != limit) {
-    const uint32_t left = Down ? pos - limit : limit - pos;
-    const uint32_t n = left < kBlock ? left : kBlock;
-    const uint32_t e = Down ? pos - 1u - lane : pos + lane;
-    const bool wanted = lane < n && (entryKeys[e] & blockBit) != 0u;
-    const uint64_t m = __ballot(wanted);
-    const uint32_t found = static_cast<uint32_t>(__popcll(m)), room = kBlock - queued;
-    const uint32_t taken = found > room ? kth_set_bit(m, room) : n; // window entries used up
-    if (wanted && lane < taken) queue[queued + static_cast<uint32_t>(__popcll(m & ((1ull << lane) - 1ull)))] = e;
-    queued += found < room ? found : room;
-    pos = Down ? pos - taken : pos + taken;
-  }
-  return queued;
-}
-
-// The queued entries: each lane stages one, and the splats that can touch a
-// pixel of the block are packed at the front of `batch` in queue order (with
-// their Gaussians in `index`, when given). Returns how many were kept.
-__device__ __forceinline__ uint32_t stage_batch(const Splat *__restrict__ splats, const uint32_t *__restrict__ entryValues,
-                                                const uint32_t *queue, uint32_t count, const BlockGeometry &geo, Staged *batch,
-                                                uint32_t *index) {
-  const uint32_t lane = threadIdx.x;
-  Staged st{};
-  uint32_t gaussian = 0;
-  bool keep = false;
-  if (lane < count) {
-    const uint32_t entry = queue[lane];
-    gaussian = entryValues[entry];
-    st = stage(load_splat(splats, gaussian), geo, entry);
-    keep = (st.cols & 0xFFu) != 0u && (st.cols >> 16) != 0u;
-  }
-  const uint64_t kept = __ballot(keep);
-  if (keep) {
-    const uint32_t slot = static_cast<uint32_t>(__popcll(kept & ((1ull << lane) - 1ull)));
-    batch[slot] = st;
-    if (index != nullptr) index[slot] = gaussian;
-  }
-  __syncthreads();
-  return static_cast<uint32_t>(__popcll(kept));
 }
 
 // The Gaussian's exponent at offset (dx, dy) (splat_at, train_types.glsl:88).
@@ -261,8 +208,9 @@ template <bool Down> struct ListWalk {
   }
   // The fetched batch: each lane stages one splat, and those that can touch a
   // pixel of the block are packed at the front of `batch` in walk order (with
-  // their Gaussians in `index`, when given). Returns how many were kept.
-  __device__ __forceinline__ uint32_t stage(const BlockGeometry &geo, Staged *batch, uint32_t *index) const {
+  // the byte offsets of their rows of rowBytes, when rowOffset is given).
+  // Returns how many were kept.
+  __device__ __forceinline__ uint32_t stage(const BlockGeometry &geo, Staged *batch, uint64_t *rowOffset, uint32_t rowBytes) const {
     Staged st{};
     bool keep = false;
     if (threadIdx.x < queued) {
@@ -273,7 +221,7 @@ template <bool Down> struct ListWalk {
     if (keep) {
       const uint32_t slot = static_cast<uint32_t>(__popcll(kept & ((1ull << threadIdx.x) - 1ull)));
       batch[slot] = st;
-      if (index != nullptr) index[slot] = gaussian;
+      if (rowOffset != nullptr) rowOffset[slot] = static_cast<uint64_t>(gaussian) * rowBytes;
     }
     return static_cast<uint32_t>(__popcll(kept));
   }
@@ -301,7 +249,7 @@ __device__ __forceinline__ void composite_block(const Splat *__restrict__ splats
     walk.request(queue);
     walk.fetch();
     while (walk.queued != 0) {
-      const uint32_t kept = walk.stage(geo, batch, nullptr);
+      const uint32_t kept = walk.stage(geo, batch, nullptr, 0u);
       // Pad the last group with splats no pixel is a candidate for (their
       // colours, which a zero weight multiplies, finite).
       if (threadIdx.x < kGroup) batch[kept + threadIdx.x] = Staged{};
@@ -442,93 +390,86 @@ __device__ __forceinline__ int64_t quantise(float v, float scale) {
   return static_cast<int64_t>(__builtin_rintf(s));
 }
 
-__device__ __forceinline__ float dpp_row_mirror(float v) { return as_float(__builtin_amdgcn_update_dpp(0, static_cast<int>(as_uint(v)), 0x140, 0xF, 0xF, false)); }
-__device__ __forceinline__ float dpp_half_mirror(float v) { return as_float(__builtin_amdgcn_update_dpp(0, static_cast<int>(as_uint(v)), 0x141, 0xF, 0xF, false)); }
-__device__ __forceinline__ float dpp_xor2(float v) { return as_float(__builtin_amdgcn_update_dpp(0, static_cast<int>(as_uint(v)), 0x4E, 0xF, 0xF, false)); }
-__device__ __forceinline__ float dpp_xor1(float v) { return as_float(__builtin_amdgcn_update_dpp(0, static_cast<int>(as_uint(v)), 0xB1, 0xF, 0xF, false)); }
+// The totals of a splat's values over the wave: each value through the same
+// tree over the lanes (partners l ^ 32, 16, 15, 7, 2, 1 in turn; a + b and b + a
+// are the same float). The first two steps are permlane swaps, each followed by
+// one add for two values. (Moving the values through LDS instead, with no
+// swaps, was slower: its traffic is more than the LDS carries.) The last four
+// steps are DPP adds within 16-lane rows, two of them merging a pair of values
+// by bank masks (lanes with bit 3, then bit 2, set keep the second) where a
+// selection of what to keep and what to send took two instructions more each.
 
-// Twelve values per lane to the wave's twelve totals, every value through the
-// same tree (partners l ^ 32, 16, 15, 7, 2, 1 in turn; a + b and b + a are the
-// same float). Afterwards lane l holds in v[0] the total of value
-// reduced_value(l); wave_emits(l) picks one lane per value.
-__device__ __forceinline__ void reduce_wave(float (&v)[12], uint32_t lane) {
-  // Partner l ^ 32: lanes 0-31 keep values 0-5, lanes 32-63 values 6-11.
-#pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    const auto p = __builtin_amdgcn_permlane32_swap(as_uint(v[i]), as_uint(v[i + 6]), false, false);
-    v[i] = as_float(p[0]) + as_float(p[1]);
-  }
-  // Partner l ^ 16: rows 0 and 2 keep their first three, rows 1 and 3 the others.
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const auto p = __builtin_amdgcn_permlane16_swap(as_uint(v[i]), as_uint(v[i + 3]), false, false);
-    v[i] = as_float(p[0]) + as_float(p[1]);
-  }
-  // Partner l ^ 15 (row mirror), all three kept.
-#pragma unroll
-  for (int i = 0; i < 3; ++i) v[i] = v[i] + dpp_row_mirror(v[i]);
-  // Partner l ^ 7 (half-row mirror): lanes with bit 2 clear keep the first of
-  // the first two, the others the second; all keep the third.
-  {
-    const bool upper = (lane & 4u) != 0u;
-    const float send = upper ? v[0] : v[1];
-    const float keep = upper ? v[1] : v[0];
-    v[0] = keep + dpp_half_mirror(send);
-    v[2] = v[2] + dpp_half_mirror(v[2]);
-  }
-  // Partner l ^ 2: lanes with bit 1 clear keep the one they kept, the others the third.
-  {
-    const bool upper = (lane & 2u) != 0u;
-    const float send = upper ? v[0] : v[2];
-    const float keep = upper ? v[2] : v[0];
-    v[0] = keep + dpp_xor2(send);
-  }
-  v[0] = v[0] + dpp_xor1(v[0]);
-}
-// Sixteen values per lane to one total per lane group, for the scored pass's
-// fourteen sums: afterwards lane l holds the wave's total of value (l >> 2) & 15
-// in v[0]. The same partner tree as reduce_wave.
-__device__ __forceinline__ void reduce_wave16(float (&v)[16], uint32_t lane) {
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const auto p = __builtin_amdgcn_permlane32_swap(as_uint(v[i]), as_uint(v[i + 8]), false, false);
-    v[i] = as_float(p[0]) + as_float(p[1]);
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const auto p = __builtin_amdgcn_permlane16_swap(as_uint(v[i]), as_uint(v[i + 4]), false, false);
-    v[i] = as_float(p[0]) + as_float(p[1]);
-  }
-  {
-    const bool upper = (lane & 8u) != 0u;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const float send = upper ? v[i] : v[i + 2];
-      const float keep = upper ? v[i + 2] : v[i];
-      v[i] = keep + dpp_row_mirror(send);
-    }
-  }
-  {
-    const bool upper = (lane & 4u) != 0u;
-    const float send = upper ? v[0] : v[1];
-    const float keep = upper ? v[1] : v[0];
-    v[0] = keep + dpp_half_mirror(send);
-  }
-  v[0] = v[0] + dpp_xor2(v[0]);
-  v[0] = v[0] + dpp_xor1(v[0]);
+// A DPP add reads a register two wait states after a vector instruction wrote
+// it, which the compiler does not see inside the block: hence the s_nops.
+__device__ __forceinline__ float reduce_row3(float a, float b, float c) {
+  float t, u, w;
+  asm("s_nop 1\n\t"
+      "v_add_f32_dpp %0, %3, %3 row_mirror row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %1, %5, %5 row_mirror row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %0, %4, %4 row_mirror row_mask:0xf bank_mask:0xc\n\t"
+      "s_nop 0\n\t"
+      "v_add_f32_dpp %2, %1, %1 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %2, %0, %0 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+      "s_nop 1\n\t"
+      "v_add_f32_dpp %2, %2, %2 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_add_f32_dpp %2, %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+      : "=&v"(t), "=&v"(u), "=&v"(w)
+      : "v"(a), "v"(b), "v"(c));
+  return w;
 }
 
-// The value whose total lane l holds after reduce_wave: 6 b5 + 3 b4 + (b1 ? 2 : b2),
+__device__ __forceinline__ float swap32_add(float a, float b) {
+  const auto p = __builtin_amdgcn_permlane32_swap(as_uint(a), as_uint(b), false, false);
+  return as_float(p[0]) + as_float(p[1]);
+}
+__device__ __forceinline__ float swap16_add(float a, float b) {
+  const auto p = __builtin_amdgcn_permlane16_swap(as_uint(a), as_uint(b), false, false);
+  return as_float(p[0]) + as_float(p[1]);
+}
+
+// Twelve values per lane to the wave's twelve totals: lane l ends with the total
+// of value reduced_value(l); wave_emits(l) picks one lane per value.
+__device__ __forceinline__ float reduce_wave(const float (&v)[12]) {
+  float u[6];
+#pragma unroll
+  for (int i = 0; i < 6; ++i) u[i] = swap32_add(v[i], v[i + 6]); // lanes 0-31 keep values 0-5
+  return reduce_row3(swap16_add(u[0], u[3]), swap16_add(u[1], u[4]), swap16_add(u[2], u[5]));
+}
+
+// Sixteen values per lane, for the scored pass's fourteen sums: lane l ends with
+// the total of value reduced_value16(l).
+__device__ __forceinline__ float reduce_wave16(const float (&v)[16]) {
+  float u[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) u[i] = swap32_add(v[i], v[i + 8]);
+  const float last = swap16_add(u[3], u[7]);
+  const float w = reduce_row3(swap16_add(u[0], u[4]), swap16_add(u[1], u[5]), swap16_add(u[2], u[6]));
+  const float z = reduce_row3(last, last, last);
+  return (threadIdx.x & 12u) == 12u ? z : w;
+}
+
+// The value whose total lane l holds after reduce_wave: 3 (l / 16) + (b2 ? 2 : b3),
 // with bk bit k of l.
 __device__ __forceinline__ uint32_t reduced_value(uint32_t lane) {
-  return 6u * ((lane >> 5) & 1u) + 3u * ((lane >> 4) & 1u) + (((lane >> 1) & 1u) != 0u ? 2u : (lane >> 2) & 1u);
+  return 3u * (lane >> 4) + ((lane & 4u) != 0u ? 2u : (lane >> 3) & 1u);
 }
-// One lane per value: bits 0 and 3 clear, and not both bits 1 and 2 (those
+// One lane per value: bits 0 and 1 clear, and not both bits 2 and 3 (those
 // lanes hold the third value twice).
-__device__ __forceinline__ bool wave_emits(uint32_t lane) { return (lane & 9u) == 0u && (lane & 6u) != 6u; }
+__device__ __forceinline__ bool wave_emits(uint32_t lane) { return (lane & 3u) == 0u && (lane & 12u) != 12u; }
+// After reduce_wave16: 4 (l / 16) + the third or the fourth where bit 2 is set, by bit 3.
+__device__ __forceinline__ uint32_t reduced_value16(uint32_t lane) {
+  return 4u * (lane >> 4) + ((lane & 4u) != 0u ? ((lane & 8u) != 0u ? 3u : 2u) : (lane >> 3) & 1u);
+}
 
 // Back to front over the tile's list (train_backward.glsl:78-158), for the
-// block's pixels, from the block's lowest stop. With Recompute the pixel's log
+// block's pixels, from the block's lowest stop. Bound by the vector unit: a
+// splat's evaluation, gradient terms, reduction and emission are about 105
+// instructions, the permlane swaps and the reciprocal among them at a third of
+// an fma's rate. At 1M Gaussians and 1280x720 (32x32 lists, fixed point) 205 us
+// before the walk's loads ran ahead, the evaluations were grouped, the reduction
+// merged by bank masks and the emission shortened (a row's byte offset staged
+// once, the halves of sums 3 to 5 taken last); 179 us with them. With Recompute the pixel's log
 // transmittance and stop come from a front-to-back sweep of its own instead
 // of the forward pass's image and stops, which are then not read. With Score
 // (a scored view) the last two sums are filled too: the pixel's high-error
@@ -542,7 +483,7 @@ __device__ __forceinline__ void backward_block(uint32_t item, const Splat *__res
                                                const float4 *__restrict__ adjoint, const uint32_t *__restrict__ stops,
                                                float fixedScale, unsigned long long *__restrict__ rawFixed,
                                                float *__restrict__ rawFloat, const float *__restrict__ edge, Staged *batch,
-                                               uint32_t *batchIndex, uint32_t *queue) {
+                                               uint64_t *rowOffset, uint32_t *queue) {
   uint32_t tile;
   const BlockGeometry geo = block_geometry<TW, TH>(item, gridW, width, height, tile);
   if (geo.x0 >= width || geo.y0 >= height) return; // a block past the image's edge (uniform)
@@ -583,97 +524,113 @@ __device__ __forceinline__ void backward_block(uint32_t item, const Splat *__res
   float Br = bgR, Bg = bgG, Bb = bgB;
   float Tbehind = exp_finite(logTotal);
 
-  const uint32_t blockBit = 1u << (tileBits + geo.block);
   const uint64_t insideLanes = vote(inside);
-  for (uint32_t pos = first < range.y ? first : range.y; pos < range.y;) {
-    __syncthreads(); // the previous batch and queue are read
-    const uint32_t queued = gather_entries<false>(entryKeys, blockBit, pos, range.y, queue);
+  // What this lane adds of a splat's totals: value `value` of its row, in steps
+  // or as it is; values 3 to 5 are reduced twice their size (exact halving last).
+  // Values 12 and 13 of the kRawPerSplat slots are zero without scoring.
+  const uint32_t value = Score ? reduced_value16(lane) : reduced_value(lane);
+  const uint64_t emitLanes = vote(Score ? (lane & 3u) == 0 && value < kRawPerSplat : wave_emits(lane));
+  const float emitScale = (value >= 3u && value <= 5u ? 0.5f : 1.0f) * (Fixed ? fixedScale : 1.0f);
+  uint8_t *const emitBase = Fixed ? reinterpret_cast<uint8_t *>(rawFixed + value) : reinterpret_cast<uint8_t *>(rawFloat + value);
+  if (first >= range.y) return;
+  ListWalk<false> walk{splats, entryKeys, entryValues, 1u << (tileBits + geo.block), range.y, first};
+  walk.load_window();
+  walk.request(queue);
+  walk.fetch();
+  while (walk.queued != 0) {
+    const uint32_t kept = walk.stage(geo, batch, rowOffset, kRawPerSplat * (Fixed ? 8u : 4u));
+    if (lane < kGroup) batch[kept + lane] = Staged{}; // the last group padded with splats no pixel is a candidate for
     __syncthreads();
-    const uint32_t kept = stage_batch(splats, entryValues, queue, queued, geo, batch, batchIndex);
-    for (uint32_t k = 0; k < kept; ++k) {
-      const Staged s = batch[k];
-      const bool live = s.entry >= stop, covered = covers(s, bits);
-      const uint64_t candidates = insideLanes & vote(live) & vote(covered);
-      if (candidates == 0) continue;
-      const bool candidate = inside && live && covered;
-      const float dx = px - s.cx, dy = py - s.cy;
-      const float power = power_at(s, dx, dy);
-      const float e = exp_finite(power);
-      const float a = s.o * e;
-      const float alpha = a < 0.99f ? a : 0.99f;
-      const bool front = !(power > 0.0f), visible = alpha >= kMinAlpha;
-      if ((candidates & vote(front) & vote(visible)) == 0) continue;
-      const bool ok = candidate && front && visible;
-      // Used where ok only: there 0.01 <= 1 - alpha <= 1 and the transmittance
-      // is at least the pixel's final one, which the forward keeps at or above
-      // 1e-4, so the short division is exact `Tbehind / (1 - alpha)`.
-      const float T = div_in_range(Tbehind, 1.0f - alpha);
-      // A lane that takes nothing from the splat carries zero factors, so its
-      // values below are all zero (every other factor is finite); the sign of
-      // a zero cannot change a total that is not zero.
-      const float Ta = ok ? T * alpha : 0.0f;
-      // At the 0.99 clamp alpha no longer depends on the parameters.
-      const bool free = ok && a < 0.99f;
-      const float dAlpha = free ? T * fma32(adj.z, s.b - Bb, fma32(adj.y, s.g - Bg, adj.x * (s.r - Br))) : 0.0f;
-      const float dPower = dAlpha * alpha;
-      const float vx = fma32(s.qy, dy, s.qx * dx), vy = fma32(s.qz, dy, s.qy * dx);
-      const float g1 = dPower * vx, g2 = dPower * vy;
-      const float hp = 0.5f * dPower;
-      constexpr int kValues = Score ? 16 : 12;
-      float v[kValues];
-      v[0] = dAlpha * e;
-      v[1] = g1;
-      v[2] = g2;
-      v[3] = (hp * vx) * vx;
-      v[4] = (hp * vx) * vy;
-      v[5] = (hp * vy) * vy;
-      v[6] = Ta * adj.x;
-      v[7] = Ta * adj.y;
-      v[8] = Ta * adj.z;
-      v[9] = Ta * perPixel;
-      v[10] = fabsf(g1);
-      v[11] = fabsf(g2);
-      if constexpr (Score) {
-        v[12] = ok ? adj.w * perPixel : 0.0f;
-        v[13] = (edgeWeight * Ta) * perPixel;
-        v[14] = v[15] = 0.0f;
+    walk.request(queue);
+    bool fetched = false;
+    for (uint32_t k = 0; k < kept; k += kGroup) {
+      if (!fetched && k * 2u >= kept) {
+        walk.fetch();
+        fetched = true;
       }
-      // The colour behind and the transmittance in front: unchanged where alpha is taken as 0.
-      const float alphaBehind = ok ? alpha : 0.0f;
-      Br = fma32(alphaBehind, s.r - Br, Br);
-      Bg = fma32(alphaBehind, s.g - Bg, Bg);
-      Bb = fma32(alphaBehind, s.b - Bb, Bb);
-      Tbehind = ok ? T : Tbehind;
-      uint32_t value;
-      bool emits;
-      if constexpr (Score) {
-        reduce_wave16(v, lane);
-        value = lane >> 2;
-        emits = (lane & 3u) == 0 && value < kRawPerSplat;
-      } else {
-        // Values 12 and 13 of the kRawPerSplat slots are zero without scoring.
-        reduce_wave(v, lane);
-        value = reduced_value(lane);
-        emits = wave_emits(lane);
+      uint64_t oks[kGroup];
+      float falloff[kGroup];
+#pragma unroll
+      for (uint32_t j = 0; j < kGroup; ++j) {
+        const Staged &s = batch[k + j];
+        const float power = power_at(s, px - s.cx, py - s.cy);
+        const float e = exp_finite(power);
+        falloff[j] = e;
+        oks[j] = insideLanes & vote(s.entry >= stop) & vote((s.cols & bits) == bits) & vote(!(power > 0.0f)) &
+                 vote(!(s.o * e < kMinAlpha));
       }
-      if (emits) {
-        const size_t slot = static_cast<size_t>(batchIndex[k]) * kRawPerSplat + value;
+#pragma unroll
+      for (uint32_t j = 0; j < kGroup; ++j) {
+        if (oks[j] == 0) continue;
+        const Staged s = batch[k + j];
+        const float dx = px - s.cx, dy = py - s.cy;
+        const float e = falloff[j];
+        const float a = s.o * e;
+        // A lane that takes nothing from the splat has alpha 0: its
+        // transmittance, the colour behind it and every sum below stay as they
+        // are (T / 1 is T; every other factor is finite, and the sign of a zero
+        // cannot change a total that is not zero). Else 0.01 <= 1 - alpha <= 1,
+        // and the transmittance is at least the pixel's final one, which the
+        // forward keeps at or above 1e-4, so the short division is exact
+        // `Tbehind / (1 - alpha)`.
+        const float alpha = lane_of(oks[j]) ? (a < 0.99f ? a : 0.99f) : 0.0f;
+        const float T = div_in_range(Tbehind, 1.0f - alpha);
+        const float Ta = T * alpha;
+        // At the 0.99 clamp alpha no longer depends on the parameters.
+        const float toward = T * fma32(adj.z, s.b - Bb, fma32(adj.y, s.g - Bg, adj.x * (s.r - Br)));
+        const float dAlpha = lane_of(oks[j] & vote(a < 0.99f)) ? toward : 0.0f;
+        const float dPower = dAlpha * alpha;
+        const float vx = fma32(s.qy, dy, s.qx * dx), vy = fma32(s.qz, dy, s.qy * dx);
+        const float g1 = dPower * vx, g2 = dPower * vy;
+        constexpr int kValues = Score ? 16 : 12;
+        float v[kValues];
+        v[0] = dAlpha * e;
+        v[1] = g1;
+        v[2] = g2;
+        v[3] = g1 * vx; // twice the sum (emitScale)
+        v[4] = g1 * vy;
+        v[5] = g2 * vy;
+        v[6] = Ta * adj.x;
+        v[7] = Ta * adj.y;
+        v[8] = Ta * adj.z;
+        v[9] = Ta * perPixel;
+        v[10] = fabsf(g1);
+        v[11] = fabsf(g2);
+        if constexpr (Score) {
+          v[12] = lane_of(oks[j]) ? adj.w * perPixel : 0.0f;
+          v[13] = (edgeWeight * Ta) * perPixel;
+          v[14] = v[15] = 0.0f;
+        }
+        Br = fma32(alpha, s.r - Br, Br);
+        Bg = fma32(alpha, s.g - Bg, Bg);
+        Bb = fma32(alpha, s.b - Bb, Bb);
+        Tbehind = T;
+        float total;
+        if constexpr (Score) {
+          total = reduce_wave16(v);
+        } else {
+          total = reduce_wave(v);
+        }
+        uint8_t *const slot = emitBase + rowOffset[k + j];
+        const float scaled = total * emitScale;
         if constexpr (Fixed) {
           // Totals under 2^31 steps (nearly all) round and convert in 32 bits,
           // exactly as quantise() would; the wave takes quantise() if any is larger.
-          const float scaled = v[0] * fixedScale;
-          int64_t q;
-          if (__builtin_amdgcn_ballot_w64(!(fabsf(scaled) < 2147483648.0f)) == 0u) {
-            q = static_cast<int32_t>(__builtin_rintf(scaled));
-          } else {
-            q = quantise(v[0], fixedScale);
+          const float rounded = __builtin_rintf(scaled);
+          int64_t q = static_cast<int32_t>(rounded);
+          uint64_t send = emitLanes & vote(rounded != 0.0f);
+          if ((emitLanes & vote(!(fabsf(scaled) < 2147483648.0f))) != 0u) {
+            q = quantise(total, emitScale);
+            send = emitLanes & vote(q != 0);
           }
-          if (q != 0) atomicAdd(&rawFixed[slot], static_cast<unsigned long long>(q));
+          if (lane_of(send)) atomicAdd(reinterpret_cast<unsigned long long *>(slot), static_cast<unsigned long long>(q));
         } else {
-          if (v[0] != 0.0f) atomicAdd(&rawFloat[slot], v[0]);
+          if (lane_of(emitLanes & vote(scaled != 0.0f))) atomicAdd(reinterpret_cast<float *>(slot), scaled);
         }
       }
     }
+    if (!fetched) walk.fetch();
+    __syncthreads(); // the batch is read
   }
 }
 
@@ -688,11 +645,11 @@ __global__ __launch_bounds__(kBlock) void backward_kernel(const Splat *__restric
                                                           float *__restrict__ rawFloat, const float *__restrict__ edge,
                                                           const uint32_t *__restrict__ order) {
   __shared__ Staged batch[kBlock + kGroup];
-  __shared__ uint32_t batchIndex[kBlock];
+  __shared__ uint64_t rowOffset[kBlock];
   __shared__ uint32_t queue[kBlock];
   const uint32_t item = order != nullptr ? order[blockIdx.x] : blockIdx.x;
   backward_block<Fixed, Recompute, Score, TW, TH>(item, splats, entryKeys, entryValues, tileBits, ranges, width, height, gridW, bgR,
-                                                  bgG, bgB, image, adjoint, stops, fixedScale, rawFixed, rawFloat, edge, batch, batchIndex,
+                                                  bgG, bgB, image, adjoint, stops, fixedScale, rawFixed, rawFloat, edge, batch, rowOffset,
                                                   queue);
 }
 
@@ -701,14 +658,14 @@ __global__ __launch_bounds__(kBlock) void backward_kernel(const Splat *__restric
 template <bool Fixed, bool Recompute, uint32_t TW, uint32_t TH>
 __global__ __launch_bounds__(kBlock) void backward_views_kernel(RasterViews views, float bgR, float bgG, float bgB) {
   __shared__ Staged batch[kBlock + kGroup];
-  __shared__ uint32_t batchIndex[kBlock];
+  __shared__ uint64_t rowOffset[kBlock];
   __shared__ uint32_t queue[kBlock];
   uint32_t item = blockIdx.x;
   const RasterView &w = views.view[view_of(views, item)];
   backward_block<Fixed, Recompute, false, TW, TH>(item, w.splats, w.entryKeys, w.entryValues, w.tileBits, w.ranges, w.width, w.height,
                                                   w.gridW, bgR, bgG, bgB, w.image, w.adjoint, w.stops, w.fixedScale,
                                                   reinterpret_cast<unsigned long long *>(w.rawFixed), w.rawFloat, nullptr, batch,
-                                                  batchIndex, queue);
+                                                  rowOffset, queue);
 }
 
 constexpr uint32_t kOrderThreads = 1024;
