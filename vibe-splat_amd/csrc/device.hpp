@@ -147,12 +147,16 @@ __device__ __forceinline__ float vs_log(float x) {
 
 // vs_exp on [-87, 87] without its special cases, for arguments that are never
 // NaN: the argument is clamped into that range (one med3), where the result
-// p 2^n is a normal float (n >= -126 with p > 1 at the low end), so ldexp
-// applies 2^n exactly, as vs_exp's two multiplications do. Equal to vs_exp(x)
-// for every x in [-87, 87].
+// p 2^n is a normal float (n >= -126 with p > 1 at the low end). The rounding to
+// n is an addition of 1.5 2^23, whose last place is 1 (ties to even, as
+// __builtin_rintf's), which also leaves n in the sum's low bits, from where it is
+// added to p's exponent: for a normal result that is p 2^n exactly. Equal to
+// vs_exp(x) for every x in [-87, 87]. (v_rndne_f32, v_cvt_i32_f32 and
+// v_ldexp_f32 issue at half the rate of the add and the shift.)
 __device__ __forceinline__ float exp_finite(float x) {
   x = __builtin_amdgcn_fmed3f(x, -87.0f, 87.0f);
-  const float n = __builtin_rintf(x * 0x1.715476p+0f);
+  const float shifted = x * 0x1.715476p+0f + 12582912.0f;
+  const float n = shifted - 12582912.0f;
   float r = fma32(n, -0x1.62e4p-1f, x);
   r = fma32(n, -0x1.7f7d1cp-20f, r);
   float q = fma32(0x1.6d752p-10f, r, 0x1.120b66p-7f);
@@ -160,7 +164,7 @@ __device__ __forceinline__ float exp_finite(float x) {
   q = fma32(q, r, 0x1.5554dcp-3f);
   q = fma32(q, r, 0x1p-1f);
   const float p = fma32(r * r, q, r) + 1.0f;
-  return __builtin_ldexpf(p, static_cast<int>(n));
+  return as_float(as_uint(p) + (as_uint(shifted) << 23));
 }
 
 // vs_log for a positive normal finite x, without its special cases; equal to
