@@ -41,8 +41,8 @@ __global__ __launch_bounds__(kScanThreads) void coverage_count_kernel(const uint
     const uint32_t r = chunk * kScanTile + k * kScanThreads + threadIdx.x;
     const bool visible = r < count && keys[r] != kInvisible;
     const uint32_t v = visible ? tileCount[values[r]] : 0u;
-    if (r < count) offsets[r] = v;
-    sum += v;
+    if (r < count) offsets[r] = v; // with a big splat's mark
+    sum += v & ~kBigCount;
     seen += visible ? 1u : 0u;
   }
   uint32_t unused;
@@ -54,7 +54,8 @@ __global__ __launch_bounds__(kScanThreads) void coverage_count_kernel(const uint
   }
 }
 
-__global__ __launch_bounds__(kScanThreads) void coverage_offsets_kernel(uint32_t count, uint32_t *__restrict__ offsets,
+__global__ __launch_bounds__(kScanThreads) void coverage_offsets_kernel(const uint32_t *__restrict__ values, uint32_t count,
+                                                                        TileRecord *__restrict__ records, uint32_t *__restrict__ offsets,
                                                                         const uint32_t *__restrict__ totals, uint32_t *counters,
                                                                         uint32_t capacity, uint32_t isStep) {
   __shared__ uint32_t waveTotals[kScanThreads / 64];
@@ -77,7 +78,7 @@ __global__ __launch_bounds__(kScanThreads) void coverage_offsets_kernel(uint32_t
 #pragma unroll
   for (uint32_t k = 0; k < kScanPerThread; ++k) {
     v[k] = first + k < count ? offsets[first + k] : 0u;
-    sum += v[k];
+    sum += v[k] & ~kBigCount;
   }
   uint32_t exclusive;
   const uint32_t chunkTotal = block_exclusive_sum(sum, exclusive, waveTotals);
@@ -85,7 +86,8 @@ __global__ __launch_bounds__(kScanThreads) void coverage_offsets_kernel(uint32_t
 #pragma unroll
   for (uint32_t k = 0; k < kScanPerThread; ++k) {
     if (first + k < count) offsets[first + k] = running;
-    running += v[k];
+    if ((v[k] & kBigCount) != 0u) records[values[first + k]].maskLo = running; // for the list pass, which finds big splats by their own list
+    running += v[k] & ~kBigCount;
   }
   if (last) {
     const uint32_t visible = block_exclusive_sum(seen, unused, waveTotals);
@@ -126,25 +128,35 @@ __global__ __launch_bounds__(128) void gather_views_kernel(ViewStatus v, uint8_t
   }
 }
 
+// What ends a pass (launch_finish): one wave.
+__global__ __launch_bounds__(64) void finish_kernel(uint32_t *__restrict__ adamState, float beta1, float beta2,
+                                                    const uint32_t *__restrict__ counters, const uint32_t *__restrict__ sums,
+                                                    uint32_t *__restrict__ status) {
+  const uint32_t w = threadIdx.x;
+  if (status != nullptr && w < kViewStatusBytes / 4) status[w] = w < kCounterWords ? counters[w] : sums[w - kCounterWords];
+  if (adamState != nullptr && w == 0 && counters[kOverflow] == 0) {
+    adamState[0] += 1u;
+    adamState[1] = as_uint(as_float(adamState[1]) * beta1);
+    adamState[2] = as_uint(as_float(adamState[2]) * beta2);
+  }
+}
+
 // A wave takes 64 consecutive depth-sorted splats and walks their candidate
 // tiles 64 at a time (tiles.hpp), reading each small splat's outcome from the
 // bits the projection kept. An entry goes to its splat's first entry (the
 // scan's offset) plus the number of its splat's reached tiles before it, so a
 // round's stores are contiguous except where a big splat's run lies between
-// two small ones. A big splat's first entry is left in its record for
-// big_emit_kernel. An entry's key is its tile in the low tileBits bits and,
+// two small ones. An entry's key is its tile in the low tileBits bits and,
 // above them, the tile's 8x8 pixel blocks its splat can reach (block_mask;
 // with blockMasks off, all of them): the sort orders by the tile alone, and
 // the raster pass stages an entry only in the blocks whose bit is set.
-__global__ __launch_bounds__(256) void bin_emit_kernel(const uint32_t *__restrict__ keys, const uint32_t *__restrict__ values,
-                                                       const Splat *__restrict__ splats, TileRecord *__restrict__ records,
-                                                       uint32_t count, uint32_t gridW, TileShape shape, uint32_t width, uint32_t height,
-                                                       uint32_t tileBits, bool blockMasks, const uint32_t *__restrict__ offsets,
-                                                       const uint32_t *counters, uint32_t *__restrict__ entryKeys,
-                                                       uint32_t *__restrict__ entryValues) {
+__device__ __forceinline__ void emit_small(const uint32_t *__restrict__ keys, const uint32_t *__restrict__ values,
+                                           const Splat *__restrict__ splats, const TileRecord *__restrict__ records, uint32_t count,
+                                           uint32_t gridW, TileShape shape, uint32_t width, uint32_t height, uint32_t tileBits,
+                                           bool blockMasks, const uint32_t *__restrict__ offsets, uint32_t limit,
+                                           uint32_t *__restrict__ entryKeys, uint32_t *__restrict__ entryValues) {
   __shared__ EmitOwner owners[256]; // per wave: its small splats with candidates, packed
   __shared__ uint32_t flags[256];   // per wave: the walk's round marks
-  if (counters[kOverflow] != 0) return; // the same for every thread of the launch
   const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x & ~63u;
   uint32_t candidates = 0, i = 0;
@@ -154,10 +166,7 @@ __global__ __launch_bounds__(256) void bin_emit_kernel(const uint32_t *__restric
     rec = records[i];
     candidates = (rec.size & 0xFFFFu) * (rec.size >> 16);
   }
-  if (candidates > kMaskTiles) {
-    records[i].maskLo = offsets[r]; // a big splat: listed by big_emit_kernel
-    candidates = 0;
-  }
+  if (candidates > kMaskTiles) candidates = 0; // a big splat: emit_big lists it
   const bool owner = candidates != 0;
   const uint64_t owning = __ballot(owner);
   const uint32_t end = wave_inclusive_sum(candidates, lane);
@@ -178,7 +187,6 @@ __global__ __launch_bounds__(256) void bin_emit_kernel(const uint32_t *__restric
   }
   const uint32_t allBlocks = (1u << ((shape.w >> 3) * (shape.h >> 3))) - 1u;
   __builtin_amdgcn_wave_barrier();
-  const uint32_t limit = counters[kEntriesUsed];
   uint32_t before = 0;
   for (uint32_t base = 0; base < total; base += 64) {
     const uint32_t k = walk_round(flags + wave, lane, base, owner, start, before);
@@ -209,14 +217,12 @@ __global__ __launch_bounds__(256) void bin_emit_kernel(const uint32_t *__restric
 // prefix count from the splat's first entry. The listed splats are dealt out
 // over all the waves. Their entries mark every 8x8 block of the tile (the
 // tiles inside a big box are covered whole).
-__global__ __launch_bounds__(256) void big_emit_kernel(const Splat *__restrict__ splats, const TileRecord *__restrict__ records,
-                                                       const uint32_t *__restrict__ bigList, const uint64_t *__restrict__ bigBits,
-                                                       uint32_t gridW, TileShape shape, uint32_t tileBits, const uint32_t *counters,
-                                                       uint32_t *__restrict__ entryKeys, uint32_t *__restrict__ entryValues) {
-  if (counters[kOverflow] != 0) return; // the same for every thread of the launch
+__device__ __forceinline__ void emit_big(uint32_t block, uint32_t blocks, const Splat *__restrict__ splats,
+                                         const TileRecord *__restrict__ records, const uint32_t *__restrict__ bigList, uint32_t listed,
+                                         const uint64_t *__restrict__ bigBits, uint32_t gridW, TileShape shape, uint32_t tileBits,
+                                         uint32_t limit, uint32_t *__restrict__ entryKeys, uint32_t *__restrict__ entryValues) {
   const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t waves = gridDim.x * (blockDim.x / 64u), wave = (blockIdx.x * blockDim.x + threadIdx.x) / 64u;
-  const uint32_t listed = counters[kBigSplats], limit = counters[kEntriesUsed];
+  const uint32_t waves = blocks * 4u, wave = block * 4u + threadIdx.x / 64u;
   const uint32_t allBlocks = ((1u << ((shape.w >> 3) * (shape.h >> 3))) - 1u) << tileBits;
   // Wave w takes listed splats w, w + waves, w + 2 waves, ..., 64 at a time (one
   // per lane), so that a short list still spreads over every wave.
@@ -257,6 +263,26 @@ __global__ __launch_bounds__(256) void big_emit_kernel(const Splat *__restrict__
         cursor.advance();
       }
     }
+  }
+}
+
+// Both kinds of splats in one launch, side by side: the first smallBlocks
+// workgroups list the small splats (256 each), the others the big ones.
+__global__ __launch_bounds__(256) void bin_emit_kernel(const uint32_t *__restrict__ keys, const uint32_t *__restrict__ values,
+                                                       const Splat *__restrict__ splats, const TileRecord *__restrict__ records,
+                                                       uint32_t count, uint32_t gridW, TileShape shape, uint32_t width, uint32_t height,
+                                                       uint32_t tileBits, bool blockMasks, const uint32_t *__restrict__ offsets,
+                                                       const uint32_t *__restrict__ bigList, const uint64_t *__restrict__ bigBits,
+                                                       uint32_t smallBlocks, const uint32_t *counters, uint32_t *__restrict__ entryKeys,
+                                                       uint32_t *__restrict__ entryValues) {
+  if (counters[kOverflow] != 0) return; // the same for every thread of the launch
+  const uint32_t limit = counters[kEntriesUsed];
+  if (blockIdx.x < smallBlocks) {
+    emit_small(keys, values, splats, records, count, gridW, shape, width, height, tileBits, blockMasks, offsets, limit, entryKeys,
+               entryValues);
+  } else {
+    emit_big(blockIdx.x - smallBlocks, gridDim.x - smallBlocks, splats, records, bigList, counters[kBigSplats], bigBits, gridW, shape,
+             tileBits, limit, entryKeys, entryValues);
   }
 }
 
@@ -302,11 +328,11 @@ __global__ __launch_bounds__(256) void tile_ranges_kernel(const uint32_t *__rest
 size_t coverage_scan_words(uint32_t count) { return 2 * static_cast<size_t>(count == 0 ? 1 : (count + kScanTile - 1) / kScanTile); }
 
 void launch_coverage_scan(hipStream_t stream, const uint32_t *keys, const uint32_t *values, const uint32_t *tileCount, uint32_t count,
-                          uint32_t *offsets, uint32_t *counters, uint32_t capacity, bool isStep, uint32_t *totals) {
+                          TileRecord *records, uint32_t *offsets, uint32_t *counters, uint32_t capacity, bool isStep, uint32_t *totals) {
   const uint32_t chunks = count == 0 ? 1 : (count + kScanTile - 1) / kScanTile;
   hipLaunchKernelGGL(coverage_count_kernel, dim3(chunks), dim3(kScanThreads), 0, stream, keys, values, tileCount, count, offsets, totals);
-  hipLaunchKernelGGL(coverage_offsets_kernel, dim3(chunks), dim3(kScanThreads), 0, stream, count, offsets, totals, counters, capacity,
-                     isStep ? 1u : 0u);
+  hipLaunchKernelGGL(coverage_offsets_kernel, dim3(chunks), dim3(kScanThreads), 0, stream, values, count, records, offsets,
+                     totals, counters, capacity, isStep ? 1u : 0u);
 }
 
 void launch_gather_views(hipStream_t stream, const ViewStatus &views, uint8_t *slots, uint32_t *status) {
@@ -314,7 +340,13 @@ void launch_gather_views(hipStream_t stream, const ViewStatus &views, uint8_t *s
   hipLaunchKernelGGL(gather_views_kernel, dim3(1), dim3(128), 0, stream, views, slots, status);
 }
 
-void launch_bin_emit(hipStream_t stream, const uint32_t *keys, const uint32_t *values, const Splat *splats, TileRecord *records,
+void launch_finish(hipStream_t stream, uint32_t *adamState, float beta1, float beta2, const uint32_t *counters, const double *sums,
+                   uint32_t *status) {
+  hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(64), 0, stream, adamState, beta1, beta2, counters, reinterpret_cast<const uint32_t *>(sums),
+                     status);
+}
+
+void launch_bin_emit(hipStream_t stream, const uint32_t *keys, const uint32_t *values, const Splat *splats, const TileRecord *records,
                      uint32_t count, uint32_t gridW, uint32_t tileW, uint32_t tileH, uint32_t width, uint32_t height, uint32_t tileBits,
                      const uint32_t *offsets, const uint32_t *counters, const uint32_t *bigList, const uint64_t *bigBits,
                      uint32_t *entryKeys, uint32_t *entryValues) {
@@ -323,10 +355,10 @@ void launch_bin_emit(hipStream_t stream, const uint32_t *keys, const uint32_t *v
   // skipping the entries that miss it saves more raster time than marking
   // costs the list pass; smaller tiles mark every block.
   const bool blockMasks = (tileW / 8u) * (tileH / 8u) >= 16u;
-  hipLaunchKernelGGL(bin_emit_kernel, dim3((count + 255) / 256), dim3(256), 0, stream, keys, values, splats, records, count, gridW,
-                     TileShape{tileW, tileH}, width, height, tileBits, blockMasks, offsets, counters, entryKeys, entryValues);
-  hipLaunchKernelGGL(big_emit_kernel, dim3(kBigSplatBlocks), dim3(256), 0, stream, splats, records, bigList, bigBits, gridW,
-                     TileShape{tileW, tileH}, tileBits, counters, entryKeys, entryValues);
+  const uint32_t smallBlocks = (count + 255) / 256;
+  hipLaunchKernelGGL(bin_emit_kernel, dim3(smallBlocks + big_splat_blocks(count)), dim3(256), 0, stream, keys, values, splats, records, count,
+                     gridW, TileShape{tileW, tileH}, width, height, tileBits, blockMasks, offsets, bigList, bigBits, smallBlocks, counters,
+                     entryKeys, entryValues);
 }
 
 void launch_tile_ranges(hipStream_t stream, const uint32_t *entryKeys, const uint32_t *counters, uint32_t capacity, uint32_t tileBits,

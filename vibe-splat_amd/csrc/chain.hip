@@ -958,14 +958,6 @@ __global__ __launch_bounds__(256) void sh_adam_kernel(uint32_t *__restrict__ shW
   if (changed) shWords[w] = word;
 }
 
-// After a step's last kernel: one more step taken, unless the step was skipped.
-__global__ void advance_adam_kernel(uint32_t *state, float beta1, float beta2, const uint32_t *counters) {
-  if (counters[kOverflow] != 0) return;
-  state[0] += 1u;
-  state[1] = as_uint(as_float(state[1]) * beta1);
-  state[2] = as_uint(as_float(state[2]) * beta2);
-}
-
 // After a scored view (train_score.comp:17-26): each Gaussian's marked pixels
 // (raw sum 12, over 3 pixels of the image like the derivatives, times
 // toPixels), that count times the view's loss, and its edge score (raw sum 13
@@ -1123,9 +1115,6 @@ void launch_chain(hipStream_t stream, const ChainBuffers &buffers, const ViewPar
     const uint64_t words = static_cast<uint64_t>(view.count) * view.shWords;
     hipLaunchKernelGGL(sh_step_kernel, dim3(static_cast<uint32_t>((words + 255) / 256)), dim3(256), 0, stream, buffers.shWords,
                        buffers.stateSh, buffers.shPass, view, params, counters);
-    if (params.mode == kModeStep && params.adamState != nullptr) {
-      hipLaunchKernelGGL(advance_adam_kernel, dim3(1), dim3(1), 0, stream, params.adamState, params.beta1, params.beta2, counters);
-    }
   }
 }
 
@@ -1145,9 +1134,6 @@ void launch_sh_adam(hipStream_t stream, const ChainBuffers &buffers, const ViewP
   const uint64_t words = static_cast<uint64_t>(view.count) * view.shWords;
   hipLaunchKernelGGL(sh_adam_kernel, dim3(static_cast<uint32_t>((words + 255) / 256)), dim3(256), 0, stream, buffers.shWords,
                      buffers.stateSh, buffers.gradSh, view, params, counters);
-  if (params.adamState != nullptr) {
-    hipLaunchKernelGGL(advance_adam_kernel, dim3(1), dim3(1), 0, stream, params.adamState, params.beta1, params.beta2, counters);
-  }
 }
 
 void launch_noise(hipStream_t stream, const ChainBuffers &buffers, uint32_t count, float scaler, const uint32_t *iterationDev,
@@ -1195,9 +1181,6 @@ void launch_adam(hipStream_t stream, const ChainBuffers &buffers, const ViewPara
   const uint64_t words = static_cast<uint64_t>(view.count) * view.shWords;
   hipLaunchKernelGGL(sh_adam_kernel, dim3(static_cast<uint32_t>((words + 255) / 256)), dim3(256), 0, stream, buffers.shWords,
                      buffers.stateSh, buffers.gradSh, view, params, counters);
-  if (params.adamState != nullptr) {
-    hipLaunchKernelGGL(advance_adam_kernel, dim3(1), dim3(1), 0, stream, params.adamState, params.beta1, params.beta2, counters);
-  }
 }
 
 } // namespace vsplat

@@ -77,9 +77,12 @@ struct ChainViews {
 
 struct TileRecord;
 
-// Workgroups (of four waves) of the kernels that count and list the big splats
-// (boxes of more than kMaskTiles tiles), whose waves take the listed splats in turn.
-constexpr uint32_t kBigSplatBlocks = 2048;
+// Workgroups (of four waves) that count and list the big splats (boxes of more
+// than kMaskTiles tiles), whose waves take the listed splats in turn: enough to
+// fill the chip, fewer for clouds too small to need them.
+inline uint32_t big_splat_blocks(uint32_t count) { return count / 16 < 64 ? 64u : (count / 16 < 2048 ? count / 16 : 2048u); }
+// A big splat's tile count carries this bit, so that the coverage scan knows it.
+constexpr uint32_t kBigCount = 0x80000000u;
 
 // Projection and tile coverage: splats, depth keys and values (the identity),
 // and per Gaussian the tile count and TileRecord; adds the visible count. The
@@ -95,10 +98,20 @@ void launch_project(hipStream_t stream, const float *positions, const float *sca
 
 // Scratch for launch_radix_sort over up to capacity keys.
 size_t radix_sort_scratch_words(uint64_t capacity);
+// Whether a sort by this many bits takes an odd number of passes: its input is
+// then read from tmpKeys and tmpValues, so that the result ends in keys and values.
+bool radix_sort_from_tmp(uint32_t bits);
 void launch_radix_sort(hipStream_t stream, uint32_t *keys, uint32_t *values, uint32_t *tmpKeys, uint32_t *tmpValues,
                        const uint32_t *countDev, uint32_t capacity, uint32_t bits, uint32_t *scratch);
-void launch_copy_u32(hipStream_t stream, const uint32_t *src, uint32_t *dst, const uint32_t *countDev, uint32_t capacity);
 void launch_fill_u32(hipStream_t stream, uint32_t *dst, uint64_t count, uint32_t value);
+// Two arrays cleared in one launch.
+void launch_clear_two(hipStream_t stream, uint32_t *a, uint64_t aCount, uint32_t *b, uint64_t bCount);
+// What ends a pass, in one small kernel: with adamState the step counted (one
+// more step taken, unless the pass was skipped), and with status the pass's
+// counters and loss sums (kViewStatusBytes) written to it, host memory that the
+// device writes to.
+void launch_finish(hipStream_t stream, uint32_t *adamState, float beta1, float beta2, const uint32_t *counters, const double *sums,
+                   uint32_t *status);
 
 // One per-Gaussian array for launch_gather: `stride` 32-bit words per Gaussian.
 struct GatherArray {
@@ -115,12 +128,12 @@ void launch_gather(hipStream_t stream, const int32_t *source, uint32_t gaussians
 // entries and its visible splats; written before it is read).
 size_t coverage_scan_words(uint32_t count);
 // Offsets of each depth-sorted splat's entries, the visible and entry counts
-// and the capacity check.
+// and the capacity check. A big splat's first entry goes to its record too (maskLo).
 void launch_coverage_scan(hipStream_t stream, const uint32_t *keys, const uint32_t *values, const uint32_t *tileCount, uint32_t count,
-                          uint32_t *offsets, uint32_t *counters, uint32_t capacity, bool isStep, uint32_t *totals);
+                          TileRecord *records, uint32_t *offsets, uint32_t *counters, uint32_t capacity, bool isStep, uint32_t *totals);
 // A batch's views' status, up to kStatusViewsPerLaunch views (views first ..
 // first + count - 1) a launch: each view's counters and loss sums copied to its
-// kViewStatusBytes slot of `slots`, then status[overflow] (the first view's
+// kViewStatusBytes slot of `slots` (host memory that the device writes to), then status[overflow] (the first view's
 // counters) |= every other view's.
 constexpr uint32_t kStatusViewsPerLaunch = 8, kViewStatusBytes = 48;
 struct ViewStatus {
@@ -129,13 +142,13 @@ struct ViewStatus {
   uint32_t first, count;
 };
 void launch_gather_views(hipStream_t stream, const ViewStatus &views, uint8_t *slots, uint32_t *status);
-// The tile lists in depth order: the small splats' entries from their bits,
-// then the big splats' (bigList, with the bits launch_project kept). records is written: a
-// big splat's first entry is kept in its maskLo for the second kernel.
+// The tile lists in depth order, in one launch: the small splats' entries from
+// their bits, and the big splats' (bigList, with the bits launch_project kept) from
+// the first entry the coverage scan left in their records.
 // The tile entries (keys: the tile in the low tileBits bits, above them the
 // tile's 8x8 blocks the splat reaches, marked for 32x32 tiles and all set for
 // the others; values: the Gaussian), for a view of width x height pixels.
-void launch_bin_emit(hipStream_t stream, const uint32_t *keys, const uint32_t *values, const Splat *splats, TileRecord *records,
+void launch_bin_emit(hipStream_t stream, const uint32_t *keys, const uint32_t *values, const Splat *splats, const TileRecord *records,
                      uint32_t count, uint32_t gridW, uint32_t tileW, uint32_t tileH, uint32_t width, uint32_t height, uint32_t tileBits,
                      const uint32_t *offsets, const uint32_t *counters, const uint32_t *bigList, const uint64_t *bigBits,
                      uint32_t *entryKeys, uint32_t *entryValues);
@@ -149,6 +162,10 @@ constexpr uint32_t kRasterXcds = 8;
 inline uint32_t raster_blocks(uint32_t tiles, uint32_t tileW, uint32_t tileH) {
   return (tiles + kRasterXcds - 1) / kRasterXcds * kRasterXcds * (tileW / 8u) * (tileH / 8u);
 }
+
+// The most blocks a view's raster passes launch in index order rather than
+// heaviest first: those that are resident at once.
+constexpr uint32_t kRasterResident = 4096;
 
 // One view of a batched raster launch (its buffers and sizes), and up to
 // kRasterViewsPerLaunch of them, passed by value as the kernel's argument.
@@ -209,7 +226,10 @@ void launch_list_order(hipStream_t stream, const uint2 *ranges, uint32_t tiles, 
 // and the target's edge weights, and the adjoint's fourth value the pixel's
 // error; both null otherwise.
 void launch_loss(hipStream_t stream, const float4 *image, const uint8_t *target, uint32_t width, uint32_t height, float lambda,
-                 float *fields, float4 *adjoint, float2 *tileTotals, double *sums, uint32_t *errorMax, float *edge);
+                 float *fields, float4 *adjoint, float2 *tileTotals, uint32_t *errorMax, float *edge);
+// The tiles' totals summed (sums[0] SSIM, sums[1] L1), and `words` words of the
+// raw sums (16-byte aligned) cleared for the backward pass, in one launch.
+void launch_total_and_clear(hipStream_t stream, const float2 *tileTotals, uint32_t tiles, double *sums, uint32_t *raw, uint64_t words);
 
 // A view's affine colour transform (Trainer::set_exposure): rows of (r, g, b, 1).
 struct Exposure {
@@ -228,7 +248,7 @@ void launch_error_mask(hipStream_t stream, float4 *adjoint, const uint32_t *erro
 // Adam step from them and stores the SH sums for launch_sh_adam.
 void launch_chain_views(hipStream_t stream, const ChainBuffers &buffers, const ChainViews &views, const ChainParams &params,
                         const uint32_t *counters);
-// Adam for the SH coefficients from the stored SH gradients, then the step count advanced.
+// Adam for the SH coefficients from the stored SH gradients.
 void launch_sh_adam(hipStream_t stream, const ChainBuffers &buffers, const ViewParams &view, const ChainParams &params,
                     const uint32_t *counters);
 // One Adam step of every parameter from the stored gradients in buffers.grad*

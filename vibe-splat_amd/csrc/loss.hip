@@ -362,9 +362,20 @@ __global__ __launch_bounds__(256) void error_mask_kernel(float4 *__restrict__ ad
   adjoint[i].w = worst > 0u && adjoint[i].w >= limit ? 1.0f : 0.0f;
 }
 
-// Sums the tiles' totals in double, in a fixed order: thread t adds tiles t,
-// t + 256, ..., then a tree over the threads. sums[0] SSIM, sums[1] L1.
-__global__ __launch_bounds__(256) void total_kernel(const float2 *__restrict__ tileTotals, uint32_t tiles, double *__restrict__ sums) {
+// Block 0 sums the tiles' totals in double, in a fixed order: thread t adds
+// tiles t, t + 256, ..., then a tree over the threads (sums[0] SSIM, sums[1] L1).
+// The other blocks clear the raw sums, vec4 of them sixteen bytes at a time and
+// the `tail` words after them, so that the one busy block costs no launch and no
+// time of its own.
+__global__ __launch_bounds__(256) void total_and_clear_kernel(const float2 *__restrict__ tileTotals, uint32_t tiles,
+                                                              double *__restrict__ sums, uint4 *__restrict__ raw, uint64_t vec4,
+                                                              uint32_t tail) {
+  if (blockIdx.x != 0) {
+    const uint64_t stride = (gridDim.x - 1) * 256ull, t = (blockIdx.x - 1) * 256ull + threadIdx.x;
+    for (uint64_t i = t; i < vec4; i += stride) raw[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (t < tail) reinterpret_cast<uint32_t *>(raw + vec4)[t] = 0u;
+    return;
+  }
   __shared__ double s[2][256];
   double ssim = 0.0, l1 = 0.0;
   for (uint32_t t = threadIdx.x; t < tiles; t += 256) {
@@ -390,15 +401,21 @@ __global__ __launch_bounds__(256) void total_kernel(const float2 *__restrict__ t
 } // namespace
 
 void launch_loss(hipStream_t stream, const float4 *image, const uint8_t *target, uint32_t width, uint32_t height, float lambda,
-                 float *fields, float4 *adjoint, float2 *tileTotals, double *sums, uint32_t *errorMax, float *edge) {
-  const uint32_t gridW = (width + 15) / 16, tiles = gridW * ((height + 15) / 16);
+                 float *fields, float4 *adjoint, float2 *tileTotals, uint32_t *errorMax, float *edge) {
+  const uint32_t gridW = (width + 15) / 16;
   const uint32_t ssimStrips = gridW * ((height + kSsimRows - 1) / kSsimRows), lossStrips = gridW * ((height + kLossRows - 1) / kLossRows);
   const uchar4 *t = reinterpret_cast<const uchar4 *>(target);
   hipLaunchKernelGGL(ssim_kernel<kSsimRows>, dim3(ssimStrips), dim3(16 * kSsimRows), 0, stream, image, t, width, height, gridW, fields,
                      tileTotals);
   hipLaunchKernelGGL(loss_kernel<kLossRows>, dim3(lossStrips), dim3(16 * kLossRows), 0, stream, image, t, width, height, gridW, lambda,
                      fields, adjoint, tileTotals, errorMax, edge);
-  hipLaunchKernelGGL(total_kernel, dim3(1), dim3(256), 0, stream, tileTotals, tiles, sums);
+}
+
+void launch_total_and_clear(hipStream_t stream, const float2 *tileTotals, uint32_t tiles, double *sums, uint32_t *raw, uint64_t words) {
+  const uint64_t blocks64 = (words / 4 + 255) / 256;
+  const uint32_t blocks = blocks64 < 1 ? 1u : (blocks64 < 4096 ? static_cast<uint32_t>(blocks64) : 4096u);
+  hipLaunchKernelGGL(total_and_clear_kernel, dim3(blocks + 1), dim3(256), 0, stream, tileTotals, tiles, sums, reinterpret_cast<uint4 *>(raw),
+                     words / 4, static_cast<uint32_t>(words % 4));
 }
 
 uint32_t exposure_groups(uint32_t pixels) { return (pixels + 255) / 256; }

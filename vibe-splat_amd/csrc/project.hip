@@ -364,7 +364,7 @@ __global__ __launch_bounds__(256) void big_count_kernel(const Splat *__restrict_
       if (lane == j) myHits = hits;
     }
     if (mineAt < listed) {
-      tileCount[mine.gaussian] = myHits;
+      tileCount[mine.gaussian] = myHits | kBigCount;
       records[mine.gaussian].maskHi = mine.first; // where its bits are, for the list pass
     }
   }
@@ -396,7 +396,7 @@ void launch_project(hipStream_t stream, const float *positions, const float *sca
 #undef VSPLAT_PROJECT_DEGREE
 #undef VSPLAT_PROJECT
   // The big splats' counts; the grid takes them in turn (how many there are is only known on the device).
-  hipLaunchKernelGGL(big_count_kernel, dim3(kBigSplatBlocks), dim3(256), 0, stream, splats, records, bigList, counters,
+  hipLaunchKernelGGL(big_count_kernel, dim3(big_splat_blocks(view.count)), dim3(256), 0, stream, splats, records, bigList, counters,
                      TileShape{view.tileW, view.tileH}, bigBits, bitCapacity, tileCount);
 }
 

@@ -216,16 +216,20 @@ size_t radix_sort_scratch_words(uint64_t capacity) {
   return 256 + static_cast<size_t>(div_up(capacity, kSortThreads * kSortPerThreadSmall)) * 256u;
 }
 
-// Sorts (keys, values) stably by the low `bits` bits of the keys (bits <= 32),
-// in ceil(bits / 8) passes of equal width. The result ends in keys/values;
-// tmpKeys/tmpValues are the other half of each pass. countDev, when given,
-// holds the element count (at most capacity).
+bool radix_sort_from_tmp(uint32_t bits) { return div_up(bits, 8) % 2 != 0; }
+
+// Sorts (keys, values) stably by the low `bits` bits of the keys (1 <= bits <=
+// 32), in ceil(bits / 8) passes of equal width. The result ends in keys/values;
+// tmpKeys/tmpValues are the other half of each pass, and hold the input when the
+// number of passes is odd (radix_sort_from_tmp), so that nothing is copied.
+// countDev, when given, holds the element count (at most capacity).
 void launch_radix_sort(hipStream_t stream, uint32_t *keys, uint32_t *values, uint32_t *tmpKeys, uint32_t *tmpValues,
                        const uint32_t *countDev, uint32_t capacity, uint32_t bits, uint32_t *scratch) {
-  if (capacity <= 1 || bits == 0) return;
+  if (capacity == 0 || bits == 0) return;
   const uint32_t passes = div_up(bits, 8);
   const uint32_t digit = div_up(bits, passes); // even split, at most 8 bits a pass
-  uint32_t *srcK = keys, *srcV = values, *dstK = tmpKeys, *dstV = tmpValues;
+  const bool odd = radix_sort_from_tmp(bits);
+  uint32_t *srcK = odd ? tmpKeys : keys, *srcV = odd ? tmpValues : values, *dstK = odd ? keys : tmpKeys, *dstV = odd ? values : tmpValues;
   for (uint32_t p = 0; p < passes; ++p) {
     // The last pass takes the bits that are left, so that no bit above `bits`
     // (which may carry other data) takes part in the order.
@@ -247,22 +251,6 @@ void launch_radix_sort(hipStream_t stream, uint32_t *keys, uint32_t *values, uin
     srcV = dstV;
     dstV = t;
   }
-  if (srcK != keys) {
-    // An odd number of passes: the result is in the temporaries.
-    launch_copy_u32(stream, srcK, keys, countDev, capacity);
-    launch_copy_u32(stream, srcV, values, countDev, capacity);
-  }
-}
-
-__global__ void copy_u32_kernel(const uint32_t *__restrict__ src, uint32_t *__restrict__ dst, const uint32_t *countDev, uint32_t countHost) {
-  const uint32_t count = count_of(countDev, countHost);
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) dst[i] = src[i];
-}
-
-void launch_copy_u32(hipStream_t stream, const uint32_t *src, uint32_t *dst, const uint32_t *countDev, uint32_t capacity) {
-  if (capacity == 0) return;
-  const uint32_t blocks = div_up(capacity, 256) < 4096 ? div_up(capacity, 256) : 4096;
-  hipLaunchKernelGGL(copy_u32_kernel, dim3(blocks), dim3(256), 0, stream, src, dst, countDev, capacity);
 }
 
 __global__ void fill_u32_kernel(uint32_t *__restrict__ dst, uint64_t count, uint32_t value) {
@@ -277,6 +265,23 @@ void launch_fill_u32(hipStream_t stream, uint32_t *dst, uint64_t count, uint32_t
   const uint64_t blocks64 = (count + 255) / 256;
   const uint32_t blocks = blocks64 < 8192 ? static_cast<uint32_t>(blocks64) : 8192;
   hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks), dim3(256), 0, stream, dst, count, value);
+}
+
+__global__ __launch_bounds__(256) void clear_two_kernel(uint32_t *__restrict__ a, uint64_t aCount, uint32_t *__restrict__ b, uint64_t bCount) {
+  for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < aCount + bCount; i += gridDim.x * 256ull) {
+    if (i < aCount) {
+      a[i] = 0u;
+    } else {
+      b[i - aCount] = 0u;
+    }
+  }
+}
+
+void launch_clear_two(hipStream_t stream, uint32_t *a, uint64_t aCount, uint32_t *b, uint64_t bCount) {
+  const uint64_t blocks64 = (aCount + bCount + 255) / 256;
+  if (blocks64 == 0) return;
+  hipLaunchKernelGGL(clear_two_kernel, dim3(blocks64 < 1024 ? static_cast<uint32_t>(blocks64) : 1024u), dim3(256), 0, stream, a, aCount, b,
+                     bCount);
 }
 
 } // namespace vsplat

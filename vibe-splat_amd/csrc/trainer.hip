@@ -23,6 +23,7 @@ namespace vsplat {
 // 1 / (3 W H), which 3 W H undoes, then kFixedSteps steps per unit
 // (trainer.cpp:586-591 has 64 steps; the sums here are 64-bit).
 static float fixed_scale(const ViewParams &v) { return 3.0f * static_cast<float>(v.width) * static_cast<float>(v.height) * kFixedSteps; }
+constexpr float kBeta1 = 0.9f, kBeta2 = 0.999f; // Adam's
 // The curvature's Hutchinson adjoint is +-1 per value, without the 1 / (3 W H).
 static float curvature_fixed_scale() { return kFixedSteps; }
 
@@ -152,7 +153,8 @@ Trainer::Trainer(const vsplat_cloud &c, const vsplat_trainer_options &options) :
     launch_fill_u32(stream_, state_[g].as<uint32_t>(), stateFloats[g], 0u);
   }
   allocate_per_gaussian();
-  readback_.ensure(kCounterWords * 4 + 2 * sizeof(double));
+  readback_.ensure(2 * kStatusSlot);
+  std::memset(readback_.as<uint8_t>(), 0, 2 * kStatusSlot);
   adamState_.ensure(4 * 4);
   const uint32_t adamStart[4] = {0u, 0x3F800000u, 0x3F800000u, 0u}; // no steps; beta^0 = 1
   check(hipMemcpy(adamState_.as<uint32_t>(), adamStart, sizeof(adamStart), hipMemcpyHostToDevice), "adam state");
@@ -388,6 +390,7 @@ std::pair<uint32_t, uint32_t> Trainer::autotune_tiles(const vsplat_camera &camer
       uint64_t entries = 0;
       for (int attempt = 0;; ++attempt) {
         enqueue_passes(b, v, deviceTarget, kModeGradients, nullptr, false, false);
+        finish_pass(b, false);
         bool overflow = false;
         const vsplat_step_stats stats = read_stats(overflow);
         entries = stats.tile_entries;
@@ -458,6 +461,7 @@ void Trainer::autotune_views(uint32_t n, const vsplat_camera *cameras, const uin
     // One run sizes the tile-entry buffers for these shapes (also down).
     for (int attempt = 0;; ++attempt) {
       enqueue_batch_passes(n, cameras, targets, params.data());
+      finish_pass(*views_[0], false);
       bool overflow = false;
       synchronize_views(stats.data(), n, overflow);
       if (!overflow) break;
@@ -661,13 +665,16 @@ void Trainer::enqueue_passes(ViewBuffers &b, const ViewParams &view, const uint8
   // Each pass's 8x8 blocks launch heaviest first on their XCD: the forward's by
   // their tiles' list lengths, the backward's by the work the forward found.
   const bool backward = mode != kModeRender;
-  uint32_t *listOrder = b.listOrder.as<uint32_t>(); // none in the allocation-free render
+  const bool ordered = launch_ordered(b);
+  uint32_t *listOrder = ordered ? b.listOrder.as<uint32_t>() : nullptr; // none in the allocation-free render
   if (listOrder != nullptr) launch_list_order(b.stream, b.ranges.as<uint2>(), b.tiles, b.tileW, b.tileH, listOrder);
   launch_forward(b.stream, b.splats.as<Splat>(), b.entryKeys.as<uint32_t>(), b.entryValues.as<uint32_t>(), b.tileBits, b.ranges.as<uint2>(),
                  v.width, v.height, b.tileW, b.tileH, options_.background, b.image.as<float4>(),
                  options_.recompute_transmittance != 0 ? nullptr : b.stops.as<uint32_t>(), backward ? b.blockWork.as<uint32_t>() : nullptr,
                  listOrder);
-  if (backward) launch_work_order(b.stream, b.blockWork.as<uint32_t>(), raster_blocks(b.tiles, b.tileW, b.tileH), b.blockOrder.as<uint32_t>());
+  if (backward && ordered) {
+    launch_work_order(b.stream, b.blockWork.as<uint32_t>(), raster_blocks(b.tiles, b.tileW, b.tileH), b.blockOrder.as<uint32_t>());
+  }
   mark("composite");
   if (!backward) return;
   enqueue_loss(b, v, deviceTarget);
@@ -679,12 +686,18 @@ void Trainer::enqueue_passes(ViewBuffers &b, const ViewParams &view, const uint8
                   b.entryValues.as<uint32_t>(), b.tileBits, b.ranges.as<uint2>(), v.width, v.height, b.tileW, b.tileH, options_.background,
                   b.image.as<float4>(),
                   b.adjoint.as<float4>(), b.stops.as<uint32_t>(), fixed_scale(v), b.rawFixed.as<int64_t>(), b.rawFloat.as<float>(),
-                  scoring ? b.edge.as<float>() : nullptr, b.blockOrder.as<uint32_t>());
+                  scoring ? b.edge.as<float>() : nullptr, ordered ? b.blockOrder.as<uint32_t>() : nullptr);
   mark("backward");
   if (!chain) return;
   enqueue_chain(b, v, mode, rates, b.stream, b.counters.as<uint32_t>());
   mark(mode == kModeStep ? "chain rule and step" : "chain rule");
 }
+
+// Whether the raster passes of a view launch their blocks heaviest first. A view
+// whose blocks all fit the chip at once (the raster kernels hold seven waves a
+// SIMD, over 1024 SIMDs) has no late starters to bring forward: its two order
+// kernels, 4 to 5 us each, are left out.
+bool Trainer::launch_ordered(const ViewBuffers &b) { return raster_blocks(b.tiles, b.tileW, b.tileH) > kRasterResident; }
 
 ViewParams Trainer::with_tiles(const ViewBuffers &b, const ViewParams &view) const {
   ViewParams v = view;
@@ -698,7 +711,8 @@ ViewParams Trainer::with_tiles(const ViewBuffers &b, const ViewParams &view) con
 void Trainer::enqueue_lists(ViewBuffers &b, const ViewParams &v, uint32_t mode, bool marks) {
   hipStream_t s = b.stream;
   uint32_t *counters = b.counters.as<uint32_t>();
-  launch_fill_u32(s, counters, kClearedPerPass, 0u); // not the sticky overflow word
+  // The counters (not the sticky overflow word) and the tiles' ranges.
+  launch_clear_two(s, counters, kClearedPerPass, b.ranges.as<uint32_t>(), static_cast<uint64_t>(b.tiles) * 2);
   launch_project(s, positions_.as<float>(), scales_.as<float>(), rotations_.as<float>(), opacities_.as<float>(),
                  shWordsBuf_.as<uint32_t>(), filterSet_ ? filter3d_.as<float>() : nullptr, v, options_.mip_filter_2d != 0, dropoutNow_,
                  shRetained_, shSeed_, b.gridW, b.gridH, b.splats.as<Splat>(), b.keys.as<uint32_t>(), b.values.as<uint32_t>(),
@@ -708,15 +722,15 @@ void Trainer::enqueue_lists(ViewBuffers &b, const ViewParams &v, uint32_t mode, 
   launch_radix_sort(s, b.keys.as<uint32_t>(), b.values.as<uint32_t>(), b.tmpKeys.as<uint32_t>(), b.tmpValues.as<uint32_t>(), nullptr, count_,
                     32, b.sortScratch.as<uint32_t>());
   if (marks) mark("depth sort");
-  launch_coverage_scan(s, b.keys.as<uint32_t>(), b.values.as<uint32_t>(), b.tileCount.as<uint32_t>(), count_, b.coverage.as<uint32_t>(),
-                       counters, static_cast<uint32_t>(b.entryCapacity), mode == kModeStep, b.scanScratch.as<uint32_t>());
+  launch_coverage_scan(s, b.keys.as<uint32_t>(), b.values.as<uint32_t>(), b.tileCount.as<uint32_t>(), count_,
+                       b.tileRecords.as<TileRecord>(), b.coverage.as<uint32_t>(), counters, static_cast<uint32_t>(b.entryCapacity), mode == kModeStep, b.scanScratch.as<uint32_t>());
   if (marks) mark("count tiles");
-  launch_fill_u32(s, b.ranges.as<uint32_t>(), static_cast<uint64_t>(b.tiles) * 2, 0u);
   if (b.entryCapacity > 0) {
+    const bool fromTmp = radix_sort_from_tmp(b.tileBits);
     launch_bin_emit(s, b.keys.as<uint32_t>(), b.values.as<uint32_t>(), b.splats.as<Splat>(), b.tileRecords.as<TileRecord>(), count_, b.gridW,
                     b.tileW, b.tileH, static_cast<uint32_t>(b.width), static_cast<uint32_t>(b.height), b.tileBits,
-                    b.coverage.as<uint32_t>(), counters, b.bigList.as<uint32_t>(), b.bigBits.as<uint64_t>(), b.entryKeys.as<uint32_t>(),
-                    b.entryValues.as<uint32_t>());
+                    b.coverage.as<uint32_t>(), counters, b.bigList.as<uint32_t>(), b.bigBits.as<uint64_t>(),
+                    (fromTmp ? b.tmpEntryKeys : b.entryKeys).as<uint32_t>(), (fromTmp ? b.tmpEntryValues : b.entryValues).as<uint32_t>());
     launch_radix_sort(s, b.entryKeys.as<uint32_t>(), b.entryValues.as<uint32_t>(), b.tmpEntryKeys.as<uint32_t>(), b.tmpEntryValues.as<uint32_t>(),
                       counters + kEntriesUsed, static_cast<uint32_t>(b.entryCapacity), b.tileBits, b.sortScratch.as<uint32_t>());
     launch_tile_ranges(s, b.entryKeys.as<uint32_t>(), counters, static_cast<uint32_t>(b.entryCapacity), b.tileBits, b.ranges.as<uint2>());
@@ -749,17 +763,15 @@ void Trainer::enqueue_loss(ViewBuffers &b, const ViewParams &v, const uint8_t *d
   const bool scoring = scoreShare_ > 0.0f;
   if (scoring) launch_fill_u32(s, b.errorMax.as<uint32_t>(), 1, 0u);
   launch_loss(s, seen, deviceTarget, v.width, v.height, options_.lambda_ssim, b.fields.as<float>(), b.adjoint.as<float4>(),
-              b.tileTotals.as<float2>(), b.sums.as<double>(), scoring ? b.errorMax.as<uint32_t>() : nullptr,
+              b.tileTotals.as<float2>(), scoring ? b.errorMax.as<uint32_t>() : nullptr,
               scoring ? b.edge.as<float>() : nullptr);
   if (exposing_) {
     launch_exposure_backward(s, b.image.as<float4>(), b.adjoint.as<float4>(), pixels, exposure_, b.exposureTotals.as<float>());
   }
   if (scoring) launch_error_mask(s, b.adjoint.as<float4>(), b.errorMax.as<uint32_t>(), pixels, scoreShare_);
-  if (fixedPoint_) {
-    launch_fill_u32(s, b.rawFixed.as<uint32_t>(), static_cast<uint64_t>(count_) * kRawPerSplat * 2, 0u);
-  } else {
-    launch_fill_u32(s, b.rawFloat.as<uint32_t>(), static_cast<uint64_t>(count_) * kRawPerSplat, 0u);
-  }
+  launch_total_and_clear(s, b.tileTotals.as<float2>(), b.lossTiles, b.sums.as<double>(),
+                         fixedPoint_ ? b.rawFixed.as<uint32_t>() : b.rawFloat.as<uint32_t>(),
+                         static_cast<uint64_t>(count_) * kRawPerSplat * (fixedPoint_ ? 2u : 1u));
 }
 
 ChainParams Trainer::chain_params(const ViewParams &v, uint32_t mode, const vsplat_learning_rates *rates) const {
@@ -786,8 +798,8 @@ ChainParams Trainer::chain_params(const ViewParams &v, uint32_t mode, const vspl
     p.seed = curvatureUpdates_;
     p.perValue = 1.0f / (3.0f * static_cast<float>(v.width) * static_cast<float>(v.height));
   }
-  p.beta1 = 0.9f;
-  p.beta2 = 0.999f;
+  p.beta1 = kBeta1;
+  p.beta2 = kBeta2;
   p.epsilon = 1e-15f; // trainer.cpp:23
   p.adamState = adamState_.as<uint32_t>();
   if (mode == kModeStep) {
@@ -847,7 +859,16 @@ void Trainer::enqueue_chain(const ViewBuffers &b, const ViewParams &v, uint32_t 
   if (pose) launch_fill_u32(stream, poseTerms_.as<uint32_t>(), static_cast<uint64_t>(count_) * 6, 0u);
   launch_chain(stream, chain_buffers(b), v, chain_params(v, mode, rates), counters);
   if (pose) launch_pose_totals(stream, poseTerms_.as<float>(), count_, poseTotals_.as<float>());
+  if (mode == kModeCurvature) return;
+  finish_pass(b, mode == kModeStep);
   if (mode == kModeStep) enqueue_noise(b, rates, stream, counters);
+}
+
+// Ends a pass on b's stream: a step counted, and the pass's counters and loss
+// sums written to host memory for read_stats.
+void Trainer::finish_pass(const ViewBuffers &b, bool step) {
+  launch_finish(b.stream, step ? adamState_.as<uint32_t>() : nullptr, kBeta1, kBeta2, b.counters.as<uint32_t>(), b.sums.as<double>(),
+                readback_.as<uint32_t>());
 }
 
 // After a step with TrainerOptions::position_noise set (trainer.cpp:601): the
@@ -875,18 +896,17 @@ void Trainer::reset_opacity(float maximum) {
   check(hipStreamSynchronize(stream_), "reset opacity");
 }
 
+// Waits for the trainer's stream and reads what the last finish_pass on it wrote
+// (an overflow once: the caller clears the device's).
 vsplat_step_stats Trainer::read_stats(bool &overflow) {
-  ViewBuffers &b = *views_[0];
-  uint8_t *host = readback_.as<uint8_t>();
-  check(hipMemcpyAsync(host, b.counters.as<uint32_t>(), kCounterWords * 4, hipMemcpyDeviceToHost, stream_), "read counters");
-  check(hipMemcpyAsync(host + kCounterWords * 4, b.sums.as<double>(), 2 * sizeof(double), hipMemcpyDeviceToHost, stream_), "read sums");
   check(hipStreamSynchronize(stream_), "step");
   uint32_t counters[kCounterWords];
   double sums[2];
-  std::memcpy(counters, host, sizeof(counters));
-  std::memcpy(sums, host + kCounterWords * 4, sizeof(sums));
+  std::memcpy(counters, readback_.as<uint8_t>(), sizeof(counters));
+  std::memcpy(sums, readback_.as<uint8_t>() + sizeof(counters), sizeof(sums));
   overflow = counters[kOverflow] != 0;
-  return make_stats(counters, sums, b.width, b.height);
+  readback_.as<uint32_t>()[kOverflow] = 0;
+  return make_stats(counters, sums, views_[0]->width, views_[0]->height);
 }
 
 vsplat_step_stats Trainer::make_stats(const uint32_t *counters, const double *sums, int width, int height) const {
@@ -1032,6 +1052,7 @@ void Trainer::render(const vsplat_camera &camera, float *out) {
   const ViewParams v = view_params(camera);
   for (int attempt = 0;; ++attempt) {
     enqueue_passes(b, v, nullptr, kModeRender, nullptr, false);
+    finish_pass(b, false);
     bool overflow = false;
     const vsplat_step_stats stats = read_stats(overflow);
     if (!overflow) break;
@@ -1099,8 +1120,10 @@ void Trainer::render_into(const vsplat_camera &camera, float *deviceOut, uint64_
   launch_fill_u32(stream_, b.counters.as<uint32_t>(), kCounterWords, 0u);
   dropoutNow_ = 0.0f; // as render(): the whole model
   enqueue_passes(b, view_params(camera), nullptr, kModeRender, nullptr, false);
-  uint32_t *host = readback_.as<uint32_t>(); // pinned at construction
-  check(hipMemcpyAsync(host, b.counters.as<uint32_t>(), kCounterWords * 4, hipMemcpyDeviceToHost, stream_), "read counters");
+  // The counters to a slot of their own in host memory (pinned at construction):
+  // a queued step's status stays for synchronize(). (The sums are not this pass's.)
+  uint32_t *host = reinterpret_cast<uint32_t *>(readback_.as<uint8_t>() + kStatusSlot);
+  launch_finish(stream_, nullptr, 0.0f, 0.0f, b.counters.as<uint32_t>(), views_[0]->sums.as<double>(), host);
   check(hipStreamSynchronize(stream_), "render");
   if (host[kOverflow] != 0) {
     throw Error(VSPLAT_BUDGET_EXCEEDED, std::to_string(host[kEntries]) + " tile entries: the allocation-free render lists at most " +
@@ -1117,6 +1140,7 @@ void Trainer::apply_gradients(const vsplat_learning_rates &rates) {
   // Adam from the stored gradients: the same rule and rounding as the chain
   // rule's own step, and it also serves a batch's summed gradients.
   launch_adam(stream_, chain_buffers(*views_[0]), lastView_, chain_params(lastView_, kModeStep, &rates), views_[0]->counters.as<uint32_t>());
+  launch_finish(stream_, adamState_.as<uint32_t>(), kBeta1, kBeta2, views_[0]->counters.as<uint32_t>(), views_[0]->sums.as<double>(), nullptr);
   mark("adam step");
   check(hipStreamSynchronize(stream_), "apply gradients");
   drain_timing();
@@ -1180,7 +1204,10 @@ void Trainer::prepare_views(uint32_t n, const vsplat_camera *cameras, const uint
     ensure_size(view_buffers(k), cameras[k].width, cameras[k].height);
   }
   ensure_gradients();
-  viewStats_.ensure(static_cast<size_t>(n) * kViewStatsBytes);
+  if (viewStats_.bytes() < static_cast<size_t>(n) * kViewStatsBytes) {
+    check(hipStreamSynchronize(stream_), "view stats"); // a queued batch may still write the old one
+    viewStats_.ensure(static_cast<size_t>(n) * kViewStatsBytes);
+  }
 }
 
 // Each view's passes up to its backward pass, on the view's stream, after
@@ -1354,8 +1381,10 @@ void Trainer::enqueue_views(uint32_t n, const vsplat_camera *cameras, const uint
   lastViewIndex_ = n - 1;
   if (mode == kModeStep) {
     launch_sh_adam(stream_, buffers, lastView_, chain_params(lastView_, kModeStep, rates), status);
+    finish_pass(*views_[0], true);
     enqueue_noise(*views_[0], rates, stream_, status);
   } else {
+    finish_pass(*views_[0], false);
     haveGradients_ = true;
   }
 }
@@ -1374,9 +1403,9 @@ uint64_t Trainer::capture_key(uint32_t n) const {
     mix(reinterpret_cast<uintptr_t>(a.as<void>()));
     mix(a.bytes());
   };
-  for (const DeviceArray *a : {&positions_, &scales_, &rotations_, &opacities_, &shWordsBuf_, &adamState_, &shPass_, &stats_, &filter3d_,
-                               &viewStats_})
+  for (const DeviceArray *a : {&positions_, &scales_, &rotations_, &opacities_, &shWordsBuf_, &adamState_, &shPass_, &stats_, &filter3d_})
     array(*a);
+  mix(reinterpret_cast<uintptr_t>(viewStats_.as<void>()));
   for (int g = 0; g < 5; ++g) {
     array(state_[g]);
     array(grad_[g]);
@@ -1471,13 +1500,12 @@ uint32_t Trainer::synchronize_views(vsplat_step_stats *stats, uint32_t capacity,
   (void)read_stats(overflow);
   drain_timing();
   const uint32_t n = static_cast<uint32_t>(queuedViewSizes_.size());
-  std::vector<uint8_t> host(static_cast<size_t>(n) * kViewStatsBytes);
-  if (n > 0) check(hipMemcpy(host.data(), viewStats_.as<uint8_t>(), host.size(), hipMemcpyDeviceToHost), "read view stats");
+  const uint8_t *host = viewStats_.as<uint8_t>();
   for (uint32_t k = 0; k < n && k < capacity && stats != nullptr; ++k) {
     uint32_t counters[kCounterWords];
     double sums[2];
-    std::memcpy(counters, host.data() + static_cast<size_t>(k) * kViewStatsBytes, sizeof(counters));
-    std::memcpy(sums, host.data() + static_cast<size_t>(k) * kViewStatsBytes + kCounterWords * 4, sizeof(sums));
+    std::memcpy(counters, host + static_cast<size_t>(k) * kViewStatsBytes, sizeof(counters));
+    std::memcpy(sums, host + static_cast<size_t>(k) * kViewStatsBytes + kCounterWords * 4, sizeof(sums));
     stats[k] = make_stats(counters, sums, queuedViewSizes_[k].first, queuedViewSizes_[k].second);
   }
   if (overflow) clear_overflow();
@@ -1719,7 +1747,7 @@ uint64_t Trainer::bytes_per_gaussian() const {
 
 uint64_t Trainer::gpu_bytes() const {
   // One view's per-Gaussian share is in bytes_per_gaussian; the others' are added as allocated.
-  uint64_t total = bytes_per_gaussian() * count_ + target_.bytes() + viewStats_.bytes();
+  uint64_t total = bytes_per_gaussian() * count_ + target_.bytes();
   for (size_t k = 0; k < views_.size(); ++k) {
     const ViewBuffers &b = *views_[k];
     for (const DeviceArray *a : {&b.image, &b.stops, &b.adjoint, &b.fields, &b.ranges, &b.tileTotals, &b.listOrder, &b.blockWork,
@@ -1791,6 +1819,10 @@ void Trainer::inspect(const std::string &name, void *out, uint64_t capacity, uin
     if (name != item.name) continue;
     if (bytes != nullptr) *bytes = item.size;
     const uint64_t copy = std::min(item.size, capacity);
+    if ((name == "list_order" || name == "block_order") && !launch_ordered(b)) {
+      for (uint64_t k = 0; k < copy / 4 && out != nullptr; ++k) static_cast<uint32_t *>(out)[k] = static_cast<uint32_t>(k);
+      return;
+    }
     if (out != nullptr && copy > 0) {
       check(hipStreamSynchronize(stream_), "inspect");
       check(hipMemcpy(out, item.array->as<void>(), copy, hipMemcpyDeviceToHost), "inspect copy");

@@ -194,6 +194,8 @@ private:
   void allocate_per_gaussian();
   void ensure_size(ViewBuffers &b, int width, int height);
   void gather_view_status(uint32_t n);
+  static bool launch_ordered(const ViewBuffers &b);
+  void finish_pass(const ViewBuffers &b, bool step);
   void ensure_layout(ViewBuffers &b, int width, int height, uint32_t tileW, uint32_t tileH);
   static void set_geometry(ViewBuffers &b, int width, int height, uint32_t tileW, uint32_t tileH);
   std::pair<uint32_t, uint32_t> tile_shape_for(int width, int height) const;
@@ -248,7 +250,7 @@ private:
   bool poseNext_ = false;      // the next chain pass writes the pose terms (the synchronous calls, with pose_gradients)
   DeviceArray poseTerms_, poseTotals_; // 6 floats per Gaussian, and per group of 256
   bool accumulateNext_ = false; // the next chain pass (gradients mode) adds to the gradient sums
-  // Per queued view of a batch: its counters and loss sums, copied on the device.
+  // Per queued view of a batch: its counters and loss sums, written by the device.
   static constexpr size_t kViewStatsBytes = kViewStatusBytes;
   std::vector<std::pair<int, int>> queuedViewSizes_;
   ViewParams lastView_{};   // the camera of the last view that ran (width 0: none)
@@ -275,9 +277,13 @@ private:
   uint64_t reservedEntries_ = 0; // what reserve_entries asked for, for views made later
   std::map<std::pair<int, int>, std::pair<uint32_t, uint32_t>> tuned_; // view size -> tile shape the autotuner chose
   uint64_t batchTunedKey_ = 0; // sizes_key of the batch autotune_views last tuned
-  DeviceArray target_, viewStats_;
+  DeviceArray target_;
   std::vector<std::unique_ptr<DeviceArray>> viewTargets_; // step_views' targets, one per view
-  PinnedArray staging_, next_, readback_;
+  PinnedArray staging_, next_;
+  // Written by the device: the last pass's counters and loss sums (and the last
+  // allocation-free render's, kStatusSlot bytes on), and each queued view's.
+  static constexpr size_t kStatusSlot = 64;
+  PinnedArray readback_, viewStats_;
 
   // The next step's target (the reference's prefetch, trainer.cpp:539-564):
   // one asynchronous host copy into pinned memory (next_) per prefetch, of the
