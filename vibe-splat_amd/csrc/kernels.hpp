@@ -106,6 +106,16 @@ void launch_radix_sort(hipStream_t stream, uint32_t *keys, uint32_t *values, uin
 void launch_fill_u32(hipStream_t stream, uint32_t *dst, uint64_t count, uint32_t value);
 // Two arrays cleared in one launch.
 void launch_clear_two(hipStream_t stream, uint32_t *a, uint64_t aCount, uint32_t *b, uint64_t bCount);
+// Up to kMaxCopies runs of words copied in one launch (to host memory that the
+// device writes to).
+constexpr uint32_t kMaxCopies = 8;
+struct WordCopies {
+  const uint32_t *from[kMaxCopies];
+  uint32_t *to[kMaxCopies];
+  uint32_t words[kMaxCopies];
+  uint32_t count;
+};
+void launch_copy_words(hipStream_t stream, const WordCopies &copies);
 // What ends a pass, in one small kernel: with adamState the step counted (one
 // more step taken, unless the pass was skipped), and with status the pass's
 // counters and loss sums (kViewStatusBytes) written to it, host memory that the

@@ -267,6 +267,25 @@ void launch_fill_u32(hipStream_t stream, uint32_t *dst, uint64_t count, uint32_t
   hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks), dim3(256), 0, stream, dst, count, value);
 }
 
+// blockIdx.y is the run; a run whose ends are 16-byte aligned goes four words at a time.
+__global__ __launch_bounds__(256) void copy_words_kernel(WordCopies c) {
+  const uint32_t *from = c.from[blockIdx.y];
+  uint32_t *to = c.to[blockIdx.y];
+  const uint32_t words = c.words[blockIdx.y], t = blockIdx.x * 256u + threadIdx.x, stride = gridDim.x * 256u;
+  const bool wide = ((reinterpret_cast<uintptr_t>(from) | reinterpret_cast<uintptr_t>(to)) & 15u) == 0u;
+  const uint32_t vec4 = wide ? words / 4u : 0u;
+  for (uint32_t i = t; i < vec4; i += stride) reinterpret_cast<uint4 *>(to)[i] = reinterpret_cast<const uint4 *>(from)[i];
+  for (uint32_t i = vec4 * 4u + t; i < words; i += stride) to[i] = from[i];
+}
+
+void launch_copy_words(hipStream_t stream, const WordCopies &copies) {
+  uint32_t most = 0;
+  for (uint32_t k = 0; k < copies.count; ++k) most = copies.words[k] > most ? copies.words[k] : most;
+  if (most == 0) return;
+  const uint32_t blocks = div_up(most, 1024) < 256 ? div_up(most, 1024) : 256;
+  hipLaunchKernelGGL(copy_words_kernel, dim3(blocks, copies.count), dim3(256), 0, stream, copies);
+}
+
 __global__ __launch_bounds__(256) void clear_two_kernel(uint32_t *__restrict__ a, uint64_t aCount, uint32_t *__restrict__ b, uint64_t bCount) {
   for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < aCount + bCount; i += gridDim.x * 256ull) {
     if (i < aCount) {

@@ -14,6 +14,7 @@
 #include "tiles.hpp"
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 
@@ -113,6 +114,114 @@ void PinnedArray::release() {
   bytes_ = 0;
 }
 
+Downloads::~Downloads() {
+  for (hipEvent_t e : landed_)
+    if (e != nullptr) (void)hipEventDestroy(e);
+}
+
+template <class Wanted> bool Downloads::run(hipStream_t stream, const std::vector<Segment> &segments, Wanted &&wanted) {
+  // The segments as one run of bytes, cut into chunks of a slot each: pieces of segments.
+  struct Piece {
+    Segment part;
+    size_t at; // in its slot
+  };
+  std::vector<std::vector<Piece>> chunks;
+  size_t total = 0;
+  for (const Segment &s : segments) {
+    for (size_t done = 0; done < s.bytes;) {
+      const size_t at = total % kChunk, take = std::min(kChunk - at, s.bytes - done);
+      if (at == 0) chunks.emplace_back();
+      chunks.back().push_back({{static_cast<uint8_t *>(s.to) + done, static_cast<const uint8_t *>(s.from) + done, take}, at});
+      done += take;
+      total += take;
+    }
+  }
+  const size_t n = chunks.size();
+  slots_.ensure(kChunk * std::min(std::max<size_t>(n, 1), kSlots));
+  for (size_t k = 0; k < std::min(n, kSlots); ++k)
+    if (landed_[k] == nullptr) check(hipEventCreateWithFlags(&landed_[k], hipEventDisableTiming), "hipEventCreate");
+  uint8_t *pinned = slots_.as<uint8_t>();
+  const auto fetch = [&](size_t k) {
+    WordCopies c{};
+    for (const Piece &p : chunks[k]) {
+      c.from[c.count] = static_cast<const uint32_t *>(p.part.from);
+      c.to[c.count] = reinterpret_cast<uint32_t *>(pinned + (k % kSlots) * kChunk + p.at);
+      c.words[c.count++] = static_cast<uint32_t>(p.part.bytes / 4);
+    }
+    launch_copy_words(stream, c);
+    check(hipEventRecord(landed_[k % kSlots], stream), "hipEventRecord");
+  };
+  const auto empty = [&](size_t k) {
+    for (const Piece &p : chunks[k]) std::memcpy(p.part.to, pinned + (k % kSlots) * kChunk + p.at, p.part.bytes);
+  };
+  // Chunks below `landed` are in their slots; a helper takes the next one and says when it has emptied the slot.
+  std::atomic<size_t> landed{0}, next{0};
+  std::vector<std::atomic<uint8_t>> emptied(n);
+  std::atomic<bool> stop{false};
+  std::vector<std::thread> helpers;
+  struct Join {
+    std::atomic<bool> &stop;
+    std::vector<std::thread> &threads;
+    ~Join() {
+      stop = true;
+      for (auto &t : threads) t.join();
+    }
+  } join{stop, helpers};
+  for (size_t k = 0; k < std::min(n, kSlots); ++k) fetch(k);
+  for (size_t h = 0; h < kHelpers && total >= kHelped; ++h) {
+    helpers.emplace_back([&] {
+      for (uint32_t spins = 0; !stop;) {
+        size_t k = next;
+        if (k >= n) return;
+        if (k >= landed) {
+          if (++spins < 4096) {
+            std::this_thread::yield();
+          } else {
+            std::this_thread::sleep_for(std::chrono::microseconds(50)); // a long pass is before the copy
+          }
+          continue;
+        }
+        if (!next.compare_exchange_weak(k, k + 1)) continue;
+        empty(k);
+        emptied[k] = 1;
+      }
+    });
+  }
+  bool copied = true;
+  size_t waited = 0; // chunks known to be emptied
+  for (size_t k = 0; k < n; ++k) {
+    check(hipEventSynchronize(landed_[k % kSlots]), "download");
+    if (k == 0 && !wanted()) {
+      copied = false;
+      break;
+    }
+    landed = k + 1;
+    if (helpers.empty()) {
+      empty(k);
+      if (k + kSlots < n) fetch(k + kSlots);
+    } else if (k + kSlots < n) {
+      for (; waited <= k; ++waited)
+        while (emptied[waited] == 0) std::this_thread::yield();
+      fetch(k + kSlots);
+    }
+  }
+  if (!copied || n == 0) {
+    check(hipStreamSynchronize(stream), "download"); // what was fetched is left in its slots
+    if (n == 0) copied = wanted();
+    return copied;
+  }
+  // The last chunk has landed, so the stream is through; the rest is emptied here too.
+  for (size_t k = next; !helpers.empty() && k < n; k = next) {
+    if (next.compare_exchange_weak(k, k + 1)) {
+      empty(k);
+      emptied[k] = 1;
+    }
+  }
+  for (; !helpers.empty() && waited < n; ++waited)
+    while (emptied[waited] == 0) std::this_thread::yield();
+  return true;
+}
+
 Trainer::Trainer(const vsplat_cloud &c, const vsplat_trainer_options &options) : options_(options) {
   if (c.count == 0) throw Error(VSPLAT_RUNTIME_ERROR, "nothing to train: the cloud is empty");
   if (c.sh_degree < 0 || c.sh_degree > 3) throw Error(VSPLAT_INVALID_ARGUMENT, "the SH degree must be 0 to 3");
@@ -140,6 +249,8 @@ Trainer::Trainer(const vsplat_cloud &c, const vsplat_trainer_options &options) :
   // Float atomics are the default on this GPU, as on any with them (trainer.cpp:181).
   fixedPoint_ = options.force_fixed_point != 0;
   check(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking), "hipStreamCreate");
+  check(hipStreamCreateWithFlags(&uploadStream_, hipStreamNonBlocking), "hipStreamCreate");
+  check(hipEventCreateWithFlags(&uploaded_, hipEventDisableTiming), "hipEventCreate");
   slots_.resize(kTimingSlots);
   for (auto &slot : slots_)
     for (auto &e : slot.events) check(hipEventCreate(&e), "hipEventCreate");
@@ -223,6 +334,11 @@ Trainer::~Trainer() {
   if (prefetchCopy_.valid()) prefetchCopy_.wait();
   release_captured();
   release_views();
+  if (uploadStream_ != nullptr) {
+    (void)hipStreamSynchronize(uploadStream_);
+    (void)hipStreamDestroy(uploadStream_);
+  }
+  if (uploaded_ != nullptr) (void)hipEventDestroy(uploaded_);
   if (batchStart_ != nullptr) (void)hipEventDestroy(batchStart_);
   if (batchRaster_ != nullptr) (void)hipEventDestroy(batchRaster_);
   for (auto &slot : slots_)
@@ -760,6 +876,7 @@ void Trainer::enqueue_loss(ViewBuffers &b, const ViewParams &v, const uint8_t *d
     launch_exposure(s, b.image.as<float4>(), b.exposed.as<float4>(), pixels, exposure_);
     seen = b.exposed.as<float4>();
   }
+  if (uploadPending_) check(hipStreamWaitEvent(s, uploaded_, 0), "hipStreamWaitEvent");
   const bool scoring = scoreShare_ > 0.0f;
   if (scoring) launch_fill_u32(s, b.errorMax.as<uint32_t>(), 1, 0u);
   launch_loss(s, seen, deviceTarget, v.width, v.height, options_.lambda_ssim, b.fields.as<float>(), b.adjoint.as<float4>(),
@@ -900,6 +1017,10 @@ void Trainer::reset_opacity(float maximum) {
 // (an overflow once: the caller clears the device's).
 vsplat_step_stats Trainer::read_stats(bool &overflow) {
   check(hipStreamSynchronize(stream_), "step");
+  return take_status(overflow);
+}
+
+vsplat_step_stats Trainer::take_status(bool &overflow) {
   uint32_t counters[kCounterWords];
   double sums[2];
   std::memcpy(counters, readback_.as<uint8_t>(), sizeof(counters));
@@ -938,7 +1059,11 @@ void Trainer::prefetch_target(const uint8_t *target, size_t bytes) {
   prefetchCopy_ = std::async(std::launch::async, [into, target, bytes] { std::memcpy(into, target, bytes); });
 }
 
+// The target into pinned memory, and from there to the device on the upload
+// stream: only the loss waits for it (enqueue_loss), so the transfer (75 us for
+// 1280x720) runs beside the projection and the sorts instead of before them.
 void Trainer::stage_target(const uint8_t *target, size_t bytes) {
+  settle_upload();
   if (prefetched_ == target && prefetchedBytes_ == bytes) {
     // Started during the previous step (trainer.cpp:572-576).
     wait_prefetch();
@@ -949,7 +1074,15 @@ void Trainer::stage_target(const uint8_t *target, size_t bytes) {
     std::memcpy(staging_.as<uint8_t>(), target, bytes);
   }
   target_.ensure(bytes);
-  check(hipMemcpyAsync(target_.as<uint8_t>(), staging_.as<uint8_t>(), bytes, hipMemcpyHostToDevice, stream_), "upload target");
+  check(hipMemcpyAsync(target_.as<uint8_t>(), staging_.as<uint8_t>(), bytes, hipMemcpyHostToDevice, uploadStream_), "upload target");
+  check(hipEventRecord(uploaded_, uploadStream_), "hipEventRecord");
+  uploadPending_ = true;
+}
+
+// Waits for an upload that no pass has been waited for with (a call that threw).
+void Trainer::settle_upload() {
+  if (uploadPending_) check(hipEventSynchronize(uploaded_), "upload");
+  uploadPending_ = false;
 }
 
 vsplat_step_stats Trainer::run(const vsplat_camera &camera, const uint8_t *target, size_t bytes, uint32_t mode,
@@ -963,7 +1096,10 @@ vsplat_step_stats Trainer::run(const vsplat_camera &camera, const uint8_t *targe
   dropoutNow_ = rates != nullptr ? shDropout_ : 0.0f;
   stage_target(target, bytes);
   if (next != nullptr && nextBytes > 0) prefetch_target(next, nextBytes);
-  if (needs_tuning(camera.width, camera.height)) autotune_tiles(camera, target_.as<uint8_t>(), 2);
+  if (needs_tuning(camera.width, camera.height)) {
+    settle_upload();
+    autotune_tiles(camera, target_.as<uint8_t>(), 2);
+  }
   const ViewParams v = view_params(camera);
   statisticsNext_ = true; // run() always adds to the densification statistics (trainer.cpp:600)
   // The pose gradient (trainer.cpp:455, 630-637), from the chain rule's pass.
@@ -988,6 +1124,7 @@ vsplat_step_stats Trainer::run(const vsplat_camera &camera, const uint8_t *targe
     grow_entries(b, stats.tile_entries);
   }
   drain_timing();
+  uploadPending_ = false; // the loss waited for it, and the stream is through
   if (exposing_) {
     // dL/d(transform): the workgroups' totals summed in double in order (trainer.cpp:620-628).
     const uint32_t groups = exposure_groups(static_cast<uint32_t>(camera.width) * static_cast<uint32_t>(camera.height));
@@ -1050,11 +1187,17 @@ void Trainer::render(const vsplat_camera &camera, float *out) {
   ensure_size(b, camera.width, camera.height);
   dropoutNow_ = 0.0f; // reports and evaluation see the whole model
   const ViewParams v = view_params(camera);
+  const size_t pixels = static_cast<size_t>(b.width) * static_cast<size_t>(b.height);
   for (int attempt = 0;; ++attempt) {
     enqueue_passes(b, v, nullptr, kModeRender, nullptr, false);
     finish_pass(b, false);
+    // The download is queued behind the passes; nothing reaches `out` if they did not fit.
+    vsplat_step_stats stats{};
     bool overflow = false;
-    const vsplat_step_stats stats = read_stats(overflow);
+    downloads_.run(stream_, {{out, b.image.as<float4>(), pixels * 16}}, [&] {
+      stats = take_status(overflow);
+      return !overflow;
+    });
     if (!overflow) break;
     launch_fill_u32(stream_, b.counters.as<uint32_t>() + kOverflow, 2, 0u); // overflow and skipped
     if (attempt > 0 && stats.tile_entries <= b.entryCapacity) throw Error(VSPLAT_DEVICE_ERROR, "tile entries overflowed twice");
@@ -1063,8 +1206,6 @@ void Trainer::render(const vsplat_camera &camera, float *out) {
   // As the reference's render uploads its camera, a curvature update now takes this view.
   lastView_ = v;
   lastViewIndex_ = 0;
-  const size_t pixels = static_cast<size_t>(b.width) * static_cast<size_t>(b.height);
-  check(hipMemcpy(out, b.image.as<float4>(), pixels * 16, hipMemcpyDeviceToHost), "download image");
 }
 
 // render() without allocating (vsplat_render_noalloc). The per-Gaussian,
@@ -1453,6 +1594,7 @@ void Trainer::release_captured() {
 void Trainer::capture_views(uint32_t n, const vsplat_camera *cameras, const uint8_t *const *targets, uint32_t mode,
                             const vsplat_learning_rates *rates) {
   release_captured();
+  settle_upload(); // a capture must not wait for an event from outside it
   if (options_.tile_shape == VSPLAT_TILES_AUTO && n > 0 && cameras != nullptr && targets != nullptr &&
       sizes_key(n, cameras) != batchTunedKey_) {
     autotune_views(n, cameras, targets, 2, nullptr, nullptr);
@@ -1519,16 +1661,27 @@ uint32_t Trainer::step_views(uint32_t n, const vsplat_camera *cameras, const uin
   }
   while (viewTargets_.size() < n) viewTargets_.push_back(std::make_unique<DeviceArray>());
   std::vector<const uint8_t *> device(n);
+  settle_upload();
+  size_t staged = 0;
+  for (uint32_t k = 0; k < n; ++k) staged += bytes[k];
+  viewStaging_.ensure(staged);
+  uint8_t *stage = viewStaging_.as<uint8_t>();
   for (uint32_t k = 0; k < n; ++k) {
     const size_t expected = static_cast<size_t>(cameras[k].width) * static_cast<size_t>(cameras[k].height) * 4;
     if (cameras[k].width <= 0 || cameras[k].height <= 0 || targets[k] == nullptr || bytes[k] != expected) {
       throw Error(VSPLAT_RUNTIME_ERROR, "a target image does not match its camera");
     }
     viewTargets_[k]->ensure(bytes[k]);
-    check(hipMemcpyAsync(viewTargets_[k]->as<uint8_t>(), targets[k], bytes[k], hipMemcpyHostToDevice, stream_), "upload target");
+    // Through pinned memory on the upload stream, as stage_target: only the losses wait.
+    std::memcpy(stage, targets[k], bytes[k]);
+    check(hipMemcpyAsync(viewTargets_[k]->as<uint8_t>(), stage, bytes[k], hipMemcpyHostToDevice, uploadStream_), "upload target");
+    stage += bytes[k];
     device[k] = viewTargets_[k]->as<uint8_t>();
   }
+  check(hipEventRecord(uploaded_, uploadStream_), "hipEventRecord");
+  uploadPending_ = true;
   if (options_.tile_shape == VSPLAT_TILES_AUTO && sizes_key(n, cameras) != batchTunedKey_) {
+    settle_upload();
     autotune_views(n, cameras, device.data(), 2, nullptr, nullptr);
   }
   std::vector<vsplat_step_stats> all(n);
@@ -1544,6 +1697,7 @@ uint32_t Trainer::step_views(uint32_t n, const vsplat_camera *cameras, const uin
     }
     if (attempt > 0 && !grew) throw Error(VSPLAT_DEVICE_ERROR, "tile entries overflowed twice");
   }
+  uploadPending_ = false; // every view's loss waited for it, and the batch is through
   if (stats != nullptr) std::copy(all.begin(), all.end(), stats);
   return n;
 }
@@ -1553,21 +1707,24 @@ void Trainer::gradients(float *positions, float *scales, float *rotations, float
   const size_t n = count_;
   float *out[5] = {positions, scales, rotations, opacities, sh};
   const size_t floats[5] = {n * 3, n * 3, n * 4, n, n * shFloats_};
-  for (int g = 0; g < 5; ++g) {
-    if (out[g] != nullptr) check(hipMemcpy(out[g], grad_[g].as<float>(), floats[g] * 4, hipMemcpyDeviceToHost), "download gradients");
-  }
+  std::vector<Downloads::Segment> segments;
+  for (int g = 0; g < 5; ++g)
+    if (out[g] != nullptr) segments.push_back({out[g], grad_[g].as<float>(), floats[g] * 4});
+  downloads_.run(stream_, segments, [] { return true; });
 }
 
 void Trainer::cloud(float *positions, float *scales, float *rotations, float *opacities, float *sh) const {
   const size_t n = count_;
-  check(hipStreamSynchronize(stream_), "cloud");
-  if (positions) check(hipMemcpy(positions, positions_.as<float>(), n * 12, hipMemcpyDeviceToHost), "download positions");
-  if (scales) check(hipMemcpy(scales, scales_.as<float>(), n * 12, hipMemcpyDeviceToHost), "download scales");
-  if (rotations) check(hipMemcpy(rotations, rotations_.as<float>(), n * 16, hipMemcpyDeviceToHost), "download rotations");
-  if (opacities) check(hipMemcpy(opacities, opacities_.as<float>(), n * 4, hipMemcpyDeviceToHost), "download opacities");
+  float *out[4] = {positions, scales, rotations, opacities};
+  const DeviceArray *from[4] = {&positions_, &scales_, &rotations_, &opacities_};
+  const size_t floats[4] = {3, 3, 4, 1};
+  std::vector<uint32_t> words(sh != nullptr ? n * shWords_ : 0);
+  std::vector<Downloads::Segment> segments;
+  for (int g = 0; g < 4; ++g)
+    if (out[g] != nullptr) segments.push_back({out[g], from[g]->as<float>(), n * floats[g] * 4});
+  if (sh != nullptr) segments.push_back({words.data(), shWordsBuf_.as<uint32_t>(), words.size() * 4});
+  downloads_.run(stream_, segments, [] { return true; });
   if (sh) {
-    std::vector<uint32_t> words(n * shWords_);
-    check(hipMemcpy(words.data(), shWordsBuf_.as<uint32_t>(), words.size() * 4, hipMemcpyDeviceToHost), "download SH");
     for (size_t i = 0; i < n; ++i) {
       const uint32_t *in = words.data() + i * shWords_;
       float *to = sh + i * shFloats_;
@@ -1582,8 +1739,7 @@ void Trainer::cloud(float *positions, float *scales, float *rotations, float *op
 }
 
 void Trainer::densify_stats(float *out) const {
-  check(hipStreamSynchronize(stream_), "densify stats");
-  check(hipMemcpy(out, stats_.as<float>(), static_cast<size_t>(count_) * 32, hipMemcpyDeviceToHost), "download stats");
+  downloads_.run(stream_, {{out, stats_.as<float>(), static_cast<size_t>(count_) * 32}}, [] { return true; });
 }
 
 // Trainer::apply_changes (trainer.cpp:749-787): the Gaussians replaced by a

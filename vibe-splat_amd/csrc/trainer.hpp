@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <future>
 #include <map>
 #include <memory>
@@ -79,6 +80,33 @@ public:
 private:
   void *ptr_ = nullptr;
   size_t bytes_ = 0;
+};
+
+// Copies from the device to ordinary host memory, through pinned memory that a
+// kernel fills slot by slot while host threads empty the slots. (hipMemcpy into
+// such memory copies each chunk on one thread before the next is fetched, and
+// fresh memory's page faults alone take that thread as long as the transfer.)
+class Downloads {
+public:
+  struct Segment { // a whole number of words each, at most kMaxCopies of them
+    void *to;
+    const void *from;
+    size_t bytes;
+  };
+  Downloads() = default;
+  Downloads(const Downloads &) = delete;
+  Downloads &operator=(const Downloads &) = delete;
+  ~Downloads();
+  // Copies the segments after the work queued on `stream`, and waits. When the
+  // work is through, `wanted` is asked: if false nothing is copied to the host.
+  template <class Wanted> bool run(hipStream_t stream, const std::vector<Segment> &segments, Wanted &&wanted);
+
+private:
+  static constexpr size_t kChunk = 1u << 20, kSlots = 12;
+  // Helper threads for a transfer of kHelped bytes and more; below, starting them costs what they save.
+  static constexpr size_t kHelpers = 3, kHelped = 3u << 20;
+  PinnedArray slots_;
+  hipEvent_t landed_[kSlots] = {};
 };
 
 // Everything one view's passes write: the per-Gaussian, per-pixel and
@@ -204,6 +232,7 @@ private:
   void fit_entries(ViewBuffers &b, uint64_t entries);
   uint64_t big_bit_words_for(uint64_t entries) const;
   void stage_target(const uint8_t *target, size_t bytes);
+  void settle_upload();
   // The passes up to the backward pass on b's stream, then (chain) the chain rule.
   void enqueue_passes(ViewBuffers &b, const ViewParams &view, const uint8_t *deviceTarget, uint32_t mode,
                       const vsplat_learning_rates *rates, bool timed, bool chain = true);
@@ -231,6 +260,7 @@ private:
   void drain_timing();
   void wait_prefetch();
   vsplat_step_stats read_stats(bool &overflow);
+  vsplat_step_stats take_status(bool &overflow);
 
   vsplat_trainer_options options_;
   uint32_t count_ = 0;
@@ -284,6 +314,13 @@ private:
   // allocation-free render's, kStatusSlot bytes on), and each queued view's.
   static constexpr size_t kStatusSlot = 64;
   PinnedArray readback_, viewStats_;
+  mutable Downloads downloads_;
+  // Targets go to the device on a stream of their own, beside the passes before
+  // the loss, which waits for uploaded_ while uploadPending_.
+  hipStream_t uploadStream_ = nullptr;
+  hipEvent_t uploaded_ = nullptr;
+  bool uploadPending_ = false;
+  PinnedArray viewStaging_; // step_views' targets
 
   // The next step's target (the reference's prefetch, trainer.cpp:539-564):
   // one asynchronous host copy into pinned memory (next_) per prefetch, of the

@@ -334,7 +334,7 @@ class Trainer:
 
     # --- the per-step surface
     def render(self, camera: Camera) -> np.ndarray:
-        out = np.zeros((camera.height * camera.width, 4), np.float32)
+        out = np.empty((camera.height * camera.width, 4), np.float32)
         cam = camera_to_c(camera)
         _raise(self._lib.vsplat_render(self._h, C.byref(cam), _p(out)), "render")
         return out
@@ -416,8 +416,8 @@ class Trainer:
     def gradients(self) -> Gradients:
         n = self.count
         coefficients = (self.sh_degree + 1) ** 2
-        g = Gradients(np.zeros((n, 3), np.float32), np.zeros((n, 3), np.float32), np.zeros((n, 4), np.float32),
-                      np.zeros(n, np.float32), np.zeros((n, coefficients, 3), np.float32))
+        g = Gradients(np.empty((n, 3), np.float32), np.empty((n, 3), np.float32), np.empty((n, 4), np.float32),
+                      np.empty(n, np.float32), np.empty((n, coefficients, 3), np.float32))
         _raise(self._lib.vsplat_get_gradients(self._h, _p(g.positions), _p(g.scales), _p(g.rotations), _p(g.opacities), _p(g.sh)),
                "gradients")
         return g
@@ -429,7 +429,7 @@ class Trainer:
         return c
 
     def densify_stats(self) -> np.ndarray:
-        out = np.zeros((self.count, 8), np.float32)
+        out = np.empty((self.count, 8), np.float32)
         _raise(self._lib.vsplat_get_densify_stats(self._h, _p(out)), "densify_stats")
         return out
 
