@@ -1,0 +1,58 @@
+"""The depth sort and the tile lists at the sizes where the counted passes (one
+launch each, tiles of 4096 keys, up to 2^18 keys) begin and end, for depths all
+different, all equal and mostly out of view: the keys sorted, equal keys in
+their first order, and each tile's entries in depth order."""
+import numpy as np
+import pytest
+
+from vsplat import fixtures as F
+import vsplat
+
+pytestmark = pytest.mark.gpu
+
+
+def _check_lists(t, stats):
+    keys, values = t.inspect("keys").astype(np.int64), t.inspect("values").astype(np.int64)
+    n = len(keys)
+    assert np.array_equal(np.sort(values), np.arange(n))
+    assert np.array_equal(np.lexsort((values, keys)), np.arange(n))  # sorted by key, equal keys by Gaussian
+    assert np.count_nonzero(keys != 0xFFFFFFFF) == stats.visible_splats
+    tiles, splats = t.inspect("entry_keys").astype(np.int64), t.inspect("entry_values").astype(np.int64)
+    assert len(tiles) == stats.tile_entries
+    rank = np.empty(n, np.int64)
+    rank[values] = np.arange(n)
+    assert np.array_equal(np.lexsort((rank[splats], tiles)), np.arange(len(tiles)))
+    ranges = t.inspect("ranges").astype(np.int64)
+    assert np.array_equal(ranges[:, 1] - ranges[:, 0], np.bincount(tiles, minlength=len(ranges)))
+    assert np.array_equal(np.bincount(splats, minlength=n), _counts(t, rank, stats))
+
+
+def _counts(t, rank, stats):
+    """Each Gaussian's entries, from the offsets in depth order."""
+    offsets = t.inspect("coverage").astype(np.int64)
+    counts = np.diff(np.append(offsets, stats.tile_entries))
+    return counts[rank]
+
+
+@pytest.mark.parametrize("scene", ["spread", "equal", "behind"])
+@pytest.mark.parametrize("count", [1, 2, 255, 4095, 4096, 4097, 8193, 70_000, 262_143, 262_144, 262_145])
+def test_depth_order(count, scene):
+    cloud = F.synthetic_cloud(count, 0, 11, log_scale=(-5.0, 0.5))
+    if scene == "equal":
+        cloud.positions[:, 2] = 0.25
+    if scene == "behind":
+        cloud.positions[count // 8:, 2] = -9.0
+    cam = F.look_at((0, 0, -3), (0, 0, 0), (0.0, -1.0, 0.0), 60.0, 130, 97)
+    with vsplat.Trainer(cloud) as t:
+        _check_lists(t, t.compute_gradients(cam, F.smooth_target(130, 97, 3)))
+
+
+@pytest.mark.parametrize("tiles", [vsplat.TILES_8X8, vsplat.TILES_16X16, vsplat.TILES_32X8, vsplat.TILES_32X32])
+@pytest.mark.parametrize("width,height", [(9, 7), (128, 128), (256, 256), (272, 256), (1000, 620), (2500, 1700)])
+def test_tile_lists(width, height, tiles):
+    """One to three passes over the tile bits, an odd number and an even one, with splats large enough for their own kernels."""
+    cloud = F.synthetic_cloud(3000, 0, 13, log_scale=(-4.0, 1.0))
+    cloud.scales[::500] = -0.5
+    cam = F.look_at((0, 0, -3), (0, 0, 0), (0.0, -1.0, 0.0), 60.0, width, height)
+    with vsplat.Trainer(cloud, vsplat.TrainerOptions(tile_shape=tiles)) as t:
+        _check_lists(t, t.compute_gradients(cam, F.smooth_target(width, height, 3)))

@@ -3,6 +3,7 @@
 // entries after the stable sort by tile (train_tile_ranges.comp:11-22). The
 // counts themselves come from the projection (project.hip).
 #include "device.hpp"
+#include "digit_count.hpp"
 #include "kernels.hpp"
 #include "blockscan.hpp"
 #include "tiles.hpp"
@@ -154,9 +155,21 @@ __device__ __forceinline__ void emit_small(const uint32_t *__restrict__ keys, co
                                            const Splat *__restrict__ splats, const TileRecord *__restrict__ records, uint32_t count,
                                            uint32_t gridW, TileShape shape, uint32_t width, uint32_t height, uint32_t tileBits,
                                            bool blockMasks, const uint32_t *__restrict__ offsets, uint32_t limit,
-                                           uint32_t *__restrict__ entryKeys, uint32_t *__restrict__ entryValues) {
+                                           uint32_t *__restrict__ entryKeys, uint32_t *__restrict__ entryValues,
+                                           uint32_t *__restrict__ entryCounts, uint32_t firstMask) {
   __shared__ EmitOwner owners[256]; // per wave: its small splats with candidates, packed
   __shared__ uint32_t flags[256];   // per wave: the walk's round marks
+  // The tile sort's first digits, counted for the kLocalTiles tiles of its keys
+  // from the workgroup's first entry on (its 256 splats' entries lie side by
+  // side but for the big splats between them), then added to the view's.
+  constexpr uint32_t kLocalTiles = 6;
+  __shared__ uint32_t local[kLocalTiles * 256];
+  uint32_t firstTile = 0;
+  if (entryCounts != nullptr) {
+    firstTile = offsets[blockIdx.x * blockDim.x] / kCountedTile;
+    for (uint32_t x = threadIdx.x; x < kLocalTiles * 256u; x += 256u) local[x] = 0u;
+    __syncthreads();
+  }
   const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x & ~63u;
   uint32_t candidates = 0, i = 0;
@@ -171,7 +184,6 @@ __device__ __forceinline__ void emit_small(const uint32_t *__restrict__ keys, co
   const uint64_t owning = __ballot(owner);
   const uint32_t end = wave_inclusive_sum(candidates, lane);
   const uint32_t total = __shfl(end, 63, 64);
-  if (total == 0) return; // nothing in this wave; no barrier follows
   const uint32_t start = end - candidates;
   if (owner) {
     const uint32_t boxWidth = rec.size & 0xFFFFu, tx0 = rec.origin & 0xFFFFu, ty0 = rec.origin >> 16;
@@ -191,6 +203,7 @@ __device__ __forceinline__ void emit_small(const uint32_t *__restrict__ keys, co
   for (uint32_t base = 0; base < total; base += 64) {
     const uint32_t k = walk_round(flags + wave, lane, base, owner, start, before);
     const uint32_t j = base + lane;
+    uint32_t at = limit, tile = 0;
     if (j < total) {
       const EmitOwner &o = owners[wave + k];
       const uint32_t local = j - o.start;
@@ -198,15 +211,29 @@ __device__ __forceinline__ void emit_small(const uint32_t *__restrict__ keys, co
       if (((mask >> local) & 1ull) != 0) {
         uint32_t tx, ty;
         box_tile(o, local, tx, ty);
-        const uint32_t at = o.offset + static_cast<uint32_t>(__popcll(mask & ((1ull << local) - 1ull)));
+        tile = ty * gridW + tx;
+        at = o.offset + static_cast<uint32_t>(__popcll(mask & ((1ull << local) - 1ull)));
         // The hits are the ones the projection counted, so at < limit; the test only guards the buffer.
         if (at < limit) {
           const uint32_t blocks = blockMasks ? block_mask(o.edges, tx, ty, o.tx0, o.ty0, o.last & 0xFFFFu, o.last >> 16, shape) : allBlocks;
-          entryKeys[at] = (ty * gridW + tx) | (blocks << tileBits);
+          entryKeys[at] = tile | (blocks << tileBits);
           entryValues[at] = o.gaussian;
         }
       }
     }
+    if (entryCounts != nullptr && at < limit) {
+      const uint32_t from = at / kCountedTile - firstTile;
+      if (from < kLocalTiles) {
+        atomicAdd(&local[from * 256u + (tile & firstMask)], 1u);
+      } else {
+        atomicAdd(&entryCounts[at / kCountedTile * kCountedStride + (tile & firstMask)], 1u);
+      }
+    }
+  }
+  if (entryCounts == nullptr) return;
+  __syncthreads();
+  for (uint32_t x = threadIdx.x; x < kLocalTiles * 256u; x += 256u) {
+    if (local[x] != 0u) atomicAdd(&entryCounts[(firstTile + x / 256u) * kCountedStride + (x & 255u)], local[x]);
   }
 }
 
@@ -220,7 +247,8 @@ __device__ __forceinline__ void emit_small(const uint32_t *__restrict__ keys, co
 __device__ __forceinline__ void emit_big(uint32_t block, uint32_t blocks, const Splat *__restrict__ splats,
                                          const TileRecord *__restrict__ records, const uint32_t *__restrict__ bigList, uint32_t listed,
                                          const uint64_t *__restrict__ bigBits, uint32_t gridW, TileShape shape, uint32_t tileBits,
-                                         uint32_t limit, uint32_t *__restrict__ entryKeys, uint32_t *__restrict__ entryValues) {
+                                         uint32_t limit, uint32_t *__restrict__ entryKeys, uint32_t *__restrict__ entryValues,
+                                         uint32_t *__restrict__ entryCounts, uint32_t firstMask) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t waves = blocks * 4u, wave = block * 4u + threadIdx.x / 64u;
   const uint32_t allBlocks = ((1u << ((shape.w >> 3) * (shape.h >> 3))) - 1u) << tileBits;
@@ -259,6 +287,7 @@ __device__ __forceinline__ void emit_big(uint32_t block, uint32_t blocks, const 
           entryKeys[at] = (ty * gridW + tx) | allBlocks;
           entryValues[at] = b.gaussian;
         }
+        if (entryCounts != nullptr) count_digit(entryCounts, at, (ty * gridW + tx) & firstMask, hit && at < limit);
         next += static_cast<uint32_t>(__popcll(mask));
         cursor.advance();
       }
@@ -274,15 +303,16 @@ __global__ __launch_bounds__(256) void bin_emit_kernel(const uint32_t *__restric
                                                        uint32_t tileBits, bool blockMasks, const uint32_t *__restrict__ offsets,
                                                        const uint32_t *__restrict__ bigList, const uint64_t *__restrict__ bigBits,
                                                        uint32_t smallBlocks, const uint32_t *counters, uint32_t *__restrict__ entryKeys,
-                                                       uint32_t *__restrict__ entryValues) {
+                                                       uint32_t *__restrict__ entryValues, uint32_t *__restrict__ entryCounts,
+                                                       uint32_t firstMask) {
   if (counters[kOverflow] != 0) return; // the same for every thread of the launch
   const uint32_t limit = counters[kEntriesUsed];
   if (blockIdx.x < smallBlocks) {
     emit_small(keys, values, splats, records, count, gridW, shape, width, height, tileBits, blockMasks, offsets, limit, entryKeys,
-               entryValues);
+               entryValues, entryCounts, firstMask);
   } else {
     emit_big(blockIdx.x - smallBlocks, gridDim.x - smallBlocks, splats, records, bigList, counters[kBigSplats], bigBits, gridW, shape,
-             tileBits, limit, entryKeys, entryValues);
+             tileBits, limit, entryKeys, entryValues, entryCounts, firstMask);
   }
 }
 
@@ -349,7 +379,7 @@ void launch_finish(hipStream_t stream, uint32_t *adamState, float beta1, float b
 void launch_bin_emit(hipStream_t stream, const uint32_t *keys, const uint32_t *values, const Splat *splats, const TileRecord *records,
                      uint32_t count, uint32_t gridW, uint32_t tileW, uint32_t tileH, uint32_t width, uint32_t height, uint32_t tileBits,
                      const uint32_t *offsets, const uint32_t *counters, const uint32_t *bigList, const uint64_t *bigBits,
-                     uint32_t *entryKeys, uint32_t *entryValues) {
+                     uint32_t *entryKeys, uint32_t *entryValues, uint32_t *entryCounts) {
   if (count == 0) return;
   // Blocks are marked per entry for tiles of 16 blocks (32x32), where a block
   // skipping the entries that miss it saves more raster time than marking
@@ -358,7 +388,7 @@ void launch_bin_emit(hipStream_t stream, const uint32_t *keys, const uint32_t *v
   const uint32_t smallBlocks = (count + 255) / 256;
   hipLaunchKernelGGL(bin_emit_kernel, dim3(smallBlocks + big_splat_blocks(count)), dim3(256), 0, stream, keys, values, splats, records, count,
                      gridW, TileShape{tileW, tileH}, width, height, tileBits, blockMasks, offsets, bigList, bigBits, smallBlocks, counters,
-                     entryKeys, entryValues);
+                     entryKeys, entryValues, entryCounts, radix_first_mask(tileBits));
 }
 
 void launch_tile_ranges(hipStream_t stream, const uint32_t *entryKeys, const uint32_t *counters, uint32_t capacity, uint32_t tileBits,

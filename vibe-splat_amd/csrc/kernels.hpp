@@ -90,22 +90,36 @@ constexpr uint32_t kBigCount = 0x80000000u;
 // counted by their own kernel. bigList holds one word per Gaussian; bigBits
 // (bitCapacity words) receives their reached-tile bits, one word per 64
 // candidates, for the list pass (a splat that finds no room keeps none).
+// depthCounts, when set, receives the depth sort's first digits.
 void launch_project(hipStream_t stream, const float *positions, const float *scales, const float *rotations, const float *opacities,
                     const uint32_t *shWords, const float *filter3d, const ViewParams &view, bool mipFilter2d, float shDropout,
                     uint32_t shRetained, uint32_t shSeed, uint32_t gridW, uint32_t gridH, Splat *splats, uint32_t *keys,
                     uint32_t *values, uint32_t *tileCount, TileRecord *records, uint32_t *counters, uint32_t *bigList,
-                    uint64_t *bigBits, uint32_t bitCapacity);
+                    uint64_t *bigBits, uint32_t bitCapacity, uint32_t *depthCounts);
 
 // Scratch for launch_radix_sort over up to capacity keys.
 size_t radix_sort_scratch_words(uint64_t capacity);
 // Whether a sort by this many bits takes an odd number of passes: its input is
 // then read from tmpKeys and tmpValues, so that the result ends in keys and values.
 bool radix_sort_from_tmp(uint32_t bits);
+// Sorts of at most this many keys take their digit counts from the keys' writers
+// (digit_count.hpp): kCountedStride words per tile of kCountedTile keys and pass,
+// radix_count_words in all (0 for larger sorts), cleared beforehand; the writer
+// counts the first pass's digits, the bits under radix_first_mask.
+constexpr uint32_t kCountedSortKeys = 1u << 18, kCountedTile = 4096, kCountedStride = 256;
+size_t radix_count_words(uint64_t capacity, uint32_t bits);
+uint32_t radix_first_mask(uint32_t bits);
 void launch_radix_sort(hipStream_t stream, uint32_t *keys, uint32_t *values, uint32_t *tmpKeys, uint32_t *tmpValues,
-                       const uint32_t *countDev, uint32_t capacity, uint32_t bits, uint32_t *scratch);
+                       const uint32_t *countDev, uint32_t capacity, uint32_t bits, uint32_t *scratch, uint32_t *counts);
 void launch_fill_u32(hipStream_t stream, uint32_t *dst, uint64_t count, uint32_t value);
-// Two arrays cleared in one launch.
-void launch_clear_two(hipStream_t stream, uint32_t *a, uint64_t aCount, uint32_t *b, uint64_t bCount);
+// Up to kMaxClears arrays cleared in one launch.
+constexpr uint32_t kMaxClears = 4;
+struct WordClears {
+  uint32_t *to[kMaxClears];
+  uint32_t words[kMaxClears];
+  uint32_t count;
+};
+void launch_clear_words(hipStream_t stream, const WordClears &clears);
 // Up to kMaxCopies runs of words copied in one launch (to host memory that the
 // device writes to).
 constexpr uint32_t kMaxCopies = 8;
@@ -158,10 +172,11 @@ void launch_gather_views(hipStream_t stream, const ViewStatus &views, uint8_t *s
 // The tile entries (keys: the tile in the low tileBits bits, above them the
 // tile's 8x8 blocks the splat reaches, marked for 32x32 tiles and all set for
 // the others; values: the Gaussian), for a view of width x height pixels.
+// entryCounts, when set, receives the tile sort's first digits.
 void launch_bin_emit(hipStream_t stream, const uint32_t *keys, const uint32_t *values, const Splat *splats, const TileRecord *records,
                      uint32_t count, uint32_t gridW, uint32_t tileW, uint32_t tileH, uint32_t width, uint32_t height, uint32_t tileBits,
                      const uint32_t *offsets, const uint32_t *counters, const uint32_t *bigList, const uint64_t *bigBits,
-                     uint32_t *entryKeys, uint32_t *entryValues);
+                     uint32_t *entryKeys, uint32_t *entryValues, uint32_t *entryCounts);
 void launch_tile_ranges(hipStream_t stream, const uint32_t *entryKeys, const uint32_t *counters, uint32_t capacity, uint32_t tileBits,
                         uint2 *ranges);
 

@@ -9,6 +9,7 @@
 // still in registers, by the wave's shared walk over candidate tiles
 // (tiles.hpp); the bits it finds are kept for the list pass.
 #include "device.hpp"
+#include "digit_count.hpp"
 #include "kernels.hpp"
 #include "tiles.hpp"
 
@@ -189,7 +190,8 @@ __global__ __launch_bounds__(256) void project_kernel(const float *__restrict__ 
                                                       ViewParams c, ProjectOptions opt, uint32_t gridW, uint32_t gridH,
                                                       Splat *__restrict__ splats, uint32_t *__restrict__ keys,
                                                       uint32_t *__restrict__ values, uint32_t *__restrict__ tileCount,
-                                                      TileRecord *__restrict__ records, uint32_t *counters, uint32_t *__restrict__ bigList) {
+                                                      TileRecord *__restrict__ records, uint32_t *counters, uint32_t *__restrict__ bigList,
+                                                      uint32_t *__restrict__ depthCounts) {
   // The block's SH words, staged with coalesced loads; afterwards the walk's owners.
   __shared__ uint32_t stage[kProjectThreads * kMaxShWords];
   __shared__ uint32_t flags[kProjectThreads]; // per wave: the walk's round marks
@@ -240,6 +242,7 @@ __global__ __launch_bounds__(256) void project_kernel(const float *__restrict__ 
   Splat s{};
   uint32_t key = kInvisible;
   const bool visible = i < c.count && project_one<Degree, Format>(i, g, stage + threadIdx.x * c.shWords, c, opt, s, key);
+  if (depthCounts != nullptr) count_digit(depthCounts, i, key & 0xFFu, i < c.count);
   if (i < c.count) {
     keys[i] = key;
     values[i] = i;
@@ -374,13 +377,14 @@ void launch_project(hipStream_t stream, const float *positions, const float *sca
                     const uint32_t *shWords, const float *filter3d, const ViewParams &view, bool mipFilter2d, float shDropout,
                     uint32_t shRetained, uint32_t shSeed, uint32_t gridW, uint32_t gridH, Splat *splats, uint32_t *keys,
                     uint32_t *values, uint32_t *tileCount, TileRecord *records, uint32_t *counters, uint32_t *bigList,
-                    uint64_t *bigBits, uint32_t bitCapacity) {
+                    uint64_t *bigBits, uint32_t bitCapacity, uint32_t *depthCounts) {
   if (view.count == 0) return;
   const ProjectOptions opt{mipFilter2d ? 1u : 0u, shDropout, shRetained, shSeed};
   const dim3 grid((view.count + 255) / 256), block(256);
 #define VSPLAT_PROJECT(D, F)                                                                                                       \
   hipLaunchKernelGGL((project_kernel<D, F>), grid, block, 0, stream, positions, scales, rotations, opacities, shWords, filter3d,    \
-                     view, opt, gridW, gridH, splats, keys, values, tileCount, records, counters, bigList)
+                     view, opt, gridW, gridH, splats, keys, values, tileCount, records, counters, bigList,     \
+                     depthCounts)
 #define VSPLAT_PROJECT_DEGREE(F)                                                                                                   \
   switch (view.shDegree) {                                                                                                         \
   case 0: VSPLAT_PROJECT(0, F); break;                                                                                             \

@@ -21,9 +21,21 @@
 //
 // Counts may live in device memory (the tile entries are only known on the
 // device): grids are sized for the capacity and tiles past the count exit.
+//
+// Up to kCountedSortKeys keys the same passes take one launch each
+// (radix_pass_kernel): whoever writes the keys also counts each pass's digits per
+// tile of 4096 keys, with atomics (digit_count.hpp), the first pass's as the keys
+// are made and every later one's as the pass before stores them, and a tile sums
+// the tiles' counts itself. At these sizes a launch's own 4 us is most of a pass:
+// the kernels of the depth sort took 66 us for 100k keys in 12 launches and take
+// 46 in 4, 61 and 41 for 30k. Past it every tile sums too many tiles' counts, one
+// after another, and the three-launch passes are the faster ones.
 #include "device.hpp"
 #include "kernels.hpp"
 #include "blockscan.hpp"
+#include "digit_count.hpp"
+
+#include <utility>
 
 namespace vsplat {
 
@@ -184,7 +196,161 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(const uint3
   }
 }
 
+constexpr uint32_t kPassThreads = 512, kPassPerThread = kCountedTile / kPassThreads;
+
+// One whole pass over a tile of kCountedTile keys: `counts` holds every tile's
+// digits (kCountedStride words a tile), nextCounts receives those of the next
+// pass, whose digit is the bits from nextShift under nextMask (none: the last pass).
+template <uint32_t Bits>
+__global__ __launch_bounds__(kPassThreads) void radix_pass_kernel(const uint32_t *__restrict__ keysIn, const uint32_t *__restrict__ valsIn,
+                                                                  uint32_t *__restrict__ keysOut, uint32_t *__restrict__ valsOut,
+                                                                  const uint32_t *countDev, uint32_t countHost, uint32_t shift,
+                                                                  const uint32_t *__restrict__ counts, uint32_t nextShift, uint32_t nextMask,
+                                                                  uint32_t *__restrict__ nextCounts) {
+  constexpr uint32_t kRadix = 1u << Bits, kWaves = kPassThreads / 64, kGroups = kPassThreads / kRadix;
+  constexpr uint32_t kWaveKeys = kCountedTile / kWaves; // consecutive keys per wave
+  __shared__ uint32_t digitBase[kRadix]; // the digit's global start for this tile, less its start within the tile
+  __shared__ uint32_t waveCount[kWaves][kRadix];
+  __shared__ uint32_t waveTotals[kWaves];
+  __shared__ uint32_t sorted[2 * kCountedTile];
+  uint32_t *const sortedKeys = sorted, *const sortedValues = sorted + kCountedTile;
+  const uint32_t count = count_of(countDev, countHost);
+  const uint32_t tileStart = blockIdx.x * kCountedTile;
+  if (tileStart >= count) return; // the same for the whole workgroup
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+
+  // The tile's keys, in flight while the counts are summed.
+  uint32_t key[kPassPerThread], val[kPassPerThread], rank[kPassPerThread];
+  const uint32_t first = tileStart + wave * kWaveKeys + lane;
+#pragma unroll
+  for (uint32_t r = 0; r < kPassPerThread; ++r) {
+    const uint32_t i = first + r * 64;
+    key[r] = i < count ? keysIn[i] : 0u;
+    val[r] = i < count ? valsIn[i] : 0u;
+  }
+  // Each digit's keys in the tiles before this one and in all, kGroups threads a
+  // digit (their partial sums meet in sortedKeys, which is not in use yet).
+  {
+    const uint32_t tiles = (count + kCountedTile - 1u) / kCountedTile, d = threadIdx.x % kRadix;
+    uint32_t before = 0, all = 0;
+#pragma unroll 8
+    for (uint32_t t = threadIdx.x / kRadix; t < tiles; t += kGroups) {
+      const uint32_t c = counts[t * kCountedStride + d];
+      before += t < blockIdx.x ? c : 0u;
+      all += c;
+    }
+    sortedKeys[threadIdx.x] = before;
+    sortedKeys[kPassThreads + threadIdx.x] = all;
+  }
+  for (uint32_t x = threadIdx.x; x < kWaves * kRadix; x += kPassThreads) (&waveCount[0][0])[x] = 0;
+  __syncthreads();
+  uint32_t before = 0, total = 0;
+  if (threadIdx.x < kRadix) {
+#pragma unroll 4
+    for (uint32_t g = 0; g < kGroups; ++g) {
+      before += sortedKeys[g * kRadix + threadIdx.x];
+      total += sortedKeys[kPassThreads + g * kRadix + threadIdx.x];
+    }
+  }
+  uint32_t start;
+  block_exclusive_sum(total, start, waveTotals);
+  if (threadIdx.x < kRadix) digitBase[threadIdx.x] = start + before;
+
+  // Rank within the wave's keys, in order.
+  const uint64_t below = (uint64_t{1} << lane) - 1u;
+#pragma unroll
+  for (uint32_t r = 0; r < kPassPerThread; ++r) {
+    const bool valid = first + r * 64 < count;
+    const uint32_t digit = (key[r] >> shift) & (kRadix - 1u);
+    uint64_t same = __ballot(valid);
+#pragma unroll
+    for (uint32_t b = 0; b < Bits; ++b) {
+      const uint64_t ones = __ballot((digit >> b) & 1u);
+      same &= ((digit >> b) & 1u) ? ones : ~ones;
+    }
+    const uint32_t lower = static_cast<uint32_t>(__popcll(same & below));
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t prior = waveCount[wave][digit];
+    rank[r] = prior + lower;
+    __builtin_amdgcn_wave_barrier();
+    if (valid && lower == 0) waveCount[wave][digit] = prior + static_cast<uint32_t>(__popcll(same));
+  }
+  __syncthreads();
+  {
+    const uint32_t d = threadIdx.x;
+    uint32_t tileCount = 0;
+    if (d < kRadix) {
+#pragma unroll
+      for (uint32_t w = 0; w < kWaves; ++w) tileCount += waveCount[w][d];
+    }
+    uint32_t localStart;
+    block_exclusive_sum(tileCount, localStart, waveTotals);
+    if (d < kRadix) {
+      digitBase[d] -= localStart;
+      uint32_t running = localStart;
+#pragma unroll
+      for (uint32_t w = 0; w < kWaves; ++w) {
+        const uint32_t c = waveCount[w][d];
+        waveCount[w][d] = running;
+        running += c;
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = 0; r < kPassPerThread; ++r) {
+    if (first + r * 64 < count) {
+      const uint32_t at = waveCount[wave][(key[r] >> shift) & (kRadix - 1u)] + rank[r];
+      sortedKeys[at] = key[r];
+      sortedValues[at] = val[r];
+    }
+  }
+  __syncthreads();
+  const uint32_t inTile = count - tileStart < kCountedTile ? count - tileStart : kCountedTile;
+  uint32_t slot[kPassPerThread]; // the counter of the next pass that the key adds to
+#pragma unroll
+  for (uint32_t r = 0; r < kPassPerThread; ++r) {
+    const uint32_t j = r * kPassThreads + threadIdx.x;
+    if (j < inTile) {
+      const uint32_t k = sortedKeys[j];
+      const uint32_t dst = digitBase[(k >> shift) & (kRadix - 1u)] + j;
+      keysOut[dst] = k;
+      valsOut[dst] = sortedValues[j];
+      slot[r] = (dst / kCountedTile) * (nextMask + 1u) + ((k >> nextShift) & nextMask);
+    }
+  }
+  if (nextMask == 0u) return; // the last pass (uniform)
+  // The next pass's digits by destination tile: counted in LDS, two 16-bit
+  // counters a word (a tile holds 4096 keys), then added to the view's.
+  uint32_t *const tally = sortedKeys;
+  static_assert(kCountedSortKeys / kCountedTile * kCountedStride / 2 <= 2 * kCountedTile, "the tally fits the sorted keys and values");
+  const uint32_t words = ((count + kCountedTile - 1u) / kCountedTile * (nextMask + 1u) + 1u) / 2u;
+  __syncthreads();
+  for (uint32_t x = threadIdx.x; x < words; x += kPassThreads) tally[x] = 0u;
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = 0; r < kPassPerThread; ++r) {
+    if (r * kPassThreads + threadIdx.x < inTile) atomicAdd(&tally[slot[r] / 2u], (slot[r] & 1u) ? 0x10000u : 1u);
+  }
+  __syncthreads();
+  for (uint32_t x = threadIdx.x; x < words; x += kPassThreads) {
+    const uint32_t two = tally[x];
+#pragma unroll
+    for (uint32_t h = 0; h < 2; ++h) {
+      const uint32_t n = h == 0 ? two & 0xFFFFu : two >> 16, at = 2u * x + h;
+      if (n != 0u) atomicAdd(&nextCounts[at / (nextMask + 1u) * kCountedStride + (at & nextMask)], n);
+    }
+  }
+}
+
 uint32_t div_up(uint64_t a, uint32_t b) { return static_cast<uint32_t>((a + b - 1) / b); }
+
+template <uint32_t Bits>
+void counted_pass(hipStream_t stream, const uint32_t *kIn, const uint32_t *vIn, uint32_t *kOut, uint32_t *vOut, const uint32_t *countDev,
+                  uint32_t capacity, uint32_t shift, const uint32_t *counts, uint32_t nextShift, uint32_t nextMask, uint32_t *nextCounts) {
+  hipLaunchKernelGGL(radix_pass_kernel<Bits>, dim3(div_up(capacity, kCountedTile)), dim3(kPassThreads), 0, stream, kIn, vIn, kOut, vOut,
+                     countDev, capacity, shift, counts, nextShift, nextMask, nextCounts);
+}
 
 template <uint32_t Bits, uint32_t PerThread>
 void sort_pass(hipStream_t stream, const uint32_t *kIn, const uint32_t *vIn, uint32_t *kOut, uint32_t *vOut, const uint32_t *countDev,
@@ -216,40 +382,56 @@ size_t radix_sort_scratch_words(uint64_t capacity) {
   return 256 + static_cast<size_t>(div_up(capacity, kSortThreads * kSortPerThreadSmall)) * 256u;
 }
 
+size_t radix_count_words(uint64_t capacity, uint32_t bits) {
+  if (capacity > kCountedSortKeys) return 0;
+  return static_cast<size_t>(div_up(bits, 8)) * div_up(capacity, kCountedTile) * kCountedStride;
+}
+uint32_t radix_first_mask(uint32_t bits) { return (1u << div_up(bits, div_up(bits, 8))) - 1u; }
+
 bool radix_sort_from_tmp(uint32_t bits) { return div_up(bits, 8) % 2 != 0; }
 
 // Sorts (keys, values) stably by the low `bits` bits of the keys (1 <= bits <=
 // 32), in ceil(bits / 8) passes of equal width. The result ends in keys/values;
 // tmpKeys/tmpValues are the other half of each pass, and hold the input when the
 // number of passes is odd (radix_sort_from_tmp), so that nothing is copied.
-// countDev, when given, holds the element count (at most capacity).
+// countDev, when given, holds the element count (at most capacity). counts: the
+// first pass's digits as the keys' writer counted them, the other passes' words
+// zero (radix_count_words of them; null where that is 0).
 void launch_radix_sort(hipStream_t stream, uint32_t *keys, uint32_t *values, uint32_t *tmpKeys, uint32_t *tmpValues,
-                       const uint32_t *countDev, uint32_t capacity, uint32_t bits, uint32_t *scratch) {
+                       const uint32_t *countDev, uint32_t capacity, uint32_t bits, uint32_t *scratch, uint32_t *counts) {
   if (capacity == 0 || bits == 0) return;
   const uint32_t passes = div_up(bits, 8);
   const uint32_t digit = div_up(bits, passes); // even split, at most 8 bits a pass
-  const bool odd = radix_sort_from_tmp(bits);
+  const bool odd = radix_sort_from_tmp(bits), counted = radix_count_words(capacity, bits) != 0;
+  const size_t passCounts = static_cast<size_t>(div_up(capacity, kCountedTile)) * kCountedStride;
   uint32_t *srcK = odd ? tmpKeys : keys, *srcV = odd ? tmpValues : values, *dstK = odd ? keys : tmpKeys, *dstV = odd ? values : tmpValues;
   for (uint32_t p = 0; p < passes; ++p) {
     // The last pass takes the bits that are left, so that no bit above `bits`
     // (which may carry other data) takes part in the order.
-    const uint32_t shift = p * digit;
+    const uint32_t shift = p * digit, next = shift + digit;
+    const uint32_t nextBits = next >= bits ? 0u : (digit < bits - next ? digit : bits - next);
+    uint32_t *mine = counted ? counts + p * passCounts : nullptr;
+#define VSPLAT_SORT_PASS(BITS)                                                                                                     \
+  case BITS:                                                                                                                       \
+    if (counted) {                                                                                                                 \
+      counted_pass<BITS>(stream, srcK, srcV, dstK, dstV, countDev, capacity, shift, mine, next, (1u << nextBits) - 1u, mine + passCounts); \
+    } else {                                                                                                                       \
+      sort_pass<BITS>(stream, srcK, srcV, dstK, dstV, countDev, capacity, shift, scratch);                                         \
+    }                                                                                                                              \
+    break;
     switch (digit < bits - shift ? digit : bits - shift) {
-    case 1: sort_pass<1>(stream, srcK, srcV, dstK, dstV, countDev, capacity, shift, scratch); break;
-    case 2: sort_pass<2>(stream, srcK, srcV, dstK, dstV, countDev, capacity, shift, scratch); break;
-    case 3: sort_pass<3>(stream, srcK, srcV, dstK, dstV, countDev, capacity, shift, scratch); break;
-    case 4: sort_pass<4>(stream, srcK, srcV, dstK, dstV, countDev, capacity, shift, scratch); break;
-    case 5: sort_pass<5>(stream, srcK, srcV, dstK, dstV, countDev, capacity, shift, scratch); break;
-    case 6: sort_pass<6>(stream, srcK, srcV, dstK, dstV, countDev, capacity, shift, scratch); break;
-    case 7: sort_pass<7>(stream, srcK, srcV, dstK, dstV, countDev, capacity, shift, scratch); break;
-    default: sort_pass<8>(stream, srcK, srcV, dstK, dstV, countDev, capacity, shift, scratch); break;
+      VSPLAT_SORT_PASS(1)
+      VSPLAT_SORT_PASS(2)
+      VSPLAT_SORT_PASS(3)
+      VSPLAT_SORT_PASS(4)
+      VSPLAT_SORT_PASS(5)
+      VSPLAT_SORT_PASS(6)
+      VSPLAT_SORT_PASS(7)
+      VSPLAT_SORT_PASS(8)
     }
-    uint32_t *t = srcK;
-    srcK = dstK;
-    dstK = t;
-    t = srcV;
-    srcV = dstV;
-    dstV = t;
+#undef VSPLAT_SORT_PASS
+    std::swap(srcK, dstK);
+    std::swap(srcV, dstV);
   }
 }
 
@@ -286,21 +468,18 @@ void launch_copy_words(hipStream_t stream, const WordCopies &copies) {
   hipLaunchKernelGGL(copy_words_kernel, dim3(blocks, copies.count), dim3(256), 0, stream, copies);
 }
 
-__global__ __launch_bounds__(256) void clear_two_kernel(uint32_t *__restrict__ a, uint64_t aCount, uint32_t *__restrict__ b, uint64_t bCount) {
-  for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < aCount + bCount; i += gridDim.x * 256ull) {
-    if (i < aCount) {
-      a[i] = 0u;
-    } else {
-      b[i - aCount] = 0u;
-    }
-  }
+// blockIdx.y is the run.
+__global__ __launch_bounds__(256) void clear_words_kernel(WordClears c) {
+  uint32_t *to = c.to[blockIdx.y];
+  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < c.words[blockIdx.y]; i += gridDim.x * 256u) to[i] = 0u;
 }
 
-void launch_clear_two(hipStream_t stream, uint32_t *a, uint64_t aCount, uint32_t *b, uint64_t bCount) {
-  const uint64_t blocks64 = (aCount + bCount + 255) / 256;
-  if (blocks64 == 0) return;
-  hipLaunchKernelGGL(clear_two_kernel, dim3(blocks64 < 1024 ? static_cast<uint32_t>(blocks64) : 1024u), dim3(256), 0, stream, a, aCount, b,
-                     bCount);
+void launch_clear_words(hipStream_t stream, const WordClears &clears) {
+  uint32_t most = 0;
+  for (uint32_t k = 0; k < clears.count; ++k) most = clears.words[k] > most ? clears.words[k] : most;
+  if (most == 0) return;
+  const uint32_t blocks = div_up(most, 1024) < 256 ? div_up(most, 1024) : 256;
+  hipLaunchKernelGGL(clear_words_kernel, dim3(blocks, clears.count), dim3(256), 0, stream, clears);
 }
 
 } // namespace vsplat

@@ -80,6 +80,9 @@ float half_to_float(uint32_t h) {
 
 uint64_t div_up(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 
+// The most words of digit counts a tile sort takes: 24-bit tiles in three passes.
+const size_t kEntryCountWords = radix_count_words(kCountedSortKeys, 24);
+
 // The big splats' bit words a view keeps room for: one per Gaussian and one per
 // 16 tile entries (boxes with up to four candidates per listed entry keep
 // their bits; the rest are tested again when listed).
@@ -379,6 +382,7 @@ ViewBuffers &Trainer::view_buffers(size_t k) {
     }
     v->scanScratch.ensure(coverage_scan_words(static_cast<uint32_t>(n)) * 4);
     v->sortScratch.ensure(radix_sort_scratch_words(n) * 4);
+    v->sortCounts.ensure((radix_count_words(n, 32) + kEntryCountWords) * 4);
     v->counters.ensure(kCounterWords * 4);
     launch_fill_u32(v->stream, v->counters.as<uint32_t>(), kCounterWords, 0u);
     v->sums.ensure(2 * sizeof(double));
@@ -827,16 +831,21 @@ ViewParams Trainer::with_tiles(const ViewBuffers &b, const ViewParams &view) con
 void Trainer::enqueue_lists(ViewBuffers &b, const ViewParams &v, uint32_t mode, bool marks) {
   hipStream_t s = b.stream;
   uint32_t *counters = b.counters.as<uint32_t>();
-  // The counters (not the sticky overflow word) and the tiles' ranges.
-  launch_clear_two(s, counters, kClearedPerPass, b.ranges.as<uint32_t>(), static_cast<uint64_t>(b.tiles) * 2);
+  // The counters (not the sticky overflow word), the tiles' ranges and the sorts' digit counts.
+  const size_t depthWords = radix_count_words(count_, 32), entryWords = radix_count_words(b.entryCapacity, b.tileBits);
+  uint32_t *depthCounts = depthWords != 0 ? b.sortCounts.as<uint32_t>() : nullptr;
+  uint32_t *entryCounts = entryWords != 0 ? b.sortCounts.as<uint32_t>() + depthWords : nullptr;
+  launch_clear_words(s, WordClears{{counters, b.ranges.as<uint32_t>(), b.sortCounts.as<uint32_t>()},
+                                   {kClearedPerPass, b.tiles * 2u, static_cast<uint32_t>(depthWords + entryWords)},
+                                   3});
   launch_project(s, positions_.as<float>(), scales_.as<float>(), rotations_.as<float>(), opacities_.as<float>(),
                  shWordsBuf_.as<uint32_t>(), filterSet_ ? filter3d_.as<float>() : nullptr, v, options_.mip_filter_2d != 0, dropoutNow_,
                  shRetained_, shSeed_, b.gridW, b.gridH, b.splats.as<Splat>(), b.keys.as<uint32_t>(), b.values.as<uint32_t>(),
                  b.tileCount.as<uint32_t>(), b.tileRecords.as<TileRecord>(), counters, b.bigList.as<uint32_t>(),
-                 b.bigBits.as<uint64_t>(), big_bit_words(b));
+                 b.bigBits.as<uint64_t>(), big_bit_words(b), depthCounts);
   if (marks) mark("project");
   launch_radix_sort(s, b.keys.as<uint32_t>(), b.values.as<uint32_t>(), b.tmpKeys.as<uint32_t>(), b.tmpValues.as<uint32_t>(), nullptr, count_,
-                    32, b.sortScratch.as<uint32_t>());
+                    32, b.sortScratch.as<uint32_t>(), depthCounts);
   if (marks) mark("depth sort");
   launch_coverage_scan(s, b.keys.as<uint32_t>(), b.values.as<uint32_t>(), b.tileCount.as<uint32_t>(), count_,
                        b.tileRecords.as<TileRecord>(), b.coverage.as<uint32_t>(), counters, static_cast<uint32_t>(b.entryCapacity), mode == kModeStep, b.scanScratch.as<uint32_t>());
@@ -846,9 +855,11 @@ void Trainer::enqueue_lists(ViewBuffers &b, const ViewParams &v, uint32_t mode, 
     launch_bin_emit(s, b.keys.as<uint32_t>(), b.values.as<uint32_t>(), b.splats.as<Splat>(), b.tileRecords.as<TileRecord>(), count_, b.gridW,
                     b.tileW, b.tileH, static_cast<uint32_t>(b.width), static_cast<uint32_t>(b.height), b.tileBits,
                     b.coverage.as<uint32_t>(), counters, b.bigList.as<uint32_t>(), b.bigBits.as<uint64_t>(),
-                    (fromTmp ? b.tmpEntryKeys : b.entryKeys).as<uint32_t>(), (fromTmp ? b.tmpEntryValues : b.entryValues).as<uint32_t>());
+                    (fromTmp ? b.tmpEntryKeys : b.entryKeys).as<uint32_t>(), (fromTmp ? b.tmpEntryValues : b.entryValues).as<uint32_t>(),
+                    entryCounts);
     launch_radix_sort(s, b.entryKeys.as<uint32_t>(), b.entryValues.as<uint32_t>(), b.tmpEntryKeys.as<uint32_t>(), b.tmpEntryValues.as<uint32_t>(),
-                      counters + kEntriesUsed, static_cast<uint32_t>(b.entryCapacity), b.tileBits, b.sortScratch.as<uint32_t>());
+                      counters + kEntriesUsed, static_cast<uint32_t>(b.entryCapacity), b.tileBits, b.sortScratch.as<uint32_t>(),
+                      entryCounts);
     launch_tile_ranges(s, b.entryKeys.as<uint32_t>(), counters, static_cast<uint32_t>(b.entryCapacity), b.tileBits, b.ranges.as<uint2>());
   }
   if (marks) mark("tile lists");
@@ -1254,6 +1265,7 @@ void Trainer::render_into(const vsplat_camera &camera, float *deviceOut, uint64_
   carve(b.ranges, uint64_t{VSPLAT_NOALLOC_MAX_TILES} * 8);
   carve(b.sortScratch, radix_sort_scratch_words(std::max(entries, n)) * 4);
   carve(b.scanScratch, coverage_scan_words(static_cast<uint32_t>(n)) * 4);
+  carve(b.sortCounts, (radix_count_words(n, 32) + kEntryCountWords) * 4);
   carve(b.counters, kCounterWords * 4);
   b.image.borrow(deviceOut, capacity);
   b.entryCapacity = entries;
@@ -1557,7 +1569,7 @@ uint64_t Trainer::capture_key(uint32_t n) const {
     for (const DeviceArray *a : {&b.splats, &b.keys, &b.values, &b.tmpKeys, &b.tmpValues, &b.coverage, &b.tileCount, &b.tileRecords,
                                  &b.bigList, &b.bigBits, &b.rawFixed, &b.rawFloat, &b.entryKeys, &b.entryValues, &b.tmpEntryKeys, &b.tmpEntryValues, &b.image,
                                  &b.stops, &b.adjoint, &b.fields, &b.ranges, &b.tileTotals, &b.listOrder, &b.blockWork, &b.blockOrder, &b.sortScratch,
-                                 &b.scanScratch, &b.counters, &b.sums})
+                                 &b.sortCounts, &b.scanScratch, &b.counters, &b.sums})
       array(*a);
     mix(b.entryCapacity);
     mix(static_cast<uint64_t>(b.width) << 32 | static_cast<uint32_t>(b.height));
@@ -1913,7 +1925,7 @@ uint64_t Trainer::gpu_bytes() const {
     }
     if (k == 0) continue;
     for (const DeviceArray *a : {&b.splats, &b.keys, &b.values, &b.tmpKeys, &b.tmpValues, &b.coverage, &b.tileCount, &b.tileRecords,
-                                 &b.bigList, &b.rawFixed, &b.rawFloat, &b.sortScratch, &b.scanScratch}) {
+                                 &b.bigList, &b.rawFixed, &b.rawFloat, &b.sortScratch, &b.sortCounts, &b.scanScratch}) {
       total += a->bytes();
     }
   }

@@ -136,7 +136,7 @@ struct ViewBuffers {
   // edge weights, the exposure backward's workgroup totals, the worst error.
   DeviceArray exposed, edge, exposureTotals, errorMax;
   // Scratch and counters.
-  DeviceArray sortScratch, scanScratch, counters, sums;
+  DeviceArray sortScratch, sortCounts, scanScratch, counters, sums;
 };
 
 class Trainer {
