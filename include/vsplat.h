@@ -374,7 +374,7 @@ int vsplat_autotune_views(vsplat_trainer *trainer, uint32_t n, const vsplat_came
  * block), "block_order" and "list_order" (the backward's and the forward's
  * launch orders: permutations of those indices, heaviest first on each XCD,
  * by block work and by tile list length; in index order for views of at most
- * 4096 blocks), "raw" (14 int64 per Gaussian with fixed point, else 14 float), "counters" (8 words: visible splats, entries, entries listed, big splats, big-splat bit words, overflow, skipped steps, unused),
+ * 1280 blocks in the backward and 7168 in the forward), "raw" (14 int64 per Gaussian with fixed point, else 14 float), "counters" (8 words: visible splats, entries, entries listed, big splats, big-splat bit words, overflow, skipped steps, unused),
  * "state_positions", "state_scales", "state_rotations", "state_opacities",
  * "state_sh" (Adam's state, one word per parameter: bf16 m low, bf16 v high),
  * "stats" (8 floats per Gaussian). *bytes

@@ -188,9 +188,21 @@ inline uint32_t raster_blocks(uint32_t tiles, uint32_t tileW, uint32_t tileH) {
   return (tiles + kRasterXcds - 1) / kRasterXcds * kRasterXcds * (tileW / 8u) * (tileH / 8u);
 }
 
-// The most blocks a view's raster passes launch in index order rather than
-// heaviest first: those that are resident at once.
-constexpr uint32_t kRasterResident = 4096;
+// The most blocks that a view's forward and its backward launch in index order
+// rather than heaviest first: an order takes a launch of 4 to 6 us, and pays
+// where heavy blocks would start late. The one-wave forward holds seven waves a
+// SIMD, 7168 blocks; with and without its order (us, 60k Gaussians): 6400 blocks
+// 52.5 + 4.2 and 56.8, 9216 blocks 54.6 + 5.3 and 63.0. The backward's blocks take twice as
+// long and its four-wave kernel holds about 1280: 1024 blocks (10k) 36.3 + 4.0
+// and 40.5, 1600 blocks (60k) 79.5 + 4.1 and 92.5, 4096 blocks (60k) 96.8 + 4.1
+// and 120.
+constexpr uint32_t kForwardUnordered = 7168, kBackwardUnordered = 1280;
+// Views of at most this many blocks have four waves work each block (raster.hip),
+// twelve waves a SIMD: past that one wave a block is as fast and does less work.
+// Forward and ordered backward of 60k Gaussians with four waves and with one
+// (us): 1600 blocks 45.4, 79.5 and 67.2, 118; 2304 blocks 50.4, 91.8 and 58.5,
+// 102; 3136 blocks 57.2, 99.2 and 55.4, 101; 4096 blocks 63.8, 117 and 55.1, 97.
+constexpr uint32_t kWideBlocks = 3072;
 
 // One view of a batched raster launch (its buffers and sizes), and up to
 // kRasterViewsPerLaunch of them, passed by value as the kernel's argument.

@@ -494,6 +494,81 @@ __device__ __forceinline__ uint32_t reduced_value16(uint32_t lane) {
   return 4u * (lane >> 4) + ((lane & 4u) != 0u ? ((lane & 8u) != 0u ? 3u : 2u) : (lane >> 3) & 1u);
 }
 
+// What a wave adds to a splat's row of raw sums, given the splat and the pixel's
+// alpha (0 where it takes nothing), transmittance in front and colour behind.
+// Lane l adds value `value` of the row, in fixed-point steps or as it is; values 3
+// to 5 are reduced twice their size (an exact halving in the scale). Values 12 and
+// 13 of the kRawPerSplat slots are zero without scoring.
+template <bool Fixed, bool Score> struct Emitter {
+  float4 adj;
+  float perPixel, edgeWeight, scale;
+  uint64_t lanes;
+  uint8_t *base;
+
+  __device__ __forceinline__ Emitter(const float4 &adjoint, float edge, float perPixelShare, float fixedScale,
+                                     unsigned long long *rawFixed, float *rawFloat)
+      : adj(adjoint), perPixel(perPixelShare), edgeWeight(edge) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t value = Score ? reduced_value16(lane) : reduced_value(lane);
+    lanes = vote(Score ? (lane & 3u) == 0 && value < kRawPerSplat : wave_emits(lane));
+    scale = (value >= 3u && value <= 5u ? 0.5f : 1.0f) * (Fixed ? fixedScale : 1.0f);
+    base = Fixed ? reinterpret_cast<uint8_t *>(rawFixed + value) : reinterpret_cast<uint8_t *>(rawFloat + value);
+  }
+
+  // ok: the lanes that take something; free: those of them whose alpha is not
+  // clamped (at the 0.99 clamp alpha no longer depends on the parameters).
+  __device__ __forceinline__ void operator()(const Staged &s, float dx, float dy, float e, float alpha, float T, float Br, float Bg, float Bb,
+                                             uint64_t ok, uint64_t free, uint64_t rowOffset) const {
+    const float Ta = T * alpha;
+    const float toward = T * fma32(adj.z, s.b - Bb, fma32(adj.y, s.g - Bg, adj.x * (s.r - Br)));
+    const float dAlpha = lane_of(free) ? toward : 0.0f;
+    const float dPower = dAlpha * alpha;
+    const float vx = fma32(s.qy, dy, s.qx * dx), vy = fma32(s.qz, dy, s.qy * dx);
+    const float g1 = dPower * vx, g2 = dPower * vy;
+    constexpr int kValues = Score ? 16 : 12;
+    float v[kValues];
+    v[0] = dAlpha * e;
+    v[1] = g1;
+    v[2] = g2;
+    v[3] = g1 * vx; // twice the sum (scale)
+    v[4] = g1 * vy;
+    v[5] = g2 * vy;
+    v[6] = Ta * adj.x;
+    v[7] = Ta * adj.y;
+    v[8] = Ta * adj.z;
+    v[9] = Ta * perPixel;
+    v[10] = fabsf(g1);
+    v[11] = fabsf(g2);
+    if constexpr (Score) {
+      v[12] = lane_of(ok) ? adj.w * perPixel : 0.0f;
+      v[13] = (edgeWeight * Ta) * perPixel;
+      v[14] = v[15] = 0.0f;
+    }
+    float total;
+    if constexpr (Score) {
+      total = reduce_wave16(v);
+    } else {
+      total = reduce_wave(v);
+    }
+    uint8_t *const slot = base + rowOffset;
+    const float scaled = total * scale;
+    if constexpr (Fixed) {
+      // Totals under 2^31 steps (nearly all) round and convert in 32 bits,
+      // exactly as quantise() would; the wave takes quantise() if any is larger.
+      const float rounded = __builtin_rintf(scaled);
+      int64_t q = static_cast<int32_t>(rounded);
+      uint64_t send = lanes & vote(rounded != 0.0f);
+      if ((lanes & vote(!(fabsf(scaled) < 2147483648.0f))) != 0u) {
+        q = quantise(total, scale);
+        send = lanes & vote(q != 0);
+      }
+      if (lane_of(send)) atomicAdd(reinterpret_cast<unsigned long long *>(slot), static_cast<unsigned long long>(q));
+    } else {
+      if (lane_of(lanes & vote(scaled != 0.0f))) atomicAdd(reinterpret_cast<float *>(slot), scaled);
+    }
+  }
+};
+
 // Back to front over the tile's list (train_backward.glsl:78-158), for the
 // block's pixels, from the block's lowest stop. Bound by the vector unit: a
 // splat's evaluation, gradient terms, reduction and emission are about 105
@@ -557,13 +632,7 @@ __device__ __forceinline__ void backward_block(uint32_t item, const Splat *__res
   float Tbehind = exp_finite(logTotal);
 
   const uint64_t insideLanes = vote(inside);
-  // What this lane adds of a splat's totals: value `value` of its row, in steps
-  // or as it is; values 3 to 5 are reduced twice their size (exact halving last).
-  // Values 12 and 13 of the kRawPerSplat slots are zero without scoring.
-  const uint32_t value = Score ? reduced_value16(lane) : reduced_value(lane);
-  const uint64_t emitLanes = vote(Score ? (lane & 3u) == 0 && value < kRawPerSplat : wave_emits(lane));
-  const float emitScale = (value >= 3u && value <= 5u ? 0.5f : 1.0f) * (Fixed ? fixedScale : 1.0f);
-  uint8_t *const emitBase = Fixed ? reinterpret_cast<uint8_t *>(rawFixed + value) : reinterpret_cast<uint8_t *>(rawFloat + value);
+  const Emitter<Fixed, Score> emit(adj, edgeWeight, perPixel, fixedScale, rawFixed, rawFloat);
   if (first >= range.y) return;
   ListWalk<false> walk{splats, entryKeys, entryValues, 1u << (tileBits + geo.block), range.y, first};
   walk.load_window();
@@ -607,58 +676,11 @@ __device__ __forceinline__ void backward_block(uint32_t item, const Splat *__res
         // `Tbehind / (1 - alpha)`.
         const float alpha = lane_of(oks[j]) ? (a < 0.99f ? a : 0.99f) : 0.0f;
         const float T = div_in_range(Tbehind, 1.0f - alpha);
-        const float Ta = T * alpha;
-        // At the 0.99 clamp alpha no longer depends on the parameters.
-        const float toward = T * fma32(adj.z, s.b - Bb, fma32(adj.y, s.g - Bg, adj.x * (s.r - Br)));
-        const float dAlpha = lane_of(oks[j] & vote(a < 0.99f)) ? toward : 0.0f;
-        const float dPower = dAlpha * alpha;
-        const float vx = fma32(s.qy, dy, s.qx * dx), vy = fma32(s.qz, dy, s.qy * dx);
-        const float g1 = dPower * vx, g2 = dPower * vy;
-        constexpr int kValues = Score ? 16 : 12;
-        float v[kValues];
-        v[0] = dAlpha * e;
-        v[1] = g1;
-        v[2] = g2;
-        v[3] = g1 * vx; // twice the sum (emitScale)
-        v[4] = g1 * vy;
-        v[5] = g2 * vy;
-        v[6] = Ta * adj.x;
-        v[7] = Ta * adj.y;
-        v[8] = Ta * adj.z;
-        v[9] = Ta * perPixel;
-        v[10] = fabsf(g1);
-        v[11] = fabsf(g2);
-        if constexpr (Score) {
-          v[12] = lane_of(oks[j]) ? adj.w * perPixel : 0.0f;
-          v[13] = (edgeWeight * Ta) * perPixel;
-          v[14] = v[15] = 0.0f;
-        }
+        emit(s, dx, dy, e, alpha, T, Br, Bg, Bb, oks[j], oks[j] & vote(a < 0.99f), rowOffset[k + j]);
         Br = fma32(alpha, s.r - Br, Br);
         Bg = fma32(alpha, s.g - Bg, Bg);
         Bb = fma32(alpha, s.b - Bb, Bb);
         Tbehind = T;
-        float total;
-        if constexpr (Score) {
-          total = reduce_wave16(v);
-        } else {
-          total = reduce_wave(v);
-        }
-        uint8_t *const slot = emitBase + rowOffset[k + j];
-        const float scaled = total * emitScale;
-        if constexpr (Fixed) {
-          // Totals under 2^31 steps (nearly all) round and convert in 32 bits,
-          // exactly as quantise() would; the wave takes quantise() if any is larger.
-          const float rounded = __builtin_rintf(scaled);
-          int64_t q = static_cast<int32_t>(rounded);
-          uint64_t send = emitLanes & vote(rounded != 0.0f);
-          if ((emitLanes & vote(!(fabsf(scaled) < 2147483648.0f))) != 0u) {
-            q = quantise(total, emitScale);
-            send = emitLanes & vote(q != 0);
-          }
-          if (lane_of(send)) atomicAdd(reinterpret_cast<unsigned long long *>(slot), static_cast<unsigned long long>(q));
-        } else {
-          if (lane_of(emitLanes & vote(scaled != 0.0f))) atomicAdd(reinterpret_cast<float *>(slot), scaled);
-        }
       }
     }
     if (!fetched) walk.fetch();
@@ -698,6 +720,328 @@ __global__ __launch_bounds__(kBlock) void backward_views_kernel(RasterViews view
                                                   w.gridW, bgR, bgG, bgB, w.image, w.adjoint, w.stops, w.fixedScale,
                                                   reinterpret_cast<unsigned long long *>(w.rawFixed), w.rawFloat, nullptr, batch,
                                                   rowOffset, queue);
+}
+
+// ---- Small views: four waves a block.
+//
+// A view of few blocks leaves most SIMDs with one wave or none, and a lone wave
+// issues at half the rate and waits out every latency: its time is the length of
+// its heaviest block's chain of splats. There a block is worked by kWideWaves
+// waves on the same 64 pixels, which share what does not depend on the order of
+// the splats: a window of 256 entries is staged by 256 threads; of each chunk of
+// kWideChunk staged splats every wave evaluates a quarter, leaving the alphas
+// (0 where a pixel takes nothing) in LDS; then every wave follows the whole chain
+// from the alphas, a few instructions a splat, the forward's waves for one colour
+// channel each, the backward's emitting the sums of the splats they evaluated.
+// Every float is formed as in the one-wave kernels, so the results are the same
+// bits. It does more work in all (the chain four times over), so it is for views
+// of at most kWideBlocks blocks. Forward and backward against one wave a block:
+// 10k Gaussians at 256x256 (1024 blocks) 18.5 and 40.5 us, before 32 and 59; a
+// batch's 1504-block view of 10k 47 and 87 us, before 86 and 150.
+constexpr uint32_t kWideWaves = 4, kWideThreads = kWideWaves * 64, kWideChunk = 32, kWideShare = kWideChunk / kWideWaves;
+
+struct WideShared {
+  Staged batch[kWideThreads + kWideChunk];
+  uint64_t rowOffset[kWideThreads];
+  float alpha[2][kWideChunk][64];
+  uint32_t kept[kWideWaves];
+};
+
+// block_geometry for a tile shape known at run time.
+__device__ __forceinline__ BlockGeometry wide_geometry(uint32_t h, uint32_t tileW, uint32_t tileH, uint32_t gridW, uint32_t width,
+                                                       uint32_t height, uint32_t &tile) {
+  const uint32_t across = tileW >> 3, perTile = across * (tileH >> 3), u = h / kRasterXcds;
+  tile = (u / perTile) * kRasterXcds + h % kRasterXcds;
+  const uint32_t q = u % perTile;
+  const uint32_t x0 = (tile % gridW) * tileW + (q % across) * 8u, y0 = (tile / gridW) * tileH + (q / across) * 8u;
+  return {x0, y0, x0 + 8u < width ? x0 + 8u : width, y0 + 8u < height ? y0 + 8u : height, q, perTile > 1u};
+}
+
+// The walk of a block's four waves over its tile's list, a window of 256 entries
+// at a time: the next window's splats and the keys and Gaussians of the one
+// after are in flight while a window is worked.
+template <bool Down> struct WideWalk {
+  const Splat *__restrict__ splats;
+  const uint32_t *__restrict__ entryKeys;
+  const uint32_t *__restrict__ entryValues;
+  uint32_t blockBit, limit, pos;
+  uint32_t entryNext, key, value; // this thread's entry of the window at pos
+  uint32_t entry, gaussian;
+  bool wanted, more;
+  float4 a, b, c;
+
+  __device__ __forceinline__ void load_window() {
+    const uint32_t left = Down ? pos - limit : limit - pos;
+    const bool valid = threadIdx.x < left;
+    entryNext = Down ? pos - 1u - threadIdx.x : pos + threadIdx.x;
+    key = valid ? entryKeys[entryNext] : 0u;
+    value = valid ? entryValues[entryNext] : 0u;
+  }
+  // Takes the window at pos, starts the load of its splats and of the next window.
+  __device__ __forceinline__ void take() {
+    more = pos != limit;
+    if (!more) return;
+    wanted = (key & blockBit) != 0u;
+    gaussian = value;
+    entry = entryNext;
+    if (wanted) {
+      const float4 *p = reinterpret_cast<const float4 *>(splats + gaussian);
+      a = p[0];
+      b = p[1];
+      c = p[2];
+    }
+    const uint32_t left = Down ? pos - limit : limit - pos, n = left < kWideThreads ? left : kWideThreads;
+    pos = Down ? pos - n : pos + n;
+    load_window();
+  }
+  // The taken window's splats staged, those that can touch the block packed in
+  // walk order; padded to whole chunks. Returns how many. (Two barriers: every
+  // thread calls it; the batch may be read after it.)
+  __device__ __forceinline__ uint32_t stage(const BlockGeometry &geo, WideShared &shared, uint32_t rowBytes) const {
+    Staged st{};
+    bool keep = false;
+    if (wanted) {
+      st = vsplat::stage(Splat{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, c.x, c.y, c.z, c.w}, geo, entry);
+      keep = (st.cols & 0xFFu) != 0u && (st.cols >> 16) != 0u;
+    }
+    const uint64_t mine = __ballot(keep);
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    if (lane == 0) shared.kept[wave] = static_cast<uint32_t>(__popcll(mine));
+    __syncthreads();
+    uint32_t before = 0, total = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kWideWaves; ++w) {
+      const uint32_t n = shared.kept[w];
+      before += w < wave ? n : 0u;
+      total += n;
+    }
+    if (keep) {
+      const uint32_t slot = before + static_cast<uint32_t>(__popcll(mine & ((1ull << lane) - 1ull)));
+      shared.batch[slot] = st;
+      shared.rowOffset[slot] = static_cast<uint64_t>(gaussian) * rowBytes;
+    }
+    if (threadIdx.x < kWideChunk) shared.batch[total + threadIdx.x] = Staged{};
+    __syncthreads();
+    return total;
+  }
+};
+
+// This wave's share of a chunk of staged splats evaluated: the alphas of splats
+// at + share .. into `out` rows, 0 where the lane's pixel (in `live`, with stop or
+// beyond it when Stops) takes nothing, and each splat's falloff, 0 likewise.
+template <bool Stops>
+__device__ __forceinline__ void evaluate_share(const Staged *batch, uint32_t at, float (*out)[64], float px, float py, uint32_t bits,
+                                               uint64_t live, uint32_t stop, float (&falloff)[kWideShare]) {
+  const uint32_t lane = threadIdx.x & 63u, share = (threadIdx.x >> 6) * kWideShare;
+#pragma unroll
+  for (uint32_t j = 0; j < kWideShare; ++j) {
+    const Staged &s = batch[at + share + j];
+    const float power = power_at(s, px - s.cx, py - s.cy);
+    const float e = exp_finite(power);
+    const float a = s.o * e;
+    uint64_t ok = live & vote((s.cols & bits) == bits) & vote(!(power > 0.0f)) & vote(!(a < kMinAlpha));
+    if constexpr (Stops) ok &= vote(s.entry >= stop);
+    falloff[j] = lane_of(ok) ? e : 0.0f;
+    out[share + j][lane] = lane_of(ok) ? (a < 0.99f ? a : 0.99f) : 0.0f;
+  }
+}
+
+// composite_block by four waves: every lane ends with its pixel's transmittance
+// and stop; `colour` is the channel of the calling wave (0 to 2: r, g, b; the
+// fourth wave's is not used).
+__device__ __forceinline__ void composite_wide(const Splat *__restrict__ splats, const uint32_t *__restrict__ entryKeys,
+                                               const uint32_t *__restrict__ entryValues, uint32_t blockBit, uint2 range,
+                                               const BlockGeometry &geo, WideShared &shared, bool inside, float px, float py, uint32_t bits,
+                                               float &colour, float &T, float &logT, uint32_t &stop) {
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, channel = wave < 3u ? wave : 0u;
+  stop = range.x;
+  uint64_t doneLanes = ~vote(inside);
+  colour = 0.0f;
+  T = 1.0f;
+  float Tlive = inside ? 1.0f : 0.0f; // T, or 0 once the pixel is finished
+  WideWalk<true> walk{splats, entryKeys, entryValues, blockBit, range.x, range.y};
+  walk.load_window();
+  for (walk.take(); walk.more && doneLanes != ~0ull;) {
+    const uint32_t kept = walk.stage(geo, shared, 0u);
+    walk.take();
+    float falloff[kWideShare];
+    uint32_t buffer = 0;
+    if (kept != 0) evaluate_share<false>(shared.batch, 0, shared.alpha[0], px, py, bits, ~0ull, 0u, falloff);
+    for (uint32_t at = 0; at < kept && doneLanes != ~0ull; at += kWideChunk, buffer ^= 1u) {
+      __syncthreads(); // this chunk's alphas are in place, and the chunk before is read
+      if (at + kWideChunk < kept) {
+        evaluate_share<false>(shared.batch, at + kWideChunk, shared.alpha[buffer ^ 1u], px, py, bits, ~0ull, 0u, falloff);
+      }
+#pragma unroll 2
+      for (uint32_t k = 0; k < kWideChunk; k += kGroup) {
+        float alpha[kGroup], c[kGroup], front[kGroup + 1];
+        front[0] = Tlive;
+#pragma unroll
+        for (uint32_t j = 0; j < kGroup; ++j) {
+          alpha[j] = shared.alpha[buffer][k + j][lane];
+          c[j] = (&shared.batch[at + k + j].r)[channel];
+          front[j + 1] = front[j] * (1.0f - alpha[j]);
+        }
+        // The transmittance only falls: if no pixel is under the bound after the group, none stops in it.
+        if ((vote(front[kGroup] < kMinTransmittance) & ~doneLanes) == 0) {
+#pragma unroll
+          for (uint32_t j = 0; j < kGroup; ++j) colour = fma32(front[j] * alpha[j], c[j], colour);
+          Tlive = front[kGroup];
+          continue;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kGroup; ++j) {
+          const float Tnext = Tlive * (1.0f - alpha[j]);
+          const uint64_t stops = vote(Tnext < kMinTransmittance) & ~doneLanes;
+          // These lanes stop at the splat and do not take it.
+          const bool stopped = lane_of(stops);
+          const float w = stopped ? 0.0f : Tlive * alpha[j];
+          T = stopped ? Tlive : T;
+          stop = stopped ? shared.batch[at + k + j].entry + 1u : stop;
+          Tlive = stopped ? 0.0f : Tnext;
+          doneLanes |= stops;
+          colour = fma32(w, c[j], colour);
+        }
+      }
+    }
+    __syncthreads(); // the batch is read
+  }
+  T = lane_of(doneLanes) ? T : Tlive;
+  logT = log_normal(T); // T in [1e-4, 1]: a normal float
+}
+
+__global__ __launch_bounds__(kWideThreads) void forward_wide_kernel(const Splat *__restrict__ splats, const uint32_t *__restrict__ entryKeys,
+                                                                    const uint32_t *__restrict__ entryValues, uint32_t tileBits,
+                                                                    const uint2 *__restrict__ ranges, uint32_t width, uint32_t height,
+                                                                    uint32_t tileW, uint32_t tileH, uint32_t gridW, float bgR, float bgG,
+                                                                    float bgB, float *__restrict__ image, uint32_t *__restrict__ stops,
+                                                                    uint32_t *__restrict__ work, const uint32_t *__restrict__ order) {
+  __shared__ WideShared shared;
+  const uint32_t item = order != nullptr ? order[blockIdx.x] : blockIdx.x;
+  uint32_t tile;
+  const BlockGeometry geo = wide_geometry(item, tileW, tileH, gridW, width, height, tile);
+  if (geo.x0 >= width || geo.y0 >= height) { // a block past the image's edge (uniform)
+    if (work != nullptr && threadIdx.x == 0) work[item] = 0;
+    return;
+  }
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, lx = lane & 7u, ly = lane >> 3;
+  const uint32_t x = geo.x0 + lx, y = geo.y0 + ly;
+  const bool inside = x < width && y < height;
+  float colour, T, logT;
+  uint32_t stop;
+  const uint2 range = ranges[tile];
+  composite_wide(splats, entryKeys, entryValues, 1u << (tileBits + geo.block), range, geo, shared, inside, static_cast<float>(x) + 0.5f,
+                 static_cast<float>(y) + 0.5f, lane_bits(lx, ly), colour, T, logT, stop);
+  if (inside) {
+    const uint32_t at = y * width + x;
+    const float background = wave == 0u ? bgR : (wave == 1u ? bgG : bgB);
+    image[at * 4u + wave] = wave < 3u ? fma32(T, background, colour) : logT;
+    if (wave == 3u && stops != nullptr) stops[at] = stop;
+  }
+  if (work != nullptr && wave == 0u) {
+    uint32_t low = inside ? stop : range.y;
+#pragma unroll
+    for (uint32_t d = 32; d >= 1; d >>= 1) {
+      const uint32_t other = static_cast<uint32_t>(__shfl_xor(static_cast<int>(low), static_cast<int>(d), 64));
+      low = other < low ? other : low;
+    }
+    if (lane == 0) work[item] = range.y - low;
+  }
+}
+
+// backward_block by four waves.
+template <bool Fixed, bool Recompute, bool Score>
+__global__ __launch_bounds__(kWideThreads) void backward_wide_kernel(const Splat *__restrict__ splats, const uint32_t *__restrict__ entryKeys,
+                                                                     const uint32_t *__restrict__ entryValues, uint32_t tileBits,
+                                                                     const uint2 *__restrict__ ranges, uint32_t width, uint32_t height,
+                                                                     uint32_t tileW, uint32_t tileH, uint32_t gridW, float bgR, float bgG,
+                                                                     float bgB, const float4 *__restrict__ image,
+                                                                     const float4 *__restrict__ adjoint, const uint32_t *__restrict__ stops,
+                                                                     float fixedScale, unsigned long long *__restrict__ rawFixed,
+                                                                     float *__restrict__ rawFloat, const float *__restrict__ edge,
+                                                                     const uint32_t *__restrict__ order) {
+  __shared__ WideShared shared;
+  uint32_t tile;
+  const BlockGeometry geo = wide_geometry(order != nullptr ? order[blockIdx.x] : blockIdx.x, tileW, tileH, gridW, width, height, tile);
+  if (geo.x0 >= width || geo.y0 >= height) return; // a block past the image's edge (uniform)
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, lx = lane & 7u, ly = lane >> 3;
+  const uint32_t bits = lane_bits(lx, ly);
+  const uint32_t x = geo.x0 + lx, y = geo.y0 + ly;
+  const bool inside = x < width && y < height;
+  const float px = static_cast<float>(x) + 0.5f, py = static_cast<float>(y) + 0.5f;
+  const uint32_t at = inside ? y * width + x : 0u;
+  const float4 adj = inside ? adjoint[at] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const float edgeWeight = Score && inside ? edge[at] : 0.0f;
+  const float perPixel = 1.0f / (3.0f * static_cast<float>(width) * static_cast<float>(height));
+  const uint2 range = ranges[tile];
+  const uint32_t blockBit = 1u << (tileBits + geo.block);
+  float logTotal;
+  uint32_t stop;
+  if constexpr (Recompute) {
+    float colour, T;
+    composite_wide(splats, entryKeys, entryValues, blockBit, range, geo, shared, inside, px, py, bits, colour, T, logTotal, stop);
+    if (!inside) {
+      stop = range.y;
+      logTotal = 0.0f;
+    }
+  } else {
+    logTotal = inside ? image[at].w : 0.0f;
+    stop = inside ? stops[at] : range.y;
+  }
+  uint32_t first = stop;
+#pragma unroll
+  for (uint32_t d = 32; d >= 1; d >>= 1) {
+    const uint32_t other = static_cast<uint32_t>(__shfl_xor(static_cast<int>(first), static_cast<int>(d), 64));
+    first = other < first ? other : first;
+  }
+  if (first >= range.y) return; // the same for the four waves
+  float Br = bgR, Bg = bgG, Bb = bgB;
+  float Tbehind = exp_finite(logTotal);
+  const uint64_t insideLanes = vote(inside);
+  const Emitter<Fixed, Score> emit(adj, edgeWeight, perPixel, fixedScale, rawFixed, rawFloat);
+  WideWalk<false> walk{splats, entryKeys, entryValues, blockBit, range.y, first};
+  walk.load_window();
+  for (walk.take(); walk.more;) {
+    const uint32_t kept = walk.stage(geo, shared, kRawPerSplat * (Fixed ? 8u : 4u));
+    walk.take();
+    uint32_t buffer = 0;
+    float falloff[kWideShare], next[kWideShare];
+    if (kept != 0) evaluate_share<true>(shared.batch, 0, shared.alpha[0], px, py, bits, insideLanes, stop, next);
+    for (uint32_t start = 0; start < kept; start += kWideChunk, buffer ^= 1u) {
+      __syncthreads(); // this chunk's alphas are in place, and the chunk before is read
+#pragma unroll
+      for (uint32_t j = 0; j < kWideShare; ++j) falloff[j] = next[j];
+      if (start + kWideChunk < kept) {
+        evaluate_share<true>(shared.batch, start + kWideChunk, shared.alpha[buffer ^ 1u], px, py, bits, insideLanes, stop, next);
+      }
+      // The chain over the chunk, share by share; the sums of this wave's own on the way.
+#pragma unroll 1
+      for (uint32_t w = 0; w < kWideWaves; ++w) {
+        const uint32_t share = w * kWideShare;
+        float alpha[kWideShare];
+#pragma unroll
+        for (uint32_t j = 0; j < kWideShare; ++j) alpha[j] = shared.alpha[buffer][share + j][lane];
+#pragma unroll
+        for (uint32_t j = 0; j < kWideShare; ++j) {
+          const Staged &s = shared.batch[start + share + j];
+          const float T = div_in_range(Tbehind, 1.0f - alpha[j]);
+          if (w == wave) {
+            const uint64_t ok = vote(alpha[j] != 0.0f);
+            if (ok != 0) {
+              const Staged own = s;
+              emit(own, px - own.cx, py - own.cy, falloff[j], alpha[j], T, Br, Bg, Bb, ok, ok & vote(alpha[j] < 0.99f),
+                   shared.rowOffset[start + share + j]);
+            }
+          }
+          Br = fma32(alpha[j], s.r - Br, Br);
+          Bg = fma32(alpha[j], s.g - Bg, Bg);
+          Bb = fma32(alpha[j], s.b - Bb, Bb);
+          Tbehind = T;
+        }
+      }
+    }
+    __syncthreads(); // the batch is read
+  }
 }
 
 constexpr uint32_t kOrderThreads = 1024;
@@ -819,6 +1163,12 @@ void launch_forward(hipStream_t stream, const Splat *splats, const uint32_t *ent
                     const uint2 *ranges, uint32_t width, uint32_t height, uint32_t tileW, uint32_t tileH, const float background[3],
                     float4 *image, uint32_t *stops, uint32_t *work, const uint32_t *order) {
   const uint32_t gridW = (width + tileW - 1) / tileW, gridH = (height + tileH - 1) / tileH;
+  if (raster_blocks(gridW * gridH, tileW, tileH) <= kWideBlocks) {
+    hipLaunchKernelGGL(forward_wide_kernel, dim3(raster_blocks(gridW * gridH, tileW, tileH)), dim3(kWideThreads), 0, stream, splats, entryKeys,
+                       entryValues, tileBits, ranges, width, height, tileW, tileH, gridW, background[0], background[1], background[2],
+                       reinterpret_cast<float *>(image), stops, work, order);
+    return;
+  }
 #define VSPLAT_FORWARD(W, H)                                                                                                       \
   hipLaunchKernelGGL((forward_kernel<W, H>), dim3(raster_blocks(gridW * gridH, W, H)), dim3(kBlock), 0, stream, splats, entryKeys,   \
                      entryValues, tileBits, ranges, width, height, gridW, background[0], background[1], background[2], image, stops, work,  \
@@ -832,6 +1182,26 @@ void launch_backward(hipStream_t stream, bool fixedPoint, bool recompute, const 
                      uint32_t tileH, const float background[3], const float4 *image, const float4 *adjoint, const uint32_t *stops,
                      float fixedScale, int64_t *rawFixed, float *rawFloat, const float *edge, const uint32_t *order) {
   const uint32_t gridW = (width + tileW - 1) / tileW, gridH = (height + tileH - 1) / tileH;
+  const bool score = edge != nullptr;
+  const int variant = (fixedPoint ? 4 : 0) | (recompute ? 2 : 0) | (score ? 1 : 0);
+  if (raster_blocks(gridW * gridH, tileW, tileH) <= kWideBlocks) {
+#define VSPLAT_BACKWARD_WIDE(F, R, S)                                                                                               \
+  hipLaunchKernelGGL((backward_wide_kernel<F, R, S>), dim3(raster_blocks(gridW * gridH, tileW, tileH)), dim3(kWideThreads), 0, stream, \
+                     splats, entryKeys, entryValues, tileBits, ranges, width, height, tileW, tileH, gridW, background[0], background[1], \
+                     background[2], image, adjoint, stops, fixedScale, reinterpret_cast<unsigned long long *>(rawFixed), rawFloat, edge, order)
+    switch (variant) {
+    case 7: VSPLAT_BACKWARD_WIDE(true, true, true); break;
+    case 6: VSPLAT_BACKWARD_WIDE(true, true, false); break;
+    case 5: VSPLAT_BACKWARD_WIDE(true, false, true); break;
+    case 4: VSPLAT_BACKWARD_WIDE(true, false, false); break;
+    case 3: VSPLAT_BACKWARD_WIDE(false, true, true); break;
+    case 2: VSPLAT_BACKWARD_WIDE(false, true, false); break;
+    case 1: VSPLAT_BACKWARD_WIDE(false, false, true); break;
+    default: VSPLAT_BACKWARD_WIDE(false, false, false); break;
+    }
+#undef VSPLAT_BACKWARD_WIDE
+    return;
+  }
 #define VSPLAT_BACKWARD_SHAPE(F, R, S, W, H)                                                                                       \
   hipLaunchKernelGGL((backward_kernel<F, R, S, W, H>), dim3(raster_blocks(gridW * gridH, W, H)), dim3(kBlock), 0, stream, splats,   \
                      entryKeys, entryValues, tileBits, ranges, width, height, gridW, background[0], background[1], background[2], image, \
@@ -844,8 +1214,6 @@ void launch_backward(hipStream_t stream, bool fixedPoint, bool recompute, const 
 #define VSPLAT_BACKWARD_FTF(W, H) VSPLAT_BACKWARD_SHAPE(false, true, false, W, H)
 #define VSPLAT_BACKWARD_FFT(W, H) VSPLAT_BACKWARD_SHAPE(false, false, true, W, H)
 #define VSPLAT_BACKWARD_FFF(W, H) VSPLAT_BACKWARD_SHAPE(false, false, false, W, H)
-  const bool score = edge != nullptr;
-  const int variant = (fixedPoint ? 4 : 0) | (recompute ? 2 : 0) | (score ? 1 : 0);
   switch (variant) {
   case 7: VSPLAT_TILE_DISPATCH(tileW, tileH, VSPLAT_BACKWARD_TTT) break;
   case 6: VSPLAT_TILE_DISPATCH(tileW, tileH, VSPLAT_BACKWARD_TTF) break;

@@ -785,16 +785,15 @@ void Trainer::enqueue_passes(ViewBuffers &b, const ViewParams &view, const uint8
   // Each pass's 8x8 blocks launch heaviest first on their XCD: the forward's by
   // their tiles' list lengths, the backward's by the work the forward found.
   const bool backward = mode != kModeRender;
-  const bool ordered = launch_ordered(b);
-  uint32_t *listOrder = ordered ? b.listOrder.as<uint32_t>() : nullptr; // none in the allocation-free render
+  const uint32_t blocks = raster_blocks(b.tiles, b.tileW, b.tileH);
+  uint32_t *listOrder = blocks > kForwardUnordered ? b.listOrder.as<uint32_t>() : nullptr; // none in the allocation-free render
   if (listOrder != nullptr) launch_list_order(b.stream, b.ranges.as<uint2>(), b.tiles, b.tileW, b.tileH, listOrder);
   launch_forward(b.stream, b.splats.as<Splat>(), b.entryKeys.as<uint32_t>(), b.entryValues.as<uint32_t>(), b.tileBits, b.ranges.as<uint2>(),
                  v.width, v.height, b.tileW, b.tileH, options_.background, b.image.as<float4>(),
                  options_.recompute_transmittance != 0 ? nullptr : b.stops.as<uint32_t>(), backward ? b.blockWork.as<uint32_t>() : nullptr,
                  listOrder);
-  if (backward && ordered) {
-    launch_work_order(b.stream, b.blockWork.as<uint32_t>(), raster_blocks(b.tiles, b.tileW, b.tileH), b.blockOrder.as<uint32_t>());
-  }
+  uint32_t *blockOrder = backward && blocks > kBackwardUnordered ? b.blockOrder.as<uint32_t>() : nullptr;
+  if (blockOrder != nullptr) launch_work_order(b.stream, b.blockWork.as<uint32_t>(), blocks, blockOrder);
   mark("composite");
   if (!backward) return;
   enqueue_loss(b, v, deviceTarget);
@@ -806,18 +805,12 @@ void Trainer::enqueue_passes(ViewBuffers &b, const ViewParams &view, const uint8
                   b.entryValues.as<uint32_t>(), b.tileBits, b.ranges.as<uint2>(), v.width, v.height, b.tileW, b.tileH, options_.background,
                   b.image.as<float4>(),
                   b.adjoint.as<float4>(), b.stops.as<uint32_t>(), fixed_scale(v), b.rawFixed.as<int64_t>(), b.rawFloat.as<float>(),
-                  scoring ? b.edge.as<float>() : nullptr, ordered ? b.blockOrder.as<uint32_t>() : nullptr);
+                  scoring ? b.edge.as<float>() : nullptr, blockOrder);
   mark("backward");
   if (!chain) return;
   enqueue_chain(b, v, mode, rates, b.stream, b.counters.as<uint32_t>());
   mark(mode == kModeStep ? "chain rule and step" : "chain rule");
 }
-
-// Whether the raster passes of a view launch their blocks heaviest first. A view
-// whose blocks all fit the chip at once (the raster kernels hold seven waves a
-// SIMD, over 1024 SIMDs) has no late starters to bring forward: its two order
-// kernels, 4 to 5 us each, are left out.
-bool Trainer::launch_ordered(const ViewBuffers &b) { return raster_blocks(b.tiles, b.tileW, b.tileH) > kRasterResident; }
 
 ViewParams Trainer::with_tiles(const ViewBuffers &b, const ViewParams &view) const {
   ViewParams v = view;
@@ -1987,7 +1980,8 @@ void Trainer::inspect(const std::string &name, void *out, uint64_t capacity, uin
     if (name != item.name) continue;
     if (bytes != nullptr) *bytes = item.size;
     const uint64_t copy = std::min(item.size, capacity);
-    if ((name == "list_order" || name == "block_order") && !launch_ordered(b)) {
+    const uint32_t blocks = raster_blocks(b.tiles, b.tileW, b.tileH);
+    if ((name == "list_order" && blocks <= kForwardUnordered) || (name == "block_order" && blocks <= kBackwardUnordered)) {
       for (uint64_t k = 0; k < copy / 4 && out != nullptr; ++k) static_cast<uint32_t *>(out)[k] = static_cast<uint32_t>(k);
       return;
     }

@@ -222,7 +222,6 @@ private:
   void allocate_per_gaussian();
   void ensure_size(ViewBuffers &b, int width, int height);
   void gather_view_status(uint32_t n);
-  static bool launch_ordered(const ViewBuffers &b);
   void finish_pass(const ViewBuffers &b, bool step);
   void ensure_layout(ViewBuffers &b, int width, int height, uint32_t tileW, uint32_t tileH);
   static void set_geometry(ViewBuffers &b, int width, int height, uint32_t tileW, uint32_t tileH);
