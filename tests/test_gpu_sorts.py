@@ -56,3 +56,17 @@ def test_tile_lists(width, height, tiles):
     cam = F.look_at((0, 0, -3), (0, 0, 0), (0.0, -1.0, 0.0), 60.0, width, height)
     with vsplat.Trainer(cloud, vsplat.TrainerOptions(tile_shape=tiles)) as t:
         _check_lists(t, t.compute_gradients(cam, F.smooth_target(width, height, 3)))
+
+
+@pytest.mark.parametrize("tiles", [vsplat.TILES_8X8, vsplat.TILES_16X16, vsplat.TILES_32X8, vsplat.TILES_32X32])
+@pytest.mark.parametrize("width,height", [(9, 7), (256, 256), (264, 256), (512, 512), (1000, 620), (1040, 520), (2500, 1700)])
+@pytest.mark.parametrize("count,scale", [(3, -2.0), (3000, -4.0), (60_000, -2.5)])
+def test_large_tile_lists(count, scale, width, height, tiles):
+    """Lists sized for more than 2^18 entries, few or many of which there are, on one to 67k tiles: the one-pass sort's chunks of 8192 and 16384
+    entries (up to 2^10 and 2^11 tiles), and the passes of eight bits past them."""
+    cloud = F.synthetic_cloud(count, 0, 17, log_scale=(scale, 0.7))
+    cam = F.look_at((0, 0, -3), (0, 0, 0), (0.0, -1.0, 0.0), 60.0, width, height)
+    with vsplat.Trainer(cloud, vsplat.TrainerOptions(tile_shape=tiles)) as t:
+        t.reserve_entries(262_145)
+        for _ in range(2):
+            _check_lists(t, t.compute_gradients(cam, F.smooth_target(width, height, 3)))

@@ -320,9 +320,9 @@ __global__ __launch_bounds__(256) void bin_emit_kernel(const uint32_t *__restric
 // (train_tile_ranges.comp:11-22). A thread takes four consecutive keys with one
 // 16-byte load, and the keys either side of them; a key's tile is its low bits
 // (tileMask), its block bits above them.
-__global__ __launch_bounds__(256) void tile_ranges_kernel(const uint32_t *__restrict__ entryKeys, const uint32_t *counters,
+__global__ __launch_bounds__(256) void tile_ranges_kernel(const uint32_t *__restrict__ entryKeys, const uint32_t *__restrict__ countDev,
                                                           uint32_t tileMask, uint2 *__restrict__ ranges) {
-  const uint32_t count = counters[kEntriesUsed];
+  const uint32_t count = *countDev;
   const uint32_t quads = (count + 3u) / 4u;
   for (uint32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < quads; q += gridDim.x * blockDim.x) {
     const uint32_t k0 = q * 4u;
@@ -391,12 +391,12 @@ void launch_bin_emit(hipStream_t stream, const uint32_t *keys, const uint32_t *v
                      entryKeys, entryValues, entryCounts, radix_first_mask(tileBits));
 }
 
-void launch_tile_ranges(hipStream_t stream, const uint32_t *entryKeys, const uint32_t *counters, uint32_t capacity, uint32_t tileBits,
+void launch_tile_ranges(hipStream_t stream, const uint32_t *entryKeys, const uint32_t *countDev, uint32_t capacity, uint32_t tileBits,
                         uint2 *ranges) {
   if (capacity == 0) return;
   const uint32_t quads = (capacity + 3) / 4;
   const uint32_t blocks = (quads + 255) / 256 < 16384 ? (quads + 255) / 256 : 16384;
-  hipLaunchKernelGGL(tile_ranges_kernel, dim3(blocks), dim3(256), 0, stream, entryKeys, counters, (1u << tileBits) - 1u, ranges);
+  hipLaunchKernelGGL(tile_ranges_kernel, dim3(blocks), dim3(256), 0, stream, entryKeys, countDev, (1u << tileBits) - 1u, ranges);
 }
 
 } // namespace vsplat

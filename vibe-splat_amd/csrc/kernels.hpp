@@ -111,6 +111,16 @@ size_t radix_count_words(uint64_t capacity, uint32_t bits);
 uint32_t radix_first_mask(uint32_t bits);
 void launch_radix_sort(hipStream_t stream, uint32_t *keys, uint32_t *values, uint32_t *tmpKeys, uint32_t *tmpValues,
                        const uint32_t *countDev, uint32_t capacity, uint32_t bits, uint32_t *scratch, uint32_t *counts);
+// The tile entries sorted by tile, and the tiles' ranges (cleared beforehand). The
+// entries start in tmpKeys and tmpValues if tile_sort_from_tmp. More than
+// kCountedSortKeys entries on at most kTileSortTiles tiles are sorted in one pass
+// (sort.hip). scratch: tile_sort_scratch_words.
+constexpr uint32_t kTileSortTiles = 2048;
+size_t tile_sort_scratch_words(uint64_t capacity, uint32_t tiles);
+bool tile_sort_from_tmp(uint64_t capacity, uint32_t tileBits, uint32_t tiles);
+void launch_tile_sort(hipStream_t stream, uint32_t *keys, uint32_t *values, uint32_t *tmpKeys, uint32_t *tmpValues,
+                      const uint32_t *countDev, uint32_t capacity, uint32_t tileBits, uint32_t tiles, uint32_t *scratch, uint32_t *counts,
+                      uint2 *ranges);
 void launch_fill_u32(hipStream_t stream, uint32_t *dst, uint64_t count, uint32_t value);
 // Up to kMaxClears arrays cleared in one launch.
 constexpr uint32_t kMaxClears = 4;
@@ -177,7 +187,7 @@ void launch_bin_emit(hipStream_t stream, const uint32_t *keys, const uint32_t *v
                      uint32_t count, uint32_t gridW, uint32_t tileW, uint32_t tileH, uint32_t width, uint32_t height, uint32_t tileBits,
                      const uint32_t *offsets, const uint32_t *counters, const uint32_t *bigList, const uint64_t *bigBits,
                      uint32_t *entryKeys, uint32_t *entryValues, uint32_t *entryCounts);
-void launch_tile_ranges(hipStream_t stream, const uint32_t *entryKeys, const uint32_t *counters, uint32_t capacity, uint32_t tileBits,
+void launch_tile_ranges(hipStream_t stream, const uint32_t *entryKeys, const uint32_t *countDev, uint32_t capacity, uint32_t tileBits,
                         uint2 *ranges);
 
 // The raster launches' workgroups for a view of `tiles` list tiles of TW x TH

@@ -457,6 +457,7 @@ void Trainer::ensure_layout(ViewBuffers &b, int width, int height, uint32_t tile
   b.listOrder.ensure(blocks * 4);
   b.blockWork.ensure(blocks * 4);
   b.blockOrder.ensure(blocks * 4);
+  ensure_sort_scratch(b);
 }
 
 // The tile grid of a view size and tile shape (no buffers).
@@ -675,9 +676,9 @@ void Trainer::grow_entries(ViewBuffers &b, uint64_t entries) {
     a->release();
     a->ensure(capacity * 4);
   }
-  b.sortScratch.ensure(std::max(radix_sort_scratch_words(capacity), radix_sort_scratch_words(count_)) * 4);
   b.bigBits.ensure(big_bit_words_for(capacity) * 8);
   b.entryCapacity = capacity;
+  ensure_sort_scratch(b);
 }
 
 // A view's tile-entry buffers sized for `entries` by grow_entries' rule (half
@@ -699,11 +700,16 @@ void Trainer::fit_entries(ViewBuffers &b, uint64_t entries) {
     a->release();
     a->ensure(wanted * 4);
   }
-  b.sortScratch.release();
-  b.sortScratch.ensure(std::max(radix_sort_scratch_words(wanted), radix_sort_scratch_words(count_)) * 4);
   b.bigBits.release();
   b.bigBits.ensure(big_bit_words_for(wanted) * 8);
   b.entryCapacity = wanted;
+  b.sortScratch.release();
+  ensure_sort_scratch(b);
+}
+
+// The scratch of the view's sorts, one after the other: by depth, then by tile.
+void Trainer::ensure_sort_scratch(ViewBuffers &b) {
+  b.sortScratch.ensure(std::max(radix_sort_scratch_words(count_), tile_sort_scratch_words(b.entryCapacity, b.tiles)) * 4);
 }
 
 void Trainer::reserve_entries(uint64_t entries) {
@@ -844,16 +850,15 @@ void Trainer::enqueue_lists(ViewBuffers &b, const ViewParams &v, uint32_t mode, 
                        b.tileRecords.as<TileRecord>(), b.coverage.as<uint32_t>(), counters, static_cast<uint32_t>(b.entryCapacity), mode == kModeStep, b.scanScratch.as<uint32_t>());
   if (marks) mark("count tiles");
   if (b.entryCapacity > 0) {
-    const bool fromTmp = radix_sort_from_tmp(b.tileBits);
+    const bool fromTmp = tile_sort_from_tmp(b.entryCapacity, b.tileBits, b.tiles);
     launch_bin_emit(s, b.keys.as<uint32_t>(), b.values.as<uint32_t>(), b.splats.as<Splat>(), b.tileRecords.as<TileRecord>(), count_, b.gridW,
                     b.tileW, b.tileH, static_cast<uint32_t>(b.width), static_cast<uint32_t>(b.height), b.tileBits,
                     b.coverage.as<uint32_t>(), counters, b.bigList.as<uint32_t>(), b.bigBits.as<uint64_t>(),
                     (fromTmp ? b.tmpEntryKeys : b.entryKeys).as<uint32_t>(), (fromTmp ? b.tmpEntryValues : b.entryValues).as<uint32_t>(),
                     entryCounts);
-    launch_radix_sort(s, b.entryKeys.as<uint32_t>(), b.entryValues.as<uint32_t>(), b.tmpEntryKeys.as<uint32_t>(), b.tmpEntryValues.as<uint32_t>(),
-                      counters + kEntriesUsed, static_cast<uint32_t>(b.entryCapacity), b.tileBits, b.sortScratch.as<uint32_t>(),
-                      entryCounts);
-    launch_tile_ranges(s, b.entryKeys.as<uint32_t>(), counters, static_cast<uint32_t>(b.entryCapacity), b.tileBits, b.ranges.as<uint2>());
+    launch_tile_sort(s, b.entryKeys.as<uint32_t>(), b.entryValues.as<uint32_t>(), b.tmpEntryKeys.as<uint32_t>(), b.tmpEntryValues.as<uint32_t>(),
+                     counters + kEntriesUsed, static_cast<uint32_t>(b.entryCapacity), b.tileBits, b.tiles, b.sortScratch.as<uint32_t>(),
+                     entryCounts, b.ranges.as<uint2>());
   }
   if (marks) mark("tile lists");
 }
@@ -1256,7 +1261,7 @@ void Trainer::render_into(const vsplat_camera &camera, float *deviceOut, uint64_
   for (DeviceArray *a : {&b.entryKeys, &b.entryValues, &b.tmpEntryKeys, &b.tmpEntryValues}) carve(*a, entries * 4);
   carve(b.stops, uint64_t{VSPLAT_NOALLOC_MAX_PIXELS} * 4);
   carve(b.ranges, uint64_t{VSPLAT_NOALLOC_MAX_TILES} * 8);
-  carve(b.sortScratch, radix_sort_scratch_words(std::max(entries, n)) * 4);
+  carve(b.sortScratch, std::max(radix_sort_scratch_words(n), tile_sort_scratch_words(entries, b.tiles)) * 4);
   carve(b.scanScratch, coverage_scan_words(static_cast<uint32_t>(n)) * 4);
   carve(b.sortCounts, (radix_count_words(n, 32) + kEntryCountWords) * 4);
   carve(b.counters, kCounterWords * 4);

@@ -227,6 +227,7 @@ private:
   static void set_geometry(ViewBuffers &b, int width, int height, uint32_t tileW, uint32_t tileH);
   std::pair<uint32_t, uint32_t> tile_shape_for(int width, int height) const;
   bool needs_tuning(int width, int height) const;
+  void ensure_sort_scratch(ViewBuffers &b);
   void grow_entries(ViewBuffers &b, uint64_t entries);
   void fit_entries(ViewBuffers &b, uint64_t entries);
   uint64_t big_bit_words_for(uint64_t entries) const;
