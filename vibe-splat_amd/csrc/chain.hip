@@ -1,14 +1,16 @@
 // The chain rule from the backward pass's 14 screen-space sums per Gaussian to
 // the raw parameters, and what becomes of the result (train_gradient.comp:105-315):
 // the densification statistics only, the gradients stored (one float per
-// parameter), or Adam's step taken at once with bf16 moments. The SH
-// coefficients step in a pass of their own, one thread per packed word
-// (train_sh_step.comp:19-70), so that neighbouring threads touch neighbouring memory.
+// parameter), or Adam's step taken at once with bf16 moments, the SH coefficients'
+// one thread per packed word (train_sh_step.comp:19-70).
+//
+// A Gaussian's sums are read only where the backward pass marked it (ChainBuffers::touched).
 //
 // The fixed-point sums are converted here (train_fixed_to_float.comp:9-14):
 // int64 to double (exact), times the scale's reciprocal in double, rounded to float once.
 #include "device.hpp"
 #include "kernels.hpp"
+#include "blockscan.hpp"
 
 namespace vsplat {
 
@@ -512,40 +514,14 @@ __device__ __forceinline__ void emit_terms(const ChainBuffers &B, const ChainPar
 }
 
 constexpr uint32_t kChainThreads = 256;
-
-// The SH gradients of one Gaussian row: zero (or unchanged, accumulating) where
-// value(j) is zero; rows of a multiple of four floats go out four at a time.
-template <typename Value>
-__device__ __forceinline__ void store_sh_row(float *out, uint32_t floats, bool add, Value &&value) {
-  if ((floats & 3u) == 0u) {
-    float4 *out4 = reinterpret_cast<float4 *>(out);
-#pragma unroll
-    for (uint32_t q = 0; q < 12; ++q) {
-      if (4 * q >= floats) break;
-      float4 v = make_float4(value(4 * q), value(4 * q + 1), value(4 * q + 2), value(4 * q + 3));
-      if (add) {
-        const float4 p = out4[q];
-        v = make_float4(p.x + v.x, p.y + v.y, p.z + v.z, p.w + v.w);
-      }
-      out4[q] = v;
-    }
-  } else {
-    for (uint32_t j = 0; j < floats; ++j) out[j] = add ? out[j] + value(j) : value(j);
-  }
-}
-
-// One view, in two kernels over the Gaussians: the SH part (colour, SH
-// gradients or the SH step's inputs, and the view direction's term of the
-// position gradient, kept in dirTerms), then the geometric part with the
-// statistics and the emits. Split, each needs far fewer registers than the
-// whole: the chain rule's long dependent chains (divisions, square roots, the
-// fixed-point conversion) are hidden by more waves per SIMD. The SH part runs
-// first because a step changes the positions it reads.
-template <int Degree, uint32_t Format>
-__device__ __forceinline__ void chain_sh_gradients(const ChainBuffers &B, const ViewParams &c, const ChainParams &o, uint32_t i,
-                                                   float *shRows);
-
-// In gradients mode the SH gradient rows go through LDS (dynamic shared
+// One view's gradients, in two kernels over all the Gaussians: the SH part (the
+// SH gradients and the view direction's term of the position gradient, kept in
+// dirTerms), then the geometric part with the statistics and the emits. Split,
+// each needs far fewer registers than the whole: the chain rule's long dependent
+// chains (divisions, square roots, the fixed-point conversion) are hidden by more
+// waves per SIMD. The raw sums are read only where the Gaussian is flagged.
+//
+// The SH gradient rows go through LDS (dynamic shared
 // memory, kShRowStride floats per row, 64 rows per wave): each lane writes its
 // row there, then the block stores its rows, which lie consecutively in
 // gradSh, with consecutive lanes on consecutive floats. Stored one row per
@@ -553,73 +529,19 @@ __device__ __forceinline__ void chain_sh_gradients(const ChainBuffers &B, const 
 constexpr uint32_t kShRowStride = 49; // odd, so that a row's lanes hit distinct banks
 constexpr uint32_t kShRowsLds = kChainThreads * kShRowStride * 4;
 
+// A lane writes its row (zero for a Gaussian no pixel touched, or above the active
+// degree) to LDS, then the block's rows are stored (or added, kFlagAccumulate) in order.
 template <int Degree, uint32_t Format>
-__global__ __launch_bounds__(kChainThreads) void chain_sh_kernel(ChainBuffers B, ViewParams c, ChainParams o, const uint32_t *counters) {
+__global__ __launch_bounds__(kChainThreads) void chain_sh_gradients_kernel(ChainBuffers B, ViewParams c, ChainParams o,
+                                                                           const uint32_t *counters) {
   extern __shared__ float shRows[];
   if (counters[kOverflow] != 0) return; // a view did not fit: this pass computed nothing (uniform)
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (o.mode == kModeGradients) {
-    chain_sh_gradients<Degree, Format>(B, c, o, i, shRows);
-    return;
-  }
-  if (i >= c.count) return;
-  float g[kRawPerSplat];
-  const bool touched = load_raw(o.fixedPoint ? B.rawFixed : nullptr, B.rawFloat, o.fixedScale, i, g);
-  const bool zeros = o.mode == kModeGradients || (o.mode == kModeStep && (o.flags & kFlagSelective) == 0);
-  const bool penalties = o.opacityReg > 0.0f || o.scaleReg > 0.0f;
-  float *shPass = B.shPass + static_cast<size_t>(i) * kShPassFloats;
-  if (o.mode == kModeStatistics || !touched) {
-    // Nothing from the pixels: no SH step, and zero SH gradients where the
-    // single kernel wrote them (gradients mode, or penalties in step mode).
-    if (o.mode == kModeStep || o.mode == kModeCurvature) shPass[9] = as_float(0u);
-    if (o.mode == kModeGradients && (zeros || penalties)) {
-      store_sh_row(B.gradSh + static_cast<size_t>(i) * o.shFloats, o.shFloats, (o.flags & kFlagAccumulate) != 0,
-                   [](uint32_t) { return 0.0f; });
-    }
-    return;
-  }
-  constexpr uint32_t kCoefficients = (Degree + 1) * (Degree + 1);
-  float dirTerm[3];
-  const float position[3] = {B.positions[i * 3], B.positions[i * 3 + 1], B.positions[i * 3 + 2]};
-  view_sh_terms<Degree, Format>(c, o, i, position, B.shWords + static_cast<size_t>(i) * c.shWords, g, dirTerm,
-                                [&](const float basis[16], const float gcu[3], const float dir[3], uint32_t used) {
-    if (o.mode == kModeGradients) {
-      // Coefficients above the active degree get zero (they are stored, not trained).
-      store_sh_row(B.gradSh + static_cast<size_t>(i) * o.shFloats, o.shFloats, (o.flags & kFlagAccumulate) != 0, [&](uint32_t j) {
-        const uint32_t k = j / 3, ch = j - 3 * k;
-        return j < kCoefficients * 3 && k < used ? basis[k] * gcu[ch] : 0.0f;
-      });
-    } else {
-      // For the SH pass: the colour gradient, the direction and the coefficients used.
-      shPass[0] = gcu[0];
-      shPass[1] = gcu[1];
-      shPass[2] = gcu[2];
-      shPass[3] = dir[0];
-      shPass[4] = dir[1];
-      shPass[5] = dir[2];
-      if ((o.flags & kFlagSecondOrder) != 0) {
-        const float opacity = 1.0f / (1.0f + vs_exp(-B.opacities[i]));
-        const uint32_t *words = B.shWords + static_cast<size_t>(i) * c.shWords;
-#pragma unroll
-        for (uint32_t ch = 0; ch < 3; ++ch) shPass[6 + ch] = sh_radius(o, opacity, sh_value<Format>(words, 0, ch));
-      }
-      shPass[9] = as_float(used);
-    }
-  });
-  B.dirTerms[i] = make_float4(dirTerm[0], dirTerm[1], dirTerm[2], 0.0f);
-}
-
-// chain_sh_kernel's gradients mode: the same terms, each lane's row (zero for
-// a Gaussian no pixel touched, or above the active degree) written to LDS, then
-// the block's rows stored (or added, kFlagAccumulate) in order.
-template <int Degree, uint32_t Format>
-__device__ __forceinline__ void chain_sh_gradients(const ChainBuffers &B, const ViewParams &c, const ChainParams &o, uint32_t i,
-                                                   float *shRows) {
   const uint32_t floats = o.shFloats;
   float *row = shRows + threadIdx.x * kShRowStride;
   if (i < c.count) {
     float g[kRawPerSplat];
-    const bool touched = load_raw(o.fixedPoint ? B.rawFixed : nullptr, B.rawFloat, o.fixedScale, i, g);
+    const bool touched = B.touched[i] != 0 && load_raw(o.fixedPoint ? B.rawFixed : nullptr, B.rawFloat, o.fixedScale, i, g);
     for (uint32_t j = 0; j < floats; ++j) row[j] = 0.0f;
     if (touched) {
       constexpr uint32_t kCoefficients = (Degree + 1) * (Degree + 1);
@@ -657,55 +579,58 @@ __device__ __forceinline__ void chain_sh_gradients(const ChainBuffers &B, const 
   }
 }
 
-__global__ __launch_bounds__(kChainThreads) void chain_geometry_kernel(ChainBuffers B, ViewParams c, ChainParams o,
-                                                                      const uint32_t *counters) {
+// A Gaussian's densification statistics, when a pass keeps them.
+__device__ __forceinline__ void keep_statistics(const ChainBuffers &B, const ViewParams &c, const ChainParams &o, uint32_t i,
+                                                const float g[kRawPerSplat]) {
+  if ((o.flags & kFlagStatistics) == 0 || B.stats == nullptr) return;
+  float4 *st = reinterpret_cast<float4 *>(B.stats + static_cast<size_t>(i) * 8);
+  float4 a = st[0], b = st[1];
+  add_statistics(a, b, g, static_cast<float>(c.width), static_cast<float>(c.height), B.splats[i].radius);
+  st[0] = a;
+  st[1] = b;
+}
+
+// How the loss moves with the camera through a Gaussian's position
+// (train_gradient.comp:276-279): v = Rv gP, w = t x v.
+__device__ __forceinline__ void keep_pose_terms(const ChainBuffers &B, const ViewParams &c, const ChainParams &o, uint32_t i,
+                                                const float gP[3]) {
+  if ((o.flags & kFlagPose) == 0 || o.mode == kModeCurvature || !(gP[0] != 0.0f || gP[1] != 0.0f || gP[2] != 0.0f)) return;
+  float tx, ty, tz;
+  to_camera(c, B.positions[i * 3], B.positions[i * 3 + 1], B.positions[i * 3 + 2], tx, ty, tz);
+  const float *V = c.view;
+  float v[3];
+#pragma unroll
+  for (int r = 0; r < 3; ++r) v[r] = dot3(V[r], V[4 + r], V[8 + r], gP[0], gP[1], gP[2]);
+  float *out = B.poseTerms + static_cast<size_t>(i) * 6;
+  out[0] = fma32(ty, v[2], -(tz * v[1]));
+  out[1] = fma32(tz, v[0], -(tx * v[2]));
+  out[2] = fma32(tx, v[1], -(ty * v[0]));
+  out[3] = v[0];
+  out[4] = v[1];
+  out[5] = v[2];
+}
+
+__global__ __launch_bounds__(kChainThreads) void chain_geometry_gradients_kernel(ChainBuffers B, ViewParams c, ChainParams o,
+                                                                                 const uint32_t *counters) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= c.count) return;
   if (counters[kOverflow] != 0) return;
-  if (o.mode == kModeStep) adam_step_now(o);
   float g[kRawPerSplat];
-  const bool touched = load_raw(o.fixedPoint ? B.rawFixed : nullptr, B.rawFloat, o.fixedScale, i, g);
-  const bool zeros = o.mode == kModeGradients || (o.mode == kModeStep && (o.flags & kFlagSelective) == 0);
-  const bool penalties = o.opacityReg > 0.0f || o.scaleReg > 0.0f;
-  if ((touched && (o.flags & kFlagStatistics) != 0) && B.stats != nullptr) {
-    float4 *st = reinterpret_cast<float4 *>(B.stats + static_cast<size_t>(i) * 8);
-    float4 a = st[0], b = st[1];
-    add_statistics(a, b, g, static_cast<float>(c.width), static_cast<float>(c.height), B.splats[i].radius);
-    st[0] = a;
-    st[1] = b;
-  }
-  if (o.mode == kModeStatistics || (!touched && !zeros && !penalties)) return;
+  const bool touched = B.touched[i] != 0 && load_raw(o.fixedPoint ? B.rawFixed : nullptr, B.rawFloat, o.fixedScale, i, g);
   ViewTerms t;
-  if (!touched) {
-    // Nothing from the pixels; the penalties still apply.
-    untouched_terms(B, o, i, penalties, t);
-  } else {
+  if (touched) {
+    keep_statistics(B, c, o, i, g);
     const float4 d = B.dirTerms[i];
     const float dirTerm[3] = {d.x, d.y, d.z};
     GaussianFrame G;
     gaussian_frame(B, i, G);
     view_geometry_terms(G, c, o, g, dirTerm, c.shDegree > 0, t);
-    const float *gP = t.position;
-    if ((o.flags & kFlagPose) != 0 && o.mode != kModeCurvature && (gP[0] != 0.0f || gP[1] != 0.0f || gP[2] != 0.0f)) {
-      // How the loss moves with the camera through this Gaussian's position
-      // (train_gradient.comp:276-279): v = Rv gP, w = t x v.
-      float tx, ty, tz;
-      to_camera(c, B.positions[i * 3], B.positions[i * 3 + 1], B.positions[i * 3 + 2], tx, ty, tz);
-      const float *V = c.view;
-      float v[3];
-#pragma unroll
-      for (int r = 0; r < 3; ++r) v[r] = dot3(V[r], V[4 + r], V[8 + r], gP[0], gP[1], gP[2]);
-      float *out = B.poseTerms + static_cast<size_t>(i) * 6;
-      out[0] = fma32(ty, v[2], -(tz * v[1]));
-      out[1] = fma32(tz, v[0], -(tx * v[2]));
-      out[2] = fma32(tx, v[1], -(ty * v[0]));
-      out[3] = v[0];
-      out[4] = v[1];
-      out[5] = v[2];
-    }
+    keep_pose_terms(B, c, o, i, t.position);
+  } else {
+    // Nothing from the pixels; the penalties still apply.
+    untouched_terms(B, o, i, o.opacityReg > 0.0f || o.scaleReg > 0.0f, t);
   }
-  // Everything above read the parameters before any of them changes.
-  emit_terms(B, o, i, t, radii_of(o, B.opacities, B.scales, i));
+  emit_terms(B, o, i, t, Radii{-1.0f, -1.0f, -1.0f});
 }
 
 // The batched chain rule (no reference counterpart): for each Gaussian, every
@@ -866,43 +791,260 @@ __device__ __forceinline__ uint32_t sh_word_put(uint32_t format, uint32_t word, 
   return (word & ~(0xFFFFu << shift)) | (half_stochastic(value, s, seed ^ 0x5DEECE66u) << shift);
 }
 
-__global__ __launch_bounds__(256) void sh_step_kernel(uint32_t *__restrict__ shWords, uint32_t *__restrict__ stateSh,
-                                                      const float *__restrict__ shPass, ViewParams c, ChainParams o,
-                                                      const uint32_t *counters) {
-  const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t words = c.shWords;
-  if (w >= c.count * words) return;
-  if (counters[kOverflow] != 0) return;
-  if (o.mode == kModeStep) adam_step_now(o);
-  const uint32_t i = w / words, q = w - i * words;
-  const float *g = shPass + static_cast<size_t>(i) * kShPassFloats;
-  const uint32_t used = as_uint(g[9]);
-  const bool secondOrder = (o.flags & kFlagSecondOrder) != 0;
-  const bool zeros = o.mode == kModeStep && (o.flags & kFlagSelective) == 0 && !secondOrder;
-  if (used == 0 && !zeros) return;
-  float basis[16];
-  sh_basis(g[3], g[4], g[5], c.shDegree, basis);
-  uint32_t first, last;
-  sh_word_floats(c.shFormat, q, o.shFloats, first, last);
-  uint32_t word = shWords[w];
-  bool changed = false;
-  for (uint32_t j = first; j <= last; ++j) {
-    const uint32_t k = j / 3, ch = j - 3 * k;
-    const float gv = k < used ? basis[k] * g[ch] : 0.0f;
-    if (gv == 0.0f && !zeros) continue;
-    const uint32_t s = i * o.shFloats + j;
-    uint32_t state = stateSh[s];
+// The chain rule of the modes that store no gradients (a step, the curvature, the
+// statistics), in one kernel. A workgroup takes perBlock neighbouring Gaussians,
+// packs those that have something to do at the front of a list in LDS, and works
+// the list kStepSlots at a time. Half of its threads take a Gaussian each through
+// the SH terms, the other half through the geometric terms (two chains of
+// dependent instructions, which one thread would go through one after the other);
+// what they find stays in LDS, and all of them then step the parameters, a thread
+// per geometric parameter or packed SH word, so that neighbouring threads touch
+// neighbouring memory and several loads are on their way at once.
+//
+// Unless a mode acts on every Gaussian (Adam without `selective`, penalties) only
+// the flagged ones are listed, and the raw sums, the parameters and the moments of
+// the others are not read. Most of a large scene is hidden in a view. Three
+// kernels over all 1M Gaussians of a 1280x736 view, 4 % of them seen, took 34 (SH
+// terms), 59 (geometry) and 76 us (SH step: 26M words asked whether they step);
+// this takes 43, of 3M (1080p, 2 %) 59 for 444, of 400k 31 for 90. Where all are
+// seen it takes as long as the three did: 93 us for 93 (200k), 453 for 481 (1M),
+// 28 for 29 (30k). Then it is bound by the step's own instructions (some 200 a
+// parameter, divisions, a square root and two hashes), where few are seen by the
+// way to memory of one after the other: flags, sums, parameters, moments.
+constexpr uint32_t kStepSlots = kChainThreads / 2, kStepMost = 4096, kStepLeast = 64, kFlagged = 0x8000u;
+// What the step takes of a Gaussian. The rows' lengths are odd, so that
+// neighbouring rows lie on different banks.
+struct ShRow {
+  float colour[3], radius[3], basis[16], direction[3]; // the colour gradient; second order's radii; the direction's term of the position
+  uint32_t used;                                       // coefficients used
+  uint32_t pad;
+};
+struct GeometryRow {
+  float term[11]; // position, scale, rotation, opacity
+  float radius[3];
+  uint32_t pad;
+};
+static_assert(sizeof(ShRow) / 4 % 2 == 1 && sizeof(GeometryRow) / 4 % 2 == 1, "odd rows");
+
+// The geometric parameters of the list's Gaussians stepped, or their curvature
+// taken, a thread a parameter, the next one's loads ahead: all positions, then
+// scales, rotations and opacities. (This loop and the next are not unrolled: a
+// workgroup goes through them a few times, and code fetched for the first time
+// costs more than the jumps.)
+__device__ __forceinline__ void step_geometry(const ChainBuffers &B, const ChainParams &o, uint32_t first, const uint16_t *list, uint32_t n,
+                                              const GeometryRow *geometry, const ShRow *sh, bool withDir, bool zeros) {
+  struct Parameter {
+    uint32_t t, k, at, group; // row t's term k
+    float *values;
+    uint32_t *states;
+    float value;
+    uint32_t state;
+  };
+  const auto load = [&](uint32_t x, Parameter &p) {
+    if (x >= 11u * n) return;
+    p.group = x < 3u * n ? 0u : (x < 6u * n ? 1u : (x < 10u * n ? 2u : 3u));
+    const uint32_t each = p.group < 2u ? 3u : (p.group == 2u ? 4u : 1u), from = p.group < 3u ? 3u * p.group : 10u;
+    const uint32_t y = x - from * n;
+    p.t = p.group < 2u ? y / 3u : (p.group == 2u ? y / 4u : y);
+    const uint32_t a = y - p.t * each;
+    p.k = from + a;
+    p.at = (first + (list[p.t] & (kFlagged - 1u))) * each + a;
+    p.values = p.group == 0u ? B.positions : (p.group == 1u ? B.scales : (p.group == 2u ? B.rotations : B.opacities));
+    p.states = p.group == 0u ? B.statePos : (p.group == 1u ? B.stateScale : (p.group == 2u ? B.stateRot : B.stateOpacity));
+    p.value = p.values[p.at];
+    p.state = p.states[p.at];
+  };
+  Parameter next{};
+  load(threadIdx.x, next);
+#pragma unroll 1
+  for (uint32_t x = threadIdx.x; x < 11u * n; x += kChainThreads) {
+    Parameter p = next;
+    load(x + kChainThreads, next);
+    float g = geometry[p.t].term[p.k];
+    if (p.group == 0u && withDir && sh[p.t].used != 0u) g = g + sh[p.t].direction[p.k];
+    const float radius = p.group == 2u ? -1.0f : geometry[p.t].radius[p.group == 3u ? 2u : p.group];
     if (o.mode == kModeCurvature) {
-      stateSh[s] = with_curvature(o, state, gv, s * 5u + 4u);
-      continue;
+      if (g != 0.0f && p.group != 2u) p.states[p.at] = with_curvature(o, p.state, g, p.at * 5u + p.group);
+    } else if (g != 0.0f || (zeros && radius < 0.0f)) {
+      const float rate = p.group == 0u ? o.rates[0] : (p.group == 1u ? o.rates[1] : (p.group == 2u ? o.rates[2] : o.rates[3]));
+      step_parameter(o, p.value, p.state, g, rate, radius, p.at * 5u + p.group);
+      p.values[p.at] = p.value;
+      p.states[p.at] = p.state;
     }
-    float value = sh_word_get(c.shFormat, word, j, first);
-    step_parameter(o, value, state, gv, k == 0 ? o.rates[4] : o.rates[4] * o.restScale, secondOrder ? g[6 + ch] : -1.0f, s * 5u + 4u);
-    stateSh[s] = state;
-    word = sh_word_put(c.shFormat, word, j, first, value, s, o.seed);
-    changed = true;
   }
-  if (changed) shWords[w] = word;
+}
+
+// The packed SH words of the list's Gaussians stepped, or their curvature taken, a
+// thread a word, the next one's loads ahead.
+__device__ __forceinline__ void step_sh_words(const ChainBuffers &B, const ViewParams &c, const ChainParams &o, uint32_t first,
+                                              const uint16_t *list, uint32_t n, const ShRow *rows, bool zeros) {
+  const bool secondOrder = (o.flags & kFlagSecondOrder) != 0;
+  const uint32_t words = c.shWords, total = n * words;
+  const float perWord = 1.0f / static_cast<float>(words);
+  struct Word {
+    uint32_t t, i, q, first, last; // word q of Gaussian i (row t), its floats first .. last
+    uint32_t word, state[2];
+    bool wanted;
+  };
+  const auto load = [&](uint32_t x, Word &w) {
+    w.wanted = false;
+    if (x >= total) return;
+    // Word x of the rows (x < 2^12: the quotient by the rounded reciprocal is exact).
+    w.t = static_cast<uint32_t>((static_cast<float>(x) + 0.5f) * perWord);
+    w.q = x - w.t * words;
+    w.i = first + (list[w.t] & (kFlagged - 1u));
+    sh_word_floats(c.shFormat, w.q, o.shFloats, w.first, w.last);
+    w.wanted = zeros || rows[w.t].used != 0;
+    if (!w.wanted) return;
+    w.word = B.shWords[static_cast<size_t>(w.i) * words + w.q];
+    const uint32_t s = w.i * o.shFloats + w.first;
+    w.state[0] = B.stateSh[s];
+    w.state[1] = w.last > w.first ? B.stateSh[s + 1] : 0u;
+  };
+  Word next{};
+  load(threadIdx.x, next);
+#pragma unroll 1
+  for (uint32_t x = threadIdx.x; x < total; x += kChainThreads) {
+    Word w = next;
+    load(x + kChainThreads, next);
+    if (!w.wanted) continue;
+    const ShRow &row = rows[w.t];
+    const uint32_t used = row.used;
+    bool changed = false;
+#pragma unroll 1
+    for (uint32_t j = w.first; j <= w.last; ++j) {
+      const uint32_t b = j / 3, ch = j - 3 * b;
+      const float gv = b < used ? row.basis[b] * row.colour[ch] : 0.0f;
+      if (gv == 0.0f && !zeros) continue;
+      const uint32_t s = w.i * o.shFloats + j;
+      uint32_t state = j == w.first ? w.state[0] : w.state[1];
+      if (o.mode == kModeCurvature) {
+        B.stateSh[s] = with_curvature(o, state, gv, s * 5u + 4u);
+        continue;
+      }
+      float value = sh_word_get(c.shFormat, w.word, j, w.first);
+      step_parameter(o, value, state, gv, b == 0 ? o.rates[4] : o.rates[4] * o.restScale, secondOrder ? row.radius[ch] : -1.0f, s * 5u + 4u);
+      B.stateSh[s] = state;
+      w.word = sh_word_put(c.shFormat, w.word, j, w.first, value, s, o.seed);
+      changed = true;
+    }
+    if (changed) B.shWords[static_cast<size_t>(w.i) * words + w.q] = w.word;
+  }
+}
+
+template <int Degree, uint32_t Format>
+__global__ __launch_bounds__(kChainThreads, 4) void chain_step_kernel(ChainBuffers B, ViewParams c, ChainParams o, uint32_t perBlock,
+                                                                      const uint32_t *counters) {
+  constexpr uint32_t kRound = 4 * kChainThreads, kRounds = kStepMost / kRound;
+  __shared__ uint16_t list[kStepMost]; // the listed Gaussians' numbers in the workgroup's, with kFlagged those whose sums may not be zero
+  __shared__ ShRow sh[kStepSlots];
+  __shared__ GeometryRow geometry[kStepSlots];
+  __shared__ uint32_t waveTotals[kChainThreads / 64];
+  if (counters[kOverflow] != 0) return; // a view did not fit: this pass computed nothing (uniform)
+  const uint32_t first = blockIdx.x * perBlock;
+  const uint32_t mine = c.count - first < perBlock ? c.count - first : perBlock;
+  uint32_t flags[kRounds]; // a byte each for four neighbours (the last word of `touched` is padded)
+#pragma unroll
+  for (uint32_t r = 0; r < kRounds; ++r) {
+    const uint32_t x = r * kRound + threadIdx.x * 4u;
+    flags[r] = x < mine ? reinterpret_cast<const uint32_t *>(B.touched + first)[x / 4u] : 0u;
+  }
+  if (o.mode == kModeStep) adam_step_now(o);
+  const bool penalties = o.opacityReg > 0.0f || o.scaleReg > 0.0f, secondOrder = (o.flags & kFlagSecondOrder) != 0;
+  const bool zeros = o.mode == kModeStep && (o.flags & kFlagSelective) == 0;
+  const bool everyone = zeros || (penalties && o.mode != kModeStatistics);
+  uint32_t listed = 0;
+#pragma unroll
+  for (uint32_t r = 0; r < kRounds; ++r) {
+    if (r * kRound >= mine) break; // uniform
+    uint32_t wanted = 0, at;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+      const uint32_t x = r * kRound + threadIdx.x * 4u + k;
+      if (x < mine && (everyone || ((flags[r] >> (8u * k)) & 0xFFu) != 0)) wanted |= 1u << k;
+    }
+    const uint32_t total = block_exclusive_sum(static_cast<uint32_t>(__popc(wanted)), at, waveTotals);
+    at += listed;
+    listed += total;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+      const uint32_t x = r * kRound + threadIdx.x * 4u + k;
+      if ((wanted >> k) & 1u) list[at++] = static_cast<uint16_t>(x | (((flags[r] >> (8u * k)) & 0xFFu) != 0 ? kFlagged : 0u));
+    }
+  }
+  __syncthreads();
+  for (uint32_t from = 0; from < listed; from += kStepSlots) {
+    const uint32_t n = listed - from < kStepSlots ? listed - from : kStepSlots;
+    const uint32_t slot = threadIdx.x % kStepSlots;
+    if (slot < n) {
+      const uint32_t x = list[from + slot], i = first + (x & (kFlagged - 1u));
+      float g[kRawPerSplat];
+      const bool touched = (x & kFlagged) != 0 && load_raw(o.fixedPoint ? B.rawFixed : nullptr, B.rawFloat, o.fixedScale, i, g);
+      if (threadIdx.x < kStepSlots) {
+        GeometryRow &row = geometry[slot];
+        ViewTerms t;
+        if (touched) {
+          GaussianFrame G;
+          gaussian_frame(B, i, G);
+          const float none[3] = {0.0f, 0.0f, 0.0f};
+          view_geometry_terms(G, c, o, g, none, false, t);
+        } else {
+          untouched_terms(B, o, i, penalties, t);
+        }
+        const Radii r = radii_of(o, B.opacities, B.scales, i);
+#pragma unroll
+        for (uint32_t a = 0; a < 3; ++a) {
+          row.term[a] = t.position[a];
+          row.term[3 + a] = t.scale[a];
+        }
+#pragma unroll
+        for (uint32_t a = 0; a < 4; ++a) row.term[6 + a] = t.rotation[a];
+        row.term[10] = t.opacity;
+        row.radius[0] = r.position;
+        row.radius[1] = r.scale;
+        row.radius[2] = r.opacity;
+        if (touched) keep_statistics(B, c, o, i, g);
+      } else {
+        ShRow &row = sh[slot];
+        row.used = 0u;
+        if (touched && o.mode != kModeStatistics) {
+          const float position[3] = {B.positions[i * 3], B.positions[i * 3 + 1], B.positions[i * 3 + 2]};
+          const uint32_t *words = B.shWords + static_cast<size_t>(i) * c.shWords;
+          view_sh_terms<Degree, Format>(c, o, i, position, words, g, row.direction,
+                                        [&](const float basis[16], const float gcu[3], const float *, uint32_t used) {
+#pragma unroll
+            for (uint32_t k = 0; k < 3; ++k) row.colour[k] = gcu[k];
+            if (secondOrder) {
+              const float opacity = 1.0f / (1.0f + vs_exp(-B.opacities[i]));
+#pragma unroll
+              for (uint32_t ch = 0; ch < 3; ++ch) row.radius[ch] = sh_radius(o, opacity, sh_value<Format>(words, 0, ch));
+            }
+            row.used = used;
+#pragma unroll
+            for (uint32_t k = 0; k < (Degree + 1) * (Degree + 1); ++k) row.basis[k] = basis[k];
+          });
+        }
+      }
+    }
+    __syncthreads(); // the rows are whole; everything above read the parameters before any of them changes
+    if (o.mode != kModeStatistics) {
+      if ((o.flags & kFlagPose) != 0) {
+        if (threadIdx.x < n && sh[threadIdx.x].used != 0u) {
+          float gP[3];
+#pragma unroll
+          for (uint32_t a = 0; a < 3; ++a) {
+            gP[a] = geometry[threadIdx.x].term[a];
+            if (Degree > 0) gP[a] = gP[a] + sh[threadIdx.x].direction[a];
+          }
+          keep_pose_terms(B, c, o, first + (list[from + threadIdx.x] & (kFlagged - 1u)), gP);
+        }
+        __syncthreads();
+      }
+      step_geometry(B, o, first, list + from, n, geometry, sh, Degree > 0, zeros);
+      step_sh_words(B, c, o, first, list + from, n, sh, zeros && !secondOrder);
+    }
+    __syncthreads(); // the rows are read
+  }
 }
 
 // One Adam step from summed gradients (the batched step): thread t takes
@@ -1106,16 +1248,24 @@ void launch_chain(hipStream_t stream, const ChainBuffers &buffers, const ViewPar
                   const uint32_t *counters) {
   if (view.count == 0) return;
   const dim3 grid((view.count + 255) / 256), block(256);
-  const uint32_t rowsLds = params.mode == kModeGradients ? kShRowsLds : 0u;
-#define VSPLAT_CHAIN(D, F) hipLaunchKernelGGL((chain_sh_kernel<D, F>), grid, block, rowsLds, stream, buffers, view, params, counters)
+  if (params.mode == kModeGradients) {
+#define VSPLAT_CHAIN(D, F)                                                                                                         \
+  hipLaunchKernelGGL((chain_sh_gradients_kernel<D, F>), grid, block, kShRowsLds, stream, buffers, view, params, counters)
+    VSPLAT_SH_DISPATCH(view.shDegree, view.shFormat, VSPLAT_CHAIN)
+#undef VSPLAT_CHAIN
+    hipLaunchKernelGGL(chain_geometry_gradients_kernel, grid, block, 0, stream, buffers, view, params, counters);
+    return;
+  }
+  // Four workgroups a CU are resident: as many, with as equal shares as can be
+  // (a multiple of four Gaussians each, so that their flags are whole words).
+  constexpr uint32_t kResident = 4 * 256;
+  const uint32_t share = ((view.count + kResident - 1) / kResident + 3) / 4 * 4;
+  const uint32_t perBlock = share < kStepLeast ? kStepLeast : (share < kStepMost ? share : kStepMost);
+#define VSPLAT_CHAIN(D, F)                                                                                                         \
+  hipLaunchKernelGGL((chain_step_kernel<D, F>), dim3((view.count + perBlock - 1) / perBlock), block, 0, stream, buffers, view, params, \
+                     perBlock, counters)
   VSPLAT_SH_DISPATCH(view.shDegree, view.shFormat, VSPLAT_CHAIN)
 #undef VSPLAT_CHAIN
-  hipLaunchKernelGGL(chain_geometry_kernel, grid, block, 0, stream, buffers, view, params, counters);
-  if (params.mode == kModeStep || params.mode == kModeCurvature) {
-    const uint64_t words = static_cast<uint64_t>(view.count) * view.shWords;
-    hipLaunchKernelGGL(sh_step_kernel, dim3(static_cast<uint32_t>((words + 255) / 256)), dim3(256), 0, stream, buffers.shWords,
-                       buffers.stateSh, buffers.shPass, view, params, counters);
-  }
 }
 
 void launch_chain_views(hipStream_t stream, const ChainBuffers &buffers, const ChainViews &views, const ChainParams &params,

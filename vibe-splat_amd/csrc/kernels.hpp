@@ -19,7 +19,6 @@ constexpr uint32_t kFlagStatistics = 1, kFlagSelective = 4;
 constexpr uint32_t kFlagAccumulate = 8; // gradients mode: add to the gradient buffers instead of writing them
 constexpr uint32_t kFlagSecondOrder = 16; // step mode: the trust-region step, curvature in the states' second halves
 constexpr uint32_t kFlagPose = 32;        // gradients and step modes: each Gaussian's pose terms into poseTerms
-constexpr uint32_t kShPassFloats = 10; // per Gaussian, what the SH step needs from the chain rule
 
 struct ChainParams {
   float opacityReg, scaleReg; // per Gaussian: the option over the count
@@ -51,11 +50,11 @@ struct ChainBuffers {
   const Splat *splats;
   const int64_t *rawFixed;
   const float *rawFloat;
-  float *shPass;
+  const uint8_t *touched; // per Gaussian: nonzero where its raw sums may not be zero (launch_backward)
   float *stats; // 8 per Gaussian, or null
   uint32_t *statePos, *stateScale, *stateRot, *stateOpacity, *stateSh;
   float *gradPos, *gradScale, *gradRot, *gradOpacity, *gradSh;
-  float4 *dirTerms; // per Gaussian: the view direction's term of the position gradient (between the chain rule's two kernels)
+  float4 *dirTerms; // per Gaussian: the view direction's term of the position gradient (between the gradients' two kernels)
   float *poseTerms; // 6 per Gaussian with kFlagPose: t x v, then v = Rv dL/dp; untouched Gaussians' left as they are
 };
 
@@ -66,6 +65,7 @@ struct ChainView {
   const int64_t *rawFixed;
   const float *rawFloat;
   const Splat *splats;
+  const uint8_t *touched;
   float fixedScale;
 };
 constexpr uint32_t kChainViewsPerLaunch = 8;
@@ -228,6 +228,7 @@ struct RasterView {
   const float4 *adjoint;
   int64_t *rawFixed;
   float *rawFloat;
+  uint8_t *touched;
   float fixedScale;
   uint32_t width, height, gridW, firstBlock, blocks;
   uint32_t tileBits;
@@ -256,11 +257,14 @@ void launch_forward(hipStream_t stream, const Splat *splats, const uint32_t *ent
 // read from the forward pass (image and stops may then be null). edge: a
 // scored view's edge weights (the adjoint's fourth value its marks), which
 // fill the last two raw sums; null otherwise. order: the blocks' launch order
-// from launch_work_order, or null for raster_blocks' own.
+// from launch_work_order, or null for raster_blocks' own. touched: set to 1 for
+// every Gaussian that may have been added to, so that a pass over the Gaussians
+// need not read (or clear) the sums of the others, which are zero.
 void launch_backward(hipStream_t stream, bool fixedPoint, bool recompute, const Splat *splats, const uint32_t *entryKeys,
                      const uint32_t *entryValues, uint32_t tileBits, const uint2 *ranges, uint32_t width, uint32_t height, uint32_t tileW,
                      uint32_t tileH, const float background[3], const float4 *image, const float4 *adjoint, const uint32_t *stops,
-                     float fixedScale, int64_t *rawFixed, float *rawFloat, const float *edge = nullptr, const uint32_t *order = nullptr);
+                     float fixedScale, int64_t *rawFixed, float *rawFloat, uint8_t *touched, const float *edge = nullptr,
+                     const uint32_t *order = nullptr);
 // The backward's launch order, heaviest first on each XCD by the forward's work
 // (each block keeps its XCD): a permutation of the items = raster_blocks(tiles)
 // launch indices.
@@ -274,9 +278,11 @@ void launch_list_order(hipStream_t stream, const uint2 *ranges, uint32_t tiles, 
 // error; both null otherwise.
 void launch_loss(hipStream_t stream, const float4 *image, const uint8_t *target, uint32_t width, uint32_t height, float lambda,
                  float *fields, float4 *adjoint, float2 *tileTotals, uint32_t *errorMax, float *edge);
-// The tiles' totals summed (sums[0] SSIM, sums[1] L1), and `words` words of the
-// raw sums (16-byte aligned) cleared for the backward pass, in one launch.
-void launch_total_and_clear(hipStream_t stream, const float2 *tileTotals, uint32_t tiles, double *sums, uint32_t *raw, uint64_t words);
+// The tiles' totals summed (sums[0] SSIM, sums[1] L1; no tiles: nothing), and the
+// raw sums of the `count` Gaussians cleared for the backward pass where touched
+// says that the last one added to them, with touched, in one launch.
+void launch_total_and_clear(hipStream_t stream, const float2 *tileTotals, uint32_t tiles, double *sums, bool fixedPoint, void *raw,
+                            uint8_t *touched, uint32_t count);
 
 // A view's affine colour transform (Trainer::set_exposure): rows of (r, g, b, 1).
 struct Exposure {

@@ -240,9 +240,10 @@ template <bool Down> struct ListWalk {
   }
   // The fetched batch: each lane stages one splat, and those that can touch a
   // pixel of the block are packed at the front of `batch` in walk order (with
-  // the byte offsets of their rows of rowBytes, when rowOffset is given).
-  // Returns how many were kept.
-  __device__ __forceinline__ uint32_t stage(const BlockGeometry &geo, Staged *batch, uint64_t *rowOffset, uint32_t rowBytes) const {
+  // the byte offsets of their rows of rowBytes, when rowOffset is given, and
+  // their Gaussians marked in `touched`). Returns how many were kept.
+  __device__ __forceinline__ uint32_t stage(const BlockGeometry &geo, Staged *batch, uint64_t *rowOffset, uint32_t rowBytes,
+                                            uint8_t *__restrict__ touched) const {
     Staged st{};
     bool keep = false;
     if (threadIdx.x < queued) {
@@ -253,7 +254,10 @@ template <bool Down> struct ListWalk {
     if (keep) {
       const uint32_t slot = static_cast<uint32_t>(__popcll(kept & ((1ull << threadIdx.x) - 1ull)));
       batch[slot] = st;
-      if (rowOffset != nullptr) rowOffset[slot] = static_cast<uint64_t>(gaussian) * rowBytes;
+      if (rowOffset != nullptr) {
+        rowOffset[slot] = static_cast<uint64_t>(gaussian) * rowBytes;
+        touched[gaussian] = 1;
+      }
     }
     return static_cast<uint32_t>(__popcll(kept));
   }
@@ -281,7 +285,7 @@ __device__ __forceinline__ void composite_block(const Splat *__restrict__ splats
     walk.request(queue);
     walk.fetch();
     while (walk.queued != 0) {
-      const uint32_t kept = walk.stage(geo, batch, nullptr, 0u);
+      const uint32_t kept = walk.stage(geo, batch, nullptr, 0u, nullptr);
       // Pad the last group with splats no pixel is a candidate for (their
       // colours, which a zero weight multiplies, finite).
       if (threadIdx.x < kGroup) batch[kept + threadIdx.x] = Staged{};
@@ -589,7 +593,7 @@ __device__ __forceinline__ void backward_block(uint32_t item, const Splat *__res
                                                float bgR, float bgG, float bgB, const float4 *__restrict__ image,
                                                const float4 *__restrict__ adjoint, const uint32_t *__restrict__ stops,
                                                float fixedScale, unsigned long long *__restrict__ rawFixed,
-                                               float *__restrict__ rawFloat, const float *__restrict__ edge, Staged *batch,
+                                               float *__restrict__ rawFloat, uint8_t *__restrict__ touched, const float *__restrict__ edge, Staged *batch,
                                                uint64_t *rowOffset, uint32_t *queue) {
   uint32_t tile;
   const BlockGeometry geo = block_geometry<TW, TH>(item, gridW, width, height, tile);
@@ -639,7 +643,7 @@ __device__ __forceinline__ void backward_block(uint32_t item, const Splat *__res
   walk.request(queue);
   walk.fetch();
   while (walk.queued != 0) {
-    const uint32_t kept = walk.stage(geo, batch, rowOffset, kRawPerSplat * (Fixed ? 8u : 4u));
+    const uint32_t kept = walk.stage(geo, batch, rowOffset, kRawPerSplat * (Fixed ? 8u : 4u), touched);
     if (lane < kGroup) batch[kept + lane] = Staged{}; // the last group padded with splats no pixel is a candidate for
     __syncthreads();
     walk.request(queue);
@@ -696,14 +700,14 @@ __global__ __launch_bounds__(kBlock) void backward_kernel(const Splat *__restric
                                                           float bgR, float bgG, float bgB, const float4 *__restrict__ image,
                                                           const float4 *__restrict__ adjoint, const uint32_t *__restrict__ stops,
                                                           float fixedScale, unsigned long long *__restrict__ rawFixed,
-                                                          float *__restrict__ rawFloat, const float *__restrict__ edge,
+                                                          float *__restrict__ rawFloat, uint8_t *__restrict__ touched, const float *__restrict__ edge,
                                                           const uint32_t *__restrict__ order) {
   __shared__ Staged batch[kBlock + kGroup];
   __shared__ uint64_t rowOffset[kBlock];
   __shared__ uint32_t queue[kBlock];
   const uint32_t item = order != nullptr ? order[blockIdx.x] : blockIdx.x;
   backward_block<Fixed, Recompute, Score, TW, TH>(item, splats, entryKeys, entryValues, tileBits, ranges, width, height, gridW, bgR,
-                                                  bgG, bgB, image, adjoint, stops, fixedScale, rawFixed, rawFloat, edge, batch, rowOffset,
+                                                  bgG, bgB, image, adjoint, stops, fixedScale, rawFixed, rawFloat, touched, edge, batch, rowOffset,
                                                   queue);
 }
 
@@ -718,7 +722,7 @@ __global__ __launch_bounds__(kBlock) void backward_views_kernel(RasterViews view
   const RasterView &w = views.view[view_of(views, item)];
   backward_block<Fixed, Recompute, false, TW, TH>(item, w.splats, w.entryKeys, w.entryValues, w.tileBits, w.ranges, w.width, w.height,
                                                   w.gridW, bgR, bgG, bgB, w.image, w.adjoint, w.stops, w.fixedScale,
-                                                  reinterpret_cast<unsigned long long *>(w.rawFixed), w.rawFloat, nullptr, batch,
+                                                  reinterpret_cast<unsigned long long *>(w.rawFixed), w.rawFloat, w.touched, nullptr, batch,
                                                   rowOffset, queue);
 }
 
@@ -797,7 +801,7 @@ template <bool Down> struct WideWalk {
   // The taken window's splats staged, those that can touch the block packed in
   // walk order; padded to whole chunks. Returns how many. (Two barriers: every
   // thread calls it; the batch may be read after it.)
-  __device__ __forceinline__ uint32_t stage(const BlockGeometry &geo, WideShared &shared, uint32_t rowBytes) const {
+  __device__ __forceinline__ uint32_t stage(const BlockGeometry &geo, WideShared &shared, uint32_t rowBytes, uint8_t *__restrict__ touched) const {
     Staged st{};
     bool keep = false;
     if (wanted) {
@@ -819,6 +823,7 @@ template <bool Down> struct WideWalk {
       const uint32_t slot = before + static_cast<uint32_t>(__popcll(mine & ((1ull << lane) - 1ull)));
       shared.batch[slot] = st;
       shared.rowOffset[slot] = static_cast<uint64_t>(gaussian) * rowBytes;
+      if (touched != nullptr) touched[gaussian] = 1;
     }
     if (threadIdx.x < kWideChunk) shared.batch[total + threadIdx.x] = Staged{};
     __syncthreads();
@@ -862,7 +867,7 @@ __device__ __forceinline__ void composite_wide(const Splat *__restrict__ splats,
   WideWalk<true> walk{splats, entryKeys, entryValues, blockBit, range.x, range.y};
   walk.load_window();
   for (walk.take(); walk.more && doneLanes != ~0ull;) {
-    const uint32_t kept = walk.stage(geo, shared, 0u);
+    const uint32_t kept = walk.stage(geo, shared, 0u, nullptr);
     walk.take();
     float falloff[kWideShare];
     uint32_t buffer = 0;
@@ -958,7 +963,7 @@ __global__ __launch_bounds__(kWideThreads) void backward_wide_kernel(const Splat
                                                                      float bgB, const float4 *__restrict__ image,
                                                                      const float4 *__restrict__ adjoint, const uint32_t *__restrict__ stops,
                                                                      float fixedScale, unsigned long long *__restrict__ rawFixed,
-                                                                     float *__restrict__ rawFloat, const float *__restrict__ edge,
+                                                                     float *__restrict__ rawFloat, uint8_t *__restrict__ touched, const float *__restrict__ edge,
                                                                      const uint32_t *__restrict__ order) {
   __shared__ WideShared shared;
   uint32_t tile;
@@ -1002,7 +1007,7 @@ __global__ __launch_bounds__(kWideThreads) void backward_wide_kernel(const Splat
   WideWalk<false> walk{splats, entryKeys, entryValues, blockBit, range.y, first};
   walk.load_window();
   for (walk.take(); walk.more;) {
-    const uint32_t kept = walk.stage(geo, shared, kRawPerSplat * (Fixed ? 8u : 4u));
+    const uint32_t kept = walk.stage(geo, shared, kRawPerSplat * (Fixed ? 8u : 4u), touched);
     walk.take();
     uint32_t buffer = 0;
     float falloff[kWideShare], next[kWideShare];
@@ -1180,7 +1185,7 @@ void launch_forward(hipStream_t stream, const Splat *splats, const uint32_t *ent
 void launch_backward(hipStream_t stream, bool fixedPoint, bool recompute, const Splat *splats, const uint32_t *entryKeys,
                      const uint32_t *entryValues, uint32_t tileBits, const uint2 *ranges, uint32_t width, uint32_t height, uint32_t tileW,
                      uint32_t tileH, const float background[3], const float4 *image, const float4 *adjoint, const uint32_t *stops,
-                     float fixedScale, int64_t *rawFixed, float *rawFloat, const float *edge, const uint32_t *order) {
+                     float fixedScale, int64_t *rawFixed, float *rawFloat, uint8_t *touched, const float *edge, const uint32_t *order) {
   const uint32_t gridW = (width + tileW - 1) / tileW, gridH = (height + tileH - 1) / tileH;
   const bool score = edge != nullptr;
   const int variant = (fixedPoint ? 4 : 0) | (recompute ? 2 : 0) | (score ? 1 : 0);
@@ -1188,7 +1193,7 @@ void launch_backward(hipStream_t stream, bool fixedPoint, bool recompute, const 
 #define VSPLAT_BACKWARD_WIDE(F, R, S)                                                                                               \
   hipLaunchKernelGGL((backward_wide_kernel<F, R, S>), dim3(raster_blocks(gridW * gridH, tileW, tileH)), dim3(kWideThreads), 0, stream, \
                      splats, entryKeys, entryValues, tileBits, ranges, width, height, tileW, tileH, gridW, background[0], background[1], \
-                     background[2], image, adjoint, stops, fixedScale, reinterpret_cast<unsigned long long *>(rawFixed), rawFloat, edge, order)
+                     background[2], image, adjoint, stops, fixedScale, reinterpret_cast<unsigned long long *>(rawFixed), rawFloat, touched, edge, order)
     switch (variant) {
     case 7: VSPLAT_BACKWARD_WIDE(true, true, true); break;
     case 6: VSPLAT_BACKWARD_WIDE(true, true, false); break;
@@ -1205,7 +1210,7 @@ void launch_backward(hipStream_t stream, bool fixedPoint, bool recompute, const 
 #define VSPLAT_BACKWARD_SHAPE(F, R, S, W, H)                                                                                       \
   hipLaunchKernelGGL((backward_kernel<F, R, S, W, H>), dim3(raster_blocks(gridW * gridH, W, H)), dim3(kBlock), 0, stream, splats,   \
                      entryKeys, entryValues, tileBits, ranges, width, height, gridW, background[0], background[1], background[2], image, \
-                     adjoint, stops, fixedScale, reinterpret_cast<unsigned long long *>(rawFixed), rawFloat, edge, order)
+                     adjoint, stops, fixedScale, reinterpret_cast<unsigned long long *>(rawFixed), rawFloat, touched, edge, order)
 #define VSPLAT_BACKWARD_TTT(W, H) VSPLAT_BACKWARD_SHAPE(true, true, true, W, H)
 #define VSPLAT_BACKWARD_TTF(W, H) VSPLAT_BACKWARD_SHAPE(true, true, false, W, H)
 #define VSPLAT_BACKWARD_TFT(W, H) VSPLAT_BACKWARD_SHAPE(true, false, true, W, H)

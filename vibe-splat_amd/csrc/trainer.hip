@@ -306,11 +306,9 @@ void Trainer::upload_cloud(const vsplat_cloud &c, DeviceArray *const values[5]) 
 }
 
 // The per-Gaussian buffers the views share (trainer.cpp:242-262), cleared:
-// densification statistics, 3D filter values, the SH pass's scratch.
+// densification statistics, 3D filter values, the chain rule's scratch.
 void Trainer::allocate_per_gaussian() {
   const size_t n = count_;
-  shPass_.ensure(n * kShPassFloats * 4);
-  launch_fill_u32(stream_, shPass_.as<uint32_t>(), n * kShPassFloats, 0u);
   dirTerms_.ensure(n * 16);
   stats_.ensure(n * 32);
   launch_fill_u32(stream_, stats_.as<uint32_t>(), n * 8, 0u);
@@ -380,6 +378,8 @@ ViewBuffers &Trainer::view_buffers(size_t k) {
       v->rawFloat.ensure(n * kRawPerSplat * 4);
       launch_fill_u32(v->stream, v->rawFloat.as<uint32_t>(), n * kRawPerSplat, 0u);
     }
+    v->touched.ensure(div_up(n, 4) * 4);
+    launch_fill_u32(v->stream, v->touched.as<uint32_t>(), div_up(n, 4), 0u);
     v->scanScratch.ensure(coverage_scan_words(static_cast<uint32_t>(n)) * 4);
     v->sortScratch.ensure(radix_sort_scratch_words(n) * 4);
     v->sortCounts.ensure((radix_count_words(n, 32) + kEntryCountWords) * 4);
@@ -811,7 +811,7 @@ void Trainer::enqueue_passes(ViewBuffers &b, const ViewParams &view, const uint8
                   b.entryValues.as<uint32_t>(), b.tileBits, b.ranges.as<uint2>(), v.width, v.height, b.tileW, b.tileH, options_.background,
                   b.image.as<float4>(),
                   b.adjoint.as<float4>(), b.stops.as<uint32_t>(), fixed_scale(v), b.rawFixed.as<int64_t>(), b.rawFloat.as<float>(),
-                  scoring ? b.edge.as<float>() : nullptr, blockOrder);
+                  b.touched.as<uint8_t>(), scoring ? b.edge.as<float>() : nullptr, blockOrder);
   mark("backward");
   if (!chain) return;
   enqueue_chain(b, v, mode, rates, b.stream, b.counters.as<uint32_t>());
@@ -895,9 +895,8 @@ void Trainer::enqueue_loss(ViewBuffers &b, const ViewParams &v, const uint8_t *d
     launch_exposure_backward(s, b.image.as<float4>(), b.adjoint.as<float4>(), pixels, exposure_, b.exposureTotals.as<float>());
   }
   if (scoring) launch_error_mask(s, b.adjoint.as<float4>(), b.errorMax.as<uint32_t>(), pixels, scoreShare_);
-  launch_total_and_clear(s, b.tileTotals.as<float2>(), b.lossTiles, b.sums.as<double>(),
-                         fixedPoint_ ? b.rawFixed.as<uint32_t>() : b.rawFloat.as<uint32_t>(),
-                         static_cast<uint64_t>(count_) * kRawPerSplat * (fixedPoint_ ? 2u : 1u));
+  launch_total_and_clear(s, b.tileTotals.as<float2>(), b.lossTiles, b.sums.as<double>(), fixedPoint_, raw_sums(b), b.touched.as<uint8_t>(),
+                         count_);
 }
 
 ChainParams Trainer::chain_params(const ViewParams &v, uint32_t mode, const vsplat_learning_rates *rates) const {
@@ -950,6 +949,8 @@ void Trainer::ensure_gradients() {
   for (int g = 0; g < 5; ++g) grad_[g].ensure(floats[g] * 4);
 }
 
+void *Trainer::raw_sums(const ViewBuffers &b) const { return fixedPoint_ ? b.rawFixed.as<void>() : b.rawFloat.as<void>(); }
+
 ChainBuffers Trainer::chain_buffers(const ViewBuffers &v) const {
   ChainBuffers b{};
   b.positions = positions_.as<float>();
@@ -962,7 +963,7 @@ ChainBuffers Trainer::chain_buffers(const ViewBuffers &v) const {
   b.splats = v.splats.as<Splat>();
   b.rawFixed = v.rawFixed.as<int64_t>();
   b.rawFloat = v.rawFloat.as<float>();
-  b.shPass = shPass_.as<float>();
+  b.touched = v.touched.as<uint8_t>();
   b.stats = stats_.as<float>();
   b.statePos = state_[0].as<uint32_t>();
   b.stateScale = state_[1].as<uint32_t>();
@@ -1476,6 +1477,7 @@ void Trainer::launch_batch_raster(uint32_t n, const ViewParams *params, bool bac
       w.adjoint = b.adjoint.as<float4>();
       w.rawFixed = fixedPoint_ ? b.rawFixed.as<int64_t>() : nullptr;
       w.rawFloat = b.rawFloat.as<float>();
+      w.touched = b.touched.as<uint8_t>();
       w.fixedScale = fixed_scale(params[k]);
       w.width = b.width;
       w.height = b.height;
@@ -1510,6 +1512,7 @@ void Trainer::enqueue_view_chains(uint32_t n, const ViewParams *params, uint32_t
       w.rawFixed = fixedPoint_ ? b.rawFixed.as<int64_t>() : nullptr;
       w.rawFloat = b.rawFloat.as<float>();
       w.splats = b.splats.as<Splat>();
+      w.touched = b.touched.as<uint8_t>();
       w.fixedScale = fixed_scale(w.c);
     }
     accumulateNext_ = first > 0;
@@ -1554,7 +1557,7 @@ uint64_t Trainer::capture_key(uint32_t n) const {
     mix(reinterpret_cast<uintptr_t>(a.as<void>()));
     mix(a.bytes());
   };
-  for (const DeviceArray *a : {&positions_, &scales_, &rotations_, &opacities_, &shWordsBuf_, &adamState_, &shPass_, &stats_, &filter3d_})
+  for (const DeviceArray *a : {&positions_, &scales_, &rotations_, &opacities_, &shWordsBuf_, &adamState_, &stats_, &filter3d_})
     array(*a);
   mix(reinterpret_cast<uintptr_t>(viewStats_.as<void>()));
   for (int g = 0; g < 5; ++g) {
@@ -1565,7 +1568,7 @@ uint64_t Trainer::capture_key(uint32_t n) const {
   for (uint32_t k = 0; k < n && k < views_.size(); ++k) {
     const ViewBuffers &b = *views_[k];
     for (const DeviceArray *a : {&b.splats, &b.keys, &b.values, &b.tmpKeys, &b.tmpValues, &b.coverage, &b.tileCount, &b.tileRecords,
-                                 &b.bigList, &b.bigBits, &b.rawFixed, &b.rawFloat, &b.entryKeys, &b.entryValues, &b.tmpEntryKeys, &b.tmpEntryValues, &b.image,
+                                 &b.bigList, &b.bigBits, &b.rawFixed, &b.rawFloat, &b.touched, &b.entryKeys, &b.entryValues, &b.tmpEntryKeys, &b.tmpEntryValues, &b.image,
                                  &b.stops, &b.adjoint, &b.fields, &b.ranges, &b.tileTotals, &b.listOrder, &b.blockWork, &b.blockOrder, &b.sortScratch,
                                  &b.sortCounts, &b.scanScratch, &b.counters, &b.sums})
       array(*a);
@@ -1855,16 +1858,12 @@ void Trainer::update_curvature() {
   const uint32_t pixels = v.width * v.height;
   uint32_t *counters = b.counters.as<uint32_t>();
   launch_hutchinson(stream_, b.adjoint.as<float4>(), pixels, curvatureUpdates_);
-  if (fixedPoint_) {
-    launch_fill_u32(stream_, b.rawFixed.as<uint32_t>(), static_cast<uint64_t>(count_) * kRawPerSplat * 2, 0u);
-  } else {
-    launch_fill_u32(stream_, b.rawFloat.as<uint32_t>(), static_cast<uint64_t>(count_) * kRawPerSplat, 0u);
-  }
+  launch_total_and_clear(stream_, nullptr, 0, nullptr, fixedPoint_, raw_sums(b), b.touched.as<uint8_t>(), count_);
   launch_backward(stream_, fixedPoint_, options_.recompute_transmittance != 0, b.splats.as<Splat>(), b.entryKeys.as<uint32_t>(),
                   b.entryValues.as<uint32_t>(), b.tileBits, b.ranges.as<uint2>(), v.width, v.height, b.tileW, b.tileH, options_.background,
                   b.image.as<float4>(),
                   b.adjoint.as<float4>(), b.stops.as<uint32_t>(), curvature_fixed_scale(), b.rawFixed.as<int64_t>(),
-                  b.rawFloat.as<float>());
+                  b.rawFloat.as<float>(), b.touched.as<uint8_t>());
   const bool statistics = statisticsNext_;
   statisticsNext_ = false; // the curvature adds nothing to the densification statistics
   enqueue_chain(b, v, kModeCurvature, nullptr, stream_, counters);
@@ -1908,7 +1907,7 @@ uint64_t Trainer::bytes_per_gaussian() const {
   // splat list, tile record, sums, SH-pass data, the direction term between the
   // chain kernels, statistics.
   const uint64_t raw = fixedPoint_ ? kRawPerSplat * 8 : kRawPerSplat * 4;
-  return parameters + sizeof(Splat) + 4 * 8 + sizeof(TileRecord) + raw + kShPassFloats * 4 + 16 + 32;
+  return parameters + sizeof(Splat) + 4 * 8 + sizeof(TileRecord) + raw + 1 + 16 + 32;
 }
 
 uint64_t Trainer::gpu_bytes() const {
@@ -1923,7 +1922,7 @@ uint64_t Trainer::gpu_bytes() const {
     }
     if (k == 0) continue;
     for (const DeviceArray *a : {&b.splats, &b.keys, &b.values, &b.tmpKeys, &b.tmpValues, &b.coverage, &b.tileCount, &b.tileRecords,
-                                 &b.bigList, &b.rawFixed, &b.rawFloat, &b.sortScratch, &b.sortCounts, &b.scanScratch}) {
+                                 &b.bigList, &b.rawFixed, &b.rawFloat, &b.touched, &b.sortScratch, &b.sortCounts, &b.scanScratch}) {
       total += a->bytes();
     }
   }

@@ -127,6 +127,9 @@ struct ViewBuffers {
   uint64_t entryCapacity = 0;
   // Per Gaussian.
   DeviceArray splats, keys, values, tmpKeys, tmpValues, coverage, tileCount, tileRecords, bigList, bigBits, rawFixed, rawFloat;
+  // A byte per Gaussian, nonzero where the raw sums may not be zero: set by the
+  // backward pass, cleared with the sums before the next.
+  DeviceArray touched;
   // Per tile entry.
   DeviceArray entryKeys, entryValues, tmpEntryKeys, tmpEntryValues;
   // Per pixel and per tile; per 8x8 block (raster launch index), the backward's
@@ -222,6 +225,7 @@ private:
   void allocate_per_gaussian();
   void ensure_size(ViewBuffers &b, int width, int height);
   void gather_view_status(uint32_t n);
+  void *raw_sums(const ViewBuffers &b) const;
   void finish_pass(const ViewBuffers &b, bool step);
   void ensure_layout(ViewBuffers &b, int width, int height, uint32_t tileW, uint32_t tileH);
   static void set_geometry(ViewBuffers &b, int width, int height, uint32_t tileW, uint32_t tileH);
@@ -292,7 +296,7 @@ private:
   DeviceArray state_[5], grad_[5];
   DeviceArray adamState_; // steps taken, beta1^steps, beta2^steps (ChainParams::adamState)
   // Per Gaussian, shared by the views.
-  DeviceArray shPass_, stats_, filter3d_, dirTerms_;
+  DeviceArray stats_, filter3d_, dirTerms_;
   bool filterSet_ = false;
   // The views' buffers; the first is the single-view calls' and runs on stream_.
   std::vector<std::unique_ptr<ViewBuffers>> views_;
