@@ -66,3 +66,25 @@ def test_steps_match_the_model(count, degree, storage, selective, hidden):
                 np.testing.assert_array_equal(got, want)
         touched = np.count_nonzero((r.raw_fixed.reshape(count, 14) != 0).any(axis=1))
         print(f"{touched} of {count} touched", flush=True)
+
+
+@pytest.mark.parametrize("views", [1, 3, 9])
+@pytest.mark.parametrize("count,degree,storage", [(1, 0, vsplat.SH_HALF), (65, 3, vsplat.SH_BF16), (1025, 3, vsplat.SH_HALF), (33_000, 1, vsplat.SH_HALF),
+                                                  (600_000, 0, vsplat.SH_BF16)])
+def test_a_batch_steps_as_its_gradients_applied(count, degree, storage, views):
+    """A batch's step, which visits the Gaussians that a view saw, against its summed gradients, stored for all of them, then applied; two in a row."""
+    cloud = _cloud(count, degree, True)
+    cams = [F.look_at((0.5 * np.sin(k), 0.2 * k, -3 + 0.1 * k), (0, 0, 0), (0.0, -1.0, 0.0), 60.0, 96 + 8 * k, 80) for k in range(views)]
+    targets = [F.smooth_target(c.width, c.height, 3 + k) for k, c in enumerate(cams)]
+    options = vsplat.TrainerOptions(force_fixed_point=True, sh_storage=storage)
+    with vsplat.Trainer(cloud, options) as a, vsplat.Trainer(cloud, options) as b:
+        for _ in range(2):
+            a.step_views(cams, targets, RATES)
+            b.step_views(cams, targets)
+            b.apply_gradients(RATES)
+            x, y = a.cloud(), b.cloud()
+            for name in ("positions", "scales", "rotations", "opacities", "sh"):
+                np.testing.assert_array_equal(_bits(getattr(x, name)), _bits(getattr(y, name)))
+            for got, want in zip(_states(a), _states(b)):
+                np.testing.assert_array_equal(got, want)
+            np.testing.assert_array_equal(a.densify_stats(), b.densify_stats())

@@ -633,133 +633,6 @@ __global__ __launch_bounds__(kChainThreads) void chain_geometry_gradients_kernel
   emit_terms(B, o, i, t, Radii{-1.0f, -1.0f, -1.0f});
 }
 
-// The batched chain rule (no reference counterpart): for each Gaussian, every
-// view of the batch in turn, each view's terms added to the sums in view order
-// in float32 (the first view's are the sums' start), so the result is the
-// per-view chain rule's gradients added up in that order. Unlike the
-// single-view chain rule it stays one kernel: split, the second half would
-// read every view's raw sums and direction terms again (about 1 GB for eight
-// views at 1M Gaussians), which measured slower. What does not depend on the
-// view (the Gaussian's frame) is computed once, and each view's raw sums are
-// loaded while the view before is worked, which the kernel's low occupancy
-// (its LDS) needs to keep loads in flight. The geometric sums stay in
-// registers and the SH sums in LDS, one row per coefficient so that a wave's
-// lanes hit consecutive banks. In gradients mode the sums are stored; in step
-// mode the geometric parameters take Adam's step from them here, and the SH
-// sums are stored for the SH step.
-template <int Degree, uint32_t Format>
-__global__ __launch_bounds__(kChainThreads) void chain_views_kernel(ChainBuffers B, ChainViews views, ChainParams o,
-                                                                   const uint32_t *counters) {
-  constexpr uint32_t kCoefficients = (Degree + 1) * (Degree + 1);
-  __shared__ float shSum[kCoefficients * 3][kChainThreads];
-  __shared__ uint32_t stage[kChainThreads * 26];
-  const uint32_t lane = threadIdx.x;
-  const uint32_t i = blockIdx.x * blockDim.x + lane;
-  const uint32_t count = views.view[0].c.count, shWords = views.view[0].c.shWords;
-  if (counters[kOverflow] != 0) return;
-  {
-    // The block's SH words, read by every view: staged once through LDS with
-    // 16-byte loads (measured faster here than each view reading them again).
-    const uint32_t first = blockIdx.x * kChainThreads;
-    const uint32_t inBlock = count - first < kChainThreads ? count - first : kChainThreads;
-    stage_words<kChainThreads>(stage, B.shWords + static_cast<size_t>(first) * shWords, inBlock * shWords);
-    __syncthreads();
-  }
-  if (i >= count) return;
-  const uint32_t *words = stage + lane * shWords;
-  if (o.mode == kModeStep) adam_step_now(o);
-  const bool penalties = o.opacityReg > 0.0f || o.scaleReg > 0.0f;
-  const bool statistics = (o.flags & kFlagStatistics) != 0 && B.stats != nullptr;
-  // A later chunk of a batch continues from the sums the earlier ones stored.
-  ViewTerms sum;
-  bool started = (o.flags & kFlagAccumulate) != 0;
-  if (started) {
-#pragma unroll
-    for (uint32_t k = 0; k < 3; ++k) {
-      sum.position[k] = B.gradPos[i * 3 + k];
-      sum.scale[k] = B.gradScale[i * 3 + k];
-    }
-#pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) sum.rotation[k] = B.gradRot[i * 4 + k];
-    sum.opacity = B.gradOpacity[i];
-    const float *prev = B.gradSh + static_cast<size_t>(i) * o.shFloats;
-#pragma unroll
-    for (uint32_t j = 0; j < kCoefficients * 3; ++j) shSum[j][lane] = prev[j];
-  }
-  o.flags &= ~kFlagAccumulate; // the sums below are complete: they are stored, not added
-  float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b = a;
-  bool statsChanged = false;
-  GaussianFrame G;
-  gaussian_frame(B, i, G);
-  // Each view's raw sums are loaded kAhead views ahead of the view being worked,
-  // in kAhead register sets that the unrolled loop uses in turn: two where the
-  // kernel stays within 256 VGPRs with them (two waves per SIMD), one for
-  // degree 3 with 16-bit SH, whose larger SH terms leave no room.
-  constexpr uint32_t kAhead = Degree == 3 && Format != kShBf16 ? 1u : 2u;
-  uint32_t raw[kAhead][2 * kRawPerSplat];
-  float radius[kAhead];
-#pragma unroll
-  for (uint32_t k = 0; k < kAhead; ++k) {
-    radius[k] = 0.0f;
-    if (k < views.count) fetch_raw(views.view[k], i, statistics, raw[k], radius[k]);
-  }
-#pragma unroll
-  for (uint32_t v = 0; v < kChainViewsPerLaunch; ++v) {
-    if (v >= views.count) break;
-    const ChainView &w = views.view[v];
-    const uint32_t set = v % kAhead;
-    float g[kRawPerSplat];
-    const bool touched = convert_fetched(raw[set], w.rawFixed != nullptr, w.fixedScale, g);
-    const float viewRadius = radius[set];
-    if (v + kAhead < views.count) fetch_raw(views.view[v + kAhead], i, statistics, raw[set], radius[set]);
-    if (touched && statistics) {
-      if (!statsChanged) {
-        const float4 *st = reinterpret_cast<const float4 *>(B.stats + static_cast<size_t>(i) * 8);
-        a = st[0];
-        b = st[1];
-        statsChanged = true;
-      }
-      add_statistics(a, b, g, static_cast<float>(w.c.width), static_cast<float>(w.c.height), viewRadius);
-    }
-    ViewTerms t;
-    if (touched) {
-      view_terms<Degree, Format>(G, w.c, o, i, words, g, t, [&](const float basis[16], const float gcu[3], const float[3], uint32_t used) {
-#pragma unroll
-        for (uint32_t k = 0; k < kCoefficients; ++k)
-#pragma unroll
-          for (uint32_t ch = 0; ch < 3; ++ch) {
-            const float x = k < used ? basis[k] * gcu[ch] : 0.0f;
-            shSum[k * 3 + ch][lane] = started ? shSum[k * 3 + ch][lane] + x : x;
-          }
-      });
-    } else {
-      untouched_terms(G, o, penalties, t);
-#pragma unroll
-      for (uint32_t j = 0; j < kCoefficients * 3; ++j) shSum[j][lane] = started ? shSum[j][lane] + 0.0f : 0.0f;
-    }
-#pragma unroll
-    for (uint32_t k = 0; k < 3; ++k) {
-      sum.position[k] = started ? sum.position[k] + t.position[k] : t.position[k];
-      sum.scale[k] = started ? sum.scale[k] + t.scale[k] : t.scale[k];
-    }
-#pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) sum.rotation[k] = started ? sum.rotation[k] + t.rotation[k] : t.rotation[k];
-    sum.opacity = started ? sum.opacity + t.opacity : t.opacity;
-    started = true;
-  }
-  if (statsChanged) {
-    float4 *st = reinterpret_cast<float4 *>(B.stats + static_cast<size_t>(i) * 8);
-    st[0] = a;
-    st[1] = b;
-  }
-  // Coefficients above the active degree get zero (they are stored, not trained).
-  float *out = B.gradSh + static_cast<size_t>(i) * o.shFloats;
-#pragma unroll
-  for (uint32_t j = 0; j < kCoefficients * 3; ++j) out[j] = shSum[j][lane];
-  for (uint32_t j = kCoefficients * 3; j < o.shFloats; ++j) out[j] = 0.0f;
-  emit_terms(B, o, i, sum, Radii{-1.0f, -1.0f, -1.0f}); // a batch takes Adam's step
-}
-
 // The SH floats packed word q holds: [first, last].
 __device__ __forceinline__ void sh_word_floats(uint32_t format, uint32_t q, uint32_t shFloats, uint32_t &first, uint32_t &last) {
   if (format == kShBf16) {
@@ -811,7 +684,7 @@ __device__ __forceinline__ uint32_t sh_word_put(uint32_t format, uint32_t word, 
 // 28 for 29 (30k). Then it is bound by the step's own instructions (some 200 a
 // parameter, divisions, a square root and two hashes), where few are seen by the
 // way to memory of one after the other: flags, sums, parameters, moments.
-constexpr uint32_t kStepSlots = kChainThreads / 2, kStepMost = 4096, kStepLeast = 64, kFlagged = 0x8000u;
+constexpr uint32_t kStepSlots = kChainThreads / 2, kStepMost = 4096, kViewsMost = 1024, kStepLeast = 64, kFlagged = 0x8000u;
 // What the step takes of a Gaussian. The rows' lengths are odd, so that
 // neighbouring rows lie on different banks.
 struct ShRow {
@@ -1047,6 +920,196 @@ __global__ __launch_bounds__(kChainThreads, 4) void chain_step_kernel(ChainBuffe
   }
 }
 
+// The batched chain rule (no reference counterpart): for each Gaussian, every
+// view of the batch in turn, each view's terms added to the sums in view order
+// in float32 (the first view's are the sums' start), so the result is the
+// per-view chain rule's gradients added up in that order. What does not depend
+// on the view (the Gaussian's frame) is computed once, and each view's raw sums
+// are loaded while the view before is worked, which the kernel's low occupancy
+// (its LDS) needs to keep loads in flight. The geometric sums stay in
+// registers and the SH sums in LDS, one row per coefficient (of an odd length, so
+// that lanes on one coefficient and lanes on one Gaussian both hit distinct
+// banks). In gradients mode the sums are stored; in step mode every parameter
+// takes Adam's step from them here.
+//
+// A workgroup takes perBlock neighbouring Gaussians. Unless all have something to
+// store or to step, it packs those that a view's backward pass added to at the
+// front of a list, as chain_step_kernel does, and a view's sums are read only for
+// the Gaussians it added to. A step over eight views of 1M Gaussians: 245 us,
+// before (all Gaussians, the SH sums through memory to a kernel of their own) 606
+// and 134; gradients of three views of 40k: 25 us.
+template <int Degree, uint32_t Format>
+__global__ __launch_bounds__(kChainThreads) void chain_views_kernel(ChainBuffers B, ChainViews views, ChainParams o, uint32_t perBlock,
+                                                                   const uint32_t *counters) {
+  constexpr uint32_t kCoefficients = (Degree + 1) * (Degree + 1), kSums = kChainThreads + 1;
+  constexpr uint32_t kRound = 4 * kChainThreads, kRounds = kViewsMost / kRound;
+  __shared__ float shSum[kCoefficients * 3][kSums];
+  __shared__ uint32_t stage[kChainThreads * 26];
+  __shared__ uint16_t list[kViewsMost];
+  __shared__ uint8_t seenBy[kViewsMost]; // per listed Gaussian, the views whose sums may not be zero
+  __shared__ uint32_t waveTotals[kChainThreads / 64];
+  const uint32_t lane = threadIdx.x;
+  const uint32_t count = views.view[0].c.count, shWords = views.view[0].c.shWords;
+  if (counters[kOverflow] != 0) return;
+  const uint32_t first = blockIdx.x * perBlock;
+  const uint32_t mine = count - first < perBlock ? count - first : perBlock;
+  const bool penalties = o.opacityReg > 0.0f || o.scaleReg > 0.0f;
+  const bool zeros = (o.flags & kFlagSelective) == 0, accumulate = (o.flags & kFlagAccumulate) != 0;
+  const bool everyone = o.mode != kModeStep || zeros || penalties || accumulate;
+  uint32_t listed = 0;
+  for (uint32_t r = 0; r < kRounds && r * kRound < mine; ++r) {
+    const uint32_t x0 = r * kRound + threadIdx.x * 4u;
+    uint32_t seen = 0; // a byte each for four neighbours
+#pragma unroll
+    for (uint32_t v = 0; v < kChainViewsPerLaunch; ++v) {
+      const uint32_t flags = v < views.count && x0 < mine ? reinterpret_cast<const uint32_t *>(views.view[v].touched + first)[x0 / 4u] : 0u;
+      seen |= flags << v; // a flag is 0 or 1
+    }
+    uint32_t wanted = 0, at;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+      if (x0 + k < mine && (everyone || ((seen >> (8u * k)) & 0xFFu) != 0)) wanted |= 1u << k;
+    }
+    const uint32_t total = block_exclusive_sum(static_cast<uint32_t>(__popc(wanted)), at, waveTotals);
+    at += listed;
+    listed += total;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+      if (((wanted >> k) & 1u) == 0) continue;
+      list[at] = static_cast<uint16_t>(x0 + k);
+      seenBy[at++] = static_cast<uint8_t>(seen >> (8u * k));
+    }
+  }
+  if (o.mode == kModeStep) adam_step_now(o);
+  const bool statistics = (o.flags & kFlagStatistics) != 0 && B.stats != nullptr;
+  o.flags &= ~kFlagAccumulate; // the sums below are complete: they are stored, not added
+  for (uint32_t from = 0; from < listed; from += kChainThreads) {
+    const uint32_t n = listed - from < kChainThreads ? listed - from : kChainThreads;
+    __syncthreads(); // the list is whole, the sums before are read
+    // The SH words, read by every view, staged once through LDS.
+    const float perWord = 1.0f / static_cast<float>(shWords);
+    for (uint32_t x = lane; x < n * shWords; x += kChainThreads) {
+      const uint32_t t = static_cast<uint32_t>((static_cast<float>(x) + 0.5f) * perWord); // exact for x < 2^13
+      stage[x] = B.shWords[static_cast<size_t>(first + list[from + t]) * shWords + (x - t * shWords)];
+    }
+    __syncthreads();
+    if (lane < n) {
+      const uint32_t i = first + list[from + lane], seen = seenBy[from + lane];
+      const uint32_t *words = stage + lane * shWords;
+      // A later chunk of a batch continues from the sums the earlier ones stored.
+      ViewTerms sum;
+      bool started = accumulate;
+      if (started) {
+#pragma unroll
+        for (uint32_t k = 0; k < 3; ++k) {
+          sum.position[k] = B.gradPos[i * 3 + k];
+          sum.scale[k] = B.gradScale[i * 3 + k];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) sum.rotation[k] = B.gradRot[i * 4 + k];
+        sum.opacity = B.gradOpacity[i];
+        const float *prev = B.gradSh + static_cast<size_t>(i) * o.shFloats;
+#pragma unroll
+        for (uint32_t j = 0; j < kCoefficients * 3; ++j) shSum[j][lane] = prev[j];
+      }
+      float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b = a;
+      bool statsChanged = false;
+      GaussianFrame G;
+      gaussian_frame(B, i, G);
+      // Each view's raw sums are loaded while the view before is worked. The loop is
+      // not unrolled: eight copies of the terms are 90 KB of instructions.
+      uint32_t raw[2 * kRawPerSplat];
+      float radius = 0.0f;
+      bool shStarted = started, missed = false; // missed: a view that adds nothing
+      if ((seen & 1u) != 0) fetch_raw(views.view[0], i, statistics, raw, radius);
+#pragma unroll 1
+      for (uint32_t v = 0; v < views.count; ++v) {
+        const ChainView &w = views.view[v];
+        float g[kRawPerSplat];
+        const bool touched = ((seen >> v) & 1u) != 0 && convert_fetched(raw, w.rawFixed != nullptr, w.fixedScale, g);
+        const float viewRadius = radius;
+        if (((seen >> (v + 1u)) & 1u) != 0) fetch_raw(views.view[v + 1u], i, statistics, raw, radius);
+        if (touched && statistics) {
+          if (!statsChanged) {
+            const float4 *st = reinterpret_cast<const float4 *>(B.stats + static_cast<size_t>(i) * 8);
+            a = st[0];
+            b = st[1];
+            statsChanged = true;
+          }
+          add_statistics(a, b, g, static_cast<float>(w.c.width), static_cast<float>(w.c.height), viewRadius);
+        }
+        ViewTerms t;
+        if (touched) {
+          view_terms<Degree, Format>(G, w.c, o, i, words, g, t, [&](const float basis[16], const float gcu[3], const float[3], uint32_t used) {
+#pragma unroll
+            for (uint32_t k = 0; k < kCoefficients; ++k)
+#pragma unroll
+              for (uint32_t ch = 0; ch < 3; ++ch) {
+                const float x = k < used ? basis[k] * gcu[ch] : 0.0f;
+                shSum[k * 3 + ch][lane] = shStarted ? shSum[k * 3 + ch][lane] + x : x;
+              }
+          });
+          shStarted = true;
+        } else {
+          untouched_terms(G, o, penalties, t);
+          missed = true;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 3; ++k) {
+          sum.position[k] = started ? sum.position[k] + t.position[k] : t.position[k];
+          sum.scale[k] = started ? sum.scale[k] + t.scale[k] : t.scale[k];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) sum.rotation[k] = started ? sum.rotation[k] + t.rotation[k] : t.rotation[k];
+        sum.opacity = started ? sum.opacity + t.opacity : t.opacity;
+        started = true;
+      }
+      // The zeros that the missed views would have added to the SH sums: wherever
+      // in the order, they only make a sum of negative zeros a positive one.
+      if (missed) {
+#pragma unroll 4
+        for (uint32_t j = 0; j < kCoefficients * 3; ++j) shSum[j][lane] = shStarted ? shSum[j][lane] + 0.0f : 0.0f;
+      }
+      if (statsChanged) {
+        float4 *st = reinterpret_cast<float4 *>(B.stats + static_cast<size_t>(i) * 8);
+        st[0] = a;
+        st[1] = b;
+      }
+      emit_terms(B, o, i, sum, Radii{-1.0f, -1.0f, -1.0f}); // a batch takes Adam's step
+    }
+    __syncthreads(); // the SH sums are whole
+    if (o.mode == kModeStep) {
+      // As step_sh_words, with the gradients summed. Coefficients above the active degree have none.
+      for (uint32_t x = lane; x < n * shWords; x += kChainThreads) {
+        const uint32_t t = static_cast<uint32_t>((static_cast<float>(x) + 0.5f) * perWord), q = x - t * shWords, i = first + list[from + t];
+        uint32_t firstFloat, last, word = stage[x];
+        sh_word_floats(Format, q, o.shFloats, firstFloat, last);
+        bool changed = false;
+        for (uint32_t j = firstFloat; j <= last; ++j) {
+          const float gv = j < kCoefficients * 3 ? shSum[j][t] : 0.0f;
+          if (gv == 0.0f && !zeros) continue;
+          const uint32_t s = i * o.shFloats + j;
+          uint32_t state = B.stateSh[s];
+          float value = sh_word_get(Format, word, j, firstFloat);
+          step_parameter(o, value, state, gv, j < 3 ? o.rates[4] : o.rates[4] * o.restScale, -1.0f, s * 5u + 4u);
+          B.stateSh[s] = state;
+          word = sh_word_put(Format, word, j, firstFloat, value, s, o.seed);
+          changed = true;
+        }
+        if (changed) B.shWords[static_cast<size_t>(i) * shWords + q] = word;
+      }
+    } else {
+      // Coefficients above the active degree get zero (they are stored, not trained).
+      const uint32_t floats = o.shFloats;
+      const float perFloat = 1.0f / static_cast<float>(floats);
+      for (uint32_t x = lane; x < n * floats; x += kChainThreads) {
+        const uint32_t t = static_cast<uint32_t>((static_cast<float>(x) + 0.5f) * perFloat), j = x - t * floats; // exact for x < 2^14
+        B.gradSh[static_cast<size_t>(first + list[from + t]) * floats + j] = j < kCoefficients * 3 ? shSum[j][t] : 0.0f;
+      }
+    }
+  }
+}
+
 // One Adam step from summed gradients (the batched step): thread t takes
 // parameter t of positions, scales, rotations and opacities in turn, with the
 // same rule and the same rounding stream (index at * 5 + group) as the chain
@@ -1244,6 +1307,13 @@ __global__ __launch_bounds__(256) void keep_first_moment_kernel(uint32_t *__rest
   default: LAUNCH(3, kShBf16); break;                                                                                              \
   }
 
+// The Gaussians of a workgroup: equal shares for as many workgroups as are
+// resident, a multiple of four so that their flags are whole words.
+static uint32_t chain_share(uint32_t count, uint32_t perCu, uint32_t most) {
+  const uint32_t share = ((count + perCu * 256 - 1) / (perCu * 256) + 3) / 4 * 4;
+  return share < kStepLeast ? kStepLeast : (share < most ? share : most);
+}
+
 void launch_chain(hipStream_t stream, const ChainBuffers &buffers, const ViewParams &view, const ChainParams &params,
                   const uint32_t *counters) {
   if (view.count == 0) return;
@@ -1256,11 +1326,7 @@ void launch_chain(hipStream_t stream, const ChainBuffers &buffers, const ViewPar
     hipLaunchKernelGGL(chain_geometry_gradients_kernel, grid, block, 0, stream, buffers, view, params, counters);
     return;
   }
-  // Four workgroups a CU are resident: as many, with as equal shares as can be
-  // (a multiple of four Gaussians each, so that their flags are whole words).
-  constexpr uint32_t kResident = 4 * 256;
-  const uint32_t share = ((view.count + kResident - 1) / kResident + 3) / 4 * 4;
-  const uint32_t perBlock = share < kStepLeast ? kStepLeast : (share < kStepMost ? share : kStepMost);
+  const uint32_t perBlock = chain_share(view.count, 4, kStepMost); // four workgroups a CU are resident
 #define VSPLAT_CHAIN(D, F)                                                                                                         \
   hipLaunchKernelGGL((chain_step_kernel<D, F>), dim3((view.count + perBlock - 1) / perBlock), block, 0, stream, buffers, view, params, \
                      perBlock, counters)
@@ -1272,18 +1338,12 @@ void launch_chain_views(hipStream_t stream, const ChainBuffers &buffers, const C
                         const uint32_t *counters) {
   const uint32_t count = views.view[0].c.count;
   if (count == 0 || views.count == 0) return;
-  const dim3 grid((count + 255) / 256), block(256);
-#define VSPLAT_CHAIN(D, F) hipLaunchKernelGGL((chain_views_kernel<D, F>), grid, block, 0, stream, buffers, views, params, counters)
+  // Two workgroups a CU are resident.
+  const uint32_t perBlock = chain_share(count, 2, kViewsMost);
+  const dim3 grid((count + perBlock - 1) / perBlock), block(256);
+#define VSPLAT_CHAIN(D, F) hipLaunchKernelGGL((chain_views_kernel<D, F>), grid, block, 0, stream, buffers, views, params, perBlock, counters)
   VSPLAT_SH_DISPATCH(views.view[0].c.shDegree, views.view[0].c.shFormat, VSPLAT_CHAIN)
 #undef VSPLAT_CHAIN
-}
-
-void launch_sh_adam(hipStream_t stream, const ChainBuffers &buffers, const ViewParams &view, const ChainParams &params,
-                    const uint32_t *counters) {
-  if (view.count == 0) return;
-  const uint64_t words = static_cast<uint64_t>(view.count) * view.shWords;
-  hipLaunchKernelGGL(sh_adam_kernel, dim3(static_cast<uint32_t>((words + 255) / 256)), dim3(256), 0, stream, buffers.shWords,
-                     buffers.stateSh, buffers.gradSh, view, params, counters);
 }
 
 void launch_noise(hipStream_t stream, const ChainBuffers &buffers, uint32_t count, float scaler, const uint32_t *iterationDev,

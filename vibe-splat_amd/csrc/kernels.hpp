@@ -297,13 +297,9 @@ void launch_error_mask(hipStream_t stream, float4 *adjoint, const uint32_t *erro
 
 // The chain rule over the views of a batch chunk, summed per Gaussian in view
 // order (kFlagAccumulate: continuing from the sums an earlier chunk stored).
-// Gradients mode stores the sums; step mode takes the geometric parameters'
-// Adam step from them and stores the SH sums for launch_sh_adam.
+// Gradients mode stores the sums; step mode takes every parameter's Adam step from them.
 void launch_chain_views(hipStream_t stream, const ChainBuffers &buffers, const ChainViews &views, const ChainParams &params,
                         const uint32_t *counters);
-// Adam for the SH coefficients from the stored SH gradients.
-void launch_sh_adam(hipStream_t stream, const ChainBuffers &buffers, const ViewParams &view, const ChainParams &params,
-                    const uint32_t *counters);
 // One Adam step of every parameter from the stored gradients in buffers.grad*
 // (Trainer::apply_gradients); params.mode is kModeStep.
 void launch_adam(hipStream_t stream, const ChainBuffers &buffers, const ViewParams &view, const ChainParams &params,

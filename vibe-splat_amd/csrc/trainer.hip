@@ -1530,11 +1530,9 @@ void Trainer::enqueue_views(uint32_t n, const vsplat_camera *cameras, const uint
   enqueue_batch_passes(n, cameras, targets, params.data());
   uint32_t *status = views_[0]->counters.as<uint32_t>();
   enqueue_view_chains(n, params.data(), mode, rates);
-  const ChainBuffers buffers = chain_buffers(*views_[0]);
   lastView_ = params[n - 1];
   lastViewIndex_ = n - 1;
   if (mode == kModeStep) {
-    launch_sh_adam(stream_, buffers, lastView_, chain_params(lastView_, kModeStep, rates), status);
     finish_pass(*views_[0], true);
     enqueue_noise(*views_[0], rates, stream_, status);
   } else {
