@@ -748,28 +748,33 @@ __device__ __forceinline__ void step_geometry(const ChainBuffers &B, const Chain
 }
 
 // The packed SH words of the list's Gaussians stepped, or their curvature taken, a
-// thread a word, the next one's loads ahead.
-__device__ __forceinline__ void step_sh_words(const ChainBuffers &B, const ViewParams &c, const ChainParams &o, uint32_t first,
-                                              const uint16_t *list, uint32_t n, const ShRow *rows, bool zeros) {
-  const bool secondOrder = (o.flags & kFlagSecondOrder) != 0;
-  const uint32_t words = c.shWords, total = n * words;
+// thread a word, the next one's loads ahead. wanted(t): whether row t has any
+// gradients; wordOf(x, place): word x of the rows, the one at `place`;
+// gradient(t, j): of SH float j; radius(t, ch): second order's, else -1.
+template <typename Wanted, typename WordOf, typename Gradient, typename Radius>
+__device__ __forceinline__ void step_sh_words(const ChainBuffers &B, const ChainParams &o, uint32_t format, uint32_t words, uint32_t first,
+                                              const uint16_t *list, uint32_t n, bool zeros, Wanted &&wanted, WordOf &&wordOf,
+                                              Gradient &&gradient, Radius &&radius) {
+  const uint32_t total = n * words;
   const float perWord = 1.0f / static_cast<float>(words);
   struct Word {
-    uint32_t t, i, q, first, last; // word q of Gaussian i (row t), its floats first .. last
+    uint32_t t, i, first, last; // a word of Gaussian i (row t), its floats first .. last
+    size_t at;
     uint32_t word, state[2];
     bool wanted;
   };
   const auto load = [&](uint32_t x, Word &w) {
     w.wanted = false;
     if (x >= total) return;
-    // Word x of the rows (x < 2^12: the quotient by the rounded reciprocal is exact).
+    // Word x of the rows (x < 2^13: the quotient by the rounded reciprocal is exact).
     w.t = static_cast<uint32_t>((static_cast<float>(x) + 0.5f) * perWord);
-    w.q = x - w.t * words;
+    const uint32_t q = x - w.t * words;
     w.i = first + (list[w.t] & (kFlagged - 1u));
-    sh_word_floats(c.shFormat, w.q, o.shFloats, w.first, w.last);
-    w.wanted = zeros || rows[w.t].used != 0;
+    w.at = static_cast<size_t>(w.i) * words + q;
+    sh_word_floats(format, q, o.shFloats, w.first, w.last);
+    w.wanted = zeros || wanted(w.t);
     if (!w.wanted) return;
-    w.word = B.shWords[static_cast<size_t>(w.i) * words + w.q];
+    w.word = wordOf(x, w.at);
     const uint32_t s = w.i * o.shFloats + w.first;
     w.state[0] = B.stateSh[s];
     w.state[1] = w.last > w.first ? B.stateSh[s + 1] : 0u;
@@ -781,13 +786,10 @@ __device__ __forceinline__ void step_sh_words(const ChainBuffers &B, const ViewP
     Word w = next;
     load(x + kChainThreads, next);
     if (!w.wanted) continue;
-    const ShRow &row = rows[w.t];
-    const uint32_t used = row.used;
     bool changed = false;
 #pragma unroll 1
     for (uint32_t j = w.first; j <= w.last; ++j) {
-      const uint32_t b = j / 3, ch = j - 3 * b;
-      const float gv = b < used ? row.basis[b] * row.colour[ch] : 0.0f;
+      const float gv = gradient(w.t, j);
       if (gv == 0.0f && !zeros) continue;
       const uint32_t s = w.i * o.shFloats + j;
       uint32_t state = j == w.first ? w.state[0] : w.state[1];
@@ -795,13 +797,13 @@ __device__ __forceinline__ void step_sh_words(const ChainBuffers &B, const ViewP
         B.stateSh[s] = with_curvature(o, state, gv, s * 5u + 4u);
         continue;
       }
-      float value = sh_word_get(c.shFormat, w.word, j, w.first);
-      step_parameter(o, value, state, gv, b == 0 ? o.rates[4] : o.rates[4] * o.restScale, secondOrder ? row.radius[ch] : -1.0f, s * 5u + 4u);
+      float value = sh_word_get(format, w.word, j, w.first);
+      step_parameter(o, value, state, gv, j < 3 ? o.rates[4] : o.rates[4] * o.restScale, radius(w.t, j % 3u), s * 5u + 4u);
       B.stateSh[s] = state;
-      w.word = sh_word_put(c.shFormat, w.word, j, w.first, value, s, o.seed);
+      w.word = sh_word_put(format, w.word, j, w.first, value, s, o.seed);
       changed = true;
     }
-    if (changed) B.shWords[static_cast<size_t>(w.i) * words + w.q] = w.word;
+    if (changed) B.shWords[w.at] = w.word;
   }
 }
 
@@ -914,7 +916,11 @@ __global__ __launch_bounds__(kChainThreads, 4) void chain_step_kernel(ChainBuffe
         __syncthreads();
       }
       step_geometry(B, o, first, list + from, n, geometry, sh, Degree > 0, zeros);
-      step_sh_words(B, c, o, first, list + from, n, sh, zeros && !secondOrder);
+      step_sh_words(
+          B, o, c.shFormat, c.shWords, first, list + from, n, zeros && !secondOrder, [&](uint32_t t) { return sh[t].used != 0; },
+          [&](uint32_t, size_t at) { return B.shWords[at]; },
+          [&](uint32_t t, uint32_t j) { return j / 3 < sh[t].used ? sh[t].basis[j / 3] * sh[t].colour[j % 3] : 0.0f; },
+          [&](uint32_t t, uint32_t ch) { return secondOrder ? sh[t].radius[ch] : -1.0f; });
     }
     __syncthreads(); // the rows are read
   }
@@ -935,11 +941,13 @@ __global__ __launch_bounds__(kChainThreads, 4) void chain_step_kernel(ChainBuffe
 // A workgroup takes perBlock neighbouring Gaussians. Unless all have something to
 // store or to step, it packs those that a view's backward pass added to at the
 // front of a list, as chain_step_kernel does, and a view's sums are read only for
-// the Gaussians it added to. A step over eight views of 1M Gaussians: 245 us,
+// the Gaussians it added to. A step over eight views of 1M Gaussians: 234 us,
 // before (all Gaussians, the SH sums through memory to a kernel of their own) 606
-// and 134; gradients of three views of 40k: 25 us.
+// and 134; gradients of three views of 40k: 24 us. Where all are seen the step is
+// bound by its instructions at two waves a SIMD: 360 us against 310 for four
+// views of 500k, gradients 177 against 156.
 template <int Degree, uint32_t Format>
-__global__ __launch_bounds__(kChainThreads) void chain_views_kernel(ChainBuffers B, ChainViews views, ChainParams o, uint32_t perBlock,
+__global__ __launch_bounds__(kChainThreads, 2) void chain_views_kernel(ChainBuffers B, ChainViews views, ChainParams o, uint32_t perBlock,
                                                                    const uint32_t *counters) {
   constexpr uint32_t kCoefficients = (Degree + 1) * (Degree + 1), kSums = kChainThreads + 1;
   constexpr uint32_t kRound = 4 * kChainThreads, kRounds = kViewsMost / kRound;
@@ -986,11 +994,27 @@ __global__ __launch_bounds__(kChainThreads) void chain_views_kernel(ChainBuffers
   for (uint32_t from = 0; from < listed; from += kChainThreads) {
     const uint32_t n = listed - from < kChainThreads ? listed - from : kChainThreads;
     __syncthreads(); // the list is whole, the sums before are read
-    // The SH words, read by every view, staged once through LDS.
-    const float perWord = 1.0f / static_cast<float>(shWords);
-    for (uint32_t x = lane; x < n * shWords; x += kChainThreads) {
-      const uint32_t t = static_cast<uint32_t>((static_cast<float>(x) + 0.5f) * perWord); // exact for x < 2^13
-      stage[x] = B.shWords[static_cast<size_t>(first + list[from + t]) * shWords + (x - t * shWords)];
+    // The SH words, read by every view, staged once through LDS: with 16-byte loads
+    // where the Gaussians are neighbours (`first` is a multiple of four), else
+    // several loads at a time.
+    if (everyone) {
+      stage_words<kChainThreads>(stage, B.shWords + static_cast<size_t>(first + from) * shWords, n * shWords);
+    } else {
+      constexpr uint32_t kBatch = 8;
+      const float perWord = 1.0f / static_cast<float>(shWords);
+      for (uint32_t x0 = lane; x0 < n * shWords; x0 += kBatch * kChainThreads) {
+        uint32_t word[kBatch];
+#pragma unroll
+        for (uint32_t k = 0; k < kBatch; ++k) {
+          const uint32_t x = x0 + k * kChainThreads < n * shWords ? x0 + k * kChainThreads : x0;
+          const uint32_t t = static_cast<uint32_t>((static_cast<float>(x) + 0.5f) * perWord); // exact for x < 2^13
+          word[k] = B.shWords[static_cast<size_t>(first + list[from + t]) * shWords + (x - t * shWords)];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kBatch; ++k) {
+          if (x0 + k * kChainThreads < n * shWords) stage[x0 + k * kChainThreads] = word[k];
+        }
+      }
     }
     __syncthreads();
     if (lane < n) {
@@ -1079,32 +1103,28 @@ __global__ __launch_bounds__(kChainThreads) void chain_views_kernel(ChainBuffers
     }
     __syncthreads(); // the SH sums are whole
     if (o.mode == kModeStep) {
-      // As step_sh_words, with the gradients summed. Coefficients above the active degree have none.
-      for (uint32_t x = lane; x < n * shWords; x += kChainThreads) {
-        const uint32_t t = static_cast<uint32_t>((static_cast<float>(x) + 0.5f) * perWord), q = x - t * shWords, i = first + list[from + t];
-        uint32_t firstFloat, last, word = stage[x];
-        sh_word_floats(Format, q, o.shFloats, firstFloat, last);
-        bool changed = false;
-        for (uint32_t j = firstFloat; j <= last; ++j) {
-          const float gv = j < kCoefficients * 3 ? shSum[j][t] : 0.0f;
-          if (gv == 0.0f && !zeros) continue;
-          const uint32_t s = i * o.shFloats + j;
-          uint32_t state = B.stateSh[s];
-          float value = sh_word_get(Format, word, j, firstFloat);
-          step_parameter(o, value, state, gv, j < 3 ? o.rates[4] : o.rates[4] * o.restScale, -1.0f, s * 5u + 4u);
-          B.stateSh[s] = state;
-          word = sh_word_put(Format, word, j, firstFloat, value, s, o.seed);
-          changed = true;
-        }
-        if (changed) B.shWords[static_cast<size_t>(i) * shWords + q] = word;
-      }
+      // Coefficients above the active degree have no gradients.
+      step_sh_words(
+          B, o, Format, shWords, first, list + from, n, zeros, [](uint32_t) { return true; }, [&](uint32_t x, size_t) { return stage[x]; },
+          [&](uint32_t t, uint32_t j) { return j < kCoefficients * 3 ? shSum[j][t] : 0.0f; }, [](uint32_t, uint32_t) { return -1.0f; });
     } else {
-      // Coefficients above the active degree get zero (they are stored, not trained).
+      // The rows, which lie consecutively (everyone is listed), with consecutive lanes
+      // on consecutive floats; coefficients above the active degree get zero (they
+      // are stored, not trained). Float x of the rows is column col of row t, kept
+      // incrementally as x advances by the block size.
       const uint32_t floats = o.shFloats;
-      const float perFloat = 1.0f / static_cast<float>(floats);
+      float *out = B.gradSh + static_cast<size_t>(first + from) * floats;
+      uint32_t t = lane / floats, col = lane - t * floats;
+      const uint32_t stepRows = kChainThreads / floats, stepCols = kChainThreads - stepRows * floats;
+#pragma unroll 4
       for (uint32_t x = lane; x < n * floats; x += kChainThreads) {
-        const uint32_t t = static_cast<uint32_t>((static_cast<float>(x) + 0.5f) * perFloat), j = x - t * floats; // exact for x < 2^14
-        B.gradSh[static_cast<size_t>(first + list[from + t]) * floats + j] = j < kCoefficients * 3 ? shSum[j][t] : 0.0f;
+        out[x] = col < kCoefficients * 3 ? shSum[col][t] : 0.0f;
+        t += stepRows;
+        col += stepCols;
+        if (col >= floats) {
+          col -= floats;
+          ++t;
+        }
       }
     }
   }
@@ -1338,8 +1358,7 @@ void launch_chain_views(hipStream_t stream, const ChainBuffers &buffers, const C
                         const uint32_t *counters) {
   const uint32_t count = views.view[0].c.count;
   if (count == 0 || views.count == 0) return;
-  // Two workgroups a CU are resident.
-  const uint32_t perBlock = chain_share(count, 2, kViewsMost);
+  const uint32_t perBlock = chain_share(count, 2, kViewsMost); // two workgroups a CU are resident
   const dim3 grid((count + perBlock - 1) / perBlock), block(256);
 #define VSPLAT_CHAIN(D, F) hipLaunchKernelGGL((chain_views_kernel<D, F>), grid, block, 0, stream, buffers, views, params, perBlock, counters)
   VSPLAT_SH_DISPATCH(views.view[0].c.shDegree, views.view[0].c.shFormat, VSPLAT_CHAIN)
