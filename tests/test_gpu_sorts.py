@@ -1,6 +1,7 @@
 """The depth sort and the tile lists at the sizes where the counted passes (one
-launch each, tiles of 4096 keys, up to 2^18 keys) begin and end, for depths all
-different, all equal and mostly out of view: the keys sorted, equal keys in
+launch each, tiles of 4096 keys, up to 2^18 keys) and the wide ones past them
+begin and end, for depths all different, all equal, mostly out of view and (a near
+plane at or behind the camera) negative: the keys sorted, equal keys in
 their first order, and each tile's entries in depth order."""
 import numpy as np
 import pytest
@@ -34,16 +35,21 @@ def _counts(t, rank, stats):
     return counts[rank]
 
 
+@pytest.mark.parametrize("near", [0.01, 0.0, -5.0])
 @pytest.mark.parametrize("scene", ["spread", "equal", "behind"])
-@pytest.mark.parametrize("count", [1, 2, 255, 4095, 4096, 4097, 8193, 70_000, 262_143, 262_144, 262_145])
-def test_depth_order(count, scene):
+@pytest.mark.parametrize("count", [1, 2, 255, 4095, 4096, 4097, 8193, 70_000, 262_143, 262_144, 262_145, 401_409])
+def test_depth_order(count, scene, near):
     cloud = F.synthetic_cloud(count, 0, 11, log_scale=(-5.0, 0.5))
     if scene == "equal":
         cloud.positions[:, 2] = 0.25
     if scene == "behind":
         cloud.positions[count // 8:, 2] = -9.0
     cam = F.look_at((0, 0, -3), (0, 0, 0), (0.0, -1.0, 0.0), 60.0, 130, 97)
-    with vsplat.Trainer(cloud) as t:
+    if scene == "behind" and near <= 0.0:
+        cloud.positions[::3, 2] = np.random.default_rng(3).uniform(-7.0, -3.0, len(cloud.positions[::3]))  # negative depths, some kept
+        cloud.positions[1::3, 2] = -3.0  # depth 0
+        cloud.opacities[:] = -3.0
+    with vsplat.Trainer(cloud, vsplat.TrainerOptions(near_plane=near)) as t:
         _check_lists(t, t.compute_gradients(cam, F.smooth_target(130, 97, 3)))
 
 

@@ -111,6 +111,15 @@ size_t radix_count_words(uint64_t capacity, uint32_t bits);
 uint32_t radix_first_mask(uint32_t bits);
 void launch_radix_sort(hipStream_t stream, uint32_t *keys, uint32_t *values, uint32_t *tmpKeys, uint32_t *tmpValues,
                        const uint32_t *countDev, uint32_t capacity, uint32_t bits, uint32_t *scratch, uint32_t *counts);
+// The depth sort: `count` keys with the identity as their values. More than
+// kCountedSortKeys keys take three passes (sort.hip), which start in tmpKeys and need no
+// values (depth_sort_three_pass); fewer are launch_radix_sort's, from keys and
+// values. signs: whether depths can be negative or -0 (a near plane not above 0).
+// scratch: depth_sort_scratch_words.
+bool depth_sort_three_pass(uint64_t count);
+size_t depth_sort_scratch_words(uint64_t count);
+void launch_depth_sort(hipStream_t stream, uint32_t *keys, uint32_t *values, uint32_t *tmpKeys, uint32_t *tmpValues, uint32_t count,
+                       bool signs, uint32_t *scratch, uint32_t *counts);
 // The tile entries sorted by tile, and the tiles' ranges (cleared beforehand). The
 // entries start in tmpKeys and tmpValues if tile_sort_from_tmp. More than
 // kCountedSortKeys entries on at most kTileSortTiles tiles are sorted in one pass

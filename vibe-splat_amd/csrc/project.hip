@@ -245,7 +245,7 @@ __global__ __launch_bounds__(256) void project_kernel(const float *__restrict__ 
   if (depthCounts != nullptr) count_digit(depthCounts, i, key & 0xFFu, i < c.count);
   if (i < c.count) {
     keys[i] = key;
-    values[i] = i;
+    if (values != nullptr) values[i] = i;
     if (visible) {
       float4 *out = reinterpret_cast<float4 *>(splats + i);
       out[0] = make_float4(s.qx, s.qy, s.qz, s.o);

@@ -349,29 +349,33 @@ __global__ __launch_bounds__(kPassThreads) void radix_pass_kernel(const uint32_t
   }
 }
 
-// ---- The tile sort of more than kCountedSortKeys entries on a grid of at most
-// kTileSortTiles tiles, in one pass whose digit is the whole tile:
+// ---- Passes with a digit of up to 11 bits, for sorts of more than kCountedSortKeys
+// keys: the tile sort on a grid of at most kTileSortTiles tiles, in one pass whose
+// digit is the whole tile, and the depth sort in three (10, 10 and 11 bits; 11, 11 and 10 where depths can be negative):
 //
-//   count    per chunk of entries, how many each tile has (hist[chunk * stride + tile]);
-//   scan     the exclusive sums over the chunks, in place, and each tile's entries;
-//   scatter  the ranks as in radix_scatter_kernel, and from the tiles' totals
-//            each tile's range, which has no kernel of its own then.
+//   count    per chunk of keys, how many have each digit (hist[chunk * stride + digit]);
+//   scan     the exclusive sums over the chunks, in place, and each digit's keys;
+//   scatter  the ranks as in radix_scatter_kernel, and from the totals each tile's
+//            range, which has no kernel of its own then.
 //
-// A chunk is 8 entries a tile (8192 for up to 2^10 tiles, 16384 for up to 2^11), so
-// that the counts stay an eighth of the entries; the scatter takes it in parts
-// of 8192, a workgroup each. Each XCD takes consecutive chunks, so that a tile's
-// neighbouring runs meet in one XCD's cache. What bounds it is the ranking's
+// The tile sort's chunk is 8 entries a tile (8192 for up to 2^10 tiles, 16384 for up
+// to 2^11), so that the counts stay an eighth of the entries; the scatter takes it in
+// parts of 8192, a workgroup each. The depth sort's is 4096 keys: 1M keys are then
+// 245 workgroups. Each XCD takes consecutive chunks, so that a digit's
+// neighbouring runs meet in one XCD's cache. What bounds them is the ranking's
 // instructions and the runs' partial lines; three workgroups a CU (80
 // registers) hide the one behind the other, two took a tenth longer.
 //
-// Against two passes of 5 or 6 bits and the kernel for the ranges (us): 63 to 33
-// for 3.4M entries on 920 tiles, 186 to 119 for 15.4M and 305 to 184 for 25M on 2040
-// tiles (400 MB read and written, 77 at the rate of a copy). At 2646 tiles (2.6M
+// The tile sort against two passes of 5 or 6 bits and the kernel for the ranges (us):
+// 63 to 33 for 3.4M entries on 920 tiles, 186 to 119 for 15.4M and 305 to 184 for 25M
+// on 2040 tiles (400 MB read and written, 77 at the rate of a copy). At 2646 tiles (2.6M
 // entries, counts of 2^12 tiles, one workgroup a CU) it is 57 against 53, and up to
-// kCountedSortKeys entries the counted passes need no more launches.
-constexpr uint32_t kChunkThreads = 512, kPartPerThread = 16;
-constexpr uint32_t kScanTiles = 16;
-__host__ __device__ __forceinline__ uint32_t tile_stride(uint32_t tiles) { return (tiles + kScanTiles - 1u) / kScanTiles * kScanTiles; }
+// kCountedSortKeys entries the counted passes need no more launches. The depth sort
+// against four passes of 8 bits: 85 to 67 for 1M keys, 145 to 107 for 3M, 70 to 58 for
+// 400k (11 bits in every pass: 75, 126, 63).
+constexpr uint32_t kChunkThreads = 512, kDepthChunk = 4096;
+constexpr uint32_t kScanDigits = 16;
+__host__ __device__ __forceinline__ uint32_t digit_stride(uint32_t digits) { return (digits + kScanDigits - 1u) / kScanDigits * kScanDigits; }
 typedef uint16_t __attribute__((may_alias)) Half;
 
 // The chunk of a workgroup (one past the last where it has none): XCD x, which runs
@@ -382,12 +386,13 @@ template <uint32_t Parts> __device__ __forceinline__ uint32_t chunk_of_block(uin
   return k < each ? (blockIdx.x % kRasterXcds) * each + k : chunks;
 }
 
-template <uint32_t Bits>
-__global__ __launch_bounds__(kChunkThreads) void tile_sort_count_kernel(const uint32_t *__restrict__ keys, const uint32_t *__restrict__ countDev,
-                                                                        uint32_t tiles, uint32_t tileMask, uint32_t *__restrict__ hist) {
-  constexpr uint32_t kChunk = 8u << Bits, kQuads = kChunk / kChunkThreads / 4;
+template <uint32_t Bits, uint32_t kChunk>
+__global__ __launch_bounds__(kChunkThreads) void digit_count_kernel(const uint32_t *__restrict__ keys, const uint32_t *__restrict__ countDev,
+                                                                    uint32_t countHost, uint32_t shift, uint32_t digits, uint32_t mask,
+                                                                    uint32_t *__restrict__ hist) {
+  constexpr uint32_t kQuads = kChunk / kChunkThreads / 4;
   __shared__ uint32_t counts[1u << Bits];
-  const uint32_t count = *countDev, chunks = chunks_of(count, kChunk), chunk = chunk_of_block<1>(chunks);
+  const uint32_t count = count_of(countDev, countHost), chunks = chunks_of(count, kChunk), chunk = chunk_of_block<1>(chunks);
   if (chunk >= chunks) return; // the same for the whole workgroup
   const uint32_t inChunk = count - chunk * kChunk < kChunk ? count - chunk * kChunk : kChunk;
   const uint32_t *const chunkKeys = keys + chunk * kChunk;
@@ -401,31 +406,31 @@ __global__ __launch_bounds__(kChunkThreads) void tile_sort_count_kernel(const ui
       k[r] = make_uint4(i < inChunk ? chunkKeys[i] : 0u, i + 1u < inChunk ? chunkKeys[i + 1u] : 0u, i + 2u < inChunk ? chunkKeys[i + 2u] : 0u, 0u);
     }
   }
-  for (uint32_t d = threadIdx.x; d < tiles; d += kChunkThreads) counts[d] = 0u;
+  for (uint32_t d = threadIdx.x; d < digits; d += kChunkThreads) counts[d] = 0u;
   __syncthreads();
 #pragma unroll
   for (uint32_t r = 0; r < kQuads; ++r) {
     const uint32_t i = (r * kChunkThreads + threadIdx.x) * 4u;
-    if (i < inChunk) atomicAdd(&counts[k[r].x & tileMask], 1u);
-    if (i + 1u < inChunk) atomicAdd(&counts[k[r].y & tileMask], 1u);
-    if (i + 2u < inChunk) atomicAdd(&counts[k[r].z & tileMask], 1u);
-    if (i + 3u < inChunk) atomicAdd(&counts[k[r].w & tileMask], 1u);
+    if (i < inChunk) atomicAdd(&counts[(k[r].x >> shift) & mask], 1u);
+    if (i + 1u < inChunk) atomicAdd(&counts[(k[r].y >> shift) & mask], 1u);
+    if (i + 2u < inChunk) atomicAdd(&counts[(k[r].z >> shift) & mask], 1u);
+    if (i + 3u < inChunk) atomicAdd(&counts[(k[r].w >> shift) & mask], 1u);
   }
   __syncthreads();
-  for (uint32_t d = threadIdx.x; d < tiles; d += kChunkThreads) hist[static_cast<size_t>(chunk) * tile_stride(tiles) + d] = counts[d];
+  for (uint32_t d = threadIdx.x; d < digits; d += kChunkThreads) hist[static_cast<size_t>(chunk) * digit_stride(digits) + d] = counts[d];
 }
 
-// A workgroup takes kScanTiles neighbouring tiles; the chunks are dealt out in
+// A workgroup takes kScanDigits neighbouring digits; the chunks are dealt out in
 // runs to its 64 groups of as many threads.
-constexpr uint32_t kScanGroups = kScanThreads / kScanTiles;
-__global__ __launch_bounds__(kScanThreads) void tile_sort_scan_kernel(uint32_t *__restrict__ hist, const uint32_t *__restrict__ countDev,
-                                                                      uint32_t chunkSize, uint32_t tiles, uint32_t *__restrict__ totals) {
-  __shared__ uint32_t sums[kScanGroups][kScanTiles];
-  const uint32_t chunks = chunks_of(*countDev, chunkSize), stride = tile_stride(tiles);
-  const uint32_t t = threadIdx.x % kScanTiles, g = threadIdx.x / kScanTiles, tile = blockIdx.x * kScanTiles + t;
+constexpr uint32_t kScanGroups = kScanThreads / kScanDigits;
+__global__ __launch_bounds__(kScanThreads) void digit_scan_kernel(uint32_t *__restrict__ hist, const uint32_t *__restrict__ countDev, uint32_t countHost,
+                                                                  uint32_t chunkSize, uint32_t digits, uint32_t *__restrict__ totals) {
+  __shared__ uint32_t sums[kScanGroups][kScanDigits];
+  const uint32_t chunks = chunks_of(count_of(countDev, countHost), chunkSize), stride = digit_stride(digits);
+  const uint32_t t = threadIdx.x % kScanDigits, g = threadIdx.x / kScanDigits, digit = blockIdx.x * kScanDigits + t;
   const uint32_t each = (chunks + kScanGroups - 1u) / kScanGroups;
   const uint32_t begin = g * each < chunks ? g * each : chunks, end = begin + each < chunks ? begin + each : chunks;
-  uint32_t *const column = hist + tile;
+  uint32_t *const column = hist + digit;
   uint32_t sum = 0;
 #pragma unroll 16
   for (uint32_t c = begin; c < end; ++c) sum += column[static_cast<size_t>(c) * stride];
@@ -444,7 +449,7 @@ __global__ __launch_bounds__(kScanThreads) void tile_sort_scan_kernel(uint32_t *
     column[static_cast<size_t>(c) * stride] = running;
     running += v;
   }
-  if (g == 0 && tile < tiles) totals[tile] = total;
+  if (g == 0 && digit < digits) totals[digit] = total;
 }
 
 // A chunk's word by a 32-bit offset from its (uniform) start.
@@ -452,51 +457,51 @@ __device__ __forceinline__ uint32_t word_at(const uint32_t *__restrict__ chunk, 
   return *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(chunk) + i * 4u);
 }
 
-template <uint32_t Bits>
-__global__ __launch_bounds__(kChunkThreads, 6) void tile_sort_scatter_kernel(
+// valsIn may be null: the values are then the keys' places. ranges may be null.
+template <uint32_t Bits, uint32_t kChunk, uint32_t kPart>
+__global__ __launch_bounds__(kChunkThreads, 6) void digit_scatter_kernel(
     const uint32_t *__restrict__ keysIn, const uint32_t *__restrict__ valsIn, uint32_t *__restrict__ keysOut, uint32_t *__restrict__ valsOut,
-    const uint32_t *__restrict__ countDev, uint32_t tiles, uint32_t tileMask, const uint32_t *__restrict__ hist,
-    const uint32_t *__restrict__ totals, uint2 *__restrict__ ranges) {
-  constexpr uint32_t kChunk = 8u << Bits, kPart = kChunkThreads * kPartPerThread, kParts = kChunk / kPart;
+    const uint32_t *__restrict__ countDev, uint32_t countHost, uint32_t shift, uint32_t digits, uint32_t mask,
+    const uint32_t *__restrict__ hist, const uint32_t *__restrict__ totals, uint2 *__restrict__ ranges) {
+  constexpr uint32_t kPartPerThread = kPart / kChunkThreads, kParts = kChunk / kPart;
   constexpr uint32_t kWaves = kChunkThreads / 64, kRadix = 1u << Bits;
-  constexpr uint32_t kOwn = kRadix / kChunkThreads; // consecutive tiles per thread
-  constexpr uint32_t kWaveKeys = kPart / kWaves;  // consecutive entries per wave
+  constexpr uint32_t kOwn = kRadix / kChunkThreads; // consecutive digits per thread
+  constexpr uint32_t kWaveKeys = kPart / kWaves;  // consecutive keys per wave
   constexpr uint32_t kCountWords = kWaves * kRadix / 2;
-  __shared__ uint32_t tileBase[kRadix]; // where the tile's entries of this part go, less their start within the part
+  __shared__ uint32_t digitBase[kRadix]; // where the digit's keys of this part go, less their start within the part
   __shared__ uint32_t waveTotals[kWaves];
-  // Each wave's entries per tile in 16 bits (two tiles a word), then the part's
-  // keys, then its values, in tile order.
-  __shared__ uint32_t shared[kPart];
-  static_assert(kCountWords <= kPart, "the counts take no more than the keys");
-  const uint32_t count = *countDev, chunks = chunks_of(count, kChunk), chunk = chunk_of_block<kParts>(chunks);
+  // Each wave's keys per digit in 16 bits (two digits a word), then the part's
+  // keys, then its values, in digit order.
+  __shared__ uint32_t shared[kCountWords > kPart ? kCountWords : kPart];
+  const uint32_t count = count_of(countDev, countHost), chunks = chunks_of(count, kChunk), chunk = chunk_of_block<kParts>(chunks);
   const uint32_t part = blockIdx.x / kRasterXcds % kParts, at = chunk * kChunk + part * kPart;
   if (chunk >= chunks || at >= count) return; // the same for the whole workgroup
   const uint32_t inPart = count - at < kPart ? count - at : kPart;
-  const uint32_t *const partKeys = keysIn + at, *const partValues = valsIn + at;
+  const uint32_t *const partKeys = keysIn + at;
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, first = wave * kWaveKeys + lane;
   Half *const waveCount = reinterpret_cast<Half *>(shared) + wave * kRadix;
-  uint32_t key[kPartPerThread], place[kPartPerThread / 2]; // place: each entry's rank, then its place in the part, in 16 bits
+  uint32_t key[kPartPerThread], place[kPartPerThread / 2]; // place: each key's rank, then its place in the part, in 16 bits
 #pragma unroll
   for (uint32_t r = 0; r < kPartPerThread; ++r) {
     key[r] = word_at(partKeys, first + r * 64 < inPart ? first + r * 64 : inPart - 1u);
   }
   for (uint32_t x = threadIdx.x; x < kCountWords; x += kChunkThreads) shared[x] = 0u;
 
-  // Where this part's entries of each of the thread's tiles go: past the chunk's
-  // earlier parts, whose entries are counted again here.
+  // Where this part's keys of each of the thread's digits go: past the chunk's
+  // earlier parts, whose keys are counted again here.
   const uint32_t d = kOwn * threadIdx.x;
   {
     uint32_t n[kOwn], sum = 0, start;
 #pragma unroll
     for (uint32_t o = 0; o < kOwn; ++o) {
-      n[o] = d + o < tiles ? totals[d + o] : 0u;
+      n[o] = d + o < digits ? totals[d + o] : 0u;
       sum += n[o];
     }
     block_exclusive_sum(sum, start, waveTotals);
 #pragma unroll
     for (uint32_t o = 0; o < kOwn; ++o) {
-      if (d + o < tiles) tileBase[d + o] = start + hist[static_cast<size_t>(chunk) * tile_stride(tiles) + d + o];
-      if (chunk == 0 && n[o] != 0u) ranges[d + o] = make_uint2(start, start + n[o]);
+      if (d + o < digits) digitBase[d + o] = start + hist[static_cast<size_t>(chunk) * digit_stride(digits) + d + o];
+      if (ranges != nullptr && chunk == 0 && n[o] != 0u) ranges[d + o] = make_uint2(start, start + n[o]);
       start += n[o];
     }
   }
@@ -504,33 +509,33 @@ __global__ __launch_bounds__(kChunkThreads, 6) void tile_sort_scatter_kernel(
   if (kParts > 1) {
     for (uint32_t i = threadIdx.x * 4u; i < part * kPart; i += kChunkThreads * 4u) {
       const uint4 k = *reinterpret_cast<const uint4 *>(keysIn + chunk * kChunk + i);
-      atomicAdd(&tileBase[k.x & tileMask], 1u);
-      atomicAdd(&tileBase[k.y & tileMask], 1u);
-      atomicAdd(&tileBase[k.z & tileMask], 1u);
-      atomicAdd(&tileBase[k.w & tileMask], 1u);
+      atomicAdd(&digitBase[(k.x >> shift) & mask], 1u);
+      atomicAdd(&digitBase[(k.y >> shift) & mask], 1u);
+      atomicAdd(&digitBase[(k.z >> shift) & mask], 1u);
+      atomicAdd(&digitBase[(k.w >> shift) & mask], 1u);
     }
     __syncthreads(); // before the starts within the part are taken off
   }
 
-  // Rank within the wave's entries, in order.
+  // Rank within the wave's keys, in order.
   const uint64_t below = (uint64_t{1} << lane) - 1u;
 #pragma unroll
   for (uint32_t r = 0; r < kPartPerThread; ++r) {
     const bool valid = first + r * 64 < inPart;
-    const uint32_t tile = key[r] & tileMask;
-    const uint64_t same = lanes_of_digit<Bits>(tile, valid);
+    const uint32_t digit = (key[r] >> shift) & mask;
+    const uint64_t same = lanes_of_digit<Bits>(digit, valid);
     const uint32_t lower = static_cast<uint32_t>(__popcll(same & below));
     __builtin_amdgcn_wave_barrier();
-    const uint32_t prior = waveCount[tile];
+    const uint32_t prior = waveCount[digit];
     place[r / 2] = r % 2 == 0 ? prior + lower : place[r / 2] | ((prior + lower) << 16);
     // The rank is formed here and the counter's address again later: kept for
     // later, the lanes' masks and the addresses take 48 registers more.
     asm volatile("" : "+v"(place[r / 2]), "+v"(key[r]));
     __builtin_amdgcn_wave_barrier();
-    if (valid && lower == 0) waveCount[tile] = static_cast<Half>(prior + static_cast<uint32_t>(__popcll(same)));
+    if (valid && lower == 0) waveCount[digit] = static_cast<Half>(prior + static_cast<uint32_t>(__popcll(same)));
   }
   __syncthreads();
-  // Per tile: where its entries start within the part, and each wave's start from there.
+  // Per digit: where its keys start within the part, and each wave's start from there.
   {
     uint32_t n[kOwn] = {}, sum = 0, start;
 #pragma unroll
@@ -547,8 +552,8 @@ __global__ __launch_bounds__(kChunkThreads, 6) void tile_sort_scatter_kernel(
 #pragma unroll
     for (uint32_t o = 0; o < kOwn; o += 2) {
       uint32_t low = start, high = start + n[o];
-      tileBase[d + o] -= low;
-      tileBase[d + o + 1] -= high;
+      digitBase[d + o] -= low;
+      digitBase[d + o + 1] -= high;
       start = high + n[o + 1];
 #pragma unroll
       for (uint32_t w = 0; w < kWaves; ++w) {
@@ -562,12 +567,13 @@ __global__ __launch_bounds__(kChunkThreads, 6) void tile_sort_scatter_kernel(
   __syncthreads();
 #pragma unroll
   for (uint32_t r = 0; r < kPartPerThread; ++r) {
-    place[r / 2] += static_cast<uint32_t>(waveCount[key[r] & tileMask]) << (r % 2 * 16);
+    place[r / 2] += static_cast<uint32_t>(waveCount[(key[r] >> shift) & mask]) << (r % 2 * 16);
   }
   uint32_t val[kPartPerThread];
 #pragma unroll
   for (uint32_t r = 0; r < kPartPerThread; ++r) {
-    val[r] = word_at(partValues, first + r * 64 < inPart ? first + r * 64 : inPart - 1u);
+    const uint32_t x = first + r * 64 < inPart ? first + r * 64 : inPart - 1u;
+    val[r] = valsIn != nullptr ? word_at(valsIn + at, x) : at + x;
   }
   __syncthreads();
 #pragma unroll
@@ -581,7 +587,7 @@ __global__ __launch_bounds__(kChunkThreads, 6) void tile_sort_scatter_kernel(
     const uint32_t j = r * kChunkThreads + threadIdx.x;
     if (j < inPart) {
       const uint32_t k = shared[j];
-      dst[r] = tileBase[k & tileMask] + j;
+      dst[r] = digitBase[(k >> shift) & mask] + j;
       keysOut[dst[r]] = k;
     }
   }
@@ -600,17 +606,17 @@ __global__ __launch_bounds__(kChunkThreads, 6) void tile_sort_scatter_kernel(
 
 uint32_t div_up(uint64_t a, uint32_t b) { return static_cast<uint32_t>((a + b - 1) / b); }
 
-template <uint32_t Bits>
-void tile_sort_pass(hipStream_t stream, const uint32_t *kIn, const uint32_t *vIn, uint32_t *kOut, uint32_t *vOut, const uint32_t *countDev,
-                    uint32_t capacity, uint32_t tileBits, uint32_t tiles, uint32_t *scratch, uint2 *ranges) {
-  constexpr uint32_t kChunk = 8u << Bits;
-  const uint32_t blocks = div_up(div_up(capacity, kChunk), kRasterXcds) * kRasterXcds, tileMask = (1u << tileBits) - 1u;
-  uint32_t *totals = scratch, *hist = scratch + tile_stride(tiles);
-  hipLaunchKernelGGL(tile_sort_count_kernel<Bits>, dim3(blocks), dim3(kChunkThreads), 0, stream, kIn, countDev, tiles, tileMask, hist);
-  hipLaunchKernelGGL(tile_sort_scan_kernel, dim3(tile_stride(tiles) / kScanTiles), dim3(kScanThreads), 0, stream, hist, countDev, kChunk, tiles,
-                     totals);
-  hipLaunchKernelGGL(tile_sort_scatter_kernel<Bits>, dim3(blocks * (kChunk / kChunkThreads / kPartPerThread)), dim3(kChunkThreads), 0, stream, kIn, vIn, kOut, vOut, countDev, tiles,
-                     tileMask, hist, totals, ranges);
+template <uint32_t Bits, uint32_t Chunk, uint32_t Part>
+void digit_pass(hipStream_t stream, const uint32_t *kIn, const uint32_t *vIn, uint32_t *kOut, uint32_t *vOut, const uint32_t *countDev,
+                uint32_t capacity, uint32_t shift, uint32_t bits, uint32_t digits, uint32_t *scratch, uint2 *ranges) {
+  const uint32_t blocks = div_up(div_up(capacity, Chunk), kRasterXcds) * kRasterXcds, mask = (1u << bits) - 1u;
+  uint32_t *totals = scratch, *hist = scratch + digit_stride(digits);
+  hipLaunchKernelGGL((digit_count_kernel<Bits, Chunk>), dim3(blocks), dim3(kChunkThreads), 0, stream, kIn, countDev, capacity, shift, digits,
+                     mask, hist);
+  hipLaunchKernelGGL(digit_scan_kernel, dim3(digit_stride(digits) / kScanDigits), dim3(kScanThreads), 0, stream, hist, countDev, capacity, Chunk,
+                     digits, totals);
+  hipLaunchKernelGGL((digit_scatter_kernel<Bits, Chunk, Part>), dim3(blocks * (Chunk / Part)), dim3(kChunkThreads), 0, stream, kIn, vIn, kOut,
+                     vOut, countDev, capacity, shift, digits, mask, hist, totals, ranges);
 }
 
 template <uint32_t Bits>
@@ -654,7 +660,7 @@ bool tile_sort_one_pass(uint64_t capacity, uint32_t tiles) { return capacity > k
 
 size_t tile_sort_scratch_words(uint64_t capacity, uint32_t tiles) {
   if (!tile_sort_one_pass(capacity, tiles)) return radix_sort_scratch_words(capacity);
-  return static_cast<size_t>(tile_stride(tiles)) * (1 + div_up(capacity, tiles <= kTileSortTiles / 2 ? 4 * kTileSortTiles : 8 * kTileSortTiles));
+  return static_cast<size_t>(digit_stride(tiles)) * (1 + div_up(capacity, tiles <= kTileSortTiles / 2 ? 4 * kTileSortTiles : 8 * kTileSortTiles));
 }
 bool tile_sort_from_tmp(uint64_t capacity, uint32_t tileBits, uint32_t tiles) {
   return tile_sort_one_pass(capacity, tiles) || radix_sort_from_tmp(tileBits);
@@ -668,9 +674,9 @@ void launch_tile_sort(hipStream_t stream, uint32_t *keys, uint32_t *values, uint
     launch_radix_sort(stream, keys, values, tmpKeys, tmpValues, countDev, capacity, tileBits, scratch, counts);
     launch_tile_ranges(stream, keys, countDev, capacity, tileBits, ranges);
   } else if (tiles <= kTileSortTiles / 2) {
-    tile_sort_pass<10>(stream, tmpKeys, tmpValues, keys, values, countDev, capacity, tileBits, tiles, scratch, ranges);
+    digit_pass<10, 8192, 8192>(stream, tmpKeys, tmpValues, keys, values, countDev, capacity, 0, tileBits, tiles, scratch, ranges);
   } else {
-    tile_sort_pass<11>(stream, tmpKeys, tmpValues, keys, values, countDev, capacity, tileBits, tiles, scratch, ranges);
+    digit_pass<11, 16384, 8192>(stream, tmpKeys, tmpValues, keys, values, countDev, capacity, 0, tileBits, tiles, scratch, ranges);
   }
 }
 
@@ -725,6 +731,29 @@ void launch_radix_sort(hipStream_t stream, uint32_t *keys, uint32_t *values, uin
     std::swap(srcK, dstK);
     std::swap(srcV, dstV);
   }
+}
+
+bool depth_sort_three_pass(uint64_t count) { return count > kCountedSortKeys; }
+
+size_t depth_sort_scratch_words(uint64_t count) {
+  if (!depth_sort_three_pass(count)) return radix_sort_scratch_words(count);
+  return size_t{2048} * (1 + div_up(count, kDepthChunk));
+}
+
+void launch_depth_sort(hipStream_t stream, uint32_t *keys, uint32_t *values, uint32_t *tmpKeys, uint32_t *tmpValues, uint32_t count,
+                       bool signs, uint32_t *scratch, uint32_t *counts) {
+  if (!depth_sort_three_pass(count)) {
+    launch_radix_sort(stream, keys, values, tmpKeys, tmpValues, nullptr, count, 32, scratch, counts);
+    return;
+  }
+  // A key is all ones less the depth's bits: without a sign its highest bit is set,
+  // as an invisible splat's is, and takes no part.
+  const uint32_t low = signs ? 11 : 10, digits = 1u << low;
+  const auto pass = signs ? digit_pass<11, kDepthChunk, kDepthChunk> : digit_pass<10, kDepthChunk, kDepthChunk>;
+  pass(stream, tmpKeys, nullptr, keys, values, nullptr, count, 0, low, digits, scratch, nullptr);
+  pass(stream, keys, values, tmpKeys, tmpValues, nullptr, count, low, low, digits, scratch, nullptr);
+  digit_pass<11, kDepthChunk, kDepthChunk>(stream, tmpKeys, tmpValues, keys, values, nullptr, count, 2 * low, signs ? 10 : 11,
+                                           signs ? 1024 : 2048, scratch, nullptr);
 }
 
 __global__ void fill_u32_kernel(uint32_t *__restrict__ dst, uint64_t count, uint32_t value) {

@@ -381,7 +381,7 @@ ViewBuffers &Trainer::view_buffers(size_t k) {
     v->touched.ensure(div_up(n, 4) * 4);
     launch_fill_u32(v->stream, v->touched.as<uint32_t>(), div_up(n, 4), 0u);
     v->scanScratch.ensure(coverage_scan_words(static_cast<uint32_t>(n)) * 4);
-    v->sortScratch.ensure(radix_sort_scratch_words(n) * 4);
+    v->sortScratch.ensure(depth_sort_scratch_words(n) * 4);
     v->sortCounts.ensure((radix_count_words(n, 32) + kEntryCountWords) * 4);
     v->counters.ensure(kCounterWords * 4);
     launch_fill_u32(v->stream, v->counters.as<uint32_t>(), kCounterWords, 0u);
@@ -709,7 +709,7 @@ void Trainer::fit_entries(ViewBuffers &b, uint64_t entries) {
 
 // The scratch of the view's sorts, one after the other: by depth, then by tile.
 void Trainer::ensure_sort_scratch(ViewBuffers &b) {
-  b.sortScratch.ensure(std::max(radix_sort_scratch_words(count_), tile_sort_scratch_words(b.entryCapacity, b.tiles)) * 4);
+  b.sortScratch.ensure(std::max(depth_sort_scratch_words(count_), tile_sort_scratch_words(b.entryCapacity, b.tiles)) * 4);
 }
 
 void Trainer::reserve_entries(uint64_t entries) {
@@ -837,14 +837,16 @@ void Trainer::enqueue_lists(ViewBuffers &b, const ViewParams &v, uint32_t mode, 
   launch_clear_words(s, WordClears{{counters, b.ranges.as<uint32_t>(), b.sortCounts.as<uint32_t>()},
                                    {kClearedPerPass, b.tiles * 2u, static_cast<uint32_t>(depthWords + entryWords)},
                                    3});
+  const bool threePass = depth_sort_three_pass(count_);
   launch_project(s, positions_.as<float>(), scales_.as<float>(), rotations_.as<float>(), opacities_.as<float>(),
                  shWordsBuf_.as<uint32_t>(), filterSet_ ? filter3d_.as<float>() : nullptr, v, options_.mip_filter_2d != 0, dropoutNow_,
-                 shRetained_, shSeed_, b.gridW, b.gridH, b.splats.as<Splat>(), b.keys.as<uint32_t>(), b.values.as<uint32_t>(),
+                 shRetained_, shSeed_, b.gridW, b.gridH, b.splats.as<Splat>(), (threePass ? b.tmpKeys : b.keys).as<uint32_t>(),
+                 threePass ? nullptr : b.values.as<uint32_t>(),
                  b.tileCount.as<uint32_t>(), b.tileRecords.as<TileRecord>(), counters, b.bigList.as<uint32_t>(),
                  b.bigBits.as<uint64_t>(), big_bit_words(b), depthCounts);
   if (marks) mark("project");
-  launch_radix_sort(s, b.keys.as<uint32_t>(), b.values.as<uint32_t>(), b.tmpKeys.as<uint32_t>(), b.tmpValues.as<uint32_t>(), nullptr, count_,
-                    32, b.sortScratch.as<uint32_t>(), depthCounts);
+  launch_depth_sort(s, b.keys.as<uint32_t>(), b.values.as<uint32_t>(), b.tmpKeys.as<uint32_t>(), b.tmpValues.as<uint32_t>(), count_,
+                    !(v.nearPlane > 0.0f), b.sortScratch.as<uint32_t>(), depthCounts);
   if (marks) mark("depth sort");
   launch_coverage_scan(s, b.keys.as<uint32_t>(), b.values.as<uint32_t>(), b.tileCount.as<uint32_t>(), count_,
                        b.tileRecords.as<TileRecord>(), b.coverage.as<uint32_t>(), counters, static_cast<uint32_t>(b.entryCapacity), mode == kModeStep, b.scanScratch.as<uint32_t>());
@@ -1262,7 +1264,7 @@ void Trainer::render_into(const vsplat_camera &camera, float *deviceOut, uint64_
   for (DeviceArray *a : {&b.entryKeys, &b.entryValues, &b.tmpEntryKeys, &b.tmpEntryValues}) carve(*a, entries * 4);
   carve(b.stops, uint64_t{VSPLAT_NOALLOC_MAX_PIXELS} * 4);
   carve(b.ranges, uint64_t{VSPLAT_NOALLOC_MAX_TILES} * 8);
-  carve(b.sortScratch, std::max(radix_sort_scratch_words(n), tile_sort_scratch_words(entries, b.tiles)) * 4);
+  carve(b.sortScratch, std::max(depth_sort_scratch_words(n), tile_sort_scratch_words(entries, b.tiles)) * 4);
   carve(b.scanScratch, coverage_scan_words(static_cast<uint32_t>(n)) * 4);
   carve(b.sortCounts, (radix_count_words(n, 32) + kEntryCountWords) * 4);
   carve(b.counters, kCounterWords * 4);
