@@ -193,7 +193,7 @@ void launch_gather_views(hipStream_t stream, const ViewStatus &views, uint8_t *s
 // the others; values: the Gaussian), for a view of width x height pixels.
 // entryCounts, when set, receives the tile sort's first digits.
 void launch_bin_emit(hipStream_t stream, const uint32_t *keys, const uint32_t *values, const Splat *splats, const TileRecord *records,
-                     uint32_t count, uint32_t gridW, uint32_t tileW, uint32_t tileH, uint32_t width, uint32_t height, uint32_t tileBits,
+                     uint32_t count, uint32_t gridW, uint32_t tileW, uint32_t tileH, uint32_t tileBits,
                      const uint32_t *offsets, const uint32_t *counters, const uint32_t *bigList, const uint64_t *bigBits,
                      uint32_t *entryKeys, uint32_t *entryValues, uint32_t *entryCounts);
 void launch_tile_ranges(hipStream_t stream, const uint32_t *entryKeys, const uint32_t *countDev, uint32_t capacity, uint32_t tileBits,

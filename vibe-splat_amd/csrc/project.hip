@@ -314,8 +314,15 @@ __global__ __launch_bounds__(256) void project_kernel(const float *__restrict__ 
   if (i < c.count) {
     if (!big) tileCount[i] = reached; // a big splat's count comes from big_count_kernel
     const uint32_t height = t[3] - t[1] + 1;
-    records[i] = TileRecord{static_cast<uint32_t>(bits), static_cast<uint32_t>(bits >> 32), t[0] | (t[1] << 16),
-                            visible ? (width | (height << 16)) : 0u};
+    uint32_t size = width | (height << 16);
+    if (!big) {
+      uint32_t edges = 0;
+      if (marks_blocks(TileShape{c.tileW, c.tileH})) {
+        edges = box_block_edges(splat_pixel_box(s.cx, s.cy, s.ex, s.ey), t[0], t[1], t[2], t[3], TileShape{c.tileW, c.tileH}, c.width, c.height);
+      }
+      size = small_box(width, height, edges);
+    }
+    records[i] = TileRecord{static_cast<uint32_t>(bits), static_cast<uint32_t>(bits >> 32), t[0] | (t[1] << 16), visible ? size : 0u};
   }
 }
 

@@ -245,7 +245,22 @@ constexpr uint32_t kMaskTiles = 64;
 struct TileRecord {
   uint32_t maskLo, maskHi;
   uint32_t origin; // tx0 | ty0 << 16
-  uint32_t size;   // width | height << 16, 0 when the splat is not visible
+  uint32_t size;   // width | height << 16 of a big splat (a grid has at most 2^13 tiles a side), small_box of a small one, 0 when not visible
 };
+
+// A small splat's box and its box_block_edges (each at most 4) in one word, so that
+// the list pass reads one record a splat and not the splat as well.
+constexpr uint32_t kSmallBox = 0x80000000u;
+__device__ __forceinline__ uint32_t small_box(uint32_t width, uint32_t height, uint32_t edges) {
+  return kSmallBox | width | (height << 7) | ((edges & 7u) << 14) | (((edges >> 8) & 7u) << 17) | (((edges >> 16) & 7u) << 20) |
+         ((edges >> 24) << 23);
+}
+__device__ __forceinline__ uint32_t small_box_edges(uint32_t size) {
+  return ((size >> 14) & 7u) | (((size >> 17) & 7u) << 8) | (((size >> 20) & 7u) << 16) | (((size >> 23) & 7u) << 24);
+}
+// Blocks are marked per entry for tiles of 16 blocks (32x32), where a block
+// skipping the entries that miss it saves more raster time than marking
+// costs the list pass; smaller tiles mark every block.
+__host__ __device__ __forceinline__ bool marks_blocks(TileShape shape) { return (shape.w / 8u) * (shape.h / 8u) >= 16u; }
 
 } // namespace vsplat

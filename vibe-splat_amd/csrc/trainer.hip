@@ -854,7 +854,7 @@ void Trainer::enqueue_lists(ViewBuffers &b, const ViewParams &v, uint32_t mode, 
   if (b.entryCapacity > 0) {
     const bool fromTmp = tile_sort_from_tmp(b.entryCapacity, b.tileBits, b.tiles);
     launch_bin_emit(s, b.keys.as<uint32_t>(), b.values.as<uint32_t>(), b.splats.as<Splat>(), b.tileRecords.as<TileRecord>(), count_, b.gridW,
-                    b.tileW, b.tileH, static_cast<uint32_t>(b.width), static_cast<uint32_t>(b.height), b.tileBits,
+                    b.tileW, b.tileH, b.tileBits,
                     b.coverage.as<uint32_t>(), counters, b.bigList.as<uint32_t>(), b.bigBits.as<uint64_t>(),
                     (fromTmp ? b.tmpEntryKeys : b.entryKeys).as<uint32_t>(), (fromTmp ? b.tmpEntryValues : b.entryValues).as<uint32_t>(),
                     entryCounts);
