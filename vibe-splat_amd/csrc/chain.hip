@@ -1153,7 +1153,7 @@ __global__ __launch_bounds__(256) void adam_kernel(ChainBuffers B, ViewParams c,
   }
 }
 
-// The SH part of that step, per packed word (as sh_step_kernel, with the
+// The SH part of that step, per packed word (as step_sh_words, with the
 // gradient read from the summed SH gradients).
 __global__ __launch_bounds__(256) void sh_adam_kernel(uint32_t *__restrict__ shWords, uint32_t *__restrict__ stateSh,
                                                       const float *__restrict__ gradSh, ViewParams c, ChainParams o,
