@@ -938,14 +938,15 @@ __global__ __launch_bounds__(kChainThreads, 4) void chain_step_kernel(ChainBuffe
 // banks). In gradients mode the sums are stored; in step mode every parameter
 // takes Adam's step from them here.
 //
-// A workgroup takes perBlock neighbouring Gaussians. Unless all have something to
-// store or to step, it packs those that a view's backward pass added to at the
-// front of a list, as chain_step_kernel does, and a view's sums are read only for
+// A workgroup takes perBlock neighbouring Gaussians. Unless all have terms or take
+// a step, it packs those that a view's backward pass added to at the
+// front of a list (the gradients of the others are cleared), as chain_step_kernel does, and a view's sums are read only for
 // the Gaussians it added to. A step over eight views of 1M Gaussians: 234 us,
 // before (all Gaussians, the SH sums through memory to a kernel of their own) 606
 // and 134; gradients of three views of 40k: 24 us. Where all are seen the step is
 // bound by its instructions at two waves a SIMD: 360 us against 310 for four
-// views of 500k, gradients 177 against 156.
+// views of 500k, gradients 182 against 156; of eight views of 1M, 4 % seen by each, 560
+// before the others' gradients were cleared in place of summed, 192 now.
 template <int Degree, uint32_t Format>
 __global__ __launch_bounds__(kChainThreads, 2) void chain_views_kernel(ChainBuffers B, ChainViews views, ChainParams o, uint32_t perBlock,
                                                                    const uint32_t *counters) {
@@ -963,7 +964,7 @@ __global__ __launch_bounds__(kChainThreads, 2) void chain_views_kernel(ChainBuff
   const uint32_t mine = count - first < perBlock ? count - first : perBlock;
   const bool penalties = o.opacityReg > 0.0f || o.scaleReg > 0.0f;
   const bool zeros = (o.flags & kFlagSelective) == 0, accumulate = (o.flags & kFlagAccumulate) != 0;
-  const bool everyone = o.mode != kModeStep || zeros || penalties || accumulate;
+  const bool everyone = (o.mode == kModeStep && zeros) || penalties || accumulate;
   uint32_t listed = 0;
   for (uint32_t r = 0; r < kRounds && r * kRound < mine; ++r) {
     const uint32_t x0 = r * kRound + threadIdx.x * 4u;
@@ -991,6 +992,22 @@ __global__ __launch_bounds__(kChainThreads, 2) void chain_views_kernel(ChainBuff
   if (o.mode == kModeStep) adam_step_now(o);
   const bool statistics = (o.flags & kFlagStatistics) != 0 && B.stats != nullptr;
   o.flags &= ~kFlagAccumulate; // the sums below are complete: they are stored, not added
+  if (o.mode == kModeGradients && !everyone && listed < mine) {
+    // The gradients of those that no view saw are zero: the workgroup's are cleared,
+    // 16 bytes at a time (`first` is a multiple of four), before the listed ones' are stored.
+    const auto clear = [&](float *values, uint32_t each) {
+      float4 *to = reinterpret_cast<float4 *>(values + static_cast<size_t>(first) * each);
+      const uint32_t words = mine * each;
+      for (uint32_t x = lane; x < words / 4u; x += kChainThreads) to[x] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      const uint32_t tail = words / 4u * 4u + lane;
+      if (tail < words) values[static_cast<size_t>(first) * each + tail] = 0.0f;
+    };
+    clear(B.gradSh, o.shFloats);
+    clear(B.gradPos, 3);
+    clear(B.gradScale, 3);
+    clear(B.gradRot, 4);
+    clear(B.gradOpacity, 1);
+  }
   for (uint32_t from = 0; from < listed; from += kChainThreads) {
     const uint32_t n = listed - from < kChainThreads ? listed - from : kChainThreads;
     __syncthreads(); // the list is whole, the sums before are read
@@ -1108,17 +1125,15 @@ __global__ __launch_bounds__(kChainThreads, 2) void chain_views_kernel(ChainBuff
           B, o, Format, shWords, first, list + from, n, zeros, [](uint32_t) { return true; }, [&](uint32_t x, size_t) { return stage[x]; },
           [&](uint32_t t, uint32_t j) { return j < kCoefficients * 3 ? shSum[j][t] : 0.0f; }, [](uint32_t, uint32_t) { return -1.0f; });
     } else {
-      // The rows, which lie consecutively (everyone is listed), with consecutive lanes
-      // on consecutive floats; coefficients above the active degree get zero (they
-      // are stored, not trained). Float x of the rows is column col of row t, kept
-      // incrementally as x advances by the block size.
+      // The rows with consecutive lanes on consecutive floats; coefficients above the
+      // active degree get zero (they are stored, not trained). Float x of the rows is
+      // column col of row t, kept incrementally as x advances by the block size.
       const uint32_t floats = o.shFloats;
-      float *out = B.gradSh + static_cast<size_t>(first + from) * floats;
       uint32_t t = lane / floats, col = lane - t * floats;
       const uint32_t stepRows = kChainThreads / floats, stepCols = kChainThreads - stepRows * floats;
 #pragma unroll 4
       for (uint32_t x = lane; x < n * floats; x += kChainThreads) {
-        out[x] = col < kCoefficients * 3 ? shSum[col][t] : 0.0f;
+        B.gradSh[static_cast<size_t>(first + list[from + t]) * floats + col] = col < kCoefficients * 3 ? shSum[col][t] : 0.0f;
         t += stepRows;
         col += stepCols;
         if (col >= floats) {
