@@ -1672,19 +1672,23 @@ uint32_t Trainer::step_views(uint32_t n, const vsplat_camera *cameras, const uin
   if (n == 0 || cameras == nullptr || targets == nullptr || bytes == nullptr) {
     throw Error(VSPLAT_INVALID_ARGUMENT, "a batch needs views and targets");
   }
-  while (viewTargets_.size() < n) viewTargets_.push_back(std::make_unique<DeviceArray>());
-  std::vector<const uint8_t *> device(n);
-  settle_upload();
+  // Every size against its camera before any of them sizes a buffer, and every
+  // buffer before the first copy: a refused call leaves nothing under way.
   size_t staged = 0;
-  for (uint32_t k = 0; k < n; ++k) staged += bytes[k];
-  viewStaging_.ensure(staged);
-  uint8_t *stage = viewStaging_.as<uint8_t>();
   for (uint32_t k = 0; k < n; ++k) {
     const size_t expected = static_cast<size_t>(cameras[k].width) * static_cast<size_t>(cameras[k].height) * 4;
     if (cameras[k].width <= 0 || cameras[k].height <= 0 || targets[k] == nullptr || bytes[k] != expected) {
       throw Error(VSPLAT_RUNTIME_ERROR, "a target image does not match its camera");
     }
-    viewTargets_[k]->ensure(bytes[k]);
+    staged += expected;
+  }
+  settle_upload();
+  while (viewTargets_.size() < n) viewTargets_.push_back(std::make_unique<DeviceArray>());
+  for (uint32_t k = 0; k < n; ++k) viewTargets_[k]->ensure(bytes[k]);
+  viewStaging_.ensure(staged);
+  std::vector<const uint8_t *> device(n);
+  uint8_t *stage = viewStaging_.as<uint8_t>();
+  for (uint32_t k = 0; k < n; ++k) {
     // Through pinned memory on the upload stream, as stage_target: only the losses wait.
     std::memcpy(stage, targets[k], bytes[k]);
     check(hipMemcpyAsync(viewTargets_[k]->as<uint8_t>(), stage, bytes[k], hipMemcpyHostToDevice, uploadStream_), "upload target");
