@@ -42,3 +42,21 @@ def test_a_target_of_the_wrong_size_is_refused(at, wrong):
         for got, want in zip(vars(b.gradients()).values(), vars(a.gradients()).values()):
             np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
         assert np.count_nonzero(b.gradients().positions) > 0
+
+
+def test_batches_of_more_views_after_single_steps():
+    """The stream that uploads targets makes room for the views' streams and comes back: single calls and batches in turn, each against a trainer of its own."""
+    cloud = F.synthetic_cloud(3000, 1, 3, log_scale=(-2.0, 0.5))
+    options = vsplat.TrainerOptions(force_fixed_point=True)
+    with vsplat.Trainer(cloud, options) as t:
+        for views in (0, 2, 0, 4, 3, 0):
+            cams = _cameras([(72 + 8 * k, 56) for k in range(max(views, 1))])
+            targets = [F.smooth_target(c.width, c.height, 3 + k + views) for k, c in enumerate(cams)]
+            with vsplat.Trainer(cloud, options) as fresh:
+                for x in (t, fresh):
+                    if views == 0:
+                        x.compute_gradients(cams[0], targets[0])
+                    else:
+                        x.step_views(cams, targets)
+                for got, want in zip(vars(t.gradients()).values(), vars(fresh.gradients()).values()):
+                    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))

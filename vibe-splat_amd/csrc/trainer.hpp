@@ -237,6 +237,8 @@ private:
   uint64_t big_bit_words_for(uint64_t entries) const;
   void stage_target(const uint8_t *target, size_t bytes);
   void settle_upload();
+  hipStream_t upload_stream();
+  void release_upload_stream();
   // The passes up to the backward pass on b's stream, then (chain) the chain rule.
   void enqueue_passes(ViewBuffers &b, const ViewParams &view, const uint8_t *deviceTarget, uint32_t mode,
                       const vsplat_learning_rates *rates, bool timed, bool chain = true);
@@ -253,6 +255,8 @@ private:
   ChainParams chain_params(const ViewParams &view, uint32_t mode, const vsplat_learning_rates *rates) const;
   ChainBuffers chain_buffers(const ViewBuffers &b) const;
   void ensure_gradients();
+  void check_views(uint32_t n, const vsplat_camera *cameras, const uint8_t *const *targets, uint32_t mode,
+                     const vsplat_learning_rates *rates) const;
   void prepare_views(uint32_t n, const vsplat_camera *cameras, const uint8_t *const *targets, uint32_t mode,
                      const vsplat_learning_rates *rates);
   uint64_t capture_key(uint32_t n) const;
