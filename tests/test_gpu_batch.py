@@ -1,9 +1,12 @@
-"""Batches of views: what a refused one leaves behind."""
+"""Batches of views: what a refused one leaves behind, batches beside single
+steps, and the batched chain rule where few, about half and all of the Gaussians
+are seen, with the options that act on the ones no view saw."""
 import ctypes as C
 
 import numpy as np
 import pytest
 
+from oracle import oracle as O
 from vsplat import fixtures as F
 import vsplat
 
@@ -60,3 +63,71 @@ def test_batches_of_more_views_after_single_steps():
                         x.step_views(cams, targets)
                 for got, want in zip(vars(t.gradients()).values(), vars(fresh.gradients()).values()):
                     np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+NAMES = ("positions", "scales", "rotations", "opacities", "sh")
+RATE_TUPLE = (RATES.position, RATES.scale, RATES.rotation, RATES.opacity, RATES.sh)
+
+
+def _bits(a):
+    return np.ascontiguousarray(a, np.float32).view(np.uint32).reshape(-1)
+
+
+def _states(t):
+    return [t.inspect(f"state_{k}") for k in NAMES]
+
+
+@pytest.mark.parametrize("options", [{}, {"selective_adam": False}, {"opacity_reg": 0.5, "scale_reg": 0.25}, {"active": 1},
+                                     {"selective_adam": False, "opacity_reg": 0.5, "active": 2}],
+                         ids=["plain", "every parameter", "penalties", "degree 1", "all of them"])
+@pytest.mark.parametrize("views,storage", [(2, vsplat.SH_HALF), (9, vsplat.SH_BF16)])
+@pytest.mark.parametrize("seen", [0.04, 0.5, 0.62, 1.0])
+def test_batches_by_the_share_seen(seen, views, storage, options):
+    """Gradients and a step of a batch against Oracle B's summed gradients and its Adam, and a second step against the gradients stored, then applied.
+    Workgroups of 64 Gaussians, whose shares seen lie on both sides of where a whole workgroup is listed."""
+    count, degree = 1217, 3
+    active = options.get("active", degree)
+    given = {k: v for k, v in options.items() if k != "active"}
+    regs = {k: given.get(k, 0.0) for k in ("opacity_reg", "scale_reg")}
+    selective = given.get("selective_adam", True)
+    rng = np.random.default_rng(7)
+    cloud = F.synthetic_cloud(count, degree, 23, log_scale=(-3.5, 0.4), sh_sigma=0.3)
+    cloud.positions[:] = rng.uniform(-0.6, 0.6, (count, 3)).astype(np.float32)
+    cloud.positions[rng.permutation(count)[round(seen * count):], 2] = -9.0  # behind every camera
+    cloud.opacities[:] = -2.0
+    cams = _cameras([(72 + 8 * (k % 3), 56) for k in range(views)])
+    targets = [F.smooth_target(c.width, c.height, 3 + k) for k, c in enumerate(cams)]
+    total, stats = None, np.zeros((count, 8), np.float32)
+    for cam, target in zip(cams, targets):
+        m = O.Model(cloud, cam, active_degree=active, sh_storage=storage)
+        r = m.forward()
+        m.loss(r, target, 0.2)
+        m.backward_fixed(r)
+        g, stats = m.gradients(r, stats=stats, **regs)
+        total = [x.copy() for x in g] if total is None else [a + b for a, b in zip(total, g)]
+    with vsplat.Trainer(cloud, vsplat.TrainerOptions(force_fixed_point=True, sh_storage=storage, **given)) as a, \
+         vsplat.Trainer(cloud, vsplat.TrainerOptions(force_fixed_point=True, sh_storage=storage, **given)) as b:
+        for t in (a, b):
+            t.set_active_sh_degree(active)
+        uploaded = a.cloud()
+        states = [np.zeros_like(s) for s in _states(a)]
+        pos, sc, rot, op, words = O.adam_from_gradients(uploaded, m.words, total, RATE_TUPLE, rest_scale=RATES.sh_rest_scale, selective=selective,
+                                                        sh_storage=storage, states=states)
+        b.step_views(cams, targets)
+        for name, want in zip(NAMES, total):
+            np.testing.assert_array_equal(_bits(getattr(b.gradients(), name)), _bits(want))
+        np.testing.assert_array_equal(_bits(b.densify_stats()), _bits(stats))
+        b.apply_gradients(RATES)
+        a.step_views(cams, targets, RATES)
+        after = a.cloud()
+        for name, want in zip(NAMES, (pos, sc, rot, op, F.unpack_sh(words, cloud.coefficients, storage))):
+            np.testing.assert_array_equal(_bits(getattr(after, name)), _bits(want))
+        for got, want in zip(_states(a), states):
+            np.testing.assert_array_equal(got, want)
+        a.step_views(cams, targets, RATES)
+        b.step_views(cams, targets)
+        b.apply_gradients(RATES)
+        for name in NAMES:
+            np.testing.assert_array_equal(_bits(getattr(a.cloud(), name)), _bits(getattr(b.cloud(), name)))
+        for got, want in zip(_states(a), _states(b)):
+            np.testing.assert_array_equal(got, want)

@@ -750,8 +750,9 @@ __device__ __forceinline__ void step_geometry(const ChainBuffers &B, const Chain
 // The packed SH words of the list's Gaussians stepped, or their curvature taken, a
 // thread a word, the next one's loads ahead. wanted(t): whether row t has any
 // gradients; wordOf(x, place): word x of the rows, the one at `place`;
-// gradient(t, j): of SH float j; radius(t, ch): second order's, else -1.
-template <typename Wanted, typename WordOf, typename Gradient, typename Radius>
+// gradient(t, j): of SH float j (with Ahead loaded with the word: from global memory);
+// radius(t, ch): second order's, else -1.
+template <bool Ahead = false, typename Wanted, typename WordOf, typename Gradient, typename Radius>
 __device__ __forceinline__ void step_sh_words(const ChainBuffers &B, const ChainParams &o, uint32_t format, uint32_t words, uint32_t first,
                                               const uint16_t *list, uint32_t n, bool zeros, Wanted &&wanted, WordOf &&wordOf,
                                               Gradient &&gradient, Radius &&radius) {
@@ -761,6 +762,7 @@ __device__ __forceinline__ void step_sh_words(const ChainBuffers &B, const Chain
     uint32_t t, i, first, last; // a word of Gaussian i (row t), its floats first .. last
     size_t at;
     uint32_t word, state[2];
+    float gradient[2]; // with Ahead
     bool wanted;
   };
   const auto load = [&](uint32_t x, Word &w) {
@@ -778,6 +780,10 @@ __device__ __forceinline__ void step_sh_words(const ChainBuffers &B, const Chain
     const uint32_t s = w.i * o.shFloats + w.first;
     w.state[0] = B.stateSh[s];
     w.state[1] = w.last > w.first ? B.stateSh[s + 1] : 0u;
+    if constexpr (Ahead) {
+      w.gradient[0] = gradient(w.t, w.first);
+      w.gradient[1] = w.last > w.first ? gradient(w.t, w.last) : 0.0f;
+    }
   };
   Word next{};
   load(threadIdx.x, next);
@@ -789,7 +795,7 @@ __device__ __forceinline__ void step_sh_words(const ChainBuffers &B, const Chain
     bool changed = false;
 #pragma unroll 1
     for (uint32_t j = w.first; j <= w.last; ++j) {
-      const float gv = gradient(w.t, j);
+      const float gv = Ahead ? (j == w.first ? w.gradient[0] : w.gradient[1]) : gradient(w.t, j);
       if (gv == 0.0f && !zeros) continue;
       const uint32_t s = w.i * o.shFloats + j;
       uint32_t state = j == w.first ? w.state[0] : w.state[1];
@@ -935,28 +941,36 @@ __global__ __launch_bounds__(kChainThreads, 4) void chain_step_kernel(ChainBuffe
 // (its LDS) needs to keep loads in flight. The geometric sums stay in
 // registers and the SH sums in LDS, one row per coefficient (of an odd length, so
 // that lanes on one coefficient and lanes on one Gaussian both hit distinct
-// banks). In gradients mode the sums are stored; in step mode every parameter
-// takes Adam's step from them here.
+// banks). The sums are stored; in a step the geometric parameters take Adam's
+// from the registers and only the SH sums are stored, for sh_step_views_kernel.
 //
 // A workgroup takes perBlock neighbouring Gaussians. Unless all have terms or take
-// a step, it packs those that a view's backward pass added to at the
-// front of a list (the gradients of the others are cleared), as chain_step_kernel does, and a view's sums are read only for
-// the Gaussians it added to. A step over eight views of 1M Gaussians: 234 us,
-// before (all Gaussians, the SH sums through memory to a kernel of their own) 606
-// and 134; gradients of three views of 40k: 24 us. Where all are seen the step is
-// bound by its instructions at two waves a SIMD: 360 us against 310 for four
-// views of 500k, gradients 182 against 156; of eight views of 1M, 4 % seen by each, 560
-// before the others' gradients were cleared in place of summed, 192 now.
-template <int Degree, uint32_t Format>
+// a step, it packs those that a view's backward pass added to at the front of a
+// list (the gradients of the others are cleared), as chain_step_kernel does, and
+// a view's sums are read only for the Gaussians it added to. Where most are listed
+// it lists all instead: their words are then neighbours and nothing is cleared.
+// Packed and whole at 500k and four views (degree 3, us): gradients of 51 % seen by
+// some view 168 and 166, 58 % 169 and 168, 69 % 200 and 171; the step 58 % 171 and 199,
+// 69 % 211 and 198. So half, and five eighths in a step, which clears nothing.
+//
+// With the SH sums through memory to a kernel of their own the step's share at two
+// waves a SIMD (what this kernel's LDS and registers leave) is the geometric one:
+// a step of the same 500k all seen 196 + 119 us, 359 with the SH words stepped
+// here; 20 % seen 99 + 37 for 142, of 1M and eight views 32 % seen 364 + 82 for 452. (All
+// Gaussians in both kernels: 181 + 126, 197 + 89, 661 + 163. Gradients of 500k all
+// seen 167, then 157: there the loop over the views was unrolled, eight copies of
+// the terms, 90 KB of instructions and too many registers for the packed form.)
+template <int Degree, uint32_t Format, bool Step>
 __global__ __launch_bounds__(kChainThreads, 2) void chain_views_kernel(ChainBuffers B, ChainViews views, ChainParams o, uint32_t perBlock,
                                                                    const uint32_t *counters) {
   constexpr uint32_t kCoefficients = (Degree + 1) * (Degree + 1), kSums = kChainThreads + 1;
-  constexpr uint32_t kRound = 4 * kChainThreads, kRounds = kViewsMost / kRound;
+  static_assert(kViewsMost == 4 * kChainThreads, "a thread packs four Gaussians");
   __shared__ float shSum[kCoefficients * 3][kSums];
   __shared__ uint32_t stage[kChainThreads * 26];
   __shared__ uint16_t list[kViewsMost];
   __shared__ uint8_t seenBy[kViewsMost]; // per listed Gaussian, the views whose sums may not be zero
   __shared__ uint32_t waveTotals[kChainThreads / 64];
+  o.mode = Step ? kModeStep : kModeGradients; // known when compiled
   const uint32_t lane = threadIdx.x;
   const uint32_t count = views.view[0].c.count, shWords = views.view[0].c.shWords;
   if (counters[kOverflow] != 0) return;
@@ -964,35 +978,37 @@ __global__ __launch_bounds__(kChainThreads, 2) void chain_views_kernel(ChainBuff
   const uint32_t mine = count - first < perBlock ? count - first : perBlock;
   const bool penalties = o.opacityReg > 0.0f || o.scaleReg > 0.0f;
   const bool zeros = (o.flags & kFlagSelective) == 0, accumulate = (o.flags & kFlagAccumulate) != 0;
-  const bool everyone = (o.mode == kModeStep && zeros) || penalties || accumulate;
-  uint32_t listed = 0;
-  for (uint32_t r = 0; r < kRounds && r * kRound < mine; ++r) {
-    const uint32_t x0 = r * kRound + threadIdx.x * 4u;
-    uint32_t seen = 0; // a byte each for four neighbours
+  const bool everyone = (Step && zeros) || penalties || accumulate;
+  const uint32_t x0 = threadIdx.x * 4u;
+  uint32_t seen = 0; // a byte each for four neighbours
 #pragma unroll
-    for (uint32_t v = 0; v < kChainViewsPerLaunch; ++v) {
-      const uint32_t flags = v < views.count && x0 < mine ? reinterpret_cast<const uint32_t *>(views.view[v].touched + first)[x0 / 4u] : 0u;
-      seen |= flags << v; // a flag is 0 or 1
-    }
-    uint32_t wanted = 0, at;
-#pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) {
-      if (x0 + k < mine && (everyone || ((seen >> (8u * k)) & 0xFFu) != 0)) wanted |= 1u << k;
-    }
-    const uint32_t total = block_exclusive_sum(static_cast<uint32_t>(__popc(wanted)), at, waveTotals);
-    at += listed;
-    listed += total;
-#pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) {
-      if (((wanted >> k) & 1u) == 0) continue;
-      list[at] = static_cast<uint16_t>(x0 + k);
-      seenBy[at++] = static_cast<uint8_t>(seen >> (8u * k));
-    }
+  for (uint32_t v = 0; v < kChainViewsPerLaunch; ++v) {
+    const uint32_t flags = v < views.count && x0 < mine ? reinterpret_cast<const uint32_t *>(views.view[v].touched + first)[x0 / 4u] : 0u;
+    seen |= flags << v; // a flag is 0 or 1
   }
-  if (o.mode == kModeStep) adam_step_now(o);
+  uint32_t wanted = 0, valid = 0, at;
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    if (x0 + k < mine) valid |= 1u << k;
+    if (x0 + k < mine && (everyone || ((seen >> (8u * k)) & 0xFFu) != 0)) wanted |= 1u << k;
+  }
+  uint32_t listed = block_exclusive_sum(static_cast<uint32_t>(__popc(wanted)), at, waveTotals);
+  const bool whole = listed * 8u >= mine * (Step ? 5u : 4u);
+  if (whole) {
+    wanted = valid;
+    at = x0;
+    listed = mine;
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    if (((wanted >> k) & 1u) == 0) continue;
+    list[at] = static_cast<uint16_t>(x0 + k);
+    seenBy[at++] = static_cast<uint8_t>(seen >> (8u * k));
+  }
+  if (Step) adam_step_now(o);
   const bool statistics = (o.flags & kFlagStatistics) != 0 && B.stats != nullptr;
   o.flags &= ~kFlagAccumulate; // the sums below are complete: they are stored, not added
-  if (o.mode == kModeGradients && !everyone && listed < mine) {
+  if (!Step && !whole) {
     // The gradients of those that no view saw are zero: the workgroup's are cleared,
     // 16 bytes at a time (`first` is a multiple of four), before the listed ones' are stored.
     const auto clear = [&](float *values, uint32_t each) {
@@ -1014,7 +1030,7 @@ __global__ __launch_bounds__(kChainThreads, 2) void chain_views_kernel(ChainBuff
     // The SH words, read by every view, staged once through LDS: with 16-byte loads
     // where the Gaussians are neighbours (`first` is a multiple of four), else
     // several loads at a time.
-    if (everyone) {
+    if (whole) {
       stage_words<kChainThreads>(stage, B.shWords + static_cast<size_t>(first + from) * shWords, n * shWords);
     } else {
       constexpr uint32_t kBatch = 8;
@@ -1035,7 +1051,7 @@ __global__ __launch_bounds__(kChainThreads, 2) void chain_views_kernel(ChainBuff
     }
     __syncthreads();
     if (lane < n) {
-      const uint32_t i = first + list[from + lane], seen = seenBy[from + lane];
+      const uint32_t i = first + (whole ? from + lane : list[from + lane]), seen = seenBy[from + lane];
       const uint32_t *words = stage + lane * shWords;
       // A later chunk of a batch continues from the sums the earlier ones stored.
       ViewTerms sum;
@@ -1119,21 +1135,16 @@ __global__ __launch_bounds__(kChainThreads, 2) void chain_views_kernel(ChainBuff
       emit_terms(B, o, i, sum, Radii{-1.0f, -1.0f, -1.0f}); // a batch takes Adam's step
     }
     __syncthreads(); // the SH sums are whole
-    if (o.mode == kModeStep) {
-      // Coefficients above the active degree have no gradients.
-      step_sh_words(
-          B, o, Format, shWords, first, list + from, n, zeros, [](uint32_t) { return true; }, [&](uint32_t x, size_t) { return stage[x]; },
-          [&](uint32_t t, uint32_t j) { return j < kCoefficients * 3 ? shSum[j][t] : 0.0f; }, [](uint32_t, uint32_t) { return -1.0f; });
-    } else {
-      // The rows with consecutive lanes on consecutive floats; coefficients above the
-      // active degree get zero (they are stored, not trained). Float x of the rows is
-      // column col of row t, kept incrementally as x advances by the block size.
-      const uint32_t floats = o.shFloats;
-      uint32_t t = lane / floats, col = lane - t * floats;
-      const uint32_t stepRows = kChainThreads / floats, stepCols = kChainThreads - stepRows * floats;
+    // The rows with consecutive lanes on consecutive floats; coefficients above the
+    // active degree get zero (they are stored, not trained). Float x of the rows is
+    // column col of row t, kept incrementally as x advances by the block size.
+    const uint32_t floats = o.shFloats;
+    uint32_t t = lane / floats, col = lane - t * floats;
+    const uint32_t stepRows = kChainThreads / floats, stepCols = kChainThreads - stepRows * floats;
+    const auto store = [&](auto &&rowOf) {
 #pragma unroll 4
       for (uint32_t x = lane; x < n * floats; x += kChainThreads) {
-        B.gradSh[static_cast<size_t>(first + list[from + t]) * floats + col] = col < kCoefficients * 3 ? shSum[col][t] : 0.0f;
+        B.gradSh[static_cast<size_t>(first + rowOf(t)) * floats + col] = col < kCoefficients * 3 ? shSum[col][t] : 0.0f;
         t += stepRows;
         col += stepCols;
         if (col >= floats) {
@@ -1141,7 +1152,54 @@ __global__ __launch_bounds__(kChainThreads, 2) void chain_views_kernel(ChainBuff
           ++t;
         }
       }
+    };
+    if (whole) {
+      store([&](uint32_t r) { return from + r; });
+    } else {
+      store([&](uint32_t r) { return static_cast<uint32_t>(list[from + r]); });
     }
+  }
+}
+
+// The SH coefficients' part of a batch's step, from the sums chain_views_kernel
+// stored: the Gaussians that have some packed as there, a thread per packed word.
+// Coefficients above the active degree have no gradients. Bound by the step's
+// instructions (step_sh_words), at eight waves a SIMD; where few are seen, by the
+// way to memory of one load after the other, which more, smaller workgroups
+// shorten (16 Gaussians at least for 64: 12 us for 15 at 40k, 15 for 20 at 30k).
+template <uint32_t Format>
+__global__ __launch_bounds__(kChainThreads) void sh_step_views_kernel(ChainBuffers B, ChainViews views, ChainParams o, uint32_t perBlock,
+                                                                      const uint32_t *counters) {
+  __shared__ uint16_t list[kViewsMost];
+  __shared__ uint32_t waveTotals[kChainThreads / 64];
+  const uint32_t count = views.view[0].c.count, shWords = views.view[0].c.shWords;
+  if (counters[kOverflow] != 0) return;
+  const uint32_t first = blockIdx.x * perBlock;
+  const uint32_t mine = count - first < perBlock ? count - first : perBlock;
+  // After an earlier chunk of the batch (kFlagAccumulate) its views' Gaussians have some too.
+  const bool zeros = (o.flags & kFlagSelective) == 0, everyone = zeros || (o.flags & kFlagAccumulate) != 0;
+  const uint32_t x0 = threadIdx.x * 4u;
+  uint32_t seen = 0, wanted = 0, at;
+#pragma unroll
+  for (uint32_t v = 0; v < kChainViewsPerLaunch; ++v) {
+    if (v < views.count && x0 < mine) seen |= reinterpret_cast<const uint32_t *>(views.view[v].touched + first)[x0 / 4u];
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    if (x0 + k < mine && (everyone || ((seen >> (8u * k)) & 0xFFu) != 0)) wanted |= 1u << k;
+  }
+  const uint32_t listed = block_exclusive_sum(static_cast<uint32_t>(__popc(wanted)), at, waveTotals);
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    if (((wanted >> k) & 1u) != 0) list[at++] = static_cast<uint16_t>(x0 + k);
+  }
+  adam_step_now(o);
+  __syncthreads();
+  for (uint32_t from = 0; from < listed; from += kChainThreads) {
+    const uint32_t n = listed - from < kChainThreads ? listed - from : kChainThreads;
+    step_sh_words<true>(
+        B, o, Format, shWords, first, list + from, n, zeros, [](uint32_t) { return true; }, [&](uint32_t, size_t place) { return B.shWords[place]; },
+        [&](uint32_t t, uint32_t j) { return B.gradSh[(first + list[from + t]) * o.shFloats + j]; }, [](uint32_t, uint32_t) { return -1.0f; });
   }
 }
 
@@ -1344,9 +1402,9 @@ __global__ __launch_bounds__(256) void keep_first_moment_kernel(uint32_t *__rest
 
 // The Gaussians of a workgroup: equal shares for as many workgroups as are
 // resident, a multiple of four so that their flags are whole words.
-static uint32_t chain_share(uint32_t count, uint32_t perCu, uint32_t most) {
+static uint32_t chain_share(uint32_t count, uint32_t perCu, uint32_t most, uint32_t least = kStepLeast) {
   const uint32_t share = ((count + perCu * 256 - 1) / (perCu * 256) + 3) / 4 * 4;
-  return share < kStepLeast ? kStepLeast : (share < most ? share : most);
+  return share < least ? least : (share < most ? share : most);
 }
 
 void launch_chain(hipStream_t stream, const ChainBuffers &buffers, const ViewParams &view, const ChainParams &params,
@@ -1375,9 +1433,25 @@ void launch_chain_views(hipStream_t stream, const ChainBuffers &buffers, const C
   if (count == 0 || views.count == 0) return;
   const uint32_t perBlock = chain_share(count, 2, kViewsMost); // two workgroups a CU are resident
   const dim3 grid((count + perBlock - 1) / perBlock), block(256);
-#define VSPLAT_CHAIN(D, F) hipLaunchKernelGGL((chain_views_kernel<D, F>), grid, block, 0, stream, buffers, views, params, perBlock, counters)
-  VSPLAT_SH_DISPATCH(views.view[0].c.shDegree, views.view[0].c.shFormat, VSPLAT_CHAIN)
-#undef VSPLAT_CHAIN
+#define VSPLAT_CHAIN_VIEWS(D, F, S)                                                                                                \
+  hipLaunchKernelGGL((chain_views_kernel<D, F, S>), grid, block, 0, stream, buffers, views, params, perBlock, counters)
+#define VSPLAT_CHAIN_GRADIENTS(D, F) VSPLAT_CHAIN_VIEWS(D, F, false)
+#define VSPLAT_CHAIN_STEP(D, F) VSPLAT_CHAIN_VIEWS(D, F, true)
+  if (params.mode != kModeStep) {
+    VSPLAT_SH_DISPATCH(views.view[0].c.shDegree, views.view[0].c.shFormat, VSPLAT_CHAIN_GRADIENTS)
+    return;
+  }
+  VSPLAT_SH_DISPATCH(views.view[0].c.shDegree, views.view[0].c.shFormat, VSPLAT_CHAIN_STEP)
+#undef VSPLAT_CHAIN_STEP
+#undef VSPLAT_CHAIN_GRADIENTS
+#undef VSPLAT_CHAIN_VIEWS
+  const uint32_t share = chain_share(count, 8, kViewsMost, 16); // eight workgroups a CU are resident
+  const dim3 shGrid((count + share - 1) / share);
+  if (views.view[0].c.shFormat == kShBf16) {
+    hipLaunchKernelGGL(sh_step_views_kernel<kShBf16>, shGrid, block, 0, stream, buffers, views, params, share, counters);
+  } else {
+    hipLaunchKernelGGL(sh_step_views_kernel<kShHalf>, shGrid, block, 0, stream, buffers, views, params, share, counters);
+  }
 }
 
 void launch_noise(hipStream_t stream, const ChainBuffers &buffers, uint32_t count, float scaler, const uint32_t *iterationDev,

@@ -306,7 +306,8 @@ void launch_error_mask(hipStream_t stream, float4 *adjoint, const uint32_t *erro
 
 // The chain rule over the views of a batch chunk, summed per Gaussian in view
 // order (kFlagAccumulate: continuing from the sums an earlier chunk stored).
-// Gradients mode stores the sums; step mode takes every parameter's Adam step from them.
+// Gradients mode stores the sums; step mode takes every parameter's Adam step
+// from them (the SH ones by way of gradSh).
 void launch_chain_views(hipStream_t stream, const ChainBuffers &buffers, const ChainViews &views, const ChainParams &params,
                         const uint32_t *counters);
 // One Adam step of every parameter from the stored gradients in buffers.grad*
