@@ -309,8 +309,7 @@ int vsplat_reserve_entries(vsplat_trainer *trainer, uint64_t entries);
  * the gradients summed over the views in view order (each view's objective
  * includes the penalties, and adds to the densification statistics), then for
  * mode 2 one Adam step from the sum (one step count, one bias correction); mode 1
- * keeps the sum for vsplat_get_gradients (mode 2 uses their memory: gradients stored
- * before are lost). targets[k] is view k's RGBA8 image in
+ * keeps the sum for vsplat_get_gradients. targets[k] is view k's RGBA8 image in
  * host memory, bytes[k] its size. stats (may be NULL) gets n entries. A view that
  * does not fit the tile-entry reservation grows it and the batch runs again, as
  * vsplat_step does. */

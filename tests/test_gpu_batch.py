@@ -131,3 +131,14 @@ def test_batches_by_the_share_seen(seen, views, storage, options):
             np.testing.assert_array_equal(_bits(getattr(a.cloud(), name)), _bits(getattr(b.cloud(), name)))
         for got, want in zip(_states(a), _states(b)):
             np.testing.assert_array_equal(got, want)
+
+
+def test_a_step_over_views_leaves_the_stored_gradients():
+    cloud, cams = F.synthetic_cloud(3000, 2, 3, log_scale=(-2.0, 0.5)), _cameras([(72, 56), (96, 40)])
+    targets = [F.smooth_target(c.width, c.height, 3 + k) for k, c in enumerate(cams)]
+    with vsplat.Trainer(cloud, vsplat.TrainerOptions(force_fixed_point=True)) as t:
+        t.compute_gradients(cams[0], targets[0])
+        before = vars(t.gradients())
+        t.step_views(cams, targets, RATES)
+        for name, got in vars(t.gradients()).items():
+            np.testing.assert_array_equal(_bits(got), _bits(before[name]))

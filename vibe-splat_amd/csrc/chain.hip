@@ -1141,10 +1141,11 @@ __global__ __launch_bounds__(kChainThreads, 2) void chain_views_kernel(ChainBuff
     const uint32_t floats = o.shFloats;
     uint32_t t = lane / floats, col = lane - t * floats;
     const uint32_t stepRows = kChainThreads / floats, stepCols = kChainThreads - stepRows * floats;
+    float *const sums = Step ? B.shSums : B.gradSh;
     const auto store = [&](auto &&rowOf) {
 #pragma unroll 4
       for (uint32_t x = lane; x < n * floats; x += kChainThreads) {
-        B.gradSh[static_cast<size_t>(first + rowOf(t)) * floats + col] = col < kCoefficients * 3 ? shSum[col][t] : 0.0f;
+        sums[static_cast<size_t>(first + rowOf(t)) * floats + col] = col < kCoefficients * 3 ? shSum[col][t] : 0.0f;
         t += stepRows;
         col += stepCols;
         if (col >= floats) {
@@ -1199,7 +1200,7 @@ __global__ __launch_bounds__(kChainThreads) void sh_step_views_kernel(ChainBuffe
     const uint32_t n = listed - from < kChainThreads ? listed - from : kChainThreads;
     step_sh_words<true>(
         B, o, Format, shWords, first, list + from, n, zeros, [](uint32_t) { return true; }, [&](uint32_t, size_t place) { return B.shWords[place]; },
-        [&](uint32_t t, uint32_t j) { return B.gradSh[(first + list[from + t]) * o.shFloats + j]; }, [](uint32_t, uint32_t) { return -1.0f; });
+        [&](uint32_t t, uint32_t j) { return B.shSums[(first + list[from + t]) * o.shFloats + j]; }, [](uint32_t, uint32_t) { return -1.0f; });
   }
 }
 

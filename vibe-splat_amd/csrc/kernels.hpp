@@ -54,6 +54,7 @@ struct ChainBuffers {
   float *stats; // 8 per Gaussian, or null
   uint32_t *statePos, *stateScale, *stateRot, *stateOpacity, *stateSh;
   float *gradPos, *gradScale, *gradRot, *gradOpacity, *gradSh;
+  float *shSums; // a batch's summed SH gradients on their way to its step
   float4 *dirTerms; // per Gaussian: the view direction's term of the position gradient (between the gradients' two kernels)
   float *poseTerms; // 6 per Gaussian with kFlagPose: t x v, then v = Rv dL/dp; untouched Gaussians' left as they are
 };
@@ -307,7 +308,7 @@ void launch_error_mask(hipStream_t stream, float4 *adjoint, const uint32_t *erro
 // The chain rule over the views of a batch chunk, summed per Gaussian in view
 // order (kFlagAccumulate: continuing from the sums an earlier chunk stored).
 // Gradients mode stores the sums; step mode takes every parameter's Adam step
-// from them (the SH ones by way of gradSh).
+// from them (the SH ones by way of shSums).
 void launch_chain_views(hipStream_t stream, const ChainBuffers &buffers, const ChainViews &views, const ChainParams &params,
                         const uint32_t *counters);
 // One Adam step of every parameter from the stored gradients in buffers.grad*

@@ -977,6 +977,7 @@ ChainBuffers Trainer::chain_buffers(const ViewBuffers &v) const {
   b.gradRot = grad_[2].as<float>();
   b.gradOpacity = grad_[3].as<float>();
   b.gradSh = grad_[4].as<float>();
+  b.shSums = shSums_.as<float>();
   b.dirTerms = dirTerms_.as<float4>();
   return b;
 }
@@ -1381,7 +1382,10 @@ void Trainer::prepare_views(uint32_t n, const vsplat_camera *cameras, const uint
     if (targets[k] == nullptr) throw Error(VSPLAT_INVALID_ARGUMENT, "no target for a view");
     ensure_size(view_buffers(k), cameras[k].width, cameras[k].height);
   }
-  ensure_gradients();
+  // Gradients are stored, or carried from one chunk of a long batch to the next; a
+  // step's SH sums have a place of their own, so that stored gradients stay.
+  if (mode == kModeGradients || n > kChainViewsPerLaunch) ensure_gradients();
+  if (mode == kModeStep) shSums_.ensure(static_cast<size_t>(count_) * shFloats_ * 4);
   if (viewStats_.bytes() < static_cast<size_t>(n) * kViewStatsBytes) {
     check(hipStreamSynchronize(stream_), "view stats"); // a queued batch may still write the old one
     viewStats_.ensure(static_cast<size_t>(n) * kViewStatsBytes);
@@ -1581,7 +1585,7 @@ uint64_t Trainer::capture_key(uint32_t n) const {
     mix(reinterpret_cast<uintptr_t>(a.as<void>()));
     mix(a.bytes());
   };
-  for (const DeviceArray *a : {&positions_, &scales_, &rotations_, &opacities_, &shWordsBuf_, &adamState_, &stats_, &filter3d_})
+  for (const DeviceArray *a : {&positions_, &scales_, &rotations_, &opacities_, &shWordsBuf_, &adamState_, &stats_, &filter3d_, &shSums_})
     array(*a);
   mix(reinterpret_cast<uintptr_t>(viewStats_.as<void>()));
   for (int g = 0; g < 5; ++g) {
@@ -1843,6 +1847,7 @@ void Trainer::apply_changes(const vsplat_cloud *cloud, const int64_t *source, ui
     state_[g].swap(state[g]);
     grad_[g].release();
   }
+  shSums_.release();
   count_ = count;
   haveGradients_ = false;
   accumulateNext_ = false;
@@ -1957,7 +1962,7 @@ uint64_t Trainer::gpu_bytes() const {
     }
   }
   for (const DeviceArray &a : grad_) total += a.bytes();
-  total += poseTerms_.bytes() + poseTotals_.bytes();
+  total += shSums_.bytes() + poseTerms_.bytes() + poseTotals_.bytes();
   return total;
 }
 

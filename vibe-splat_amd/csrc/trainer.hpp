@@ -298,6 +298,7 @@ private:
   // Parameters and optimiser state, in GaussianCloud's layout; SH packed as halves.
   DeviceArray positions_, scales_, rotations_, opacities_, shWordsBuf_;
   DeviceArray state_[5], grad_[5];
+  DeviceArray shSums_; // a batch's summed SH gradients, between the two kernels of its step
   DeviceArray adamState_; // steps taken, beta1^steps, beta2^steps (ChainParams::adamState)
   // Per Gaussian, shared by the views.
   DeviceArray stats_, filter3d_, dirTerms_;
