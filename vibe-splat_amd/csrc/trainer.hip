@@ -11,6 +11,7 @@
 // within the memory budget, and runs the step again. In steady state that is
 // one synchronisation per step and no host work between kernels.
 #include "trainer.hpp"
+#include "helpers.hpp"
 #include "tiles.hpp"
 
 #include <algorithm>
@@ -171,8 +172,8 @@ template <class Wanted> bool Downloads::run(hipStream_t stream, const std::vecto
     }
   } join{stop, helpers};
   for (size_t k = 0; k < std::min(n, kSlots); ++k) fetch(k);
-  for (size_t h = 0; h < kHelpers && total >= kHelped; ++h) {
-    helpers.emplace_back([&] {
+  if (total >= kHelped) {
+    start_helpers(helpers, kHelpers, [&] {
       for (uint32_t spins = 0; !stop;) {
         size_t k = next;
         if (k >= n) return;
