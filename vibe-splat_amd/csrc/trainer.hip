@@ -1857,6 +1857,8 @@ void Trainer::apply_changes(const vsplat_cloud *cloud, const int64_t *source, ui
   allocate_per_gaussian();
   view_buffers(0);
   check(hipStreamSynchronize(stream_), "per-Gaussian buffers");
+  // The status of a pass over the old cloud goes with its counters.
+  std::memset(readback_.as<uint8_t>(), 0, kStatusSlot);
 }
 
 // Trainer::enable_second_order (trainer.cpp:642-654): from now on the states'
