@@ -1,5 +1,6 @@
-"""The status a queued pass leaves in host memory, where its cloud is replaced
-before anybody has asked for it."""
+"""What a trainer says of itself: the status a queued pass leaves in host memory,
+where its cloud is replaced before anybody has asked for it, and the memory it
+holds."""
 import numpy as np
 import pytest
 
@@ -20,3 +21,11 @@ def test_a_changed_cloud_has_no_status(fits):
         stats = t.synchronize()
         assert (stats.visible_splats, stats.tile_entries) == (0, 0)
         assert t.compute_gradients(cam, F.smooth_target(320, 240, 3)).visible_splats > 0
+
+
+@pytest.mark.parametrize("count", [1, 5000])
+def test_the_sorts_digit_counts_are_memory_too(count):
+    """Per tile of 4096 keys and pass 256 words: four passes over the Gaussians, three over at most 2^18 tile entries."""
+    words = 4 * -(-count // 4096) * 256 + 3 * 64 * 256
+    with vsplat.Trainer(F.synthetic_cloud(count, 0, 3)) as t:
+        assert t.gpu_bytes() - t.bytes_per_gaussian() * count >= 4 * words

@@ -1942,8 +1942,8 @@ uint64_t Trainer::bytes_per_gaussian() const {
   // Values (SH as packed words) and one optimiser word per parameter.
   const uint64_t parameters = (floats - shFloats_ + shWords_) * 4 + floats * 4;
   // Splat, sort keys and values with copies, coverage, tile count, filter, big
-  // splat list, tile record, sums, SH-pass data, the direction term between the
-  // chain kernels, statistics.
+  // splat list, tile record, sums and whether they are set, the direction term
+  // between the chain kernels, statistics.
   const uint64_t raw = fixedPoint_ ? kRawPerSplat * 8 : kRawPerSplat * 4;
   return parameters + sizeof(Splat) + 4 * 8 + sizeof(TileRecord) + raw + 1 + 16 + 32;
 }
@@ -1955,12 +1955,12 @@ uint64_t Trainer::gpu_bytes() const {
     const ViewBuffers &b = *views_[k];
     for (const DeviceArray *a : {&b.image, &b.stops, &b.adjoint, &b.fields, &b.ranges, &b.tileTotals, &b.listOrder, &b.blockWork,
                                  &b.blockOrder, &b.entryKeys, &b.entryValues, &b.tmpEntryKeys, &b.tmpEntryValues, &b.bigBits, &b.exposed,
-                                 &b.edge, &b.exposureTotals, &b.errorMax}) {
+                                 &b.edge, &b.exposureTotals, &b.errorMax, &b.sortCounts}) {
       total += a->bytes();
     }
     if (k == 0) continue;
     for (const DeviceArray *a : {&b.splats, &b.keys, &b.values, &b.tmpKeys, &b.tmpValues, &b.coverage, &b.tileCount, &b.tileRecords,
-                                 &b.bigList, &b.rawFixed, &b.rawFloat, &b.touched, &b.sortScratch, &b.sortCounts, &b.scanScratch}) {
+                                 &b.bigList, &b.rawFixed, &b.rawFloat, &b.touched, &b.sortScratch, &b.scanScratch}) {
       total += a->bytes();
     }
   }
