@@ -1284,7 +1284,11 @@ void Trainer::render_into(const vsplat_camera &camera, float *deviceOut, uint64_
   for (DeviceArray *a : {&b.entryKeys, &b.entryValues, &b.tmpEntryKeys, &b.tmpEntryValues}) carve(*a, entries * 4);
   carve(b.stops, uint64_t{VSPLAT_NOALLOC_MAX_PIXELS} * 4);
   carve(b.ranges, uint64_t{VSPLAT_NOALLOC_MAX_TILES} * 8);
-  carve(b.sortScratch, std::max(depth_sort_scratch_words(n), tile_sort_scratch_words(entries, b.tiles)) * 4);
+  // For the largest of the tile sorts, whose scratch grows with the tiles up to the bound of each.
+  size_t sortWords = depth_sort_scratch_words(n);
+  for (uint32_t tiles : {kTileSortTiles / 2, kTileSortTiles, VSPLAT_NOALLOC_MAX_TILES})
+    sortWords = std::max(sortWords, tile_sort_scratch_words(entries, tiles));
+  carve(b.sortScratch, sortWords * 4);
   carve(b.scanScratch, coverage_scan_words(static_cast<uint32_t>(n)) * 4);
   carve(b.sortCounts, (radix_count_words(n, 32) + kEntryCountWords) * 4);
   carve(b.counters, kCounterWords * 4);
