@@ -142,3 +142,18 @@ def test_a_step_over_views_leaves_the_stored_gradients():
         t.step_views(cams, targets, RATES)
         for name, got in vars(t.gradients()).items():
             np.testing.assert_array_equal(_bits(got), _bits(before[name]))
+
+
+@pytest.mark.parametrize("sizes", [[(352, 360), (360, 368)], [(360, 368), (440, 440), (448, 448)]])
+def test_batches_on_either_side_of_the_launch_rule(sizes):
+    """Views of 1984 to 3136 8x8 blocks: four waves a block up to 2048 in a batch and up to 3072 alone; image and sums are those of the view alone."""
+    cloud, cams = F.random_cloud(600, 1, 11), [F.train_camera(w, h) for w, h in sizes]
+    targets = [F.smooth_target(c.width, c.height, 3) for c in cams]
+    options = vsplat.TrainerOptions(force_fixed_point=True, tile_shape=vsplat.TILES_8X8)
+    with vsplat.Trainer(cloud, options) as t, vsplat.Trainer(cloud, options) as one:
+        t.step_views(cams, targets)
+        for k, (cam, target) in enumerate(zip(cams, targets)):
+            one.compute_gradients(cam, target)
+            np.testing.assert_array_equal(_bits(t.inspect("image", view=k)), _bits(one.inspect("image")))
+            np.testing.assert_array_equal(t.inspect("raw", view=k), one.inspect("raw"))
+            assert np.count_nonzero(one.inspect("raw")) > 0

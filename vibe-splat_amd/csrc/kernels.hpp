@@ -217,12 +217,19 @@ inline uint32_t raster_blocks(uint32_t tiles, uint32_t tileW, uint32_t tileH) {
 // and 40.5, 1600 blocks (60k) 79.5 + 4.1 and 92.5, 4096 blocks (60k) 96.8 + 4.1
 // and 120.
 constexpr uint32_t kForwardUnordered = 7168, kBackwardUnordered = 1280;
-// Views of at most this many blocks have four waves work each block (raster.hip),
-// twelve waves a SIMD: past that one wave a block is as fast and does less work.
+// Views of at most this many blocks have four waves work each block (raster.hip): past
+// that one wave a block is as fast and does less work. (A CU holds five of the
+// four-wave workgroups at a time, 1280 blocks on the chip.)
 // Forward and ordered backward of 60k Gaussians with four waves and with one
 // (us): 1600 blocks 45.4, 79.5 and 67.2, 118; 2304 blocks 50.4, 91.8 and 58.5,
 // 102; 3136 blocks 57.2, 99.2 and 55.4, 101; 4096 blocks 63.8, 117 and 55.1, 97.
-constexpr uint32_t kWideBlocks = 3072;
+// The views of a batch fill the chip together, so there the extra work counts
+// sooner: the gradients of queued batches (us a batch): two views of 1936 blocks
+// 386 and 407, 2500 blocks 421 and 402; three of 1344 403 and 495, 2304 517 and 467;
+// four of 1936 750 and 794, 2304 1000 and 920; eight of 1344 1080 and 1390, 1936 1229
+// and 1251, 2304 1302 and 1238.
+constexpr uint32_t kWideBlocks = 3072, kWideBatchBlocks = 2048;
+inline bool wide_blocks(uint32_t blocks, bool batch) { return blocks <= (batch ? kWideBatchBlocks : kWideBlocks); }
 
 // One view of a batched raster launch (its buffers and sizes), and up to
 // kRasterViewsPerLaunch of them, passed by value as the kernel's argument.
@@ -253,12 +260,13 @@ void launch_forward_views(hipStream_t stream, const RasterViews &views, uint32_t
 void launch_backward_views(hipStream_t stream, bool fixedPoint, bool recompute, const RasterViews &views, uint32_t tileW, uint32_t tileH,
                            const float background[3]);
 
-// The raster kernels for one tile shape: 8x8, 16x16, 32x8 or 32x32 (tileW x tileH).
+// The raster kernels for one tile shape: 8x8, 16x16, 32x8 or 32x32 (tileW x tileH);
+// batch: beside those of other views (wide_blocks).
 // The lists are read as launch_bin_emit left them: entryKeys carry each
 // entry's tile (low tileBits bits) and blocks, entryValues its Gaussian.
 void launch_forward(hipStream_t stream, const Splat *splats, const uint32_t *entryKeys, const uint32_t *entryValues, uint32_t tileBits,
                     const uint2 *ranges, uint32_t width, uint32_t height, uint32_t tileW, uint32_t tileH, const float background[3],
-                    float4 *image, uint32_t *stops, uint32_t *work = nullptr, const uint32_t *order = nullptr);
+                    float4 *image, uint32_t *stops, uint32_t *work = nullptr, const uint32_t *order = nullptr, bool batch = false);
 // (stops may be null: not kept when the backward recomputes them. work, when
 // given, receives per launch index the entries the backward will walk for
 // that 8x8 block, raster_blocks(tiles) of them. order: the blocks' launch
@@ -274,7 +282,7 @@ void launch_backward(hipStream_t stream, bool fixedPoint, bool recompute, const 
                      const uint32_t *entryValues, uint32_t tileBits, const uint2 *ranges, uint32_t width, uint32_t height, uint32_t tileW,
                      uint32_t tileH, const float background[3], const float4 *image, const float4 *adjoint, const uint32_t *stops,
                      float fixedScale, int64_t *rawFixed, float *rawFloat, uint8_t *touched, const float *edge = nullptr,
-                     const uint32_t *order = nullptr);
+                     const uint32_t *order = nullptr, bool batch = false);
 // The backward's launch order, heaviest first on each XCD by the forward's work
 // (each block keeps its XCD): a permutation of the items = raster_blocks(tiles)
 // launch indices.

@@ -739,7 +739,7 @@ __global__ __launch_bounds__(kBlock) void backward_views_kernel(RasterViews view
 // channel each, the backward's emitting the sums of the splats they evaluated.
 // Every float is formed as in the one-wave kernels, so the results are the same
 // bits. It does more work in all (the chain four times over), so it is for views
-// of at most kWideBlocks blocks. Forward and backward against one wave a block:
+// of few blocks (wide_blocks). Forward and backward against one wave a block:
 // 10k Gaussians at 256x256 (1024 blocks) 18.5 and 40.5 us, before 32 and 59; a
 // batch's 1504-block view of 10k 47 and 87 us, before 86 and 150.
 constexpr uint32_t kWideWaves = 4, kWideThreads = kWideWaves * 64, kWideChunk = 32, kWideShare = kWideChunk / kWideWaves;
@@ -1166,9 +1166,9 @@ void launch_list_order(hipStream_t stream, const uint2 *ranges, uint32_t tiles, 
 
 void launch_forward(hipStream_t stream, const Splat *splats, const uint32_t *entryKeys, const uint32_t *entryValues, uint32_t tileBits,
                     const uint2 *ranges, uint32_t width, uint32_t height, uint32_t tileW, uint32_t tileH, const float background[3],
-                    float4 *image, uint32_t *stops, uint32_t *work, const uint32_t *order) {
+                    float4 *image, uint32_t *stops, uint32_t *work, const uint32_t *order, bool batch) {
   const uint32_t gridW = (width + tileW - 1) / tileW, gridH = (height + tileH - 1) / tileH;
-  if (raster_blocks(gridW * gridH, tileW, tileH) <= kWideBlocks) {
+  if (wide_blocks(raster_blocks(gridW * gridH, tileW, tileH), batch)) {
     hipLaunchKernelGGL(forward_wide_kernel, dim3(raster_blocks(gridW * gridH, tileW, tileH)), dim3(kWideThreads), 0, stream, splats, entryKeys,
                        entryValues, tileBits, ranges, width, height, tileW, tileH, gridW, background[0], background[1], background[2],
                        reinterpret_cast<float *>(image), stops, work, order);
@@ -1185,11 +1185,12 @@ void launch_forward(hipStream_t stream, const Splat *splats, const uint32_t *ent
 void launch_backward(hipStream_t stream, bool fixedPoint, bool recompute, const Splat *splats, const uint32_t *entryKeys,
                      const uint32_t *entryValues, uint32_t tileBits, const uint2 *ranges, uint32_t width, uint32_t height, uint32_t tileW,
                      uint32_t tileH, const float background[3], const float4 *image, const float4 *adjoint, const uint32_t *stops,
-                     float fixedScale, int64_t *rawFixed, float *rawFloat, uint8_t *touched, const float *edge, const uint32_t *order) {
+                     float fixedScale, int64_t *rawFixed, float *rawFloat, uint8_t *touched, const float *edge, const uint32_t *order,
+                     bool batch) {
   const uint32_t gridW = (width + tileW - 1) / tileW, gridH = (height + tileH - 1) / tileH;
   const bool score = edge != nullptr;
   const int variant = (fixedPoint ? 4 : 0) | (recompute ? 2 : 0) | (score ? 1 : 0);
-  if (raster_blocks(gridW * gridH, tileW, tileH) <= kWideBlocks) {
+  if (wide_blocks(raster_blocks(gridW * gridH, tileW, tileH), batch)) {
 #define VSPLAT_BACKWARD_WIDE(F, R, S)                                                                                               \
   hipLaunchKernelGGL((backward_wide_kernel<F, R, S>), dim3(raster_blocks(gridW * gridH, tileW, tileH)), dim3(kWideThreads), 0, stream, \
                      splats, entryKeys, entryValues, tileBits, ranges, width, height, tileW, tileH, gridW, background[0], background[1], \

@@ -784,7 +784,7 @@ std::vector<std::pair<std::string, double>> Trainer::timings() const {
 // tile lists, the forward pass, the loss and its adjoint, the backward pass,
 // and (chain) the chain rule.
 void Trainer::enqueue_passes(ViewBuffers &b, const ViewParams &view, const uint8_t *deviceTarget, uint32_t mode,
-                             const vsplat_learning_rates *rates, bool timed, bool chain) {
+                             const vsplat_learning_rates *rates, bool timed, bool chain, bool batch) {
   current_ = nullptr;
   if (timed) begin_timing(true);
   const ViewParams v = with_tiles(b, view);
@@ -798,7 +798,7 @@ void Trainer::enqueue_passes(ViewBuffers &b, const ViewParams &view, const uint8
   launch_forward(b.stream, b.splats.as<Splat>(), b.entryKeys.as<uint32_t>(), b.entryValues.as<uint32_t>(), b.tileBits, b.ranges.as<uint2>(),
                  v.width, v.height, b.tileW, b.tileH, options_.background, b.image.as<float4>(),
                  options_.recompute_transmittance != 0 ? nullptr : b.stops.as<uint32_t>(), backward ? b.blockWork.as<uint32_t>() : nullptr,
-                 listOrder);
+                 listOrder, batch);
   uint32_t *blockOrder = backward && blocks > kBackwardUnordered ? b.blockOrder.as<uint32_t>() : nullptr;
   if (blockOrder != nullptr) launch_work_order(b.stream, b.blockWork.as<uint32_t>(), blocks, blockOrder);
   mark("composite");
@@ -812,7 +812,7 @@ void Trainer::enqueue_passes(ViewBuffers &b, const ViewParams &view, const uint8
                   b.entryValues.as<uint32_t>(), b.tileBits, b.ranges.as<uint2>(), v.width, v.height, b.tileW, b.tileH, options_.background,
                   b.image.as<float4>(),
                   b.adjoint.as<float4>(), b.stops.as<uint32_t>(), fixed_scale(v), b.rawFixed.as<int64_t>(), b.rawFloat.as<float>(),
-                  b.touched.as<uint8_t>(), scoring ? b.edge.as<float>() : nullptr, blockOrder);
+                  b.touched.as<uint8_t>(), scoring ? b.edge.as<float>() : nullptr, blockOrder, batch);
   mark("backward");
   if (!chain) return;
   enqueue_chain(b, v, mode, rates, b.stream, b.counters.as<uint32_t>());
@@ -1411,7 +1411,7 @@ void Trainer::enqueue_view_passes(uint32_t n, const vsplat_camera *cameras, cons
     ViewBuffers &b = *views_[k];
     if (b.stream != stream_) check(hipStreamWaitEvent(b.stream, batchStart_, 0), "hipStreamWaitEvent");
     params[k] = view_params(cameras[k]);
-    enqueue_passes(b, params[k], targets[k], kModeGradients, nullptr, false, false);
+    enqueue_passes(b, params[k], targets[k], kModeGradients, nullptr, false, false, n > 1);
     check(hipEventRecord(b.done, b.stream), "hipEventRecord");
     queuedViewSizes_.emplace_back(cameras[k].width, cameras[k].height);
   }
@@ -1449,8 +1449,10 @@ void Trainer::enqueue_batch_passes(uint32_t n, const vsplat_camera *cameras, con
 // 8x8 pixel blocks (one per tile shape among the views, eight views a launch):
 // each view's lists on its own stream; once every view's lists are made, the
 // forward launch on the trainer's stream; each view's loss on its own stream;
-// then the backward launch. Each (view, block) pair runs the single-view
-// kernels' code, so the images, sums and gradients are the same bits.
+// then the backward launch. A block is worked by one wave, whatever the views'
+// sizes, by the single-view kernels' code for views of many blocks; the code for
+// views of few forms every float in the same way, so the images, sums and
+// gradients are the same bits.
 void Trainer::enqueue_view_passes_one_launch(uint32_t n, const vsplat_camera *cameras, const uint8_t *const *targets, ViewParams *params) {
   queuedViewSizes_.clear();
   current_ = nullptr; // no stage events in a batch

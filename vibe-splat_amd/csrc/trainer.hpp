@@ -239,9 +239,9 @@ private:
   void settle_upload();
   hipStream_t upload_stream();
   void release_upload_stream();
-  // The passes up to the backward pass on b's stream, then (chain) the chain rule.
+  // The passes up to the backward pass on b's stream (batch: beside other views'), then (chain) the chain rule.
   void enqueue_passes(ViewBuffers &b, const ViewParams &view, const uint8_t *deviceTarget, uint32_t mode,
-                      const vsplat_learning_rates *rates, bool timed, bool chain = true);
+                      const vsplat_learning_rates *rates, bool timed, bool chain = true, bool batch = false);
   ViewParams with_tiles(const ViewBuffers &b, const ViewParams &view) const;
   void enqueue_lists(ViewBuffers &b, const ViewParams &view, uint32_t mode, bool marks);
   void enqueue_loss(ViewBuffers &b, const ViewParams &view, const uint8_t *deviceTarget);
