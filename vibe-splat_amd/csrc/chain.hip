@@ -677,13 +677,15 @@ __device__ __forceinline__ uint32_t sh_word_put(uint32_t format, uint32_t word, 
 // Unless a mode acts on every Gaussian (Adam without `selective`, penalties) only
 // the flagged ones are listed, and the raw sums, the parameters and the moments of
 // the others are not read. Most of a large scene is hidden in a view. Three
-// kernels over all 1M Gaussians of a 1280x736 view, 4 % of them seen, took 34 (SH
+// kernels over all 1M Gaussians of a 1280x720 view, 3.3 % of them seen, took 34 (SH
 // terms), 59 (geometry) and 76 us (SH step: 26M words asked whether they step);
 // this takes 43, of 3M (1080p, 2 %) 59 for 444, of 400k 31 for 90. Where all are
 // seen it takes as long as the three did: 93 us for 93 (200k), 453 for 481 (1M),
 // 28 for 29 (30k). Then it is bound by the step's own instructions (some 200 a
 // parameter, divisions, a square root and two hashes), where few are seen by the
-// way to memory of one after the other: flags, sums, parameters, moments.
+// way to memory of one after the other: flags, sums, parameters, moments. At four
+// waves a SIMD (128 registers) spilled scalars take 24 bytes of scratch a lane, at
+// degree 3 with halves nine vector registers 32 more.
 constexpr uint32_t kStepSlots = kChainThreads / 2, kStepMost = 4096, kViewsMost = 1024, kStepLeast = 64, kFlagged = 0x8000u;
 // What the step takes of a Gaussian. The rows' lengths are odd, so that
 // neighbouring rows lie on different banks.
@@ -956,7 +958,8 @@ __global__ __launch_bounds__(kChainThreads, 4) void chain_step_kernel(ChainBuffe
 // With the SH sums through memory to a kernel of their own the step's share at two
 // waves a SIMD (what this kernel's LDS and registers leave) is the geometric one:
 // a step of the same 500k all seen 196 + 119 us, 359 with the SH words stepped
-// here; 20 % seen 99 + 37 for 142, of 1M and eight views 32 % seen 364 + 82 for 452. (All
+// here; 20 % seen 99 + 37 for 142; of 1M and eight views 32 % seen 364 + 82 for 452, and
+// of the ring of eight uneven views, where few are, 192 + 46 for 232. (All
 // Gaussians in both kernels: 181 + 126, 197 + 89, 661 + 163. Gradients of 500k all
 // seen 167, then 157: there the loop over the views was unrolled, eight copies of
 // the terms, 90 KB of instructions and too many registers for the packed form.)

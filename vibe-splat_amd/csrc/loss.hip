@@ -367,8 +367,8 @@ __global__ __launch_bounds__(256) void error_mask_kernel(float4 *__restrict__ ad
 // The other blocks clear the raw sums that the last backward pass added to (the
 // others are zero): a wave takes 64 Gaussians at a time, reads their flags, and
 // covers their rows, kRawPerSplat / 2 units of two sums each, with its lanes on
-// neighbouring units. Most Gaussians of a large scene are hidden: of 1M, some 4 %
-// are flagged, and clearing them takes 5 us where all rows (112 MB) took 17.
+// neighbouring units. Most Gaussians of a large scene are hidden: of 1M, 3.3 %
+// have sums, and the launch takes 7.6 us where clearing all rows (112 MB) took 17.
 template <class Unit>
 __global__ __launch_bounds__(256) void total_and_clear_kernel(const float2 *__restrict__ tileTotals, uint32_t tiles,
                                                               double *__restrict__ sums, Unit *__restrict__ raw,

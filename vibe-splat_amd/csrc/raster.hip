@@ -575,9 +575,9 @@ template <bool Fixed, bool Score> struct Emitter {
 
 // Back to front over the tile's list (train_backward.glsl:78-158), for the
 // block's pixels, from the block's lowest stop. Bound by the vector unit: a
-// splat's evaluation, gradient terms, reduction and emission are about 105
-// instructions, the permlane swaps and the reciprocal among them at a third of
-// an fma's rate. At 1M Gaussians and 1280x720 (32x32 lists, fixed point) 205 us
+// splat's evaluation is 29 instructions, its gradient terms, reduction and emission
+// where a pixel takes it 91 more, the permlane swaps and the reciprocal among them at
+// a third of an fma's rate. At 1M Gaussians and 1280x720 (32x32 lists, fixed point) 205 us
 // before the walk's loads ran ahead, the evaluations were grouped, the reduction
 // merged by bank masks and the emission shortened (a row's byte offset staged
 // once, the halves of sums 3 to 5 taken last); 179 us with them. With Recompute the pixel's log
