@@ -157,3 +157,16 @@ def test_batches_on_either_side_of_the_launch_rule(sizes):
             np.testing.assert_array_equal(_bits(t.inspect("image", view=k)), _bits(one.inspect("image")))
             np.testing.assert_array_equal(t.inspect("raw", view=k), one.inspect("raw"))
             assert np.count_nonzero(one.inspect("raw")) > 0
+
+
+@pytest.mark.parametrize("views", [2, 8, 9])
+def test_memory_of_a_trainer_that_steps_batches(views):
+    """A step holds the SH sums, or for more views than the chain rule takes at once the gradients, and not both."""
+    cloud, cams = F.synthetic_cloud(30_000, 3, 3), _cameras([(48, 40)] * views)
+    targets = [F.smooth_target(48, 40, 3)] * views
+    held = []
+    for rates in (None, RATES):
+        with vsplat.Trainer(cloud) as t:
+            t.step_views(cams, targets, rates)
+            held.append(t.gpu_bytes())
+    assert held[0] - held[1] == (30_000 * 4 * 11 if views <= 8 else 0)

@@ -564,7 +564,7 @@ std::pair<uint32_t, uint32_t> Trainer::autotune_tiles(const vsplat_camera &camer
 // state changes but the chosen shapes and the buffers sized for them.
 void Trainer::autotune_views(uint32_t n, const vsplat_camera *cameras, const uint8_t *const *targets, uint32_t repeats,
                              uint32_t *tileW, uint32_t *tileH) {
-  prepare_views(n, cameras, targets, kModeGradients, nullptr);
+  prepare_views(n, cameras, targets, kModeGradients, nullptr, false);
   std::vector<std::pair<int, int>> sizes;
   for (uint32_t k = 0; k < n; ++k) {
     const std::pair<int, int> size{cameras[k].width, cameras[k].height};
@@ -1379,18 +1379,19 @@ void Trainer::check_views(uint32_t n, const vsplat_camera *cameras, const uint8_
 }
 
 // Checks a batch's arguments and makes every buffer it needs (so that queueing
-// it allocates nothing).
+// it allocates nothing), with chain the chain rule's too.
 void Trainer::prepare_views(uint32_t n, const vsplat_camera *cameras, const uint8_t *const *targets, uint32_t mode,
-                            const vsplat_learning_rates *rates) {
+                            const vsplat_learning_rates *rates, bool chain) {
   check_views(n, cameras, targets, mode, rates);
+  const bool chunks = n > kChainViewsPerLaunch;
   for (uint32_t k = 0; k < n; ++k) {
     if (targets[k] == nullptr) throw Error(VSPLAT_INVALID_ARGUMENT, "no target for a view");
     ensure_size(view_buffers(k), cameras[k].width, cameras[k].height);
   }
-  // Gradients are stored, or carried from one chunk of a long batch to the next; a
-  // step's SH sums have a place of their own, so that stored gradients stay.
-  if (mode == kModeGradients || n > kChainViewsPerLaunch) ensure_gradients();
-  if (mode == kModeStep) shSums_.ensure(static_cast<size_t>(count_) * shFloats_ * 4);
+  // Gradients are stored, or carried from one chunk of a long batch to the next; the
+  // SH sums of any other step have a place of their own, so that stored gradients stay.
+  if (chain && (mode == kModeGradients || chunks)) ensure_gradients();
+  if (chain && mode == kModeStep && !chunks) shSums_.ensure(static_cast<size_t>(count_) * shFloats_ * 4);
   if (viewStats_.bytes() < static_cast<size_t>(n) * kViewStatsBytes) {
     check(hipStreamSynchronize(stream_), "view stats"); // a queued batch may still write the old one
     viewStats_.ensure(static_cast<size_t>(n) * kViewStatsBytes);
@@ -1536,7 +1537,8 @@ void Trainer::launch_batch_raster(uint32_t n, const ViewParams *params, bool bac
 // behind a later view's passes queued before it.)
 void Trainer::enqueue_view_chains(uint32_t n, const ViewParams *params, uint32_t mode, const vsplat_learning_rates *rates) {
   uint32_t *status = views_[0]->counters.as<uint32_t>();
-  const ChainBuffers buffers = chain_buffers(*views_[0]);
+  ChainBuffers buffers = chain_buffers(*views_[0]);
+  if (n > kChainViewsPerLaunch) buffers.shSums = buffers.gradSh; // the chunks' sums are there
   for (uint32_t first = 0; first < n; first += kChainViewsPerLaunch) {
     const uint32_t count = std::min(n - first, kChainViewsPerLaunch);
     const bool last = first + count == n;

@@ -258,7 +258,7 @@ private:
   void check_views(uint32_t n, const vsplat_camera *cameras, const uint8_t *const *targets, uint32_t mode,
                      const vsplat_learning_rates *rates) const;
   void prepare_views(uint32_t n, const vsplat_camera *cameras, const uint8_t *const *targets, uint32_t mode,
-                     const vsplat_learning_rates *rates);
+                     const vsplat_learning_rates *rates, bool chain = true);
   uint64_t capture_key(uint32_t n) const;
   void clear_overflow();
   vsplat_step_stats make_stats(const uint32_t *counters, const double *sums, int width, int height) const;
