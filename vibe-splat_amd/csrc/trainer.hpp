@@ -105,6 +105,12 @@ private:
   static constexpr size_t kChunk = 1u << 20, kSlots = 12;
   // Helper threads for a transfer of kHelped bytes and more; below, starting them costs what they save.
   static constexpr size_t kHelpers = 3, kHelped = 3u << 20;
+  // Past this hipMemcpy is the faster one: slots and destination no longer share the
+  // host's cache, and it reads straight into the caller's pages. Into new and into
+  // used memory, by slots and by it (us): 59 MB 4900, 2600 and 6000, 3470; 92 MB 8200,
+  // 4400 and 9050, 5310; 133 MB 12500-13500, 7700-9000 and 12650, 7700; 280 MB 30300,
+  // 19600 and 26800, 16100.
+  static constexpr size_t kSlotted = 96u << 20;
   PinnedArray slots_;
   hipEvent_t landed_[kSlots] = {};
 };
