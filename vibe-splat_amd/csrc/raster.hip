@@ -116,7 +116,12 @@ __device__ __forceinline__ bool reaches_block(const Splat &s, float x0, float y0
   const float fx = __builtin_fmaxf(-lowx, highx), fy = __builtin_fmaxf(-lowy, highy); // the farthest pixel centres
   const float terms = fma32(s.qz * fy, fy, s.qx * fx * fx);
   const float reach = 1.3862944f * __builtin_amdgcn_logf(255.0f * s.o); // 2 ln(255 o), v_log_f32 being log2
-  return __builtin_fminf(vertical, horizontal) <= fma32(1e-6f, terms, fma32(reach, 1.001f, 1e-3f));
+  // A splat whose determinant overflows has a conic of zeros (or next to nothing, its
+  // reciprocals infinite), with which the lists' test finds no edge that it reaches:
+  // it is its centre's block's alone, in every tile shape.
+  const bool conic = __builtin_fmaxf(s.qx, s.qz) > 0x1p-128f || s.qy != 0.0f;
+  return __builtin_fminf(vertical, horizontal) <= fma32(1e-6f, terms, fma32(reach, 1.001f, 1e-3f)) &&
+         (conic || (xn == 0.0f && yn == 0.0f));
 }
 
 // The bits lo .. hi - 1 (0 <= lo < hi <= 8) of pixels first + lo, ... (centres)
